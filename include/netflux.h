@@ -311,9 +311,8 @@ int nf_mlp_predict(nf_mlp *m, const float *x, int64_t n, float *y);
  * memory (code under HIP graph capture, serving loops): nf_mlp_predict on
  * DEVICE arrays x [n][6] -> y [n][5], at most 16384 samples per call (more:
  * NF_E_ARG), enqueued on `stream` (a hipStream_t; null: the network's own
- * stream) without synchronising and without allocating.  The activations
- * live in a fixed device array of about 17 MB per GPU, shared by every call
- * on that GPU: calls that overlap on one GPU race.  The device that was
+ * stream) without synchronising and without allocating.  One kernel, whose
+ * activations stay on the CU: calls share no buffer.  The device that was
  * current at nf_mlp_create must be current.  Same results as nf_mlp_predict,
  * bit for bit. */
 int nf_mlp_predict_noalloc(nf_mlp *m, const float *x, int64_t n, float *y, void *stream);

@@ -17,7 +17,6 @@
 #include <cstdio>
 #include <cstring>
 #include <memory>
-#include <mutex>
 #include <random>
 #include <string>
 #include <type_traits>
@@ -33,6 +32,7 @@ using nf::mlp::OUT;
 namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // flattened parameter layout: W1 [HID][IN], b1, W2 [HID][HID], b2, W3, b3,
@@ -180,8 +180,8 @@ __global__ void k_bias_gelu(float *Z, const float *b, __bf16 *A, int rows, int n
     A[i] = (__bf16)gelu(z);
 }
 
-// Y += b; for training: D = Y - T, dY = 2 D / (OUT n) (FP32 and BF16), and
-// per-block sums of D^2 for the loss
+// Y += b, D = Y - T, dY = 2 D / (OUT n) (FP32 and BF16), and per-block sums
+// of D^2 for the loss
 __global__ void k_out_loss(float *Y, const float *b, const float *T, float *dY, __bf16 *dYb, float *loss_part,
                            int n, float inv_count) {
     __shared__ float sh[4];
@@ -192,16 +192,13 @@ __global__ void k_out_loss(float *Y, const float *b, const float *T, float *dY, 
             const size_t i = (size_t)o * n + j;
             const float y = Y[i] + b[o];
             Y[i] = y;
-            if (T) {
-                const float d = y - T[i];
-                s += d * d;
-                const float g = 2.0f * d * inv_count;
-                dY[i] = g;
-                dYb[i] = (__bf16)g;
-            }
+            const float d = y - T[i];
+            s += d * d;
+            const float g = 2.0f * d * inv_count;
+            dY[i] = g;
+            dYb[i] = (__bf16)g;
         }
     }
-    if (!T) return;
     for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
     if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
     __syncthreads();
@@ -239,8 +236,8 @@ __global__ void k_sum_splits(const float *part, int splits, int64_t stride, int6
     out[i] = s;
 }
 
-// raw feature-major inputs -> normalised BF16 operand; idx (optional) picks
-// the samples of a minibatch; targets normalised alongside
+// raw feature-major inputs -> normalised BF16 operand, and targets alongside;
+// idx (optional) picks the samples of a minibatch
 __global__ void k_gather(const float *x, const float *y, int64_t n_all, const int64_t *idx, int64_t first, int n,
                          const float *in_shift, const float *in_scale, const float *out_shift,
                          const float *out_iscale, __bf16 *X0, float *T) {
@@ -248,28 +245,147 @@ __global__ void k_gather(const float *x, const float *y, int64_t n_all, const in
     if (j >= n) return;
     const int64_t s = idx ? idx[first + j] : first + j;
     for (int f = 0; f < IN; ++f) X0[(size_t)f * n + j] = (__bf16)((x[f * n_all + s] - in_shift[f]) * in_scale[f]);
-    if (T)
-        for (int o = 0; o < OUT; ++o) T[(size_t)o * n + j] = (y[o * n_all + s] - out_shift[o]) * out_iscale[o];
+    for (int o = 0; o < OUT; ++o) T[(size_t)o * n + j] = (y[o * n_all + s] - out_shift[o]) * out_iscale[o];
 }
 
-// y_raw[o][first + j] = Y[o][j] * out_scale + out_shift
-__global__ void k_denorm(const float *Y, int n, const float *out_shift, const float *out_scale, float *y,
-                         int64_t n_all, int64_t first) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= n) return;
-    for (int o = 0; o < OUT; ++o) y[o * n_all + first + j] = Y[(size_t)o * n + j] * out_scale[o] + out_shift[o];
+// ---------------------------------------------------------------------------
+// Fused network: one block of four waves takes NC x 16 samples through every
+// layer, so activations never leave the CU.  Wave w computes features
+// [32w, 32w + 32) of each hidden layer (two MFMA row tiles), keeps those rows
+// of all weights in registers as MFMA operands for as long as it lives (the
+// grid is persistent), and hands its activations to the other waves through
+// LDS as [sample][feature] BF16, so that a lane's operand fragment of the
+// next layer -- 8 consecutive features of one sample -- is one 16-byte read.
+// Every product is accumulated over k in the same steps of 32 as k_gemm's, so
+// outputs have the layer-by-layer kernels' bits.
+constexpr int LDH = HID + 8;  // row stride of the LDS activations: 16-byte aligned, 16 columns over all banks
+
+// MFMA operand fragment of row r (R real rows), columns [k, k + 8) of a
+// row-major [R][HID] BF16 matrix
+__device__ __forceinline__ bf16x8 row_frag(const __bf16 *W, int r, int k, int R) {
+    if (r < R) return *reinterpret_cast<const bf16x8 *>(W + r * HID + k);
+    bf16x8 z;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) z[e] = (__bf16)0.0f;
+    return z;
 }
-// the same normalisation from / de-normalisation to sample-major [n][w]
-// arrays (the layout of nf_mlp_predict's host arrays)
-__global__ void k_gather_aos(const float *x, int n, const float *in_shift, const float *in_scale, __bf16 *X0) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= n) return;
-    for (int f = 0; f < IN; ++f) X0[(size_t)f * n + j] = (__bf16)((x[(size_t)j * IN + f] - in_shift[f]) * in_scale[f]);
+// the same of the [HID][IN] input layer: columns IN.. are zero
+__device__ __forceinline__ bf16x8 in_frag(const __bf16 *W, int r, int k) {
+    bf16x8 v;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = k + e < IN ? W[r * IN + k + e] : (__bf16)0.0f;
+    return v;
 }
-__global__ void k_denorm_aos(const float *Y, int n, const float *out_shift, const float *out_scale, float *y) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= n) return;
-    for (int o = 0; o < OUT; ++o) y[(size_t)j * OUT + o] = Y[(size_t)o * n + j] * out_scale[o] + out_shift[o];
+
+struct Infer {
+    const __bf16 *pb;   // BF16 parameters
+    const float *p;     // FP32 parameters (biases)
+    const float *norm;  // in_shift[6], in_scale[6], out_shift[5], out_scale[5]
+    const float *x;     // x(f, j) = x[f * xf + j * xj]
+    int64_t xf, xj;
+    float *y;           // y(o, j) = y[o * yo + j * yj]
+    int64_t yo, yj;
+    int64_t n;
+};
+
+// Bound by the erf of the three GELUs (384 per sample, about 45 VALU
+// instructions each), not by the products or by memory.  Layer by layer (11
+// launches, 3.6 KB per sample through HBM) 700 samples took 38 us and
+// 1,463,340 samples 2.4 ms; one launch that moves 44 bytes per sample takes
+// 6.5 us and 0.44 ms.
+template <int NC>
+__global__ __launch_bounds__(256) void k_infer(Infer g) {
+    __shared__ __attribute__((aligned(16))) __bf16 H[2][NC * 16][LDH];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, col = lane & 15, q4 = lane >> 4;
+    const int64_t ntiles = (g.n + NC * 16 - 1) / (NC * 16);
+    bf16x8 a1[2], a2[2][4], a3[2][4], a4[4];
+    f32x4 b1[2], b2[2], b3[2];
+    float b4[4], osh[4], osc[4];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int r = 32 * w + 16 * i;
+        a1[i] = in_frag(g.pb + OFF_W1, r + col, 8 * q4);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            a2[i][q] = row_frag(g.pb + OFF_W2, r + col, 32 * q + 8 * q4, HID);
+            a3[i][q] = row_frag(g.pb + OFF_W3, r + col, 32 * q + 8 * q4, HID);
+        }
+        b1[i] = *reinterpret_cast<const f32x4 *>(g.p + OFF_B1 + r + 4 * q4);
+        b2[i] = *reinterpret_cast<const f32x4 *>(g.p + OFF_B2 + r + 4 * q4);
+        b3[i] = *reinterpret_cast<const f32x4 *>(g.p + OFF_B3 + r + 4 * q4);
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) a4[q] = row_frag(g.pb + OFF_W4, col, 32 * q + 8 * q4, OUT);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int o = 4 * q4 + r;
+        b4[r] = o < OUT ? g.p[OFF_B4 + o] : 0.f;
+        osh[r] = o < OUT ? g.norm[12 + o] : 0.f;
+        osc[r] = o < OUT ? g.norm[17 + o] : 0.f;
+    }
+    // activations of one product, [2 row tiles][NC sample tiles], to LDS
+    auto store = [&](const f32x4 (*acc)[NC], const f32x4 *b, __bf16 (*S)[LDH]) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                bf16x4 h;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) h[r] = (__bf16)gelu(acc[i][c][r] + b[i][r]);
+                *reinterpret_cast<bf16x4 *>(&S[c * 16 + col][32 * w + 16 * i + 4 * q4]) = h;
+            }
+    };
+    auto layer = [&](const bf16x8 (*a)[4], const f32x4 *b, const __bf16 (*S)[LDH], __bf16 (*D)[LDH]) {
+        f32x4 acc[2][NC];
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            acc[0][c] = acc[1][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const bf16x8 h = *reinterpret_cast<const bf16x8 *>(&S[c * 16 + col][32 * q + 8 * q4]);
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+                    acc[i][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i][q], h, acc[i][c], 0, 0, 0);
+            }
+        }
+        store(acc, b, D);
+    };
+    int p = 0;  // the buffer the input layer writes; it was last read two barriers ago
+    for (int64_t t = blockIdx.x; t < ntiles; t += gridDim.x, p ^= 1) {
+        const int64_t j0 = t * (NC * 16);
+        f32x4 acc[2][NC];
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            // padding samples repeat the last one and are not stored
+            const int64_t j = j0 + c * 16 + col < g.n ? j0 + c * 16 + col : g.n - 1;
+            bf16x8 v;
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                v[e] = q4 == 0 && e < IN ? (__bf16)((g.x[(e < IN ? e : 0) * g.xf + j * g.xj] - g.norm[e < IN ? e : 0]) *
+                                                    g.norm[6 + (e < IN ? e : 0)])
+                                         : (__bf16)0.0f;
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+                acc[i][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1[i], v, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+        }
+        store(acc, b1, H[p]);
+        __syncthreads();
+        layer(a2, b2, H[p], H[p ^ 1]);
+        __syncthreads();
+        layer(a3, b3, H[p ^ 1], H[p]);
+        __syncthreads();
+        for (int c = w; c < NC; c += 4) {
+            f32x4 y = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                y = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                    a4[q], *reinterpret_cast<const bf16x8 *>(&H[p][c * 16 + col][32 * q + 8 * q4]), y, 0, 0, 0);
+            const int64_t j = j0 + c * 16 + col;
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (4 * q4 + r < OUT && j < g.n) g.y[(4 * q4 + r) * g.yo + j * g.yj] = (y[r] + b4[r]) * osc[r] + osh[r];
+        }
+    }
 }
 
 // Adam step on the FP32 masters (bias-corrected step size lr_t), BF16 copy
@@ -320,6 +436,7 @@ struct nf_mlp {
 
 namespace {
 
+constexpr int64_t NC1_MAX = 12288;  // samples up to which inference takes 16 per block (infer)
 constexpr int KSPLIT = 512;  // batch samples per split of the weight-gradient sums
 
 int fail(nf_mlp *m, int code, const std::string &msg) {
@@ -378,36 +495,38 @@ const float *d_out_shift(const nf_mlp *m) { return m->norm + 12; }
 const float *d_out_scale(const nf_mlp *m) { return m->norm + 17; }
 const float *d_out_iscale(const nf_mlp *m) { return m->norm + 22; }
 
-// activation buffers of one forward pass, feature-major [rows][n]
-struct FwdBufs {
-    const __bf16 *X0;
-    float *Z[3];
-    __bf16 *A[3];
-    float *Y;
-};
-
-// forward of the n samples in X0 (normalised); Y = normalised outputs
-hipError_t forward_on(const nf_mlp *m, const FwdBufs &b, int n, hipStream_t s) {
+// forward of the n samples in X0 (normalised) for training, which keeps every
+// layer's pre-activations and activations; Y = normalised outputs, bias not
+// yet added
+hipError_t forward(nf_mlp *m, int n, hipStream_t s) {
     hipError_t e;
-    const __bf16 *in = b.X0;
+    const __bf16 *in = m->X0;
     int k = IN;
     const int64_t offW[3] = {OFF_W1, OFF_W2, OFF_W3}, offB[3] = {OFF_B1, OFF_B2, OFF_B3};
     for (int l = 0; l < 3; ++l) {
-        if ((e = gemm(s, m->pb + offW[l], k, 1, in, n, 1, b.Z[l], n, 1, HID, n, k))) return e;
-        hipLaunchKernelGGL(k_bias_gelu, dim3((n + 255) / 256, HID), dim3(256), 0, s, b.Z[l],
-                           (const float *)(m->p + offB[l]), b.A[l], HID, n);
+        if ((e = gemm(s, m->pb + offW[l], k, 1, in, n, 1, m->Z[l], n, 1, HID, n, k))) return e;
+        hipLaunchKernelGGL(k_bias_gelu, dim3((n + 255) / 256, HID), dim3(256), 0, s, m->Z[l],
+                           (const float *)(m->p + offB[l]), m->A[l], HID, n);
         if ((e = hipGetLastError())) return e;
-        in = b.A[l];
+        in = m->A[l];
         k = HID;
     }
-    return gemm(s, m->pb + OFF_W4, HID, 1, in, n, 1, b.Y, n, 1, OUT, n, HID);
+    return gemm(s, m->pb + OFF_W4, HID, 1, in, n, 1, m->Y, n, 1, OUT, n, HID);
 }
 
-// forward over the network's own workspace (training keeps every layer's
-// pre-activations and activations for the backward pass)
-hipError_t forward(nf_mlp *m, int n, hipStream_t s) {
-    const FwdBufs b{m->X0, {m->Z[0], m->Z[1], m->Z[2]}, {m->A[0], m->A[1], m->A[2]}, m->Y};
-    return forward_on(m, b, n, s);
+// inference of n samples on the device: x(f, j) = x[f * xf + j * xj],
+// y(o, j) = y[o * yo + j * yj]; one launch, no workspace
+hipError_t infer(const nf_mlp *m, const float *x, int64_t xf, int64_t xj, float *y, int64_t yo, int64_t yj, int64_t n,
+                 hipStream_t s) {
+    if (n < 1) return hipSuccess;
+    const Infer g{m->pb, m->p, m->norm, x, xf, xj, y, yo, yj, n};
+    // 64 samples per block share one read of the weights and activations
+    // (one block's latency 12.4 us up to 2 blocks per CU), 16 per block are
+    // done in 6.2 us while at most about 3 of them share a CU: 9.1 against
+    // 12.5 us at 8,192 samples, 16.5 against 12.5 us at 16,384
+    if (n > NC1_MAX) hipLaunchKernelGGL(k_infer<4>, dim3((unsigned)std::min<int64_t>((n + 63) / 64, 512)), dim3(256), 0, s, g);
+    else hipLaunchKernelGGL(k_infer<1>, dim3((unsigned)((n + 15) / 16)), dim3(256), 0, s, g);
+    return hipGetLastError();
 }
 
 // loss and gradient (into m->g) of the n samples in X0 / T
@@ -499,74 +618,16 @@ namespace nf {
 namespace mlp {
 
 hipError_t predict_device(nf_mlp *m, const float *x, int64_t n, float *y, hipStream_t s) {
-    constexpr int CH = 1 << 18;
-    if (ensure_ws(m, (int)std::min<int64_t>(n, CH))) return hipErrorOutOfMemory;
-    hipError_t e;
-    for (int64_t first = 0; first < n; first += CH) {
-        const int c = (int)std::min<int64_t>(CH, n - first);
-        hipLaunchKernelGGL(k_gather, dim3((c + 255) / 256), dim3(256), 0, s, x, (const float *)nullptr, n,
-                           (const int64_t *)nullptr, first, c, d_in_shift(m), d_in_scale(m), d_out_shift(m),
-                           d_out_iscale(m), m->X0, (float *)nullptr);
-        if ((e = hipGetLastError())) return e;
-        if ((e = forward(m, c, s))) return e;
-        hipLaunchKernelGGL(k_out_loss, dim3((c + 255) / 256), dim3(256), 0, s, m->Y, (const float *)(m->p + OFF_B4),
-                           (const float *)nullptr, (float *)nullptr, (__bf16 *)nullptr, (float *)nullptr, c, 0.f);
-        if ((e = hipGetLastError())) return e;
-        hipLaunchKernelGGL(k_denorm, dim3((c + 255) / 256), dim3(256), 0, s, (const float *)m->Y, c, d_out_shift(m),
-                           d_out_scale(m), y, n, first);
-        if ((e = hipGetLastError())) return e;
-    }
-    return hipSuccess;
+    return infer(m, x, n, 1, y, n, 1, n, s);
 }
 
 }  // namespace mlp
 }  // namespace nf
 
 // ============================================================================
-// ---------------------------------------------------------------------------
-// Inference that allocates nothing, for callers that may not call hipMalloc
-// (code under HIP graph capture, serving loops).  The activations of one call
-// -- normalised inputs X0 (BF16 [6][n]), one layer's pre-activations Z (FP32
-// [128][n]), two BF16 activation buffers [128][n] used in turn, and the
-// outputs Y (FP32 [5][n]) -- live in `scratch`, a file-scope device array
-// sized for NOALLOC_MAX samples (about 17 MB).  Each GPU the library runs on
-// holds its own copy until the process ends.  Host code never uses the
-// array's name as an address: nf_mlp_create looks up the copy of the current
-// device once (hipGetSymbolAddress) and the kernels take that address.  Every
-// buffer is written in full before it is read, so nothing needs clearing
-// between calls; calls that overlap on one GPU (two streams or threads)
-// share the array and race.
 namespace {
-
-constexpr int64_t NOALLOC_MAX = 16384;  // samples per call
-constexpr size_t al256(size_t b) { return (b + 255) / 256 * 256; }
-constexpr size_t NA_X0 = 0;
-constexpr size_t NA_Z = al256(NA_X0 + sizeof(__bf16) * IN * NOALLOC_MAX);
-constexpr size_t NA_A0 = al256(NA_Z + sizeof(float) * HID * NOALLOC_MAX);
-constexpr size_t NA_A1 = al256(NA_A0 + sizeof(__bf16) * HID * NOALLOC_MAX);
-constexpr size_t NA_Y = al256(NA_A1 + sizeof(__bf16) * HID * NOALLOC_MAX);
-constexpr size_t NA_BYTES = al256(NA_Y + sizeof(float) * OUT * NOALLOC_MAX);
-
-__device__ __align__(256) unsigned char scratch[NA_BYTES];
-
-constexpr int MAX_DEVICES = 64;
-std::mutex scratch_mu;
-unsigned char *scratch_ptr[MAX_DEVICES] = {};  // per device: its copy of `scratch`
-
-// once per device, with that device current (called by nf_mlp_create)
-int scratch_setup(nf_mlp *mm, int dev) {
-    if (dev < 0 || dev >= MAX_DEVICES) return fail(mm, NF_E_ARG, "device index out of range");
-    std::lock_guard<std::mutex> lk(scratch_mu);
-    if (scratch_ptr[dev]) return NF_OK;
-    void *p = nullptr;
-    const hipError_t e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
-    if (e != hipSuccess || !p)
-        return fail(mm, NF_E_HIP, std::string("hipGetSymbolAddress(scratch): ") + hipGetErrorString(e));
-    scratch_ptr[dev] = static_cast<unsigned char *>(p);
-    return NF_OK;
+constexpr int64_t NOALLOC_MAX = 16384;  // samples per nf_mlp_predict_noalloc call
 }
-
-}  // namespace
 
 extern "C" {
 
@@ -583,29 +644,7 @@ int nf_mlp_predict_noalloc(nf_mlp *mm, const float *x, int64_t n, float *y, void
     HIPM(hipGetDevice(&dev));
     if (dev != mm->device)
         return fail(mm, NF_E_ARG, "nf_mlp_predict_noalloc: the network's device must be current");
-    unsigned char *base;
-    {
-        std::lock_guard<std::mutex> lk(scratch_mu);
-        base = scratch_ptr[dev];
-    }
-    if (!base) return fail(mm, NF_E_HIP, "nf_mlp_predict_noalloc: scratch not set up on this device");
-    const int c = (int)n;
-    __bf16 *X0 = reinterpret_cast<__bf16 *>(base + NA_X0);
-    float *Z = reinterpret_cast<float *>(base + NA_Z);
-    __bf16 *A0 = reinterpret_cast<__bf16 *>(base + NA_A0), *A1 = reinterpret_cast<__bf16 *>(base + NA_A1);
-    float *Y = reinterpret_cast<float *>(base + NA_Y);
-    hipStream_t s = stream ? static_cast<hipStream_t>(stream) : mm->stream;
-    const dim3 g((c + 255) / 256), b(256);
-    hipLaunchKernelGGL(k_gather_aos, g, b, 0, s, x, c, d_in_shift(mm), d_in_scale(mm), X0);
-    HIPM(hipGetLastError());
-    // layer l reads A[l-1] and writes A[l]: A0, A1, A0
-    const FwdBufs fb{X0, {Z, Z, Z}, {A0, A1, A0}, Y};
-    HIPM(forward_on(mm, fb, c, s));
-    hipLaunchKernelGGL(k_out_loss, g, b, 0, s, Y, (const float *)(mm->p + OFF_B4), (const float *)nullptr,
-                       (float *)nullptr, (__bf16 *)nullptr, (float *)nullptr, c, 0.f);
-    HIPM(hipGetLastError());
-    hipLaunchKernelGGL(k_denorm_aos, g, b, 0, s, (const float *)Y, c, d_out_shift(mm), d_out_scale(mm), y);
-    HIPM(hipGetLastError());
+    HIPM(infer(mm, x, 1, IN, y, 1, OUT, n, stream ? static_cast<hipStream_t>(stream) : mm->stream));
     return NF_OK;
 }
 
@@ -617,8 +656,6 @@ int nf_mlp_create(uint64_t seed, nf_mlp **out) {
     std::unique_ptr<nf_mlp> hold(new nf_mlp);
     nf_mlp *mm = hold.get();
     HIPM(hipGetDevice(&mm->device));
-    int rc0 = scratch_setup(mm, mm->device);
-    if (rc0) return rc0;
     HIPM(hipStreamCreateWithFlags(&mm->stream, hipStreamNonBlocking));
     HIPM(hipMalloc(&mm->p, NPARAM * sizeof(float)));
     HIPM(hipMalloc(&mm->g, NPARAM * sizeof(float)));
@@ -707,14 +744,12 @@ int nf_mlp_predict(nf_mlp *mm, const float *x, int64_t n, float *y) {
     if (!mm || !x || !y || n < 0) return NF_E_ARG;
     if (n == 0) return NF_OK;
     int rc;
-    if ((rc = ensure_data(mm, n)) || (rc = upload_fm(mm, x, n, IN, mm->dx))) return rc;
-    const hipError_t e = nf::mlp::predict_device(mm, mm->dx, n, mm->dy, mm->stream);
-    if (e != hipSuccess) return fail(mm, NF_E_HIP, std::string("predict: ") + hipGetErrorString(e));
-    std::vector<float> fm((size_t)OUT * n);
+    // both arrays cross as they are ([n][6], [n][5]): the kernel reads samples
+    if ((rc = ensure_data(mm, n))) return rc;
+    HIPM(hipMemcpyAsync(mm->dx, x, (size_t)IN * n * sizeof(float), hipMemcpyHostToDevice, mm->stream));
+    HIPM(infer(mm, mm->dx, 1, IN, mm->dy, 1, OUT, n, mm->stream));
+    HIPM(hipMemcpyAsync(y, mm->dy, (size_t)OUT * n * sizeof(float), hipMemcpyDeviceToHost, mm->stream));
     HIPM(hipStreamSynchronize(mm->stream));
-    HIPM(hipMemcpy(fm.data(), mm->dy, fm.size() * sizeof(float), hipMemcpyDeviceToHost));
-    for (int64_t j = 0; j < n; ++j)
-        for (int o = 0; o < OUT; ++o) y[(size_t)j * OUT + o] = fm[(size_t)o * n + j];
     return NF_OK;
 }
 
