@@ -126,43 +126,98 @@ __global__ void k_reset_inst(InstState *st, int i, int uold_zero, double rref) {
     if (threadIdx.x == 0) st[i] = InstState{0.0, 0.0, rref, 0, 0, 0, 0, 0, 0, uold_zero, 0};
 }
 
-// Network features of the cells [0, n) of one instance, feature-major
-// x[6][n]: (p0, p1, centroid, distance to the nearest wall point).  The wall
-// points are streamed through LDS; every thread takes part in every pass.
-__global__ __launch_bounds__(BLOCK) void k_features(DevMesh m, uint32_t cell0, uint32_t n, const float4 *wall,
-                                                    uint32_t nw, float p0, float p1, float *x) {
-    __shared__ float4 sh[BLOCK];
-    const uint32_t c = blockIdx.x * BLOCK + threadIdx.x;
-    const bool live = c < n;
-    float cx = 0.f, cy = 0.f, cz = 0.f;
-    if (live) {
-        const uint4 q = *reinterpret_cast<const uint4 *>(m.cnodes + 4 * (size_t)(cell0 + c));
-        const uint32_t id[4] = {q.x, q.y, q.z, q.w};
-        double s[3] = {0.0, 0.0, 0.0};
-        for (int k = 0; k < 4; ++k)
-            for (int d = 0; d < 3; ++d) s[d] += m.nodes[4 * (size_t)id[k] + d];
-        cx = (float)(0.25 * s[0]);
-        cy = (float)(0.25 * s[1]);
-        cz = (float)(0.25 * s[2]);
-    }
+constexpr uint32_t WTILE = 32;  // wall points per box (16: 0.93 ms, 64: 0.81 ms where 32 takes 0.76 ms)
+
+struct FeatArgs {
+    uint32_t cell0, n;   // the instance's device cells
+    const float4 *wall;  // its wall points, Morton order, [boxes][WTILE] (the last box repeats its last point)
+    const float4 *wbox;  // [boxes][2] lower and upper corner of each box
+    uint32_t nbox;
+    float p0, p1;
+    float *x;              // x(f, c) = x[f * xf + row(c) * xj]
+    size_t xf, xj;
+    const uint32_t *perm;  // row(c): reference cell of device cell c, or null: c
+};
+
+// Network features of the cells [0, n) of one instance: (p0, p1, centroid,
+// distance to the nearest wall point).  A wave's 64 cells are neighbours, so
+// only the few boxes of wall points that can hold a nearest point of any
+// of them are searched: the box with the smallest gap to the wave's cells
+// first, then, of the boxes whose gap is below the wave's largest distance
+// after that, those with a smaller gap to some cell than its distance so
+// far.  The gap is formed with the operations of the distance itself (the
+// difference per axis, squares, the same order of sums), and rounding is
+// monotone, so a skipped box holds no point whose computed distance is
+// smaller: the result is the minimum over all wall points, bit for bit.
+// 1,463,340 cells and 34,452 wall points take 0.76 ms, where a scan of every
+// point (VALU-bound) took 17.3 ms.
+__global__ __launch_bounds__(BLOCK) void k_features(DevMesh m, FeatArgs a) {
+    const uint32_t c0 = blockIdx.x * BLOCK + threadIdx.x, lane = threadIdx.x & 63u;
+    const bool live = c0 < a.n;
+    const uint32_t c = live ? c0 : a.n - 1;
+    const uint4 q = *reinterpret_cast<const uint4 *>(m.cnodes + 4 * (size_t)(a.cell0 + c));
+    const uint32_t id[4] = {q.x, q.y, q.z, q.w};
+    double s[3] = {0.0, 0.0, 0.0};
+    for (int k = 0; k < 4; ++k)
+        for (int d = 0; d < 3; ++d) s[d] += m.nodes[4 * (size_t)id[k] + d];
+    const float cx = (float)(0.25 * s[0]), cy = (float)(0.25 * s[1]), cz = (float)(0.25 * s[2]);
+    auto wmin = [](float v) {
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) v = fminf(v, __shfl_xor(v, o, 64));
+        return v;
+    };
+    auto wmax = [](float v) {
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
+        return v;
+    };
+    const float lx = wmin(cx), ly = wmin(cy), lz = wmin(cz), hx = wmax(cx), hy = wmax(cy), hz = wmax(cz);
+    // squared gap between box b and the box (ax, ay, az) - (ex, ey, ez)
+    auto gap_to = [&](uint32_t b, float ax, float ay, float az, float ex, float ey, float ez) {
+        const float4 lo = a.wbox[2 * b], hi = a.wbox[2 * b + 1];
+        const float dx = fmaxf(fmaxf(lo.x - ex, ax - hi.x), 0.f), dy = fmaxf(fmaxf(lo.y - ey, ay - hi.y), 0.f),
+                    dz = fmaxf(fmaxf(lo.z - ez, az - hi.z), 0.f);
+        return dx * dx + dy * dy + dz * dz;
+    };
+    auto gap2 = [&](uint32_t b) { return gap_to(b, lx, ly, lz, hx, hy, hz); };
     float d2 = INFINITY;
-    for (uint32_t w0 = 0; w0 < nw; w0 += BLOCK) {
-        if (w0 + threadIdx.x < nw) sh[threadIdx.x] = wall[w0 + threadIdx.x];
-        __syncthreads();
-        const uint32_t cnt = min((uint32_t)BLOCK, nw - w0);
-        for (uint32_t k = 0; k < cnt; ++k) {
-            const float dx = sh[k].x - cx, dy = sh[k].y - cy, dz = sh[k].z - cz;
+    auto search = [&](uint32_t b) {  // b is the same in every lane
+        const float4 *w = a.wall + (size_t)__builtin_amdgcn_readfirstlane(b) * WTILE;
+#pragma unroll 8
+        for (uint32_t k = 0; k < WTILE; ++k) {
+            const float dx = w[k].x - cx, dy = w[k].y - cy, dz = w[k].z - cz;
             d2 = fminf(d2, dx * dx + dy * dy + dz * dz);
         }
-        __syncthreads();
+    };
+    if (a.nbox) {
+        float g = INFINITY;
+        uint32_t first = 0;
+        for (uint32_t b = lane; b < a.nbox; b += 64) {
+            const float t = gap2(b);
+            if (t < g) g = t, first = b;
+        }
+        const float gm = wmin(g);
+        const uint64_t at = __ballot(g == gm);
+        first = __shfl(first, at ? __ffsll((unsigned long long)at) - 1 : 0, 64);
+        search(first);
+        const float far = wmax(d2);  // (a lane whose distance stays infinite keeps every box)
+        for (uint32_t b0 = 0; b0 < a.nbox; b0 += 64) {
+            const uint32_t b = b0 + lane;
+            uint64_t todo = __ballot(b < a.nbox && b != first && !(gap2(b) >= far));
+            for (; todo; todo &= todo - 1) {
+                const uint32_t t = b0 + __builtin_amdgcn_readfirstlane(__ffsll((unsigned long long)todo) - 1);
+                if (__any(!(gap_to(t, cx, cy, cz, cx, cy, cz) >= d2))) search(t);
+            }
+        }
     }
     if (live) {
-        x[c] = p0;
-        x[n + c] = p1;
-        x[2 * (size_t)n + c] = cx;
-        x[3 * (size_t)n + c] = cy;
-        x[4 * (size_t)n + c] = cz;
-        x[5 * (size_t)n + c] = nw ? sqrtf(d2) : 0.f;
+        float *x = a.x + (a.perm ? a.perm[c] : c) * a.xj;
+        x[0] = a.p0;
+        x[a.xf] = a.p1;
+        x[2 * a.xf] = cx;
+        x[3 * a.xf] = cy;
+        x[4 * a.xf] = cz;
+        x[5 * a.xf] = a.nbox ? sqrtf(d2) : 0.f;
     }
 }
 
@@ -189,7 +244,7 @@ struct Inst {
     std::vector<uint32_t> perm;  // local device cell -> reference cell
     double Vinf[5] = {0, 0, 0, 0, 0};
     bool dt_valid = false;
-    uint32_t wall0 = 0, nwall = 0;  // wall-face centroids of the instance
+    uint32_t wbox0 = 0, nwbox = 0;  // boxes of wall-face centroids of the instance
     double rref = 0.0;              // residual reference of the drop (0: r_0)
     bool warm = false;              // state from the network, not yet fallen back
     // FP64 primvars V of the instance differ from prim(U): steps do not store
@@ -243,7 +298,7 @@ struct nf_ctx {
     double *red_dt = nullptr, *red_res = nullptr;  // per chunk
     double *hist = nullptr;                         // [instances][hist_cap]
     int hist_cap = 0;
-    float4 *wall = nullptr;                         // wall-face centroids of all instances
+    float4 *wall = nullptr, *wbox = nullptr;        // wall-face centroids of all instances and their boxes
     float *feat = nullptr, *vpred = nullptr;        // network features / prediction scratch
     uint32_t feat_cap = 0;
     double *r_eval = nullptr;                       // [instances]
@@ -697,20 +752,23 @@ int timestep_subset(nf_ctx *ctx, const std::vector<bool> &need) {
     return NF_OK;
 }
 
-// feature-major features of instance i into ctx->feat
-int features(nf_ctx *ctx, int i, const double *cp) {
+// features of instance i into ctx->feat: feature-major in device cell order
+// (the network's input), or rows [N][6] in reference cell order
+int features(nf_ctx *ctx, int i, const double *cp, bool rows) {
     const Inst &I = ctx->inst[i];
+    int rc;
     if (I.N > ctx->feat_cap) {
         uint32_t cap = 0;
         for (const Inst &J : ctx->inst) cap = std::max(cap, J.N);
-        int rc;
         if ((rc = dalloc(ctx, &ctx->feat, 6 * (size_t)cap))) return rc;
         if ((rc = dalloc(ctx, &ctx->vpred, 5 * (size_t)cap))) return rc;
         ctx->feat_cap = cap;
     }
-    hipLaunchKernelGGL(k_features, dim3((I.N + BLOCK - 1) / BLOCK), dim3(BLOCK), 0, ctx->stream, devmesh(ctx),
-                       I.cell0, I.N, (const float4 *)(ctx->wall + I.wall0), I.nwall, (float)cp[0], (float)cp[1],
-                       ctx->feat);
+    if (rows && (rc = ensure_stage(ctx))) return rc;
+    const FeatArgs a{I.cell0, I.N, ctx->wall + (size_t)I.wbox0 * WTILE, ctx->wbox + 2 * (size_t)I.wbox0, I.nwbox,
+                     (float)cp[0], (float)cp[1], ctx->feat, rows ? 1 : (size_t)I.N, rows ? 6 : (size_t)1,
+                     rows ? ctx->perm_dev + I.cell0 : nullptr};
+    hipLaunchKernelGGL(k_features, dim3((I.N + BLOCK - 1) / BLOCK), dim3(BLOCK), 0, ctx->stream, devmesh(ctx), a);
     HIPC(hipGetLastError());
     return NF_OK;
 }
@@ -749,6 +807,43 @@ int set_freestream(nf_ctx *ctx, int i) {
 }
 
 double d_node(const double *nodes, uint32_t v, int d) { return nodes[3 * (size_t)v + d]; }
+
+// appends one instance's wall points in Morton order, in boxes of WTILE, and
+// the boxes' corners (points with a NaN coordinate are never nearest and
+// widen no box)
+void wall_boxes(const std::vector<float4> &pts, std::vector<float4> &wall, std::vector<float4> &wbox) {
+    if (pts.empty()) return;
+    auto grow = [](float4 &lo, float4 &hi, const float4 &p) {
+        lo = make_float4(fminf(lo.x, p.x), fminf(lo.y, p.y), fminf(lo.z, p.z), 0.f);
+        hi = make_float4(fmaxf(hi.x, p.x), fmaxf(hi.y, p.y), fmaxf(hi.z, p.z), 0.f);
+    };
+    const float4 none_lo = make_float4(INFINITY, INFINITY, INFINITY, 0.f);
+    const float4 none_hi = make_float4(-INFINITY, -INFINITY, -INFINITY, 0.f);
+    float4 lo = none_lo, hi = none_hi;
+    for (const float4 &p : pts) grow(lo, hi, p);
+    const float ext = std::max(std::max(hi.x - lo.x, hi.y - lo.y), hi.z - lo.z);
+    const float scale = ext > 0.f ? 1023.f / ext : 0.f;
+    auto spread = [&](float v, float l) {
+        const float t = (v - l) * scale;
+        uint32_t x = t >= 0.f && t <= 1023.f ? (uint32_t)t : 0u, r = 0;
+        for (int b = 0; b < 10; ++b) r |= ((x >> b) & 1u) << (3 * b);
+        return r;
+    };
+    std::vector<std::pair<uint32_t, uint32_t>> order(pts.size());
+    for (uint32_t q = 0; q < pts.size(); ++q)
+        order[q] = {spread(pts[q].x, lo.x) | spread(pts[q].y, lo.y) << 1 | spread(pts[q].z, lo.z) << 2, q};
+    std::sort(order.begin(), order.end());
+    for (size_t q0 = 0; q0 < order.size(); q0 += WTILE) {
+        float4 blo = none_lo, bhi = none_hi;
+        for (size_t q = q0; q < q0 + WTILE; ++q) {
+            const float4 &p = pts[order[std::min(q, order.size() - 1)].second];
+            grow(blo, bhi, p);
+            wall.push_back(p);
+        }
+        wbox.push_back(blo);
+        wbox.push_back(bhi);
+    }
+}
 
 int build_red_table(nf_ctx *ctx, uint32_t B, RedTable &r) {
     std::vector<uint32_t> first, n, c0, nc;
@@ -838,7 +933,7 @@ int create(int32_t n, const nf_mesh_desc *descs, const nf_params *prms, nf_ctx *
 
     // host pipeline per instance; the device arrays are the concatenation
     std::vector<uint32_t> cnodes, nbr, fcode, bface, inst_end;
-    std::vector<float4> wall;
+    std::vector<float4> wall, wbox;
     std::vector<uint8_t> bbc;
     std::vector<double> bS3;  // [nb][3]
     std::vector<uint16_t> binst;
@@ -896,17 +991,19 @@ int create(int32_t n, const nf_mesh_desc *descs, const nf_params *prms, nf_ctx *
             binst.push_back((uint16_t)i);
         }
         // wall-face centroids (slip and no-slip patches) for the network features
-        I.wall0 = (uint32_t)wall.size();
+        std::vector<float4> pts;
         for (size_t q = 0; q < g.pfirst.size(); ++q) {
             if (g.pbc[q] == NF_BC_FARFIELD) continue;
             for (uint32_t f = g.pfirst[q]; f < g.pfirst[q] + g.pn[q]; ++f) {
                 double cf[3] = {0, 0, 0};
                 for (int k = 0; k < 3; ++k)
                     for (int e = 0; e < 3; ++e) cf[e] += d_node(d->nodes, g.fnodes[3 * (size_t)f + k], e);
-                wall.push_back(make_float4((float)(cf[0] / 3), (float)(cf[1] / 3), (float)(cf[2] / 3), 0.f));
+                pts.push_back(make_float4((float)(cf[0] / 3), (float)(cf[1] / 3), (float)(cf[2] / 3), 0.f));
             }
         }
-        I.nwall = (uint32_t)wall.size() - I.wall0;
+        I.wbox0 = (uint32_t)(wbox.size() / 2);
+        wall_boxes(pts, wall, wbox);
+        I.nwbox = (uint32_t)(wbox.size() / 2) - I.wbox0;
         for (uint32_t b = 0; b < I.Npad / BLOCK; ++b) blk_inst.push_back((uint32_t)i);
         inst_end.push_back((uint32_t)cell0 + g.N);
         for (uint32_t v = 0; v < d->n_nodes; ++v)
@@ -1025,7 +1122,11 @@ int create(int32_t n, const nf_mesh_desc *descs, const nf_params *prms, nf_ctx *
     if ((rc = dalloc(ctx, &ctx->red_res, (size_t)ctx->red128.nchunk))) return rc;
     if ((rc = dalloc(ctx, &ctx->r_eval, (size_t)n))) return rc;
     if ((rc = dalloc(ctx, &ctx->wall, wall.size()))) return rc;
-    if (!wall.empty()) HIPC(hipMemcpy(ctx->wall, wall.data(), wall.size() * sizeof(float4), hipMemcpyHostToDevice));
+    if ((rc = dalloc(ctx, &ctx->wbox, wbox.size()))) return rc;
+    if (!wall.empty()) {
+        HIPC(hipMemcpy(ctx->wall, wall.data(), wall.size() * sizeof(float4), hipMemcpyHostToDevice));
+        HIPC(hipMemcpy(ctx->wbox, wbox.data(), wbox.size() * sizeof(float4), hipMemcpyHostToDevice));
+    }
     if ((rc = ensure_hist(ctx, 1024))) return rc;
     for (int i = 0; i < n; ++i)
         if ((rc = set_freestream(ctx, i))) return rc;
@@ -1476,20 +1577,16 @@ int nf_eval_residuals(nf_ctx *ctx, double *out) {
 int nf_inst_features(nf_ctx *ctx, int32_t i, const double *cp, float *x) {
     if (!valid_inst(ctx, i) || !cp || !x) return NF_E_ARG;
     int rc;
-    if ((rc = features(ctx, i, cp))) return rc;
-    const Inst &I = ctx->inst[i];
-    std::vector<float> fm((size_t)6 * I.N);
+    if ((rc = features(ctx, i, cp, true))) return rc;
+    HIPC(hipMemcpyAsync(x, ctx->feat, (size_t)6 * ctx->inst[i].N * sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
     HIPC(hipStreamSynchronize(ctx->stream));
-    HIPC(hipMemcpy(fm.data(), ctx->feat, fm.size() * sizeof(float), hipMemcpyDeviceToHost));
-    for (uint32_t c = 0; c < I.N; ++c)
-        for (int f = 0; f < 6; ++f) x[6 * (size_t)I.perm[c] + f] = fm[(size_t)f * I.N + c];
     return NF_OK;
 }
 
 int nf_inst_warm_start(nf_ctx *ctx, int32_t i, nf_mlp *net, const double *cp, int32_t *fell_back) {
     if (!valid_inst(ctx, i) || !net || !cp) return NF_E_ARG;
     int rc;
-    if ((rc = features(ctx, i, cp))) return rc;
+    if ((rc = features(ctx, i, cp, false))) return rc;
     Inst &I = ctx->inst[i];
     HIPC(nf::mlp::predict_device(net, ctx->feat, I.N, ctx->vpred, ctx->stream));
     if ((rc = clear_flags(ctx))) return rc;
