@@ -16,9 +16,9 @@
 //   sweep B (per stage): face values -> Rusanov fluxes of the four faces,
 //            flux balance, RK stage combination, prim(U) of the new state.
 //   Boundary faces read their ghost state from small per-boundary-face
-//   buffers filled by k_ghost<false> (ghost of the cell-centre state, for the
-//   gradient and min/max) and k_ghost<true> (ghost of the reconstructed face
-//   state, for the boundary flux), so the sweeps carry no boundary code.
+//   buffers: ghosts of the cell-centre states (for the gradient and min/max)
+//   and of the reconstructed face states (for the boundary flux).  k_ghost
+//   fills them, or, on small meshes (FUSE), the end of the sweep before.
 //
 // Several meshes (instances) can share one launch: their cells are
 // concatenated, each instance padded to whole blocks of 256 cells, and every
@@ -128,6 +128,19 @@ __device__ __forceinline__ LaneCell lane_cell(const DevMesh &m, int xcd_remap) {
     const uint32_t inst = m.blk_inst[(lb * B) / BLOCK];
     const uint32_t end = m.inst_end[inst];
     return {c0 < end ? c0 : end - 1, inst, lb, c0 < end};
+}
+
+// The boundary faces of a block's cells (numbered in device cell order).
+// Loaded by a sweep before anything else, kept there by the asm: at its end
+// every block would wait for these scalar loads.
+struct BndRange {
+    uint32_t b0, b1;
+};
+template <int B>
+__device__ __forceinline__ BndRange bnd_range(const uint32_t *boff, uint32_t lb) {
+    BndRange r{boff[lb * (B / 128)], boff[(lb + 1) * (B / 128)]};
+    asm volatile("" : "+s"(r.b0), "+s"(r.b1));
+    return r;
 }
 
 struct CellGeo {
@@ -380,44 +393,57 @@ __device__ __forceinline__ void apply_stage_cell(const DevMesh &m, const ApplyAr
 
 #ifndef NF_DEVICE_HELPERS_ONLY
 // ---------------------------------------------------------------------------
-// boundary ghost states.  bface[b] = device cell | slot << 29.
-struct GhostArgs {
-    const uint32_t *bface;
-    const uint8_t *bbc;          // boundary type
+// boundary ghost states; boundary faces are numbered in device cell order
+struct BndArgs {
+    const uint32_t *bface;       // device cell | slot << 29
+    const uint32_t *boff;        // [cells/128 + 1] first boundary face of each 128 device cells
     const uint16_t *binst;       // instance
-    uint32_t nb;                 // boundary faces
-    const double *src;           // V or U [tile][5][64] (cell) or FV [tile][4][5][64] (face)
-    double *out;                 // [nb/64][5][64], tiled like V
-    const FarField<double> *fs;  // [instances]
-    int src_is_u;                // cell ghosts: src is U, the primvars are prim(U)
+    const uint8_t *bbc;          // boundary type
     const double *bS;            // [3][nb] S_ij of each boundary face (cell -> ghost)
+    uint32_t nb;                 // boundary faces
+    const FarField<double> *fs;  // [instances]
+    double *out;                 // [nb/64][5][64], tiled like V
 };
 
-// FACE = false: ghost of the cell-centre state (set_constant_ghost_values,
-// src/Solver.cpp:300-330); FACE = true: ghost of the reconstructed face state
+// what a ghost is formed from: V (set_constant_ghost_values, src/Solver.cpp:
+// 300-330), the primvars of the state U, or the reconstructed face states FV
 // (src/Solver.cpp:210-212)
-// The face vector comes precomputed from the host face graph: the same
-// cross product and sign the sweeps evaluate from the nodes, so the same bits.
-template <bool FACE>
-__global__ __launch_bounds__(BLOCK) void k_ghost(DevMesh m, GhostArgs a) {
-    const uint32_t b0 = blockIdx.x * BLOCK + threadIdx.x;
-    const bool live = b0 < a.nb;
-    const uint32_t b = live ? b0 : a.nb - 1;
-    const uint32_t inst = a.binst[b];
-    const uint32_t w = a.bface[b], c = w & 0x1FFFFFFFu, s = w >> 29;
+enum class GhostOf { V, U, FV };
+
+// The face vector comes precomputed from the host face graph: the same cross
+// product and sign the sweeps evaluate from the nodes, so the same bits.
+template <GhostOf OF>
+__device__ __forceinline__ void bnd_ghost(const BndArgs &a, uint32_t b, uint32_t inst, const double *src) {
+    const uint32_t w = a.bface[b], c = w & 0x1FFFFFFFu;
     const V3d S = {a.bS[b], a.bS[a.nb + b], a.bS[2 * (size_t)a.nb + b]};
     double Vd[5], Vg[5];
 #pragma unroll
-    for (int k = 0; k < 5; ++k) Vd[k] = FACE ? a.src[fix(c, s, k)] : a.src[tix(c, k)];
-    if (!FACE && a.src_is_u) {
+    for (int k = 0; k < 5; ++k) Vd[k] = OF == GhostOf::FV ? src[fix(c, w >> 29, k)] : src[tix(c, k)];
+    if (OF == GhostOf::U) {
         const double Ud[5] = {Vd[0], Vd[1], Vd[2], Vd[3], Vd[4]};
         cons_to_prim_d(Ud, Vd);
     }
     ghost_d((int)a.bbc[b], Vd, S, a.fs[inst], Vg);
-    if (live && !m.st[inst].stop) {
 #pragma unroll
-        for (int k = 0; k < 5; ++k) a.out[tix(b, k)] = Vg[k];
-    }
+    for (int k = 0; k < 5; ++k) a.out[tix(b, k)] = Vg[k];
+}
+
+// Ghosts of the block's boundary faces, at the end of a sweep that stored
+// src.  The block's faces are taken by its first lanes, one face per lane, so
+// the long farfield branch (two pow) runs in as few waves as it can.
+template <int B, GhostOf OF>
+__device__ __forceinline__ void bnd_ghosts(const BndArgs &a, BndRange r, uint32_t inst, const double *src) {
+    if (r.b0 == r.b1) return;  // the same for the whole block
+    __syncthreads();           // every wave's part of src is stored
+    for (uint32_t b = r.b0 + threadIdx.x; b < r.b1; b += B) bnd_ghost<OF>(a, b, inst, src);
+}
+
+// Ghosts of every boundary face in a launch of its own.  Also those of
+// stopped instances: they have to match the state when it runs again.
+template <GhostOf OF>
+__global__ __launch_bounds__(BLOCK) void k_ghost(BndArgs a, const double *src) {
+    const uint32_t b = blockIdx.x * BLOCK + threadIdx.x;
+    if (b < a.nb) bnd_ghost<OF>(a, b, a.binst[b], src);
 }
 
 // ---------------------------------------------------------------------------
@@ -431,6 +457,7 @@ struct SweepAArgs {
     int xcd_remap;
     double *grad_aux;  // [N][15] column-major 5x3 per cell, or null
     double *psi_aux;   // [N][5] or null
+    BndArgs bnd;       // FUSE: ghosts of the reconstructed face states (out: Gf)
 };
 
 // One 64-cell tile of sweep A: its loads (tileA_issue) and the rest
@@ -629,12 +656,14 @@ __device__ __forceinline__ double tileA_run(const DevMesh &m, const SweepAArgs &
     return dtc;
 }
 
-template <int ORDER, int B, bool FROM_U>
+template <int ORDER, int B, bool FROM_U, bool FUSE>
 __global__ __launch_bounds__(B) NF_SWEEP_ATTR void k_sweepA(DevMesh m, SweepAArgs a) {
     __shared__ double sh[B / 64];
     __shared__ double lds[12 * B];
     __shared__ __align__(16) double ldsv[NF_A_LDS ? 5 * B : 2];  // [wave][5][64] own states
     const LaneCell L = lane_cell<B>(m, a.xcd_remap);
+    BndRange br{0, 0};
+    if (FUSE) br = bnd_range<B>(a.bnd.boff, L.lb);
     if (m.st[L.inst].stop) return;
     TileA t;
     t.c = L.c;
@@ -643,6 +672,7 @@ __global__ __launch_bounds__(B) NF_SWEEP_ATTR void k_sweepA(DevMesh m, SweepAArg
     tileA_issue<ORDER, B, FROM_U>(m, a, t);
     __builtin_amdgcn_sched_barrier(0);
     const double dtc = tileA_run<ORDER, B, FROM_U>(m, a, t, lds, ldsv);
+    if (FUSE) bnd_ghosts<B, GhostOf::FV>(a.bnd, br, L.inst, a.FV);
     if (a.dt_part) {
         const double v = block_reduce<true, B>(dtc, sh);
         if (threadIdx.x == 0) a.dt_part[L.lb] = v;
@@ -656,7 +686,6 @@ struct SweepBArgs {
     const double *U;        // [tile][5][64] state entering the stage
     const double *Uo;       // U_old (U^n)
     double *Uout;           // (may alias U)
-    double *Vout;           // prim(Uout), or null (the next sweep A evaluates it)
     const double *dt_cell;  // per-cell step (local time stepping), or null
     int kind;               // 1: U + dt/vol R, 2: RK3 stage 2, 3: RK3 stage 3
     double *res_part;       // per-block sum of R_rho^2, or null
@@ -664,14 +693,17 @@ struct SweepBArgs {
     int xcd_remap;
     double *R_aux;          // [N][5] or null: store R, skip the update
     double *Rst, *fst;      // checked stage: R [tile][5][64] and f [cell] for k_apply, no update
+    BndArgs bnd;            // FUSE: ghosts of the updated cell states (out: Gc), where it updates
 };
 
 // FLUX: 0 Rusanov, 1 HLLC
-template <int B, int FLUX>
+template <int B, int FLUX, bool FUSE>
 __global__ __launch_bounds__(B) NF_SWEEPB_ATTR void k_sweepB(DevMesh m, SweepBArgs a) {
     __shared__ double sh[B / 64];
     __shared__ double lds[12 * B];
     const LaneCell L = lane_cell<B>(m, a.xcd_remap);
+    BndRange br{0, 0};
+    if (FUSE) br = bnd_range<B>(a.bnd.boff, L.lb);
     InstState &st = m.st[L.inst];
     if (st.stop) return;
     const uint32_t c = L.c;
@@ -773,12 +805,9 @@ __global__ __launch_bounds__(B) NF_SWEEPB_ATTR void k_sweepB(DevMesh m, SweepBAr
             if (live) {
 #pragma unroll
                 for (int k = 0; k < 5; ++k) a.Uout[tix(c, k)] = Un[k];
-                if (a.Vout) {
-#pragma unroll
-                    for (int k = 0; k < 5; ++k) a.Vout[tix(c, k)] = Vnew[k];
-                }
                 if (!(Vnew[0] > 0.0) || !(Vnew[4] > 0.0) || !(Un[4] > 0.0)) atomicAdd(&st.bad_state, 1);
             }
+            if (FUSE) bnd_ghosts<B, GhostOf::U>(a.bnd, br, L.inst, a.Uout);
         }
     }
     if (a.res_part) {

@@ -25,15 +25,14 @@ namespace mx {
 #define NF_SWEEPB_MX_ATTR
 #endif
 
-// kernel arguments
-struct GhostArgsMx {
-    const uint32_t *bface;
-    const uint8_t *bbc;
+// kernel arguments; BndArgsMx as BndArgs, the face vectors from the nodes
+struct BndArgsMx {
+    const uint32_t *bface, *boff;
     const uint16_t *binst;
+    const uint8_t *bbc;
     uint32_t nb;
-    const float *src;          // V32 [tile][5][64] (cell) or FV32 (face)
-    float *out;                // [nb/64][5][64], tiled like V
     const FarField<float> *fs; // [instances]
+    float *out;                // [nb/64][5][64], tiled like V
 };
 
 struct SweepAArgsMx {
@@ -45,6 +44,7 @@ struct SweepAArgsMx {
     double CFL;
     int xcd_remap;
     double *grad_aux, *psi_aux;
+    BndArgsMx bnd;
 };
 
 struct SweepBArgsMx {
@@ -61,6 +61,7 @@ struct SweepBArgsMx {
     int xcd_remap;
     double *R_aux;
     double *Rst, *fst;  // checked stage: R and f stored for the apply pass, no update
+    BndArgsMx bnd;
 };
 
 #ifdef NF_MIXED_KERNELS
@@ -147,35 +148,50 @@ __device__ __forceinline__ float barth_psi_f(const float *delta, float vmax, flo
 
 // ---------------------------------------------------------------------------
 
-template <bool FACE>
-__global__ __launch_bounds__(BLOCK) void k_ghost_mx(DevMesh m, GhostArgsMx a) {
-    __shared__ double lds[12 * BLOCK];
-    const uint32_t b0 = blockIdx.x * BLOCK + threadIdx.x;
-    const bool live = b0 < a.nb;
-    const uint32_t b = live ? b0 : a.nb - 1;
-    const uint32_t inst = a.binst[b];
+// ghost of boundary face b from the cell states (FACE = false) or the
+// reconstructed face states; lds: [12 * B]
+template <int B, bool FACE>
+__device__ __forceinline__ void bnd_ghost_mx(const DevMesh &m, const BndArgsMx &a, uint32_t b, uint32_t inst,
+                                             const float *src, double *lds) {
     const uint32_t w = a.bface[b], c = w & 0x1FFFFFFFu, s = w >> 29;
     CellGeo g;
     load_cell(m, c, g);
-    const NodeView nv = stage_nodes<BLOCK>(lds, g);
+    const NodeView nv = stage_nodes<B>(lds, g);
     V3f S;
     face_geo_mx(nv, g, (m.fcode[c] >> (8 * s)) & 0xFFu, S, nullptr);
     float Vd[5], Vg[5];
 #pragma unroll
-    for (int k = 0; k < 5; ++k) Vd[k] = FACE ? a.src[fix(c, s, k)] : a.src[tix(c, k)];
+    for (int k = 0; k < 5; ++k) Vd[k] = FACE ? src[fix(c, s, k)] : src[tix(c, k)];
     ghost_value<float>((int)a.bbc[b], Vd, S, a.fs[inst], Vg);
-    if (live && !m.st[inst].stop) {
 #pragma unroll
-        for (int k = 0; k < 5; ++k) a.out[tix(b, k)] = Vg[k];
-    }
+    for (int k = 0; k < 5; ++k) a.out[tix(b, k)] = Vg[k];
 }
 
-template <int ORDER, int B>
+// ghosts of the block's boundary faces at the end of a sweep (bnd_ghosts)
+template <int B, bool FACE>
+__device__ __forceinline__ void bnd_ghosts_mx(const DevMesh &m, const BndArgsMx &a, BndRange r, uint32_t inst,
+                                              const float *src, double *lds) {
+    if (r.b0 == r.b1) return;  // the same for the whole block
+    __syncthreads();           // every wave's part of src is stored, and lds is free
+    for (uint32_t b = r.b0 + threadIdx.x; b < r.b1; b += B) bnd_ghost_mx<B, FACE>(m, a, b, inst, src, lds);
+}
+
+// ghosts of every boundary face in a launch of its own (k_ghost)
+template <bool FACE>
+__global__ __launch_bounds__(BLOCK) void k_ghost_mx(DevMesh m, BndArgsMx a, const float *src) {
+    __shared__ double lds[12 * BLOCK];
+    const uint32_t b = blockIdx.x * BLOCK + threadIdx.x;
+    if (b < a.nb) bnd_ghost_mx<BLOCK, FACE>(m, a, b, a.binst[b], src, lds);
+}
+
+template <int ORDER, int B, bool FUSE>
 __global__ __launch_bounds__(B) void k_sweepA_mx(DevMesh m, SweepAArgsMx a) {
     __shared__ double sh[B / 64];
     __shared__ double lds[12 * B];
     __shared__ float ldsv[5 * B];  // [wave][5][64] own states
     const LaneCell L = lane_cell<B>(m, a.xcd_remap);
+    BndRange br{0, 0};
+    if (FUSE) br = bnd_range<B>(a.bnd.boff, L.lb);
     if (m.st[L.inst].stop) return;
     const uint32_t c = L.c;
     const bool live = L.live;
@@ -274,6 +290,7 @@ __global__ __launch_bounds__(B) void k_sweepA_mx(DevMesh m, SweepAArgsMx a) {
             }
         }
     }
+    if (FUSE) bnd_ghosts_mx<B, true>(m, a.bnd, br, L.inst, a.FV, lds);
     if (a.dt_part) {
         const V3d Sd[4] = {{S[0].x, S[0].y, S[0].z}, {S[1].x, S[1].y, S[1].z}, {S[2].x, S[2].y, S[2].z},
                            {S[3].x, S[3].y, S[3].z}};
@@ -286,11 +303,13 @@ __global__ __launch_bounds__(B) void k_sweepA_mx(DevMesh m, SweepAArgsMx a) {
     }
 }
 
-template <int B>
+template <int B, bool FUSE>
 __global__ __launch_bounds__(B) NF_SWEEPB_MX_ATTR void k_sweepB_mx(DevMesh m, SweepBArgsMx a) {
     __shared__ double sh[B / 64];
     __shared__ double lds[12 * B];
     const LaneCell L = lane_cell<B>(m, a.xcd_remap);
+    BndRange br{0, 0};
+    if (FUSE) br = bnd_range<B>(a.bnd.boff, L.lb);
     InstState &st = m.st[L.inst];
     if (st.stop) return;
     const uint32_t c = L.c;
@@ -382,6 +401,7 @@ __global__ __launch_bounds__(B) NF_SWEEPB_MX_ATTR void k_sweepB_mx(DevMesh m, Sw
                 }
                 if (!(Vnew[0] > 0.0) || !(Vnew[4] > 0.0) || !(Un[4] > 0.0)) atomicAdd(&st.bad_state, 1);
             }
+            if (FUSE) bnd_ghosts_mx<B, false>(m, a.bnd, br, L.inst, a.Vout, lds);
         }
     }
     if (a.res_part) {
@@ -407,9 +427,11 @@ __global__ __launch_bounds__(BLOCK) void k_prim_mx(const double *U, float *V, ui
 #endif  // NF_MIXED_KERNELS
 
 // host-side launchers (compiled in solver_mixed.hip)
-hipError_t launch_ghost_mx(bool face, dim3 g, hipStream_t st, const DevMesh &m, const GhostArgsMx &a);
-hipError_t launch_sweepA_mx(int order, int block, dim3 g, hipStream_t st, const DevMesh &m, const SweepAArgsMx &a);
-hipError_t launch_sweepB_mx(int block, dim3 g, hipStream_t st, const DevMesh &m, const SweepBArgsMx &a);
+hipError_t launch_ghost_mx(bool face, hipStream_t st, const DevMesh &m, const BndArgsMx &a, const float *src);
+hipError_t launch_sweepA_mx(int order, int block, bool fuse, uint32_t ncell, hipStream_t st, const DevMesh &m,
+                            const SweepAArgsMx &a);
+hipError_t launch_sweepB_mx(int block, bool fuse, uint32_t ncell, hipStream_t st, const DevMesh &m,
+                            const SweepBArgsMx &a);
 hipError_t launch_prim_mx(dim3 g, hipStream_t st, const double *U, float *V, uint32_t N);
 hipError_t launch_apply_mx(dim3 g, hipStream_t st, const DevMesh &m, const ApplyArgs &a);
 

@@ -14,6 +14,7 @@
 #include <map>
 #include <memory>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/netflux.h"
@@ -29,77 +30,100 @@ namespace {
 
 constexpr uint32_t RCHUNK = 2048;  // blocks per first-level reduction chunk
 
-// First level of the per-block partial reductions: chunk q reduces blocks
-// [first[q], first[q] + n[q]) of one instance in a fixed order.
+// The step's reductions of the sweeps' per-block partials, in a fixed order:
+// the minimum of the CFL steps and the sum of R_rho^2 of each instance.
+struct RedArgs {
+    const double *dt_part, *res_part;  // per sweep block; null: not reduced by this launch
+    const uint32_t *first, *n;         // [chunks] blocks [first, first + n) of one instance
+    const uint32_t *c0, *nc;           // [instances] its chunks
+    double *red_dt, *red_res;          // [chunks]
+    InstState *st;
+    int advance;   // dt: end of a step
+    double *hist;  // residual histories [instances][cap]
+    int cap;
+    double drop;
+    double *out;   // residuals go to out[instance] instead
+};
+
 template <bool MIN>
-__global__ __launch_bounds__(BLOCK) void k_reduce(const double *in, const uint32_t *first, const uint32_t *n,
-                                                  double *out) {
-    __shared__ double sh[BLOCK / 64];
-    const uint32_t q = blockIdx.x, b0 = first[q], nb = n[q];
+__device__ __forceinline__ double red_blocks(const double *in, uint32_t first, uint32_t n, double *sh) {
+    constexpr uint32_t Q = RCHUNK / BLOCK;  // a chunk's loads all in flight at once
     double v = MIN ? DBL_MAX : 0.0;
-    for (uint32_t i = threadIdx.x; i < nb; i += BLOCK) {
-        const double x = in[b0 + i];
-        v = MIN ? ((x < v) ? x : v) : v + x;
+    for (uint32_t i0 = threadIdx.x; i0 < n; i0 += RCHUNK) {
+        double x[Q];
+#pragma unroll
+        for (uint32_t q = 0; q < Q; ++q) x[q] = in[first + (i0 + q * BLOCK < n ? i0 + q * BLOCK : i0)];
+#pragma unroll
+        for (uint32_t q = 0; q < Q; ++q)
+            if (i0 + q * BLOCK < n) v = MIN ? ((x[q] < v) ? x[q] : v) : v + x[q];
     }
-    v = block_reduce<MIN, BLOCK>(v, sh);
-    if (threadIdx.x == 0) out[q] = v;
+    return block_reduce<MIN, BLOCK>(v, sh);
 }
 
-// Second level, one block per instance: dt = min over the instance's chunks.
-// advance = 1 at the end of a step: time += dt, nstep += 1, the first-step
-// flag clears, a converged instance stops, and the new dt (of the primvars
-// the step's last sweep A read) is installed for the next step.
-__global__ __launch_bounds__(BLOCK) void k_finalize_dt(const double *red, const uint32_t *c0, const uint32_t *nc,
-                                                       InstState *st, int advance) {
-    __shared__ double sh[BLOCK / 64];
-    const uint32_t i = blockIdx.x;
-    if (st[i].stop) return;
-    double v = DBL_MAX;
-    for (uint32_t q = threadIdx.x; q < nc[i]; q += BLOCK) {
-        const double x = red[c0[i] + q];
-        v = (x < v) ? x : v;
+// r_k = sqrt(sum) into the instance's residual history; sets `converged` once
+// r_k / ref <= drop, ref = rref if set, else r_0.  With `out`, r goes there.
+__device__ __forceinline__ void finish_res(const RedArgs &a, uint32_t i, double sum) {
+    const double r = sqrt(sum);
+    if (a.out) {
+        a.out[i] = r;
+        return;
     }
-    v = block_reduce<true, BLOCK>(v, sh);
-    if (threadIdx.x == 0) {
-        if (advance) {
-            st[i].time += st[i].dt;
-            st[i].nstep += 1;
-            st[i].uold_zero = 0;
-            if (st[i].converged) st[i].stop = 1;
-        }
-        // num_is_valid_and_pos (include/Includes.hpp:131-137)
-        const bool ok = (v - v == 0.0) && v > 0.0;
-        st[i].dt = v;
-        if (!ok) {
-            st[i].err = NF_E_INVALID_DT;
-            st[i].stop = 1;
-        }
+    InstState &st = a.st[i];
+    const int k = st.nstep;
+    double *h = a.hist + (size_t)i * a.cap;
+    if (k < a.cap) h[k] = r;
+    const double ref = st.rref > 0.0 ? st.rref : h[0];
+    if (a.drop > 0.0 && k < a.cap && ref > 0.0 && r / ref <= a.drop) st.converged = 1;
+}
+
+// dt = v.  advance = 1 at the end of a step: time += dt, nstep += 1, the
+// first-step flag clears, a converged instance stops, and the new dt (of the
+// primvars the step's last sweep A read) is installed for the next step.
+__device__ __forceinline__ void finish_dt(const RedArgs &a, uint32_t i, double v) {
+    InstState &st = a.st[i];
+    if (a.advance) {
+        st.time += st.dt;
+        st.nstep += 1;
+        st.uold_zero = 0;
+        if (st.converged) st.stop = 1;
+    }
+    // num_is_valid_and_pos (include/Includes.hpp:131-137)
+    const bool ok = (v - v == 0.0) && v > 0.0;
+    st.dt = v;
+    if (!ok) {
+        st.err = NF_E_INVALID_DT;
+        st.stop = 1;
     }
 }
 
-// r_k = sqrt(sum of the instance's partials), summed in a fixed order, into
-// the instance's residual history; sets `converged` once r_k / ref <= drop,
-// ref = rref if set, else r_0.  With `out`, r goes to out[i] instead.
-__global__ __launch_bounds__(BLOCK) void k_finalize_res(const double *red, const uint32_t *c0, const uint32_t *nc,
-                                                        InstState *st, double *hist, int cap, double drop,
-                                                        double *out) {
-    __shared__ double sh[BLOCK / 64];
+// One block per instance: everything, where no instance has more than one
+// chunk (RCHUNK blocks, 524,288 cells), from the partials (ONE); else the
+// second level, from the chunks' results of k_reduce.  The step's residual
+// and dt go through one launch (two with chunks), not two (four).
+template <bool ONE>
+__global__ __launch_bounds__(BLOCK) void k_finish(RedArgs a) {
+    __shared__ double sh[2][BLOCK / 64];
     const uint32_t i = blockIdx.x;
-    if (!out && st[i].stop) return;
-    double v = 0.0;
-    for (uint32_t q = threadIdx.x; q < nc[i]; q += BLOCK) v += red[c0[i] + q];
-    v = block_reduce<false, BLOCK>(v, sh);
+    if (!a.out && a.st[i].stop) return;
+    const uint32_t b0 = ONE ? a.first[a.c0[i]] : a.c0[i], nb = ONE ? a.n[a.c0[i]] : a.nc[i];
+    double s = 0.0, v = DBL_MAX;
+    if (a.res_part) s = red_blocks<false>(ONE ? a.res_part : a.red_res, b0, nb, sh[0]);
+    if (a.dt_part) v = red_blocks<true>(ONE ? a.dt_part : a.red_dt, b0, nb, sh[1]);
     if (threadIdx.x == 0) {
-        const double r = sqrt(v);
-        if (out) {
-            out[i] = r;
-            return;
-        }
-        const int k = st[i].nstep;
-        double *h = hist + (size_t)i * cap;
-        if (k < cap) h[k] = r;
-        const double ref = st[i].rref > 0.0 ? st[i].rref : h[0];
-        if (drop > 0.0 && k < cap && ref > 0.0 && r / ref <= drop) st[i].converged = 1;
+        if (a.res_part) finish_res(a, i, s);
+        if (a.dt_part) finish_dt(a, i, v);
+    }
+}
+
+__global__ __launch_bounds__(BLOCK) void k_reduce(RedArgs a) {
+    __shared__ double sh[2][BLOCK / 64];
+    const uint32_t q = blockIdx.x;
+    double s = 0.0, v = DBL_MAX;
+    if (a.res_part) s = red_blocks<false>(a.res_part, a.first[q], a.n[q], sh[0]);
+    if (a.dt_part) v = red_blocks<true>(a.dt_part, a.first[q], a.n[q], sh[1]);
+    if (threadIdx.x == 0) {
+        if (a.res_part) a.red_res[q] = s;
+        if (a.dt_part) a.red_dt[q] = v;
     }
 }
 
@@ -282,11 +306,12 @@ struct nf_ctx {
     double *Ua = nullptr, *Ub = nullptr, *V = nullptr, *FV = nullptr;
     float *V32 = nullptr, *FV32 = nullptr;
     uint32_t nbf = 0;
-    uint32_t *bface = nullptr;
+    uint32_t *bface = nullptr, *boff = nullptr;  // boundary faces in device cell order, their range per 128 cells
     uint8_t *bbc = nullptr;
     double *bS = nullptr;  // [3][nbf] S_ij of the boundary faces
     uint16_t *binst = nullptr;
     double *Gc = nullptr, *Gf = nullptr;
+    const double *gc_of = nullptr;  // the state (Ua or Ub) whose cell ghosts Gc (Gc32) holds, or null
     float *Gc32 = nullptr, *Gf32 = nullptr;
     FarField<double> *fs = nullptr;
     FarField<float> *fs32 = nullptr;
@@ -396,21 +421,35 @@ int refresh_v(nf_ctx *ctx) {
     return NF_OK;
 }
 
-// U: cell ghosts from prim(U) of this state instead of the stored primvars
-int run_ghost(nf_ctx *ctx, bool face, const double *U = nullptr) {
+BndArgs bnd_args(const nf_ctx *c, double *out) {
+    return {c->bface, c->boff, c->binst, c->bbc, c->bS, c->nbf, c->fs, out};
+}
+mx::BndArgsMx bnd_args_mx(const nf_ctx *c, float *out) {
+    return {c->bface, c->boff, c->binst, c->bbc, c->nbf, c->fs32, out};
+}
+
+// cell ghosts of the stored primvars, or (U set, FP64) of prim(U)
+int run_ghost_cell(nf_ctx *ctx, const double *U) {
+    ctx->gc_of = U;
     if (ctx->nbf == 0) return NF_OK;
+    if (ctx->mixed)
+        return launch_fn(ctx, "ghost_cell_mx", [&] {
+            return mx::launch_ghost_mx(false, ctx->stream, devmesh(ctx), bnd_args_mx(ctx, ctx->Gc32), ctx->V32);
+        });
     const dim3 g((ctx->nbf + BLOCK - 1) / BLOCK), b(BLOCK);
-    const DevMesh m = devmesh(ctx);
-    if (ctx->mixed) {
-        const mx::GhostArgsMx a{ctx->bface, ctx->bbc, ctx->binst, ctx->nbf, face ? ctx->FV32 : ctx->V32,
-                                face ? ctx->Gf32 : ctx->Gc32, ctx->fs32};
-        return launch_fn(ctx, face ? "ghost_face_mx" : "ghost_cell_mx",
-                         [&] { return mx::launch_ghost_mx(face, g, ctx->stream, m, a); });
-    }
-    const GhostArgs a{ctx->bface, ctx->bbc, ctx->binst, ctx->nbf, face ? ctx->FV : (U ? U : ctx->V),
-                      face ? ctx->Gf : ctx->Gc, ctx->fs, (!face && U) ? 1 : 0, ctx->bS};
-    if (face) return LAUNCH("ghost_face", k_ghost<true>, g, b, m, a);
-    return LAUNCH("ghost_cell", k_ghost<false>, g, b, m, a);
+    if (U) return LAUNCH("ghost_cell", k_ghost<GhostOf::U>, g, b, bnd_args(ctx, ctx->Gc), U);
+    return LAUNCH("ghost_cell", k_ghost<GhostOf::V>, g, b, bnd_args(ctx, ctx->Gc), (const double *)ctx->V);
+}
+
+// ghosts of the reconstructed face states
+int run_ghost_face(nf_ctx *ctx) {
+    if (ctx->nbf == 0) return NF_OK;
+    if (ctx->mixed)
+        return launch_fn(ctx, "ghost_face_mx", [&] {
+            return mx::launch_ghost_mx(true, ctx->stream, devmesh(ctx), bnd_args_mx(ctx, ctx->Gf32), ctx->FV32);
+        });
+    return LAUNCH("ghost_face", k_ghost<GhostOf::FV>, dim3((ctx->nbf + BLOCK - 1) / BLOCK), dim3(BLOCK),
+                  bnd_args(ctx, ctx->Gf), (const double *)ctx->FV);
 }
 
 int order_of(const nf_ctx *ctx) {
@@ -418,42 +457,64 @@ int order_of(const nf_ctx *ctx) {
     return ctx->prm.limiter == NF_LIMITER_NONE ? 1 : 2;
 }
 
-template <int B, bool FROM_U>
+template <int B, bool FROM_U, bool FUSE>
 hipError_t launch_sweepA(hipStream_t s, uint32_t ncell, int order, const DevMesh &m, const SweepAArgs &a) {
     const dim3 g(ncell / B), b(B);
-    if (order == 0) hipLaunchKernelGGL((k_sweepA<0, B, FROM_U>), g, b, 0, s, m, a);
-    else if (order == 1) hipLaunchKernelGGL((k_sweepA<1, B, FROM_U>), g, b, 0, s, m, a);
-    else hipLaunchKernelGGL((k_sweepA<2, B, FROM_U>), g, b, 0, s, m, a);
+    if (order == 0) hipLaunchKernelGGL((k_sweepA<0, B, FROM_U, FUSE>), g, b, 0, s, m, a);
+    else if (order == 1) hipLaunchKernelGGL((k_sweepA<1, B, FROM_U, FUSE>), g, b, 0, s, m, a);
+    else hipLaunchKernelGGL((k_sweepA<2, B, FROM_U, FUSE>), g, b, 0, s, m, a);
     return hipGetLastError();
 }
+template <int B, bool FUSE>
+hipError_t launch_sweepB(hipStream_t s, uint32_t ncell, bool hllc, const DevMesh &m, const SweepBArgs &a) {
+    const dim3 g(ncell / B), b(B);
+    if (hllc) hipLaunchKernelGGL((k_sweepB<B, 1, FUSE>), g, b, 0, s, m, a);
+    else hipLaunchKernelGGL((k_sweepB<B, 0, FUSE>), g, b, 0, s, m, a);
+    return hipGetLastError();
+}
+
+// Boundary ghosts at the end of the sweeps (FUSE) or in launches of their own:
+// a launch costs 4 to 6 us whatever it does, a boundary block's ghosts 4 to 8
+// us at the end of a sweep, hidden only while blocks do not queue for CUs.
+// Step at 63k / 196k / 303k / 584k farfield cells, us: separate 78.7 / 135 /
+// 184 / 276, fused 63.0 / 133 / 190 / 295; mixed precision 67.3 / 109 / 145 /
+// 208 and 54.5 / 97 / 145 / 217.
+constexpr uint32_t FUSE_MAX_CELLS = 1024 * BLOCK;
+bool fused_ghosts(const nf_ctx *ctx) { return ctx->Ncell <= FUSE_MAX_CELLS; }
 
 // sweep A of the current primvars, or (U set, FP64) of prim(U) of that state.
 // dt: per-block CFL minima into dt_part; dtc: per-cell CFL steps into dt_cell
 // (local time stepping); aux: keep the gradient and limiter fields.
 int run_sweepA(nf_ctx *ctx, bool dt, bool aux, bool dtc = false, const double *U = nullptr) {
     int rc;
-    if (ctx->mixed) U = nullptr;
     if (!U && !ctx->mixed && (rc = refresh_v(ctx))) return rc;
-    if ((rc = run_ghost(ctx, false, U))) return rc;
+    // (a fused sweep B before it left the ghosts of the state it wrote)
+    if ((!U || ctx->gc_of != U) && (rc = run_ghost_cell(ctx, U))) return rc;
+    if (ctx->mixed) U = nullptr;
     const DevMesh m = devmesh(ctx);
     const int order = order_of(ctx);
+    const bool fuse = fused_ghosts(ctx);
     if (ctx->mixed) {
         const mx::SweepAArgsMx x{ctx->V32, ctx->Gc32, ctx->FV32, dt ? ctx->dt_part : nullptr,
                                  dtc ? ctx->dt_cell : nullptr, ctx->prm.CFL, ctx->xcd_remap,
-                                 aux ? ctx->grad_aux : nullptr, aux ? ctx->psi_aux : nullptr};
+                                 aux ? ctx->grad_aux : nullptr, aux ? ctx->psi_aux : nullptr,
+                                 bnd_args_mx(ctx, ctx->Gf32)};
         return launch_fn(ctx, order == 2 ? "sweepA_barth_mx" : "sweepA_mx", [&] {
-            return mx::launch_sweepA_mx(order, ctx->block, dim3(ctx->Ncell / ctx->block), ctx->stream, m, x);
+            return mx::launch_sweepA_mx(order, ctx->block, fuse, ctx->Ncell, ctx->stream, m, x);
         });
     }
     const SweepAArgs a{U ? U : ctx->V, ctx->Gc, ctx->FV, dt ? ctx->dt_part : nullptr, dtc ? ctx->dt_cell : nullptr,
-                       ctx->prm.CFL, ctx->xcd_remap, aux ? ctx->grad_aux : nullptr, aux ? ctx->psi_aux : nullptr};
+                       ctx->prm.CFL, ctx->xcd_remap, aux ? ctx->grad_aux : nullptr, aux ? ctx->psi_aux : nullptr,
+                       bnd_args(ctx, ctx->Gf)};
     const char *name = order == 2 ? "sweepA_barth" : (order == 1 ? "sweepA_nolim" : "sweepA_first");
     return launch_fn(ctx, name, [&] {
-        if (U)
-            return ctx->block == 128 ? launch_sweepA<128, true>(ctx->stream, ctx->Ncell, order, m, a)
-                                     : launch_sweepA<256, true>(ctx->stream, ctx->Ncell, order, m, a);
-        return ctx->block == 128 ? launch_sweepA<128, false>(ctx->stream, ctx->Ncell, order, m, a)
-                                 : launch_sweepA<256, false>(ctx->stream, ctx->Ncell, order, m, a);
+        auto go = [&](auto from_u, auto fused) {
+            return ctx->block == 128
+                       ? launch_sweepA<128, from_u(), fused()>(ctx->stream, ctx->Ncell, order, m, a)
+                       : launch_sweepA<256, from_u(), fused()>(ctx->stream, ctx->Ncell, order, m, a);
+        };
+        if (U) return fuse ? go(std::true_type{}, std::true_type{}) : go(std::true_type{}, std::false_type{});
+        return fuse ? go(std::false_type{}, std::true_type{}) : go(std::false_type{}, std::false_type{});
     });
 }
 
@@ -464,18 +525,20 @@ int run_sweepA(nf_ctx *ctx, bool dt, bool aux, bool dtc = false, const double *U
 // untouched, as the reference throws before the update).
 int run_sweepB(nf_ctx *ctx, int kind, const double *U, double *Uout, bool res, bool aux) {
     int rc;
-    if ((rc = run_ghost(ctx, true))) return rc;
+    const bool fuse = fused_ghosts(ctx);
+    if (!fuse && (rc = run_ghost_face(ctx))) return rc;
     const DevMesh m = devmesh(ctx);
     const double *dtc = ctx->prm.local_time_step ? ctx->dt_cell : nullptr;
     const bool checked = ctx->prm.check_physical_validity && !aux;
     double *Rst = checked ? ctx->Rst : nullptr, *fst = checked ? ctx->fst : nullptr;
+    if (!aux) ctx->gc_of = fuse && !checked ? Uout : nullptr;
     const ApplyArgs ap{U, ctx->Ua, Uout, ctx->mixed ? (void *)ctx->V32 : nullptr, Rst, fst, kind};
     if (ctx->mixed) {
         const mx::SweepBArgsMx x{ctx->FV32, ctx->Gf32, U, ctx->Ua, Uout, ctx->V32, dtc, kind,
                                  res ? ctx->res_part : nullptr, ctx->prm.check_physical_validity,
-                                 ctx->xcd_remap, aux ? ctx->R_aux : nullptr, Rst, fst};
+                                 ctx->xcd_remap, aux ? ctx->R_aux : nullptr, Rst, fst, bnd_args_mx(ctx, ctx->Gc32)};
         if ((rc = launch_fn(ctx, "sweepB_mx", [&] {
-                 return mx::launch_sweepB_mx(ctx->block, dim3(ctx->Ncell / ctx->block), ctx->stream, m, x);
+                 return mx::launch_sweepB_mx(ctx->block, fuse, ctx->Ncell, ctx->stream, m, x);
              })))
             return rc;
         if (!checked) return NF_OK;
@@ -483,48 +546,39 @@ int run_sweepB(nf_ctx *ctx, int kind, const double *U, double *Uout, bool res, b
                          [&] { return mx::launch_apply_mx(dim3(ctx->Ncell / BLOCK), ctx->stream, m, ap); });
     }
     // (FP64: prim(Uout) is not stored; the next sweep A evaluates it from U)
-    const SweepBArgs a{ctx->FV, ctx->Gf, U, ctx->Ua, Uout, nullptr, dtc, kind, res ? ctx->res_part : nullptr,
-                       ctx->prm.check_physical_validity, ctx->xcd_remap, aux ? ctx->R_aux : nullptr, Rst, fst};
+    const SweepBArgs a{ctx->FV, ctx->Gf, U, ctx->Ua, Uout, dtc, kind, res ? ctx->res_part : nullptr,
+                       ctx->prm.check_physical_validity, ctx->xcd_remap, aux ? ctx->R_aux : nullptr, Rst, fst,
+                       bnd_args(ctx, ctx->Gc)};
     const bool hllc = ctx->prm.inv_flux_scheme == NF_FLUX_HLLC;
     if ((rc = launch_fn(ctx, "sweepB", [&] {
-             const dim3 g(ctx->Ncell / ctx->block), b(ctx->block);
-             if (ctx->block == 128 && hllc) hipLaunchKernelGGL((k_sweepB<128, 1>), g, b, 0, ctx->stream, m, a);
-             else if (ctx->block == 128) hipLaunchKernelGGL((k_sweepB<128, 0>), g, b, 0, ctx->stream, m, a);
-             else if (hllc) hipLaunchKernelGGL((k_sweepB<256, 1>), g, b, 0, ctx->stream, m, a);
-             else hipLaunchKernelGGL((k_sweepB<256, 0>), g, b, 0, ctx->stream, m, a);
-             return hipGetLastError();
+             auto go = [&](auto fused) {
+                 return ctx->block == 128 ? launch_sweepB<128, fused()>(ctx->stream, ctx->Ncell, hllc, m, a)
+                                          : launch_sweepB<256, fused()>(ctx->stream, ctx->Ncell, hllc, m, a);
+             };
+             return fuse ? go(std::true_type{}) : go(std::false_type{});
          })))
         return rc;
     if (!checked) return NF_OK;
     return LAUNCH("apply", k_apply, dim3(ctx->Ncell / BLOCK), dim3(BLOCK), m, ap);
 }
 
-int reduce_dt(nf_ctx *ctx, int advance) {
-    int rc;
+// reductions of the last sweeps' partials: res (into the histories, or out)
+// and dt (advance: at the end of a step)
+int reduce(nf_ctx *ctx, bool res, double drop, double *out, bool dt, int advance) {
     const RedTable &r = red(ctx);
-    if ((rc = LAUNCH("reduce_dt", k_reduce<true>, dim3(r.nchunk), dim3(BLOCK), (const double *)ctx->dt_part,
-                     (const uint32_t *)r.first, (const uint32_t *)r.n, ctx->red_dt)))
-        return rc;
-    return LAUNCH("finalize_dt", k_finalize_dt, dim3(ctx->n_inst), dim3(BLOCK), (const double *)ctx->red_dt,
-                  (const uint32_t *)r.inst_c0, (const uint32_t *)r.inst_nc, ctx->st, advance);
-}
-
-int reduce_res(nf_ctx *ctx, double drop, double *out = nullptr) {
+    const RedArgs a{dt ? ctx->dt_part : nullptr, res ? ctx->res_part : nullptr, r.first, r.n, r.inst_c0, r.inst_nc,
+                    ctx->red_dt, ctx->red_res, ctx->st, advance, ctx->hist, ctx->hist_cap, drop, out};
+    if (r.nchunk == ctx->n_inst) return LAUNCH("reduce", k_finish<true>, dim3(ctx->n_inst), dim3(BLOCK), a);
     int rc;
-    const RedTable &r = red(ctx);
-    if ((rc = LAUNCH("reduce_res", k_reduce<false>, dim3(r.nchunk), dim3(BLOCK), (const double *)ctx->res_part,
-                     (const uint32_t *)r.first, (const uint32_t *)r.n, ctx->red_res)))
-        return rc;
-    return LAUNCH("finalize_res", k_finalize_res, dim3(ctx->n_inst), dim3(BLOCK), (const double *)ctx->red_res,
-                  (const uint32_t *)r.inst_c0, (const uint32_t *)r.inst_nc, ctx->st, ctx->hist, ctx->hist_cap,
-                  drop, out);
+    if ((rc = LAUNCH("reduce_chunks", k_reduce, dim3(r.nchunk), dim3(BLOCK), a))) return rc;
+    return LAUNCH("reduce", k_finish<false>, dim3(ctx->n_inst), dim3(BLOCK), a);
 }
 
 // One step of every live instance (Solver::step, src/Solver.cpp:34-52).  The
 // last sweep A of the step evaluates the CFL dt of the primvars it reads --
 // prim(U2) for TVD-RK3, prim(U^n) for explicit Euler -- which is the state
 // the reference's next calc_timestep sees (src/Solver.cpp:248);
-// k_finalize_dt installs that dt for the following step.  U^n (= U_old after
+// k_finish installs that dt for the following step.  U^n (= U_old after
 // the first step) stays in Ua; stages write Ub, the last stage writes Ua.
 int enqueue_step(nf_ctx *ctx, double drop) {
     int rc;
@@ -533,7 +587,9 @@ int enqueue_step(nf_ctx *ctx, double drop) {
     // each stage's sweep A evaluates the primvars of its input state
     if ((rc = run_sweepA(ctx, !rk3 || lts, false, lts, ctx->Ua))) return rc;
     if ((rc = run_sweepB(ctx, 1, ctx->Ua, rk3 ? ctx->Ub : ctx->Ua, true, false))) return rc;
-    if ((rc = reduce_res(ctx, drop))) return rc;
+    // a checked instance can stop in a later stage, its residual counts
+    const bool early = ctx->prm.check_physical_validity;
+    if (early && (rc = reduce(ctx, true, drop, nullptr, false, 0))) return rc;
     if (rk3) {
         if ((rc = run_sweepA(ctx, false, false, false, ctx->Ub))) return rc;
         if ((rc = run_sweepB(ctx, 2, ctx->Ub, ctx->Ub, false, false))) return rc;
@@ -542,14 +598,14 @@ int enqueue_step(nf_ctx *ctx, double drop) {
     }
     if (!ctx->mixed)
         for (Inst &I : ctx->inst) I.v_stale = true;
-    return reduce_dt(ctx, 1);
+    return reduce(ctx, !early, drop, nullptr, true, 1);
 }
 
 // dt of the current primvars with a standalone sweep A
 int enqueue_timestep(nf_ctx *ctx) {
     int rc;
     if ((rc = run_sweepA(ctx, true, false))) return rc;
-    return reduce_dt(ctx, 0);
+    return reduce(ctx, false, 0.0, nullptr, true, 0);
 }
 
 int clear_flags(nf_ctx *ctx, bool keep_converged = false) {
@@ -698,6 +754,7 @@ int after_state_set(nf_ctx *ctx, int i, bool uold_zero) {
     I.dt_valid = false;
     I.warm = false;
     I.v_stale = false;
+    ctx->gc_of = nullptr;
     ctx->aux_valid = false;
     return NF_OK;
 }
@@ -723,7 +780,7 @@ int eval_residuals(nf_ctx *ctx, double *out) {
     if ((rc = prim_all(ctx))) return rc;
     if ((rc = run_sweepA(ctx, false, false))) return rc;
     if ((rc = run_sweepB(ctx, 1, ctx->Ua, ctx->Ub, true, false))) return rc;
-    if ((rc = reduce_res(ctx, 0.0, ctx->r_eval))) return rc;
+    if ((rc = reduce(ctx, true, 0.0, ctx->r_eval, false, 0))) return rc;
     if ((rc = prim_all(ctx))) return rc;
     HIPC(hipStreamSynchronize(ctx->stream));
     HIPC(hipMemcpy(out, ctx->r_eval, ctx->n_inst * sizeof(double), hipMemcpyDeviceToHost));
@@ -1013,6 +1070,9 @@ int create(int32_t n, const nf_mesh_desc *descs, const nf_params *prms, nf_ctx *
         node0 += d->n_nodes;
     }
     if (bface.size() > NBR_INDEX_MASK) return NF_E_ARG;
+    std::vector<uint32_t> boff(cell0 / 128 + 1, 0);
+    for (uint32_t w : bface) boff[(w & NBR_INDEX_MASK) / 128 + 1]++;
+    for (size_t q = 1; q < boff.size(); ++q) boff[q] += boff[q - 1];
     // node tables of the 64-cell groups (one per wave; instances are padded
     // to 256 cells): distinct nodes in first-use order
     std::vector<uint32_t> grp_off(1, 0);
@@ -1077,6 +1137,8 @@ int create(int32_t n, const nf_mesh_desc *descs, const nf_params *prms, nf_ctx *
         if ((rc = dalloc(ctx, &ctx->fst, NC))) return rc;
     }
     if ((rc = dalloc(ctx, &ctx->bface, ctx->nbf))) return rc;
+    if ((rc = dalloc(ctx, &ctx->boff, boff.size()))) return rc;
+    HIPC(hipMemcpy(ctx->boff, boff.data(), boff.size() * 4, hipMemcpyHostToDevice));
     if ((rc = dalloc(ctx, &ctx->bbc, ctx->nbf))) return rc;
     if ((rc = dalloc(ctx, &ctx->bS, 3 * (size_t)ctx->nbf))) return rc;
     if ((rc = dalloc(ctx, &ctx->binst, ctx->nbf))) return rc;
@@ -1194,6 +1256,10 @@ int run_loop(nf_ctx *ctx, const nf_run_opts *o, nf_run_stats *stats) {
     while (done < o->n_steps && !stopped) {
         const int chunk = std::min(K, o->n_steps - done);
         if (o->use_graph && chunk == K) {
+            // fused: a graph starts from the cell ghosts of Ua in place, whatever
+            // was the case when it was captured, and leaves gc_of as a step does
+            if (!fused_ghosts(ctx)) ctx->gc_of = nullptr;
+            else if (ctx->gc_of != ctx->Ua && (rc = run_ghost_cell(ctx, ctx->Ua))) return rc;
             if (!ctx->graph || ctx->graph_steps != K || ctx->graph_drop != drop || ctx->graph_block != ctx->block ||
                 ctx->graph_xcd != ctx->xcd_remap) {
                 if (ctx->graph) (void)hipGraphExecDestroy(ctx->graph);
@@ -1203,6 +1269,7 @@ int run_loop(nf_ctx *ctx, const nf_run_opts *o, nf_run_stats *stats) {
                 for (int s = 0; s < K; ++s)
                     if ((rc = enqueue_step(ctx, drop))) {
                         (void)hipStreamEndCapture(ctx->stream, &gr);
+                        ctx->gc_of = nullptr;
                         return rc;
                     }
                 HIPC(hipStreamEndCapture(ctx->stream, &gr));
@@ -1214,6 +1281,7 @@ int run_loop(nf_ctx *ctx, const nf_run_opts *o, nf_run_stats *stats) {
                 ctx->graph_xcd = ctx->xcd_remap;
             }
             HIPC(hipGraphLaunch(ctx->graph, ctx->stream));
+            ctx->gc_of = fused_ghosts(ctx) && !ctx->prm.check_physical_validity ? ctx->Ua : nullptr;
             if (!ctx->mixed)  // (the capture marked them once; a replay steps again)
                 for (Inst &I : ctx->inst) I.v_stale = true;
         } else {
@@ -1328,6 +1396,7 @@ int restore(nf_ctx *ctx, const Snapshot &s) {
         ctx->inst[i].dt_valid = s.dt_valid[i];
         ctx->inst[i].v_stale = s.v_stale[i];
     }
+    ctx->gc_of = nullptr;
     ctx->aux_valid = false;
     return NF_OK;
 }
@@ -1628,6 +1697,7 @@ int nf_set_precision(nf_ctx *ctx, int32_t precision) {
     HIPC(hipStreamSynchronize(ctx->stream));
     ctx->mixed = mixed;
     ctx->prm.precision = precision;
+    ctx->gc_of = nullptr;
     if (ctx->graph) {  // captured with the other precision's kernels and buffers
         (void)hipGraphExecDestroy(ctx->graph);
         ctx->graph = nullptr;

@@ -8,29 +8,38 @@
 namespace nf {
 namespace mx {
 
-hipError_t launch_ghost_mx(bool face, dim3 g, hipStream_t st, const DevMesh &m, const GhostArgsMx &a) {
-    if (face) hipLaunchKernelGGL(k_ghost_mx<true>, g, dim3(BLOCK), 0, st, m, a);
-    else hipLaunchKernelGGL(k_ghost_mx<false>, g, dim3(BLOCK), 0, st, m, a);
+hipError_t launch_ghost_mx(bool face, hipStream_t st, const DevMesh &m, const BndArgsMx &a, const float *src) {
+    const dim3 g((a.nb + BLOCK - 1) / BLOCK), b(BLOCK);
+    if (face) hipLaunchKernelGGL(k_ghost_mx<true>, g, b, 0, st, m, a, src);
+    else hipLaunchKernelGGL(k_ghost_mx<false>, g, b, 0, st, m, a, src);
     return hipGetLastError();
 }
 
-template <int B>
-static void sweepA_b(int order, dim3 g, hipStream_t st, const DevMesh &m, const SweepAArgsMx &a) {
-    if (order == 0) hipLaunchKernelGGL((k_sweepA_mx<0, B>), g, dim3(B), 0, st, m, a);
-    else if (order == 1) hipLaunchKernelGGL((k_sweepA_mx<1, B>), g, dim3(B), 0, st, m, a);
-    else hipLaunchKernelGGL((k_sweepA_mx<2, B>), g, dim3(B), 0, st, m, a);
+template <int B, bool FUSE>
+static hipError_t sweepA_b(int order, uint32_t ncell, hipStream_t st, const DevMesh &m, const SweepAArgsMx &a) {
+    const dim3 g(ncell / B), b(B);
+    if (order == 0) hipLaunchKernelGGL((k_sweepA_mx<0, B, FUSE>), g, b, 0, st, m, a);
+    else if (order == 1) hipLaunchKernelGGL((k_sweepA_mx<1, B, FUSE>), g, b, 0, st, m, a);
+    else hipLaunchKernelGGL((k_sweepA_mx<2, B, FUSE>), g, b, 0, st, m, a);
+    return hipGetLastError();
 }
-
-hipError_t launch_sweepA_mx(int order, int block, dim3 g, hipStream_t st, const DevMesh &m, const SweepAArgsMx &a) {
-    if (block == 128) sweepA_b<128>(order, g, st, m, a);
-    else sweepA_b<256>(order, g, st, m, a);
+template <int B, bool FUSE>
+static hipError_t sweepB_b(uint32_t ncell, hipStream_t st, const DevMesh &m, const SweepBArgsMx &a) {
+    hipLaunchKernelGGL((k_sweepB_mx<B, FUSE>), dim3(ncell / B), dim3(B), 0, st, m, a);
     return hipGetLastError();
 }
 
-hipError_t launch_sweepB_mx(int block, dim3 g, hipStream_t st, const DevMesh &m, const SweepBArgsMx &a) {
-    if (block == 128) hipLaunchKernelGGL(k_sweepB_mx<128>, g, dim3(128), 0, st, m, a);
-    else hipLaunchKernelGGL(k_sweepB_mx<256>, g, dim3(256), 0, st, m, a);
-    return hipGetLastError();
+hipError_t launch_sweepA_mx(int order, int block, bool fuse, uint32_t ncell, hipStream_t st, const DevMesh &m,
+                            const SweepAArgsMx &a) {
+    if (block == 128)
+        return fuse ? sweepA_b<128, true>(order, ncell, st, m, a) : sweepA_b<128, false>(order, ncell, st, m, a);
+    return fuse ? sweepA_b<256, true>(order, ncell, st, m, a) : sweepA_b<256, false>(order, ncell, st, m, a);
+}
+
+hipError_t launch_sweepB_mx(int block, bool fuse, uint32_t ncell, hipStream_t st, const DevMesh &m,
+                            const SweepBArgsMx &a) {
+    if (block == 128) return fuse ? sweepB_b<128, true>(ncell, st, m, a) : sweepB_b<128, false>(ncell, st, m, a);
+    return fuse ? sweepB_b<256, true>(ncell, st, m, a) : sweepB_b<256, false>(ncell, st, m, a);
 }
 
 hipError_t launch_prim_mx(dim3 g, hipStream_t st, const double *U, float *V, uint32_t N) {
