@@ -4,12 +4,15 @@
 // centroid x, y, z, wall distance); outputs are the primitive variables,
 // both normalised per component.
 //
-// All products -- forward Z = W X, backward dX = W^T dZ and dW = dZ X^T --
-// go through one BF16 MFMA GEMM kernel (v_mfma_f32_16x16x32_bf16) with
-// arbitrary operand strides, so the transposed operands of the backward pass
-// need no copies.  Activations are feature-major ([feature][sample]) so the
-// sample dimension is the contiguous one.  Weight gradients reduce over the
-// batch with a fixed split-K partition and a fixed-order sum (deterministic).
+// All products run on BF16 MFMA (v_mfma_f32_16x16x32_bf16).  Inference is one
+// kernel; a training step is three: the minibatch through the network and
+// back (k_train), the weight gradients dW = dZ X^T over the batch with the
+// bias and loss sums (k_wgrad), and the sum over batch splits with Adam
+// (k_update).  Activations go between them as [16-sample tile][feature][16]:
+// a block of k_train writes whole lines, and k_wgrad's operand fragments are
+// 16-byte loads of adjacent rows.  Weight gradients
+// reduce over the batch with a fixed split-K partition and a fixed-order sum
+// (deterministic).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -43,221 +46,17 @@ constexpr int64_t OFF_W3 = OFF_B2 + HID, OFF_B3 = OFF_W3 + HID * HID;
 constexpr int64_t OFF_W4 = OFF_B3 + HID, OFF_B4 = OFF_W4 + OUT * HID;
 constexpr int64_t NPARAM = OFF_B4 + OUT;
 
-// ---------------------------------------------------------------------------
-// GEMM  C(m, n) = sum_k A(m, k) B(k, n),  A(m,k) = A[m*sam + k*sak],
-// B(k,n) = B[k*sbk + n*sbn], C(m,n) = C[z*sc_split + m*scm + n*scn], where
-// blockIdx.z selects the K range [z*ksplit, (z+1)*ksplit).
-// Tile 64x64 per 256-thread block, K step 64; each wave computes 32x32 as
-// 2x2 MFMA 16x16x32 tiles.  Operand tiles are staged in LDS as [row][k]
-// (k contiguous) so each lane's MFMA fragment -- 8 consecutive k of one row
-// -- is a single 16-byte LDS read.
-constexpr int TM = 64, TN = 64, TK = 64, LDK = TK + 8;
-
-struct Gemm {
-    const __bf16 *A;
-    int64_t sam, sak;
-    const __bf16 *B;
-    int64_t sbk, sbn;
-    float *C;
-    int64_t scm, scn, sc_split;
-    int M, N, K, ksplit;
-};
-
-// tile S[r][k] = P[(r0 + r)*s_row + (k0 + k)*s_k] for r < 64, k < TK, zero
-// outside r0 + r < R, k0 + k < kend
-__device__ __forceinline__ void load_tile(const __bf16 *P, int64_t s_row, int64_t s_k, int r0, int k0, int R,
-                                          int kend, __bf16 (*S)[LDK]) {
-    const int t = threadIdx.x;
-    const bool aligned = (((uintptr_t)P) & 15) == 0;
-    const bool vec = s_k == 1 && (s_row & 7) == 0 && aligned;
-    const bool vec_rows = !vec && s_row == 1 && (s_k & 7) == 0 && aligned;
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        if (vec_rows) {
-            // rows contiguous: 16-byte loads of 8 rows at one k (a wave reads
-            // 128 contiguous bytes per k), transposed into the [row][k] tile
-            const int rr = (t & 7) * 8, kk = (t >> 3) + 32 * h;
-            const int gr = r0 + rr, gk = k0 + kk;
-            bf16x8 v;
-            if (gk < kend && gr + 8 <= R) {
-                v = *reinterpret_cast<const bf16x8 *>(P + gr + gk * s_k);
-            } else {
-#pragma unroll
-                for (int e = 0; e < 8; ++e) v[e] = (gk < kend && gr + e < R) ? P[(gr + e) + gk * s_k] : (__bf16)0.0f;
-            }
-#pragma unroll
-            for (int e = 0; e < 8; ++e) S[rr + e][kk] = v[e];
-        } else if (vec) {
-            // thread -> (row, 8 consecutive k): 16-byte loads along k
-            const int r = (t >> 3) + 32 * h, kk = (t & 7) * 8;
-            const int gr = r0 + r, gk = k0 + kk;
-            bf16x8 v;
-            if (gr < R && gk + 8 <= kend) {
-                v = *reinterpret_cast<const bf16x8 *>(P + gr * s_row + gk);
-            } else {
-#pragma unroll
-                for (int e = 0; e < 8; ++e)
-                    v[e] = (gr < R && gk + e < kend) ? P[gr * s_row + (gk + e)] : (__bf16)0.0f;
-            }
-            *reinterpret_cast<bf16x8 *>(&S[r][kk]) = v;
-        } else {
-            // thread -> (row, k block): consecutive threads take consecutive
-            // rows, which are contiguous when s_row == 1
-            const int r = t & 63, kk = (t >> 6) * 8 + 32 * h;
-            const int gr = r0 + r;
-            bf16x8 v;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const int gk = k0 + kk + e;
-                v[e] = (gr < R && gk < kend) ? P[gr * s_row + gk * s_k] : (__bf16)0.0f;
-            }
-            *reinterpret_cast<bf16x8 *>(&S[r][kk]) = v;
-        }
-    }
-}
-
-__global__ __launch_bounds__(256) void k_gemm(Gemm g) {
-    __shared__ __attribute__((aligned(16))) __bf16 As[TM][LDK];
-    __shared__ __attribute__((aligned(16))) __bf16 Bs[TN][LDK];
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-    const int wm = w >> 1, wn = w & 1;
-    const int m0 = blockIdx.y * TM, n0 = blockIdx.x * TN;
-    const int kb = blockIdx.z * g.ksplit, ke = min(g.K, kb + g.ksplit);
-    f32x4 acc[2][2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int k0 = kb; k0 < ke; k0 += TK) {
-        load_tile(g.A, g.sam, g.sak, m0, k0, g.M, ke, As);
-        load_tile(g.B, g.sbn, g.sbk, n0, k0, g.N, ke, Bs);
-        __syncthreads();
-#pragma unroll
-        for (int ks = 0; ks < TK; ks += 32) {
-            bf16x8 a[2], b[2];
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-                a[i] = *reinterpret_cast<const bf16x8 *>(&As[wm * 32 + i * 16 + (lane & 15)][ks + 8 * (lane >> 4)]);
-#pragma unroll
-            for (int j = 0; j < 2; ++j)
-                b[j] = *reinterpret_cast<const bf16x8 *>(&Bs[wn * 32 + j * 16 + (lane & 15)][ks + 8 * (lane >> 4)]);
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
-        }
-        __syncthreads();
-    }
-    // D fragment: lane holds rows 4*(lane/16) + r of column lane%16
-    float *C = g.C + blockIdx.z * g.sc_split;
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int m = m0 + wm * 32 + i * 16 + 4 * (lane >> 4) + r;
-                const int n = n0 + wn * 32 + j * 16 + (lane & 15);
-                if (m < g.M && n < g.N) C[m * g.scm + n * g.scn] = acc[i][j][r];
-            }
-}
-
-// ---------------------------------------------------------------------------
-// elementwise kernels over feature-major [rows][ld] arrays
 __device__ __forceinline__ float gelu(float x) { return 0.5f * x * (1.0f + erff(x * 0.70710678118654752f)); }
-__device__ __forceinline__ float gelu_d(float x) {
-    return 0.5f * (1.0f + erff(x * 0.70710678118654752f)) + x * 0.39894228040143268f * expf(-0.5f * x * x);
-}
-
-// Z += b (per row); A = bf16(gelu(Z))
-__global__ void k_bias_gelu(float *Z, const float *b, __bf16 *A, int rows, int n) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x, r = blockIdx.y;
-    if (j >= n || r >= rows) return;
-    const size_t i = (size_t)r * n + j;
-    const float z = Z[i] + b[r];
-    Z[i] = z;
-    A[i] = (__bf16)gelu(z);
-}
-
-// Y += b, D = Y - T, dY = 2 D / (OUT n) (FP32 and BF16), and per-block sums
-// of D^2 for the loss
-__global__ void k_out_loss(float *Y, const float *b, const float *T, float *dY, __bf16 *dYb, float *loss_part,
-                           int n, float inv_count) {
-    __shared__ float sh[4];
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    float s = 0.f;
-    if (j < n) {
-        for (int o = 0; o < OUT; ++o) {
-            const size_t i = (size_t)o * n + j;
-            const float y = Y[i] + b[o];
-            Y[i] = y;
-            const float d = y - T[i];
-            s += d * d;
-            const float g = 2.0f * d * inv_count;
-            dY[i] = g;
-            dYb[i] = (__bf16)g;
-        }
-    }
-    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
-    __syncthreads();
-    if (threadIdx.x == 0) loss_part[blockIdx.x] = (sh[0] + sh[1]) + (sh[2] + sh[3]);
-}
-
-// dZ = dA * gelu'(Z), FP32 (bias gradient) and BF16 (next product)
-__global__ void k_gelu_back(float *dA, const float *Z, __bf16 *dZb, int rows, int n) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x, r = blockIdx.y;
-    if (j >= n || r >= rows) return;
-    const size_t i = (size_t)r * n + j;
-    const float d = dA[i] * gelu_d(Z[i]);
-    dA[i] = d;
-    dZb[i] = (__bf16)d;
-}
-
-// out[r] = sum_j X[r][j] in a fixed order (one block per row)
-__global__ __launch_bounds__(256) void k_rowsum(const float *X, int n, float *out) {
-    __shared__ float sh[4];
-    const int r = blockIdx.x;
-    float s = 0.f;
-    for (int j = threadIdx.x; j < n; j += 256) s += X[(size_t)r * n + j];
-    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
-    __syncthreads();
-    if (threadIdx.x == 0) out[r] = (sh[0] + sh[1]) + (sh[2] + sh[3]);
-}
-
-// out[i] = sum over splits s (in order) of part[s*stride + i]
-__global__ void k_sum_splits(const float *part, int splits, int64_t stride, int64_t n, float *out) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    float s = 0.f;
-    for (int q = 0; q < splits; ++q) s += part[q * stride + i];
-    out[i] = s;
-}
-
-// raw feature-major inputs -> normalised BF16 operand, and targets alongside;
-// idx (optional) picks the samples of a minibatch
-__global__ void k_gather(const float *x, const float *y, int64_t n_all, const int64_t *idx, int64_t first, int n,
-                         const float *in_shift, const float *in_scale, const float *out_shift,
-                         const float *out_iscale, __bf16 *X0, float *T) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= n) return;
-    const int64_t s = idx ? idx[first + j] : first + j;
-    for (int f = 0; f < IN; ++f) X0[(size_t)f * n + j] = (__bf16)((x[f * n_all + s] - in_shift[f]) * in_scale[f]);
-    for (int o = 0; o < OUT; ++o) T[(size_t)o * n + j] = (y[o * n_all + s] - out_shift[o]) * out_iscale[o];
-}
 
 // ---------------------------------------------------------------------------
-// Fused network: one block of four waves takes NC x 16 samples through every
-// layer, so activations never leave the CU.  Wave w computes features
-// [32w, 32w + 32) of each hidden layer (two MFMA row tiles), keeps those rows
-// of all weights in registers as MFMA operands for as long as it lives (the
-// grid is persistent), and hands its activations to the other waves through
-// LDS as [sample][feature] BF16, so that a lane's operand fragment of the
-// next layer -- 8 consecutive features of one sample -- is one 16-byte read.
-// Every product is accumulated over k in the same steps of 32 as k_gemm's, so
-// outputs have the layer-by-layer kernels' bits.
+// Fused network: one block takes NC x 16 samples through every layer, so
+// activations never leave the CU.  Each of its 8 / RT waves computes RT MFMA
+// row tiles (16 RT features) of each hidden layer, keeps those rows of all
+// weights in registers as MFMA operands for as long as it lives (the grid is
+// persistent), and hands its activations to the other waves through LDS as
+// [sample][feature] BF16, so that a lane's operand fragment of the next layer
+// -- 8 consecutive features of one sample -- is one 16-byte read.  Every
+// product is accumulated over k in steps of 32 in increasing order.
 constexpr int LDH = HID + 8;  // row stride of the LDS activations: 16-byte aligned, 16 columns over all banks
 
 // MFMA operand fragment of row r (R real rows), columns [k, k + 8) of a
@@ -292,18 +91,18 @@ struct Infer {
 // instructions each), not by the products or by memory.  Layer by layer (11
 // launches, 3.6 KB per sample through HBM) 700 samples took 38 us and
 // 1,463,340 samples 2.4 ms; one launch that moves 44 bytes per sample takes
-// 6.5 us and 0.44 ms.
-template <int NC>
-__global__ __launch_bounds__(256) void k_infer(Infer g) {
+// 6.0 us and 0.44 ms.
+template <int NC, int RT>
+__global__ __launch_bounds__(512 / RT) void k_infer(Infer g) {
     __shared__ __attribute__((aligned(16))) __bf16 H[2][NC * 16][LDH];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, col = lane & 15, q4 = lane >> 4;
     const int64_t ntiles = (g.n + NC * 16 - 1) / (NC * 16);
-    bf16x8 a1[2], a2[2][4], a3[2][4], a4[4];
-    f32x4 b1[2], b2[2], b3[2];
+    bf16x8 a1[RT], a2[RT][4], a3[RT][4], a4[4];
+    f32x4 b1[RT], b2[RT], b3[RT];
     float b4[4], osh[4], osc[4];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int r = 32 * w + 16 * i;
+    for (int i = 0; i < RT; ++i) {
+        const int r = 16 * (RT * w + i);
         a1[i] = in_frag(g.pb + OFF_W1, r + col, 8 * q4);
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
@@ -326,25 +125,26 @@ __global__ __launch_bounds__(256) void k_infer(Infer g) {
     // activations of one product, [2 row tiles][NC sample tiles], to LDS
     auto store = [&](const f32x4 (*acc)[NC], const f32x4 *b, __bf16 (*S)[LDH]) {
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < RT; ++i)
 #pragma unroll
             for (int c = 0; c < NC; ++c) {
                 bf16x4 h;
 #pragma unroll
                 for (int r = 0; r < 4; ++r) h[r] = (__bf16)gelu(acc[i][c][r] + b[i][r]);
-                *reinterpret_cast<bf16x4 *>(&S[c * 16 + col][32 * w + 16 * i + 4 * q4]) = h;
+                *reinterpret_cast<bf16x4 *>(&S[c * 16 + col][16 * (RT * w + i) + 4 * q4]) = h;
             }
     };
     auto layer = [&](const bf16x8 (*a)[4], const f32x4 *b, const __bf16 (*S)[LDH], __bf16 (*D)[LDH]) {
-        f32x4 acc[2][NC];
+        f32x4 acc[RT][NC];
 #pragma unroll
         for (int c = 0; c < NC; ++c) {
-            acc[0][c] = acc[1][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int i = 0; i < RT; ++i) acc[i][c] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const bf16x8 h = *reinterpret_cast<const bf16x8 *>(&S[c * 16 + col][32 * q + 8 * q4]);
 #pragma unroll
-                for (int i = 0; i < 2; ++i)
+                for (int i = 0; i < RT; ++i)
                     acc[i][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i][q], h, acc[i][c], 0, 0, 0);
             }
         }
@@ -353,7 +153,7 @@ __global__ __launch_bounds__(256) void k_infer(Infer g) {
     int p = 0;  // the buffer the input layer writes; it was last read two barriers ago
     for (int64_t t = blockIdx.x; t < ntiles; t += gridDim.x, p ^= 1) {
         const int64_t j0 = t * (NC * 16);
-        f32x4 acc[2][NC];
+        f32x4 acc[RT][NC];
 #pragma unroll
         for (int c = 0; c < NC; ++c) {
             // padding samples repeat the last one and are not stored
@@ -365,7 +165,7 @@ __global__ __launch_bounds__(256) void k_infer(Infer g) {
                                                     g.norm[6 + (e < IN ? e : 0)])
                                          : (__bf16)0.0f;
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
+            for (int i = 0; i < RT; ++i)
                 acc[i][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1[i], v, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
         }
         store(acc, b1, H[p]);
@@ -374,7 +174,7 @@ __global__ __launch_bounds__(256) void k_infer(Infer g) {
         __syncthreads();
         layer(a3, b3, H[p ^ 1], H[p]);
         __syncthreads();
-        for (int c = w; c < NC; c += 4) {
+        for (int c = w; c < NC; c += 8 / RT) {
             f32x4 y = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int q = 0; q < 4; ++q)
@@ -388,24 +188,315 @@ __global__ __launch_bounds__(256) void k_infer(Infer g) {
     }
 }
 
-// Adam step on the FP32 masters (bias-corrected step size lr_t), BF16 copy
-__global__ void k_adam(float *p, const float *g, float *m, float *v, __bf16 *pb, int64_t n, float lr_t, float b1,
-                       float b2, float eps) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float gi = g[i];
-    const float mi = b1 * m[i] + (1.f - b1) * gi;
-    const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
-    m[i] = mi;
-    v[i] = vi;
-    const float pi = p[i] - lr_t * mi / (sqrtf(vi) + eps);
-    p[i] = pi;
-    pb[i] = (__bf16)pi;
+// ---------------------------------------------------------------------------
+// Training.  Transposed BF16 weights for the backward products (rows are the
+// layer's inputs): W2^T, W3^T [HID][HID], W4^T [HID][8], its columns OUT.. zero
+constexpr int64_t PT2 = 0, PT3 = PT2 + HID * HID, PT4 = PT3 + HID * HID, NPT = PT4 + HID * 8;
+
+__device__ __forceinline__ size_t tix(int tile, int rows, int r, int col) { return ((size_t)tile * rows + r) * 16 + col; }
+
+struct Train {
+    const __bf16 *pb, *pt;  // BF16 parameters and their transposes
+    const float *p;         // FP32 parameters (biases)
+    const float *norm;      // in_shift[6], in_scale[6], out_shift[5], out_scale[5], out_iscale[5]
+    const float *x, *y;     // raw samples [.][IN], targets [.][OUT]
+    const int64_t *idx;     // minibatch: sample idx[first + j], or null: first + j
+    int64_t first;
+    int n, ld;              // samples, and rounded up to 64: samples n.. are stored as zeros
+    float inv_count;
+    __bf16 *X0, *A[3], *dZb[3], *dYb;  // [ld / 16][rows][16]
+    float *dZ[3], *dY;                 // the same, for the bias sums
+    float *se;                         // [ld] squared error of each sample
+};
+
+// The samples of a minibatch through the network and back, 16 per block tile,
+// organised as k_infer; GELU and its derivative share one erf, and the
+// pre-activations stay in registers.  Bound by the erf and exp of 3 x 128
+// activations per sample in the few waves a minibatch has (2,048 samples:
+// 128 blocks), not by the products.  A step of 2,048 samples took 33 launches
+// and 157 us when every product, activation and sum was one; it takes 29 us
+// (k_train 15, k_wgrad 6, k_update 3.6): eight waves of one row tile each
+// (four of two: 34 us with [row][sample] activations, eight 31 us), the
+// activations in 16-sample tiles (29 us).
+__global__ __launch_bounds__(512) void k_train(Train g) {
+    constexpr int RT = 1;  // row tiles per wave
+    __shared__ __attribute__((aligned(16))) __bf16 H[2][16][LDH];
+    __shared__ __attribute__((aligned(16))) __bf16 D[16][8];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, col = lane & 15, q4 = lane >> 4;
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    bf16x8 none;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) none[e] = (__bf16)0.0f;
+    bf16x8 a1[RT], a2[RT][4], a3[RT][4], a4[4], t2[RT][4], t3[RT][4], t4[RT];
+    f32x4 b1[RT], b2[RT], b3[RT];
+#pragma unroll
+    for (int i = 0; i < RT; ++i) {
+        const int r = 16 * (RT * w + i);
+        a1[i] = in_frag(g.pb + OFF_W1, r + col, 8 * q4);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            a2[i][q] = row_frag(g.pb + OFF_W2, r + col, 32 * q + 8 * q4, HID);
+            a3[i][q] = row_frag(g.pb + OFF_W3, r + col, 32 * q + 8 * q4, HID);
+            t2[i][q] = row_frag(g.pt + PT2, r + col, 32 * q + 8 * q4, HID);
+            t3[i][q] = row_frag(g.pt + PT3, r + col, 32 * q + 8 * q4, HID);
+        }
+        t4[i] = q4 == 0 ? *reinterpret_cast<const bf16x8 *>(g.pt + PT4 + (r + col) * 8) : none;
+        b1[i] = *reinterpret_cast<const f32x4 *>(g.p + OFF_B1 + r + 4 * q4);
+        b2[i] = *reinterpret_cast<const f32x4 *>(g.p + OFF_B2 + r + 4 * q4);
+        b3[i] = *reinterpret_cast<const f32x4 *>(g.p + OFF_B3 + r + 4 * q4);
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) a4[q] = row_frag(g.pb + OFF_W4, col, 32 * q + 8 * q4, OUT);
+    int p = 0;
+    for (int t = blockIdx.x; t < g.ld / 16; t += gridDim.x, p ^= 1) {
+        const int j = t * 16 + col;
+        const bool live = j < g.n;
+        const int64_t src = g.idx ? g.idx[g.first + (live ? j : g.n - 1)] : g.first + (live ? j : g.n - 1);
+        f32x4 gd[3][RT];  // gelu' of the three layers
+        auto product = [&](const bf16x8 (*a)[4], const __bf16 (*S)[LDH], f32x4 *acc) {
+#pragma unroll
+            for (int i = 0; i < RT; ++i) acc[i] = zero;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const bf16x8 h = *reinterpret_cast<const bf16x8 *>(&S[col][32 * q + 8 * q4]);
+#pragma unroll
+                for (int i = 0; i < RT; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i][q], h, acc[i], 0, 0, 0);
+            }
+        };
+        auto activate = [&](int l, const f32x4 *acc, const f32x4 *b, __bf16 (*S)[LDH]) {
+#pragma unroll
+            for (int i = 0; i < RT; ++i) {
+                const int f = 16 * (RT * w + i) + 4 * q4;
+                bf16x4 h;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float z = acc[i][r] + b[i][r];
+                    const float e = 1.0f + erff(z * 0.70710678118654752f);
+                    h[r] = (__bf16)(0.5f * z * e);
+                    gd[l][i][r] = 0.5f * e + z * 0.39894228040143268f * expf(-0.5f * z * z);
+                    g.A[l][tix(t, HID, f + r, col)] = live ? h[r] : (__bf16)0.0f;
+                }
+                *reinterpret_cast<bf16x4 *>(&S[col][f]) = h;
+            }
+        };
+        f32x4 acc[RT];
+        {
+            bf16x8 v = none;
+            if (q4 == 0) {
+#pragma unroll
+                for (int e = 0; e < IN; ++e) {
+                    v[e] = (__bf16)((g.x[src * IN + e] - g.norm[e]) * g.norm[6 + e]);
+                    if (w == 0) g.X0[tix(t, IN, e, col)] = live ? v[e] : (__bf16)0.0f;
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < RT; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1[i], v, zero, 0, 0, 0);
+        }
+        activate(0, acc, b1, H[p]);
+        __syncthreads();
+        product(a2, H[p], acc);
+        activate(1, acc, b2, H[p ^ 1]);
+        __syncthreads();
+        product(a3, H[p ^ 1], acc);
+        activate(2, acc, b3, H[p]);
+        __syncthreads();
+        if (w == 0) {
+            // output layer: D = Y - T, dY = 2 D / (OUT n); rows OUT.. are zero
+            f32x4 y = zero;
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                y = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                    a4[q], *reinterpret_cast<const bf16x8 *>(&H[p][col][32 * q + 8 * q4]), y, 0, 0, 0);
+            float d[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int o = 4 * q4 + r;
+                d[r] = 0.f;
+                if (o < OUT) {
+                    const float T = (g.y[src * OUT + o] - g.norm[12 + o]) * g.norm[22 + o];
+                    d[r] = (y[r] + g.p[OFF_B4 + o]) - T;
+                    const float gy = 2.0f * d[r] * g.inv_count;
+                    g.dY[tix(t, OUT, o, col)] = live ? gy : 0.f;
+                    g.dYb[tix(t, OUT, o, col)] = live ? (__bf16)gy : (__bf16)0.0f;
+                    D[col][o] = (__bf16)gy;
+                } else if (o < 8) {
+                    D[col][o] = (__bf16)0.0f;
+                }
+            }
+            const float d4 = __shfl(d[0], (lane + 16) & 63, 64);
+            if (q4 == 0) g.se[j] = live ? (((d[0] * d[0] + d[1] * d[1]) + d[2] * d[2]) + d[3] * d[3]) + d4 * d4 : 0.f;
+        }
+        __syncthreads();
+        auto back = [&](int l, __bf16 (*S)[LDH]) {
+#pragma unroll
+            for (int i = 0; i < RT; ++i) {
+                const int f = 16 * (RT * w + i) + 4 * q4;
+                bf16x4 h;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float d = acc[i][r] * gd[l][i][r];
+                    h[r] = (__bf16)d;
+                    g.dZ[l][tix(t, HID, f + r, col)] = live ? d : 0.f;
+                    g.dZb[l][tix(t, HID, f + r, col)] = live ? h[r] : (__bf16)0.0f;
+                }
+                if (S) *reinterpret_cast<bf16x4 *>(&S[col][f]) = h;
+            }
+        };
+        {
+            const bf16x8 v = q4 == 0 ? *reinterpret_cast<const bf16x8 *>(&D[col][0]) : none;
+#pragma unroll
+            for (int i = 0; i < RT; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(t4[i], v, zero, 0, 0, 0);
+        }
+        back(2, H[p ^ 1]);
+        __syncthreads();
+        product(t3, H[p ^ 1], acc);
+        back(1, H[p]);
+        __syncthreads();
+        product(t2, H[p], acc);
+        back(0, nullptr);
+    }
 }
 
-__global__ void k_to_bf16(const float *p, __bf16 *pb, int64_t n) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) pb[i] = (__bf16)p[i];
+constexpr int KSPLIT = 512;  // batch samples per split of the weight-gradient sums
+
+struct Wgrad {
+    const __bf16 *X0, *A[3], *dZb[3], *dYb;
+    const float *dZ[3], *dY, *se;
+    int n, ld, splits;
+    float *part;       // [splits][NPARAM] partial weight gradients
+    float *g;          // [NPARAM] bias gradients
+    float *loss_part;  // [n / 256] sums of squared errors
+};
+
+// 16 x (16 NT) tiles of a weight gradient dW = dZ X^T over one batch split
+template <int NT>
+__device__ __forceinline__ void wgrad_tile(const __bf16 *Z, int rows, int r0, const __bf16 *X, int cols, int c0,
+                                           int k0, int k1, float *out) {
+    const int lane = threadIdx.x & 63, col = lane & 15, q4 = lane >> 4;
+    f32x4 acc[NT];
+#pragma unroll
+    for (int i = 0; i < NT; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // rows outside the matrix repeat its last one; their results are not stored
+    // the lane's 8 samples k + 8 q4 .. are half a row of tile (k + 8 q4) / 16
+    const __bf16 *zp = Z + tix(q4 >> 1, rows, min(r0 + col, rows - 1), 8 * (q4 & 1));
+    const __bf16 *xp[NT];
+#pragma unroll
+    for (int i = 0; i < NT; ++i) xp[i] = X + tix(q4 >> 1, cols, min(c0 + 16 * i + col, cols - 1), 8 * (q4 & 1));
+    auto step = [&](int k) {
+        const bf16x8 a = *reinterpret_cast<const bf16x8 *>(zp + (size_t)k * rows);
+#pragma unroll
+        for (int i = 0; i < NT; ++i)
+            acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                a, *reinterpret_cast<const bf16x8 *>(xp[i] + (size_t)k * cols), acc[i], 0, 0, 0);
+    };
+    if (k1 - k0 == KSPLIT) {  // a full split: every load in flight
+#pragma unroll
+        for (int k = 0; k < KSPLIT; k += 32) step(k0 + k);
+    } else {
+        for (int k = k0; k < k1; k += 32) step(k);
+    }
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int m = r0 + 4 * q4 + r, c = c0 + 16 * i + col;
+            if (m < rows && c < cols) out[m * cols + c] = acc[i][r];
+        }
+}
+
+// sum over 256 threads in a fixed order; valid in thread 0
+__device__ __forceinline__ float sum256(float s, float *sh) {
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
+    __syncthreads();
+    return (sh[0] + sh[1]) + (sh[2] + sh[3]);
+}
+
+constexpr int WG_UNITS = 76;  // wave tiles of all weight gradients of one split
+constexpr int wgrad_blocks(int splits) { return (WG_UNITS * splits + 3) / 4; }
+
+// Every sum over the batch in one launch: the weight gradients (one wave per
+// 16 x 32 tile and split; latency-bound, so as many waves as tiles), the bias
+// gradients (one block per row) and the loss (one block per 256 samples).
+__global__ __launch_bounds__(256) void k_wgrad(Wgrad g) {
+    __shared__ float sh[4];
+    int b = blockIdx.x;
+    const int nw = wgrad_blocks(g.splits);
+    if (b < nw) {
+        const int q = b * 4 + (threadIdx.x >> 6);
+        if (q >= WG_UNITS * g.splits) return;
+        const int z = q / WG_UNITS, u = q % WG_UNITS;
+        const int k0 = z * KSPLIT, k1 = min(g.ld, k0 + KSPLIT);
+        float *out = g.part + (size_t)z * NPARAM;
+        if (u < 32) wgrad_tile<2>(g.dZb[2], HID, 16 * (u >> 2), g.A[1], HID, 32 * (u & 3), k0, k1, out + OFF_W3);
+        else if (u < 64) wgrad_tile<2>(g.dZb[1], HID, 16 * ((u - 32) >> 2), g.A[0], HID, 32 * (u & 3), k0, k1, out + OFF_W2);
+        else if (u < 68) wgrad_tile<2>(g.dYb, OUT, 0, g.A[2], HID, 32 * (u & 3), k0, k1, out + OFF_W4);
+        else wgrad_tile<1>(g.dZb[0], HID, 16 * (u - 68), g.X0, IN, 0, k0, k1, out + OFF_W1);
+        return;
+    }
+    b -= nw;
+    if (b < 3 * HID + OUT) {
+        const int l = b / HID, r = b % HID;
+        const float *X = l < 3 ? g.dZ[l] : g.dY;
+        float s = 0.f;
+#pragma unroll 4
+        for (int j = threadIdx.x; j < g.n; j += 256) s += X[tix(j >> 4, l < 3 ? HID : OUT, r, j & 15)];
+        s = sum256(s, sh);
+        if (threadIdx.x == 0) g.g[(l == 0 ? OFF_B1 : (l == 1 ? OFF_B2 : (l == 2 ? OFF_B3 : OFF_B4))) + r] = s;
+        return;
+    }
+    b -= 3 * HID + OUT;
+    const int j = b * 256 + threadIdx.x;
+    const float s = sum256(j < g.n ? g.se[j] : 0.f, sh);
+    if (threadIdx.x == 0) g.loss_part[b] = s;
+}
+
+__device__ __forceinline__ bool is_bias(int64_t i) {
+    return (i >= OFF_B1 && i < OFF_W2) || (i >= OFF_B2 && i < OFF_W3) || (i >= OFF_B3 && i < OFF_W4) || i >= OFF_B4;
+}
+// BF16 copies of parameter i
+__device__ __forceinline__ void put_bf16(int64_t i, float v, __bf16 *pb, __bf16 *pt) {
+    const __bf16 h = (__bf16)v;
+    pb[i] = h;
+    if (i >= OFF_W2 && i < OFF_B2) pt[PT2 + (i - OFF_W2) % HID * HID + (i - OFF_W2) / HID] = h;
+    if (i >= OFF_W3 && i < OFF_B3) pt[PT3 + (i - OFF_W3) % HID * HID + (i - OFF_W3) / HID] = h;
+    if (i >= OFF_W4 && i < OFF_B4) pt[PT4 + (i - OFF_W4) % HID * 8 + (i - OFF_W4) / HID] = h;
+}
+
+struct Update {
+    const float *part;  // [splits][NPARAM]
+    int splits;
+    float *g, *p, *m, *v;
+    __bf16 *pb, *pt;
+    float lr_t, b1, b2, eps;
+};
+
+// gradient = sum over splits in order; with ADAM a step on the FP32 masters
+// (bias-corrected step size lr_t) and their BF16 copies
+template <bool ADAM>
+__global__ __launch_bounds__(256) void k_update(Update a) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= NPARAM) return;
+    float gi = 0.f;
+    if (is_bias(i)) gi = a.g[i];
+    else {
+#pragma unroll 4
+        for (int q = 0; q < a.splits; ++q) gi += a.part[(size_t)q * NPARAM + i];
+        a.g[i] = gi;
+    }
+    if (!ADAM) return;
+    const float mi = a.b1 * a.m[i] + (1.f - a.b1) * gi;
+    const float vi = a.b2 * a.v[i] + (1.f - a.b2) * gi * gi;
+    a.m[i] = mi;
+    a.v[i] = vi;
+    const float pi = a.p[i] - a.lr_t * mi / (sqrtf(vi) + a.eps);
+    a.p[i] = pi;
+    put_bf16(i, pi, a.pb, a.pt);
+}
+
+__global__ __launch_bounds__(256) void k_to_bf16(const float *p, __bf16 *pb, __bf16 *pt) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < NPARAM) put_bf16(i, p[i], pb, pt);
 }
 
 }  // namespace
@@ -415,20 +506,20 @@ struct nf_mlp {
     std::string err;
     hipStream_t stream = nullptr;
     float *p = nullptr, *g = nullptr, *m = nullptr, *v = nullptr;  // FP32 [NPARAM]
-    __bf16 *pb = nullptr;                                          // BF16 copy
+    __bf16 *pb = nullptr, *pt = nullptr;                           // BF16 copy, transposes (PT2..)
     float *norm = nullptr;  // device: in_shift[6], in_scale[6], out_shift[5], out_scale[5], out_iscale[5]
     float hnorm[27] = {};
     bool norm_set = false;  // false: training sets it from the data
     int64_t adam_t = 0;
     // workspace for batches of up to `cap` samples
     int cap = 0;
-    __bf16 *X0 = nullptr, *A[3] = {nullptr, nullptr, nullptr}, *dZb = nullptr, *dYb = nullptr;
-    float *Z[3] = {nullptr, nullptr, nullptr}, *Y = nullptr, *T = nullptr, *dY = nullptr, *dA = nullptr;
+    __bf16 *X0 = nullptr, *A[3] = {nullptr, nullptr, nullptr}, *dZb[3] = {nullptr, nullptr, nullptr}, *dYb = nullptr;
+    float *dZ[3] = {nullptr, nullptr, nullptr}, *dY = nullptr, *se = nullptr;
     float *part = nullptr, *loss_part = nullptr;
     std::vector<void *> ws;
     int device = 0;  // device current at nf_mlp_create, holding the parameters
-    // feature-major device copies of the caller's host arrays (inputs [6][n],
-    // targets or outputs [5][n], minibatch order), kept and grown as needed
+    // device copies of the caller's host arrays (inputs [n][6], targets or
+    // outputs [n][5]) and the minibatch order, kept and grown as needed
     float *dx = nullptr, *dy = nullptr;
     int64_t *didx = nullptr;
     int64_t data_cap = 0;
@@ -437,7 +528,6 @@ struct nf_mlp {
 namespace {
 
 constexpr int64_t NC1_MAX = 12288;  // samples up to which inference takes 16 per block (infer)
-constexpr int KSPLIT = 512;  // batch samples per split of the weight-gradient sums
 
 int fail(nf_mlp *m, int code, const std::string &msg) {
     if (m) m->err = msg;
@@ -449,15 +539,6 @@ int fail(nf_mlp *m, int code, const std::string &msg) {
         if (e_ != hipSuccess)                                                            \
             return fail(mm, NF_E_HIP, std::string(#expr) + ": " + hipGetErrorString(e_)); \
     } while (0)
-
-hipError_t gemm(hipStream_t s, const __bf16 *A, int64_t sam, int64_t sak, const __bf16 *B, int64_t sbk, int64_t sbn,
-                float *C, int64_t scm, int64_t scn, int M, int N, int K, int ksplit = 0, int64_t sc_split = 0) {
-    if (ksplit <= 0) ksplit = (K + TK - 1) / TK * TK;
-    const Gemm g{A, sam, sak, B, sbk, sbn, C, scm, scn, sc_split, M, N, K, ksplit};
-    const dim3 grid((N + TN - 1) / TN, (M + TM - 1) / TM, (K + ksplit - 1) / ksplit);
-    hipLaunchKernelGGL(k_gemm, grid, dim3(256), 0, s, g);
-    return hipGetLastError();
-}
 
 int ensure_ws(nf_mlp *mm, int n) {
     if (n <= mm->cap) return NF_OK;
@@ -475,43 +556,16 @@ int ensure_ws(nf_mlp *mm, int n) {
     if ((rc = al(&mm->X0, (size_t)IN * cap))) return rc;
     for (int l = 0; l < 3; ++l) {
         if ((rc = al(&mm->A[l], (size_t)HID * cap))) return rc;
-        if ((rc = al(&mm->Z[l], (size_t)HID * cap))) return rc;
+        if ((rc = al(&mm->dZb[l], (size_t)HID * cap))) return rc;
+        if ((rc = al(&mm->dZ[l], (size_t)HID * cap))) return rc;
     }
-    if ((rc = al(&mm->dZb, (size_t)HID * cap))) return rc;
-    if ((rc = al(&mm->dA, (size_t)HID * cap))) return rc;
-    if ((rc = al(&mm->Y, (size_t)OUT * cap))) return rc;
-    if ((rc = al(&mm->T, (size_t)OUT * cap))) return rc;
     if ((rc = al(&mm->dY, (size_t)OUT * cap))) return rc;
     if ((rc = al(&mm->dYb, (size_t)OUT * cap))) return rc;
-    if ((rc = al(&mm->part, (size_t)((cap + KSPLIT - 1) / KSPLIT) * HID * HID))) return rc;
+    if ((rc = al(&mm->se, (size_t)cap))) return rc;
+    if ((rc = al(&mm->part, (size_t)((cap + KSPLIT - 1) / KSPLIT) * NPARAM))) return rc;
     if ((rc = al(&mm->loss_part, (size_t)cap / 256 + 1))) return rc;
     mm->cap = cap;
     return NF_OK;
-}
-
-const float *d_in_shift(const nf_mlp *m) { return m->norm; }
-const float *d_in_scale(const nf_mlp *m) { return m->norm + 6; }
-const float *d_out_shift(const nf_mlp *m) { return m->norm + 12; }
-const float *d_out_scale(const nf_mlp *m) { return m->norm + 17; }
-const float *d_out_iscale(const nf_mlp *m) { return m->norm + 22; }
-
-// forward of the n samples in X0 (normalised) for training, which keeps every
-// layer's pre-activations and activations; Y = normalised outputs, bias not
-// yet added
-hipError_t forward(nf_mlp *m, int n, hipStream_t s) {
-    hipError_t e;
-    const __bf16 *in = m->X0;
-    int k = IN;
-    const int64_t offW[3] = {OFF_W1, OFF_W2, OFF_W3}, offB[3] = {OFF_B1, OFF_B2, OFF_B3};
-    for (int l = 0; l < 3; ++l) {
-        if ((e = gemm(s, m->pb + offW[l], k, 1, in, n, 1, m->Z[l], n, 1, HID, n, k))) return e;
-        hipLaunchKernelGGL(k_bias_gelu, dim3((n + 255) / 256, HID), dim3(256), 0, s, m->Z[l],
-                           (const float *)(m->p + offB[l]), m->A[l], HID, n);
-        if ((e = hipGetLastError())) return e;
-        in = m->A[l];
-        k = HID;
-    }
-    return gemm(s, m->pb + OFF_W4, HID, 1, in, n, 1, m->Y, n, 1, OUT, n, HID);
 }
 
 // inference of n samples on the device: x(f, j) = x[f * xf + j * xj],
@@ -522,51 +576,38 @@ hipError_t infer(const nf_mlp *m, const float *x, int64_t xf, int64_t xj, float 
     const Infer g{m->pb, m->p, m->norm, x, xf, xj, y, yo, yj, n};
     // 64 samples per block share one read of the weights and activations
     // (one block's latency 12.4 us up to 2 blocks per CU), 16 per block are
-    // done in 6.2 us while at most about 3 of them share a CU: 9.1 against
+    // done in 6.0 us while at most about 3 of them share a CU: 9.2 against
     // 12.5 us at 8,192 samples, 16.5 against 12.5 us at 16,384
-    if (n > NC1_MAX) hipLaunchKernelGGL(k_infer<4>, dim3((unsigned)std::min<int64_t>((n + 63) / 64, 512)), dim3(256), 0, s, g);
-    else hipLaunchKernelGGL(k_infer<1>, dim3((unsigned)((n + 15) / 16)), dim3(256), 0, s, g);
+    if (n > NC1_MAX) hipLaunchKernelGGL((k_infer<4, 2>), dim3((unsigned)std::min<int64_t>((n + 63) / 64, 512)), dim3(256), 0, s, g);
+    else hipLaunchKernelGGL((k_infer<1, 1>), dim3((unsigned)((n + 15) / 16)), dim3(512), 0, s, g);
     return hipGetLastError();
 }
 
-// loss and gradient (into m->g) of the n samples in X0 / T
-hipError_t backward(nf_mlp *m, int n, hipStream_t s) {
-    hipError_t e;
-    const float inv_count = 1.0f / ((float)OUT * (float)n);
-    const int nb = (n + 255) / 256;
-    hipLaunchKernelGGL(k_out_loss, dim3(nb), dim3(256), 0, s, m->Y, (const float *)(m->p + OFF_B4),
-                       (const float *)m->T, m->dY, m->dYb, m->loss_part, n, inv_count);
-    if ((e = hipGetLastError())) return e;
-    const int splits = (n + KSPLIT - 1) / KSPLIT;
-    // weight gradient dW = dZ X^T over the batch, split over samples
-    auto dW = [&](const __bf16 *dZ, int rows, const __bf16 *X, int cols, int64_t off) -> hipError_t {
-        hipError_t e2;
-        if ((e2 = gemm(s, dZ, n, 1, X, 1, n, m->part, cols, 1, rows, cols, n, KSPLIT, (int64_t)rows * cols)))
-            return e2;
-        const int64_t cnt = (int64_t)rows * cols;
-        hipLaunchKernelGGL(k_sum_splits, dim3((cnt + 255) / 256), dim3(256), 0, s, (const float *)m->part, splits,
-                           cnt, cnt, m->g + off);
-        return hipGetLastError();
-    };
-    // output layer
-    if ((e = dW(m->dYb, OUT, m->A[2], HID, OFF_W4))) return e;
-    hipLaunchKernelGGL(k_rowsum, dim3(OUT), dim3(256), 0, s, (const float *)m->dY, n, m->g + OFF_B4);
-    if ((e = hipGetLastError())) return e;
-    // dA3 = W4^T dY
-    if ((e = gemm(s, m->pb + OFF_W4, 1, HID, m->dYb, n, 1, m->dA, n, 1, HID, n, OUT))) return e;
-    const int64_t offW[3] = {OFF_W1, OFF_W2, OFF_W3}, offB[3] = {OFF_B1, OFF_B2, OFF_B3};
-    for (int l = 2; l >= 0; --l) {
-        hipLaunchKernelGGL(k_gelu_back, dim3(nb, HID), dim3(256), 0, s, m->dA, (const float *)m->Z[l], m->dZb, HID,
-                           n);
-        if ((e = hipGetLastError())) return e;
-        hipLaunchKernelGGL(k_rowsum, dim3(HID), dim3(256), 0, s, (const float *)m->dA, n, m->g + offB[l]);
-        if ((e = hipGetLastError())) return e;
-        const __bf16 *X = l ? m->A[l - 1] : m->X0;
-        const int kin = l ? HID : IN;
-        if ((e = dW(m->dZb, HID, X, kin, offW[l]))) return e;
-        if (l > 0 && (e = gemm(s, m->pb + offW[l], 1, kin, m->dZb, n, 1, m->dA, n, 1, kin, n, HID))) return e;
+// loss partials and gradient partials of n samples: first + j, or idx[first + j]
+hipError_t gradients(nf_mlp *m, const int64_t *idx, int64_t first, int n, hipStream_t s) {
+    const int ld = (n + 63) / 64 * 64, splits = (n + KSPLIT - 1) / KSPLIT;
+    Train t{m->pb, m->pt, m->p, m->norm, m->dx, m->dy, idx, first, n, ld, 1.0f / ((float)OUT * (float)n), m->X0,
+            {}, {}, m->dYb, {}, m->dY, m->se};
+    Wgrad g{m->X0, {}, {}, m->dYb, {}, m->dY, m->se, n, ld, splits, m->part, m->g, m->loss_part};
+    for (int l = 0; l < 3; ++l) {
+        g.A[l] = t.A[l] = m->A[l];
+        g.dZb[l] = t.dZb[l] = m->dZb[l];
+        g.dZ[l] = t.dZ[l] = m->dZ[l];
     }
-    return hipSuccess;
+    hipLaunchKernelGGL(k_train, dim3(std::min(ld / 16, 256)), dim3(512), 0, s, t);
+    hipError_t e = hipGetLastError();
+    if (e) return e;
+    hipLaunchKernelGGL(k_wgrad, dim3(wgrad_blocks(splits) + 3 * HID + OUT + (n + 255) / 256), dim3(256), 0, s, g);
+    return hipGetLastError();
+}
+
+// gradient from its partials; lr_t, o: an Adam step too
+template <bool ADAM>
+hipError_t update(nf_mlp *m, int n, hipStream_t s, float lr_t, const nf_train_opts *o) {
+    Update u{m->part, (n + KSPLIT - 1) / KSPLIT, m->g, m->p, m->m, m->v, m->pb, m->pt, lr_t, 0.f, 0.f, 0.f};
+    if (o) u.b1 = o->beta1, u.b2 = o->beta2, u.eps = o->eps;
+    hipLaunchKernelGGL(k_update<ADAM>, dim3((NPARAM + 255) / 256), dim3(256), 0, s, u);
+    return hipGetLastError();
 }
 
 float sum_loss(nf_mlp *m, int n) {
@@ -603,12 +644,10 @@ int ensure_data(nf_mlp *mm, int64_t n) {
     return NF_OK;
 }
 
-// a host AoS [n][w] array into a feature-major device buffer [w][n]
-int upload_fm(nf_mlp *mm, const float *aos, int64_t n, int w, float *dev) {
-    std::vector<float> fm((size_t)w * n);
-    for (int64_t j = 0; j < n; ++j)
-        for (int f = 0; f < w; ++f) fm[(size_t)f * n + j] = aos[(size_t)j * w + f];
-    HIPM(hipMemcpy(dev, fm.data(), fm.size() * sizeof(float), hipMemcpyHostToDevice));
+// the caller's samples and targets, as they are
+int upload_data(nf_mlp *mm, const float *x, const float *y, int64_t n) {
+    HIPM(hipMemcpy(mm->dx, x, (size_t)IN * n * sizeof(float), hipMemcpyHostToDevice));
+    HIPM(hipMemcpy(mm->dy, y, (size_t)OUT * n * sizeof(float), hipMemcpyHostToDevice));
     return NF_OK;
 }
 
@@ -662,6 +701,8 @@ int nf_mlp_create(uint64_t seed, nf_mlp **out) {
     HIPM(hipMalloc(&mm->m, NPARAM * sizeof(float)));
     HIPM(hipMalloc(&mm->v, NPARAM * sizeof(float)));
     HIPM(hipMalloc(&mm->pb, NPARAM * sizeof(__bf16)));
+    HIPM(hipMalloc(&mm->pt, NPT * sizeof(__bf16)));
+    HIPM(hipMemset(mm->pt, 0, NPT * sizeof(__bf16)));
     HIPM(hipMalloc(&mm->norm, 27 * sizeof(float)));
     // uniform(+-1/sqrt(fan_in)) weights and biases, a linear layer's default
     std::mt19937_64 rng(seed);
@@ -687,7 +728,7 @@ int nf_mlp_destroy(nf_mlp *mm) {
     if (!mm) return NF_OK;
     if (mm->stream) (void)hipStreamSynchronize(mm->stream);
     for (void *q : mm->ws) (void)hipFree(q);
-    for (void *q : {(void *)mm->p, (void *)mm->g, (void *)mm->m, (void *)mm->v, (void *)mm->pb, (void *)mm->norm,
+    for (void *q : {(void *)mm->p, (void *)mm->g, (void *)mm->m, (void *)mm->v, (void *)mm->pb, (void *)mm->pt, (void *)mm->norm,
                     (void *)mm->dx, (void *)mm->dy, (void *)mm->didx})
         if (q) (void)hipFree(q);
     if (mm->stream) (void)hipStreamDestroy(mm->stream);
@@ -712,7 +753,7 @@ int nf_mlp_set_params(nf_mlp *mm, const float *params) {
     HIPM(hipMemset(mm->v, 0, NPARAM * sizeof(float)));
     mm->adam_t = 0;
     hipLaunchKernelGGL(k_to_bf16, dim3((NPARAM + 255) / 256), dim3(256), 0, mm->stream, (const float *)mm->p, mm->pb,
-                       NPARAM);
+                       mm->pt);
     HIPM(hipGetLastError());
     HIPM(hipStreamSynchronize(mm->stream));
     return NF_OK;
@@ -758,14 +799,10 @@ int nf_mlp_loss_grad(nf_mlp *mm, const float *x, const float *y, int64_t n, floa
     if (!mm || !x || !y || n < 1 || n > (1 << 20)) return NF_E_ARG;
     int rc;
     if ((rc = ensure_ws(mm, (int)n)) || (rc = ensure_data(mm, n))) return rc;
-    if ((rc = upload_fm(mm, x, n, IN, mm->dx)) || (rc = upload_fm(mm, y, n, OUT, mm->dy))) return rc;
+    if ((rc = upload_data(mm, x, y, n))) return rc;
     const int c = (int)n;
-    hipLaunchKernelGGL(k_gather, dim3((c + 255) / 256), dim3(256), 0, mm->stream, (const float *)mm->dx,
-                       (const float *)mm->dy, n, (const int64_t *)nullptr, (int64_t)0, c, d_in_shift(mm),
-                       d_in_scale(mm), d_out_shift(mm), d_out_iscale(mm), mm->X0, mm->T);
-    hipError_t e = hipGetLastError();
-    if (!e) e = forward(mm, c, mm->stream);
-    if (!e) e = backward(mm, c, mm->stream);
+    hipError_t e = gradients(mm, nullptr, 0, c, mm->stream);
+    if (!e) e = update<false>(mm, c, mm->stream, 0.f, nullptr);
     if (!e) e = hipStreamSynchronize(mm->stream);
     if (e != hipSuccess) return fail(mm, NF_E_HIP, std::string("loss_grad: ") + hipGetErrorString(e));
     if (loss) *loss = sum_loss(mm, c);
@@ -803,8 +840,7 @@ int nf_mlp_train(nf_mlp *mm, const float *x, const float *y, int64_t n, const nf
         mm->norm_set = true;
     }
     if ((rc = ensure_data(mm, n))) return rc;
-    if ((rc = upload_fm(mm, x, n, IN, mm->dx)) || (rc = upload_fm(mm, y, n, OUT, mm->dy))) return rc;
-    const float *dx = mm->dx, *dy = mm->dy;
+    if ((rc = upload_data(mm, x, y, n))) return rc;
     int64_t *didx = mm->didx;
     std::vector<int64_t> idx(n);
     for (int64_t j = 0; j < n; ++j) idx[j] = j;
@@ -824,20 +860,12 @@ int nf_mlp_train(nf_mlp *mm, const float *x, const float *y, int64_t n, const nf
         const float lr = o->lr * std::pow(o->lr_decay > 0 ? o->lr_decay : 1.0f, (float)ep);
         double ep_loss = 0;
         for (int64_t q = 0; q < per_epoch && !e; ++q) {
-            hipLaunchKernelGGL(k_gather, dim3(B / 256), dim3(256), 0, mm->stream, (const float *)dx, (const float *)dy,
-                               n, (const int64_t *)didx, q * B, B, d_in_shift(mm), d_in_scale(mm), d_out_shift(mm),
-                               d_out_iscale(mm), mm->X0, mm->T);
-            e = hipGetLastError();
-            if (!e) e = forward(mm, B, mm->stream);
-            if (!e) e = backward(mm, B, mm->stream);
+            e = gradients(mm, didx, q * B, B, mm->stream);
             if (e) break;
             ++mm->adam_t;
             const double bc1 = 1.0 - std::pow((double)o->beta1, (double)mm->adam_t);
             const double bc2 = 1.0 - std::pow((double)o->beta2, (double)mm->adam_t);
-            const float lr_t = (float)(lr * std::sqrt(bc2) / bc1);
-            hipLaunchKernelGGL(k_adam, dim3((NPARAM + 255) / 256), dim3(256), 0, mm->stream, mm->p,
-                               (const float *)mm->g, mm->m, mm->v, mm->pb, NPARAM, lr_t, o->beta1, o->beta2, o->eps);
-            e = hipGetLastError();
+            e = update<true>(mm, B, mm->stream, (float)(lr * std::sqrt(bc2) / bc1), o);
             ++steps;
             if (q == 0 || q == per_epoch - 1) {
                 if (!e) e = hipStreamSynchronize(mm->stream);

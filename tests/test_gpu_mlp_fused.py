@@ -1,11 +1,15 @@
 """The fused inference kernel at the edges of its sample tiles (16 and 64 per
 block) and of the rule between them, against the FP64 restatement of the
 network with BF16 rounding at the device's rounding points."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
+from netflux_amd import _abi as A
 from oracle import mlp_ref as M
 from tests.test_gpu_mlp import _data, _net
+from tests.test_zz_no_alloc import DevBuf, _hip
 
 pytestmark = pytest.mark.gpu
 
@@ -23,3 +27,33 @@ def test_predict_at_tile_edges(n):
     # samples are independent: the last ones alone give the same bits
     k = min(n, 5)
     np.testing.assert_array_equal(net.predict(x[-k:]), y[-k:])
+
+
+def test_device_calls_overlap_on_two_streams():
+    """nf_mlp_predict_noalloc calls of two networks, in turn on two streams
+    without waiting between them, share nothing: each gives its own result."""
+    print("[case] fused predict, two networks on two streams", flush=True)
+    hip = _hip()
+    nets = [_net(seed=11)[0], _net(seed=12)[0]]
+    xs = [_data(700, seed=21 + q)[0] for q in range(2)]
+    ref = [n.predict(x) for n, x in zip(nets, xs)]
+    streams = [C.c_void_p(), C.c_void_p()]
+    bufs = [(DevBuf(hip, x.nbytes), DevBuf(hip, len(x) * 20)) for x in xs]
+    try:
+        for s in streams:
+            assert hip.hipStreamCreate(C.byref(s)) == 0  # default priority
+        for x, (xd, yd) in zip(xs, bufs):
+            xd.put(x)
+            yd.put(np.full((len(x), 5), np.nan, np.float32))
+        for _ in range(20):
+            for net, s, x, (xd, yd) in zip(nets, streams, xs, bufs):
+                assert A.lib().nf_mlp_predict_noalloc(net._h, xd.p, len(x), yd.p, s) == A.NF_OK
+        for q, s in enumerate(streams):
+            assert hip.hipStreamSynchronize(s) == 0
+            np.testing.assert_array_equal(bufs[q][1].get((len(xs[q]), 5)), ref[q])
+    finally:
+        for xd, yd in bufs:
+            xd.free()
+            yd.free()
+        for s in streams:
+            hip.hipStreamDestroy(s)
