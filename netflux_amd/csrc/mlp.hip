@@ -26,6 +26,7 @@
 #include <vector>
 
 #include "../../include/netflux.h"
+#include "host_pipe.hpp"
 #include "mlp.hpp"
 
 using nf::mlp::HID;
@@ -523,6 +524,7 @@ struct nf_mlp {
     float *dx = nullptr, *dy = nullptr;
     int64_t *didx = nullptr;
     int64_t data_cap = 0;
+    nf::HostPipe pipe;  // large arrays across the boundary
 };
 
 namespace {
@@ -646,8 +648,8 @@ int ensure_data(nf_mlp *mm, int64_t n) {
 
 // the caller's samples and targets, as they are
 int upload_data(nf_mlp *mm, const float *x, const float *y, int64_t n) {
-    HIPM(hipMemcpy(mm->dx, x, (size_t)IN * n * sizeof(float), hipMemcpyHostToDevice));
-    HIPM(hipMemcpy(mm->dy, y, (size_t)OUT * n * sizeof(float), hipMemcpyHostToDevice));
+    HIPM(mm->pipe.up(mm->dx, x, (size_t)IN * n * sizeof(float), mm->stream));
+    HIPM(mm->pipe.up(mm->dy, y, (size_t)OUT * n * sizeof(float), mm->stream));
     return NF_OK;
 }
 
@@ -787,10 +789,9 @@ int nf_mlp_predict(nf_mlp *mm, const float *x, int64_t n, float *y) {
     int rc;
     // both arrays cross as they are ([n][6], [n][5]): the kernel reads samples
     if ((rc = ensure_data(mm, n))) return rc;
-    HIPM(hipMemcpyAsync(mm->dx, x, (size_t)IN * n * sizeof(float), hipMemcpyHostToDevice, mm->stream));
+    HIPM(mm->pipe.up(mm->dx, x, (size_t)IN * n * sizeof(float), mm->stream));
     HIPM(infer(mm, mm->dx, 1, IN, mm->dy, 1, OUT, n, mm->stream));
-    HIPM(hipMemcpyAsync(y, mm->dy, (size_t)OUT * n * sizeof(float), hipMemcpyDeviceToHost, mm->stream));
-    HIPM(hipStreamSynchronize(mm->stream));
+    HIPM(mm->pipe.down(y, mm->dy, (size_t)OUT * n * sizeof(float), mm->stream));
     return NF_OK;
 }
 

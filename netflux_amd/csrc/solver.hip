@@ -18,6 +18,7 @@
 #include <vector>
 
 #include "../../include/netflux.h"
+#include "host_pipe.hpp"
 #include "kernels_fp64.hpp"
 #include "kernels_mixed.hpp"
 #include "mesh.hpp"
@@ -337,6 +338,7 @@ struct nf_ctx {
     bool timing = false;
     std::map<std::string, std::pair<double, int>> ktime;
     std::vector<std::pair<std::string, std::pair<hipEvent_t, hipEvent_t>>> pending;
+    nf::HostPipe pipe;             // large arrays across the boundary
     nf::PolyPath *poly = nullptr;  // mixed-element mesh: the polyhedral path (n_inst = 0)
 };
 
@@ -694,7 +696,7 @@ int upload_state(nf_ctx *ctx, int i, const double *aos, double *dev) {
     const Inst &I = ctx->inst[i];
     int rc;
     if ((rc = ensure_stage(ctx))) return rc;
-    HIPC(hipMemcpyAsync(ctx->stage, aos, (size_t)5 * I.N * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
+    HIPC(ctx->pipe.up(ctx->stage, aos, (size_t)5 * I.N * sizeof(double), ctx->stream));
     hipLaunchKernelGGL(k_state_in, dim3(I.Npad / BLOCK), dim3(BLOCK), 0, ctx->stream, (const double *)ctx->stage,
                        (const uint32_t *)(ctx->perm_dev + I.cell0), dev + (size_t)5 * I.cell0, I.N, I.Npad);
     HIPC(hipGetLastError());
@@ -710,8 +712,7 @@ int download_state(nf_ctx *ctx, int i, const double *dev, double *aos) {
     hipLaunchKernelGGL(k_state_out, dim3(I.Npad / BLOCK), dim3(BLOCK), 0, ctx->stream,
                        dev + (size_t)5 * I.cell0, (const uint32_t *)(ctx->perm_dev + I.cell0), ctx->stage, I.N);
     HIPC(hipGetLastError());
-    HIPC(hipMemcpyAsync(aos, ctx->stage, (size_t)5 * I.N * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-    HIPC(hipStreamSynchronize(ctx->stream));
+    HIPC(ctx->pipe.down(aos, ctx->stage, (size_t)5 * I.N * sizeof(double), ctx->stream));
     return NF_OK;
 }
 template <typename T>
@@ -835,7 +836,7 @@ int features(nf_ctx *ctx, int i, const double *cp, bool rows) {
 int set_state(nf_ctx *ctx, int i, const double *U, const double *U_old) {
     bool zero = ctx->prm.rk3_zero_old_first_step != 0;
     if (U_old) {
-        if (std::memcmp(U, U_old, (size_t)5 * ctx->inst[i].N * sizeof(double)) != 0)
+        if (U != U_old && std::memcmp(U, U_old, (size_t)5 * ctx->inst[i].N * sizeof(double)) != 0)
             return fail(ctx, NF_E_ARG, "U_old must be NULL (zero) or equal to U");
         zero = false;
     }
@@ -1647,8 +1648,7 @@ int nf_inst_features(nf_ctx *ctx, int32_t i, const double *cp, float *x) {
     if (!valid_inst(ctx, i) || !cp || !x) return NF_E_ARG;
     int rc;
     if ((rc = features(ctx, i, cp, true))) return rc;
-    HIPC(hipMemcpyAsync(x, ctx->feat, (size_t)6 * ctx->inst[i].N * sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
-    HIPC(hipStreamSynchronize(ctx->stream));
+    HIPC(ctx->pipe.down(x, ctx->feat, (size_t)6 * ctx->inst[i].N * sizeof(float), ctx->stream));
     return NF_OK;
 }
 

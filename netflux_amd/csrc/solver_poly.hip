@@ -27,6 +27,7 @@
 #include <vector>
 
 #include "fp64_math.hpp"
+#include "host_pipe.hpp"
 #include "physics.hpp"
 #include "poly.hpp"
 
@@ -420,6 +421,7 @@ struct PolyPath {
     std::map<std::string, std::pair<double, int>> ktime;
     std::vector<uint32_t> perm;  // device cell -> reference cell
     uint32_t *perm_dev = nullptr;  // the same on the device (made on first state transfer)
+    HostPipe pipe;                 // large arrays across the boundary
     double *stage = nullptr;       // [15][N] AoS staging of state and field transfers
     std::vector<double> hist;    // residual norm of each step (flux balance of U^n)
     double time = 0.0;
@@ -467,7 +469,7 @@ int put_soa(PolyPath *P, double *dst, const double *aos, int cols, std::string &
     const uint32_t N = P->m.N;
     int rc;
     if ((rc = ensure_stage(P, err))) return rc;
-    PHIP(hipMemcpyAsync(P->stage, aos, (size_t)cols * N * 8, hipMemcpyHostToDevice, P->st));
+    PHIP(P->pipe.up(P->stage, aos, (size_t)cols * N * 8, P->st));
     hipLaunchKernelGGL(k_poly_aos_in, grid(N), dim3(PB), 0, P->st, (const double *)P->stage,
                        (const uint32_t *)P->perm_dev, dst, N, cols);
     PHIP(hipGetLastError());
@@ -481,8 +483,7 @@ int get_soa(PolyPath *P, const double *src, int cols, double *aos, std::string &
     hipLaunchKernelGGL(k_poly_aos_out, grid(N), dim3(PB), 0, P->st, src, (const uint32_t *)P->perm_dev, P->stage,
                        N, cols);
     PHIP(hipGetLastError());
-    PHIP(hipMemcpyAsync(aos, P->stage, (size_t)cols * N * 8, hipMemcpyDeviceToHost, P->st));
-    PHIP(hipStreamSynchronize(P->st));
+    PHIP(P->pipe.down(aos, P->stage, (size_t)cols * N * 8, P->st));
     return NF_OK;
 }
 
@@ -721,7 +722,7 @@ int poly_set_state(PolyPath *P, const double *U, const double *U_old, std::strin
     const uint32_t N = P->m.N;
     bool zero = P->prm.rk3_zero_old_first_step != 0;
     if (U_old) {
-        if (std::memcmp(U, U_old, (size_t)5 * N * sizeof(double)) != 0) {
+        if (U != U_old && std::memcmp(U, U_old, (size_t)5 * N * sizeof(double)) != 0) {
             err = "U_old must be NULL (zero) or equal to U";
             return NF_E_ARG;
         }
