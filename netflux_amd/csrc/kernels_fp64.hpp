@@ -457,6 +457,7 @@ struct SweepAArgs {
     int xcd_remap;
     double *grad_aux;  // [N][15] column-major 5x3 per cell, or null
     double *psi_aux;   // [N][5] or null
+    const uint32_t *aux_row;  // device cell -> row of grad_aux and psi_aux (reference cell)
     BndArgs bnd;       // FUSE: ghosts of the reconstructed face states (out: Gf)
 };
 
@@ -638,10 +639,11 @@ __device__ __forceinline__ double tileA_run(const DevMesh &m, const SweepAArgs &
             }
             if (live) {
                 if (a.grad_aux) {
-                    a.grad_aux[15 * (size_t)c + k] = g0;
-                    a.grad_aux[15 * (size_t)c + k + 5] = g1;
-                    a.grad_aux[15 * (size_t)c + k + 10] = g2;
-                    a.psi_aux[5 * (size_t)c + k] = psi;
+                    const size_t row = a.aux_row[c];
+                    a.grad_aux[15 * row + k] = g0;
+                    a.grad_aux[15 * row + k + 5] = g1;
+                    a.grad_aux[15 * row + k + 10] = g2;
+                    a.psi_aux[5 * row + k] = psi;
                 }
             }
             __builtin_amdgcn_sched_barrier(0);
@@ -692,6 +694,7 @@ struct SweepBArgs {
     int check;
     int xcd_remap;
     double *R_aux;          // [N][5] or null: store R, skip the update
+    const uint32_t *aux_row;  // device cell -> row of R_aux (reference cell)
     double *Rst, *fst;      // checked stage: R [tile][5][64] and f [cell] for k_apply, no update
     BndArgs bnd;            // FUSE: ghosts of the updated cell states (out: Gc), where it updates
 };
@@ -786,7 +789,7 @@ __global__ __launch_bounds__(B) NF_SWEEPB_ATTR void k_sweepB(DevMesh m, SweepBAr
     if (a.R_aux) {
         if (live) {
 #pragma unroll
-            for (int k = 0; k < 5; ++k) a.R_aux[5 * (size_t)c + k] = R[k];
+            for (int k = 0; k < 5; ++k) a.R_aux[5 * (size_t)a.aux_row[c] + k] = R[k];
         }
     } else {
         const double dt = a.dt_cell ? a.dt_cell[c] : st.dt;
@@ -842,14 +845,24 @@ __global__ __launch_bounds__(BLOCK) void k_state_in(const double *aos, const uin
 #pragma unroll
     for (int k = 0; k < 5; ++k) dev[tix(p, k)] = p < N ? aos[r + k] : 0.0;
 }
-// and back: device tiles to reference-order AoS
-__global__ __launch_bounds__(BLOCK) void k_state_out(const double *dev, const uint32_t *perm, double *aos,
-                                                     uint32_t N) {
+// and back: device tiles (FP64, or FP32 primvars) to reference-order AoS
+template <typename T>
+__global__ __launch_bounds__(BLOCK) void k_state_out(const T *dev, const uint32_t *perm, double *aos, uint32_t N) {
     const uint32_t p = blockIdx.x * BLOCK + threadIdx.x;
     if (p >= N) return;
     const size_t r = 5 * (size_t)perm[p];
 #pragma unroll
-    for (int k = 0; k < 5; ++k) aos[r + k] = dev[tix(p, k)];
+    for (int k = 0; k < 5; ++k) aos[r + k] = (double)dev[tix(p, k)];
+}
+// one state in every cell, padding cells zero
+struct CellState {
+    double v[5];
+};
+__global__ __launch_bounds__(BLOCK) void k_state_fill(CellState s, double *dev, uint32_t N, uint32_t Npad) {
+    const uint32_t p = blockIdx.x * BLOCK + threadIdx.x;
+    if (p >= Npad) return;
+#pragma unroll
+    for (int k = 0; k < 5; ++k) dev[tix(p, k)] = p < N ? s.v[k] : 0.0;
 }
 #endif  // NF_DEVICE_HELPERS_ONLY
 

@@ -44,6 +44,7 @@ struct SweepAArgsMx {
     double CFL;
     int xcd_remap;
     double *grad_aux, *psi_aux;
+    const uint32_t *aux_row;
     BndArgsMx bnd;
 };
 
@@ -60,6 +61,7 @@ struct SweepBArgsMx {
     int check;
     int xcd_remap;
     double *R_aux;
+    const uint32_t *aux_row;
     double *Rst, *fst;  // checked stage: R and f stored for the apply pass, no update
     BndArgsMx bnd;
 };
@@ -282,10 +284,11 @@ __global__ __launch_bounds__(B) void k_sweepA_mx(DevMesh m, SweepAArgsMx a) {
 #pragma unroll
                 for (int s = 0; s < 4; ++s) a.FV[fix(c, s, k)] = Vc[k] + psi * delta[s];
                 if (a.grad_aux) {
-                    a.grad_aux[15 * (size_t)c + k] = g0;
-                    a.grad_aux[15 * (size_t)c + k + 5] = g1;
-                    a.grad_aux[15 * (size_t)c + k + 10] = g2;
-                    a.psi_aux[5 * (size_t)c + k] = psi;
+                    const size_t row = a.aux_row[c];
+                    a.grad_aux[15 * row + k] = g0;
+                    a.grad_aux[15 * row + k + 5] = g1;
+                    a.grad_aux[15 * row + k + 10] = g2;
+                    a.psi_aux[5 * row + k] = psi;
                 }
             }
         }
@@ -378,7 +381,7 @@ __global__ __launch_bounds__(B) NF_SWEEPB_MX_ATTR void k_sweepB_mx(DevMesh m, Sw
     if (a.R_aux) {
         if (live) {
 #pragma unroll
-            for (int k = 0; k < 5; ++k) a.R_aux[5 * (size_t)c + k] = R[k];
+            for (int k = 0; k < 5; ++k) a.R_aux[5 * (size_t)a.aux_row[c] + k] = R[k];
         }
     } else {
         const double dt = a.dt_cell ? a.dt_cell[c] : st.dt;

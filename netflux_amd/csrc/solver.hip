@@ -500,6 +500,7 @@ int run_sweepA(nf_ctx *ctx, bool dt, bool aux, bool dtc = false, const double *U
         const mx::SweepAArgsMx x{ctx->V32, ctx->Gc32, ctx->FV32, dt ? ctx->dt_part : nullptr,
                                  dtc ? ctx->dt_cell : nullptr, ctx->prm.CFL, ctx->xcd_remap,
                                  aux ? ctx->grad_aux : nullptr, aux ? ctx->psi_aux : nullptr,
+                                 ctx->perm_dev,
                                  bnd_args_mx(ctx, ctx->Gf32)};
         return launch_fn(ctx, order == 2 ? "sweepA_barth_mx" : "sweepA_mx", [&] {
             return mx::launch_sweepA_mx(order, ctx->block, fuse, ctx->Ncell, ctx->stream, m, x);
@@ -507,7 +508,7 @@ int run_sweepA(nf_ctx *ctx, bool dt, bool aux, bool dtc = false, const double *U
     }
     const SweepAArgs a{U ? U : ctx->V, ctx->Gc, ctx->FV, dt ? ctx->dt_part : nullptr, dtc ? ctx->dt_cell : nullptr,
                        ctx->prm.CFL, ctx->xcd_remap, aux ? ctx->grad_aux : nullptr, aux ? ctx->psi_aux : nullptr,
-                       bnd_args(ctx, ctx->Gf)};
+                       ctx->perm_dev, bnd_args(ctx, ctx->Gf)};
     const char *name = order == 2 ? "sweepA_barth" : (order == 1 ? "sweepA_nolim" : "sweepA_first");
     return launch_fn(ctx, name, [&] {
         auto go = [&](auto from_u, auto fused) {
@@ -538,7 +539,7 @@ int run_sweepB(nf_ctx *ctx, int kind, const double *U, double *Uout, bool res, b
     if (ctx->mixed) {
         const mx::SweepBArgsMx x{ctx->FV32, ctx->Gf32, U, ctx->Ua, Uout, ctx->V32, dtc, kind,
                                  res ? ctx->res_part : nullptr, ctx->prm.check_physical_validity,
-                                 ctx->xcd_remap, aux ? ctx->R_aux : nullptr, Rst, fst, bnd_args_mx(ctx, ctx->Gc32)};
+                                 ctx->xcd_remap, aux ? ctx->R_aux : nullptr, ctx->perm_dev, Rst, fst, bnd_args_mx(ctx, ctx->Gc32)};
         if ((rc = launch_fn(ctx, "sweepB_mx", [&] {
                  return mx::launch_sweepB_mx(ctx->block, fuse, ctx->Ncell, ctx->stream, m, x);
              })))
@@ -549,7 +550,7 @@ int run_sweepB(nf_ctx *ctx, int kind, const double *U, double *Uout, bool res, b
     }
     // (FP64: prim(Uout) is not stored; the next sweep A evaluates it from U)
     const SweepBArgs a{ctx->FV, ctx->Gf, U, ctx->Ua, Uout, dtc, kind, res ? ctx->res_part : nullptr,
-                       ctx->prm.check_physical_validity, ctx->xcd_remap, aux ? ctx->R_aux : nullptr, Rst, fst,
+                       ctx->prm.check_physical_validity, ctx->xcd_remap, aux ? ctx->R_aux : nullptr, ctx->perm_dev, Rst, fst,
                        bnd_args(ctx, ctx->Gc)};
     const bool hllc = ctx->prm.inv_flux_scheme == NF_FLUX_HLLC;
     if ((rc = launch_fn(ctx, "sweepB", [&] {
@@ -672,10 +673,7 @@ int ensure_hist(nf_ctx *ctx, int need) {
     return NF_OK;
 }
 
-size_t tile_index(uint32_t c, int k) { return ((size_t)(c >> 6) * 5 + k) * TILE + (c & 63u); }
-
-// reference-order AoS [N][5] of instance i -> device tiles
-// the staging buffer and the device copy of the cell maps, made on first use
+// the staging buffer and the device copy of the cell maps
 int ensure_stage(nf_ctx *ctx) {
     if (ctx->stage) return NF_OK;
     uint32_t nmax = 1;
@@ -705,35 +703,15 @@ int upload_state(nf_ctx *ctx, int i, const double *aos, double *dev) {
 }
 
 // device tiles of instance i -> reference-order AoS [N][5]
-int download_state(nf_ctx *ctx, int i, const double *dev, double *aos) {
-    const Inst &I = ctx->inst[i];
-    int rc;
-    if ((rc = ensure_stage(ctx))) return rc;
-    hipLaunchKernelGGL(k_state_out, dim3(I.Npad / BLOCK), dim3(BLOCK), 0, ctx->stream,
-                       dev + (size_t)5 * I.cell0, (const uint32_t *)(ctx->perm_dev + I.cell0), ctx->stage, I.N);
-    HIPC(hipGetLastError());
-    HIPC(ctx->pipe.down(aos, ctx->stage, (size_t)5 * I.N * sizeof(double), ctx->stream));
-    return NF_OK;
-}
 template <typename T>
 int download_state(nf_ctx *ctx, int i, const T *dev, double *aos) {
     const Inst &I = ctx->inst[i];
-    std::vector<T> d((size_t)5 * I.Npad);
-    HIPC(hipStreamSynchronize(ctx->stream));
-    HIPC(hipMemcpy(d.data(), dev + (size_t)5 * I.cell0, d.size() * sizeof(T), hipMemcpyDeviceToHost));
-    for (uint32_t c = 0; c < I.N; ++c)
-        for (int k = 0; k < 5; ++k) aos[5 * (size_t)I.perm[c] + k] = d[tile_index(c, k)];
-    return NF_OK;
-}
-
-// device-cell AoS [cells][rows] of instance i -> reference-order AoS
-int download_aos(nf_ctx *ctx, int i, const double *dev, int rows, double *aos) {
-    const Inst &I = ctx->inst[i];
-    std::vector<double> d((size_t)rows * I.N);
-    HIPC(hipStreamSynchronize(ctx->stream));
-    HIPC(hipMemcpy(d.data(), dev + (size_t)rows * I.cell0, d.size() * sizeof(double), hipMemcpyDeviceToHost));
-    for (uint32_t c = 0; c < I.N; ++c)
-        std::memcpy(aos + (size_t)rows * I.perm[c], &d[(size_t)rows * c], rows * sizeof(double));
+    int rc;
+    if ((rc = ensure_stage(ctx))) return rc;
+    hipLaunchKernelGGL(k_state_out<T>, dim3(I.Npad / BLOCK), dim3(BLOCK), 0, ctx->stream, dev + (size_t)5 * I.cell0,
+                       (const uint32_t *)(ctx->perm_dev + I.cell0), ctx->stage, I.N);
+    HIPC(hipGetLastError());
+    HIPC(ctx->pipe.down(aos, ctx->stage, (size_t)5 * I.N * sizeof(double), ctx->stream));
     return NF_OK;
 }
 
@@ -774,7 +752,7 @@ int prim_all(nf_ctx *ctx) {
 }
 
 // ||R_rho||_2 of every instance's current state into out[n] (host); the
-// update of the stage-1 sweep goes to Ub and is discarded, V = prim(U) after
+// update of the stage-1 sweep goes to Ub and is discarded, V32 = prim(U) after
 int eval_residuals(nf_ctx *ctx, double *out) {
     int rc;
     if ((rc = clear_flags(ctx))) return rc;
@@ -782,7 +760,7 @@ int eval_residuals(nf_ctx *ctx, double *out) {
     if ((rc = run_sweepA(ctx, false, false))) return rc;
     if ((rc = run_sweepB(ctx, 1, ctx->Ua, ctx->Ub, true, false))) return rc;
     if ((rc = reduce(ctx, true, 0.0, ctx->r_eval, false, 0))) return rc;
-    if ((rc = prim_all(ctx))) return rc;
+    if (ctx->mixed && (rc = prim_all(ctx))) return rc;  // (an FP64 sweep B stores no primvars)
     HIPC(hipStreamSynchronize(ctx->stream));
     HIPC(hipMemcpy(out, ctx->r_eval, ctx->n_inst * sizeof(double), hipMemcpyDeviceToHost));
     for (Inst &I : ctx->inst) I.dt_valid = false;
@@ -852,14 +830,19 @@ int set_freestream(nf_ctx *ctx, int i) {
     double V[5], U[5];
     std::memcpy(V, I.Vinf, sizeof V);
     prim_to_cons(V, U);
-    std::vector<double> aos((size_t)5 * I.N);
-    for (uint32_t c = 0; c < I.N; ++c) std::memcpy(&aos[5 * (size_t)c], U, sizeof U);
-    int rc = upload_state(ctx, i, aos.data(), ctx->Ua);
-    if (rc) return rc;
+    auto fill = [&](const double *v, double *dev) {
+        CellState cs;
+        std::memcpy(cs.v, v, sizeof cs.v);
+        hipLaunchKernelGGL(k_state_fill, dim3(I.Npad / BLOCK), dim3(BLOCK), 0, ctx->stream, cs,
+                           dev + (size_t)5 * I.cell0, I.N, I.Npad);
+        return hipGetLastError();
+    };
+    int rc;
+    HIPC(fill(U, ctx->Ua));
     if ((rc = after_state_set(ctx, i, ctx->prm.rk3_zero_old_first_step != 0))) return rc;
     if (!ctx->mixed) {
-        for (uint32_t c = 0; c < I.N; ++c) std::memcpy(&aos[5 * (size_t)c], V, sizeof V);
-        if ((rc = upload_state(ctx, i, aos.data(), ctx->V))) return rc;
+        HIPC(fill(V, ctx->V));
+        HIPC(hipStreamSynchronize(ctx->stream));
     }
     return NF_OK;
 }
@@ -1191,6 +1174,7 @@ int create(int32_t n, const nf_mesh_desc *descs, const nf_params *prms, nf_ctx *
         HIPC(hipMemcpy(ctx->wbox, wbox.data(), wbox.size() * sizeof(float4), hipMemcpyHostToDevice));
     }
     if ((rc = ensure_hist(ctx, 1024))) return rc;
+    if ((rc = ensure_stage(ctx))) return rc;
     for (int i = 0; i < n; ++i)
         if ((rc = set_freestream(ctx, i))) return rc;
     *out = hold.release();
@@ -1553,15 +1537,14 @@ int nf_eval_flux_balance(nf_ctx *ctx) {
         if ((rc = dalloc(ctx, &ctx->psi_aux, 5 * NC))) return rc;
         if ((rc = dalloc(ctx, &ctx->R_aux, 5 * NC))) return rc;
     }
+    if ((rc = ensure_stage(ctx))) return rc;
     if ((rc = clear_flags(ctx))) return rc;
     if ((rc = prim_all(ctx))) return rc;
     if ((rc = run_sweepA(ctx, false, true))) return rc;
+    // (keeping R, the sweep updates nothing.  The dt the last step left on the
+    // device, from prim(U2) for TVD-RK3, stays valid, so an evaluation between
+    // steps does not change the run.)
     if ((rc = run_sweepB(ctx, 1, ctx->Ua, ctx->Ub, false, true))) return rc;
-    // the sweep wrote prim of the discarded update: primvars = prim(U) again,
-    // which is what they were before the call.  The dt the last step left on
-    // the device (from prim(U2) for TVD-RK3) stays valid, so an evaluation
-    // between steps does not change the run.
-    if ((rc = prim_all(ctx))) return rc;
     ctx->aux_valid = true;
     return check_errors(ctx);
 }
@@ -1590,9 +1573,10 @@ int nf_get_field(nf_ctx *ctx, int32_t which, double *out) {
     case NF_FIELD_GRADIENT:
     case NF_FIELD_RESIDUAL:
         if (!ctx->aux_valid) return fail(ctx, NF_E_ARG, "call nf_eval_flux_balance first");
-        if (which == NF_FIELD_LIMITER) return download_aos(ctx, 0, ctx->psi_aux, 5, out);
-        if (which == NF_FIELD_GRADIENT) return download_aos(ctx, 0, ctx->grad_aux, 15, out);
-        return download_aos(ctx, 0, ctx->R_aux, 5, out);
+        // (the sweeps stored them in reference order)
+        HIPC(ctx->pipe.down(out, which == NF_FIELD_LIMITER ? ctx->psi_aux : (which == NF_FIELD_GRADIENT ? ctx->grad_aux : ctx->R_aux),
+                            (which == NF_FIELD_GRADIENT ? 15 : 5) * (size_t)ctx->inst[0].N * sizeof(double), ctx->stream));
+        return NF_OK;
     default:
         return fail(ctx, NF_E_ARG, "unknown field");
     }
