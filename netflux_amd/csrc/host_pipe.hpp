@@ -10,113 +10,169 @@
 // 11.3 ms (14 of them the comparison of U with U_old when both are the same
 // array), nf_get_state into fresh pages 49.0 -> 12.3 ms.
 //
-// Not thread-safe, like the context that owns it; its pinned chunks (at most
-// 32 MB) are made on the first large copy and live as long as their owner.
+// The pinned pieces (8 of 4 MB for each device) belong to a pool, since making
+// them takes longer (1.3 ms) than most copies: a copy borrows those it can
+// get, under a lock, and returns them when its last piece has left; a copy that
+// gets none is a plain one.  The pool is given back with its last user.
 #pragma once
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <atomic>
 #include <cstring>
+#include <map>
 #include <mutex>
 #include <thread>
 #include <vector>
 
 namespace nf {
 
-class HostPipe {
+class PinnedPool {
   public:
-    HostPipe() = default;
-    HostPipe(const HostPipe &) = delete;
-    HostPipe &operator=(const HostPipe &) = delete;
-    ~HostPipe() {
-        for (Slot &q : slot_) {
-            if (q.busy) (void)hipEventSynchronize(q.ev);
-            (void)hipEventDestroy(q.ev);
-            (void)hipHostFree(q.mem);
-        }
-    }
-
-    // device -> host after the work enqueued on s so far; returns when dst holds the data
-    hipError_t down(void *dst, const void *src, size_t bytes, hipStream_t s) {
-        if (bytes >= MIN && ready(bytes)) return run<true>(static_cast<char *>(dst), static_cast<const char *>(src), bytes, s);
-        const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s);
-        return e ? e : hipStreamSynchronize(s);
-    }
-    // host -> device, ordered on s; returns when src may change
-    hipError_t up(void *dst, const void *src, size_t bytes, hipStream_t s) {
-        if (bytes >= MIN && ready(bytes)) return run<false>(static_cast<char *>(dst), static_cast<const char *>(src), bytes, s);
-        const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s);
-        return e ? e : hipStreamSynchronize(s);
-    }
-
-  private:
-    static constexpr size_t CHUNK = 4u << 20, MIN = 2u << 20;  // below MIN the threads cost more than they save
-    static constexpr int SLOTS = 8;
+    static constexpr size_t PIECE = 4u << 20;
     struct Slot {
         char *mem = nullptr;
         hipEvent_t ev = nullptr;
-        bool busy = false;  // the event marks a copy that may still read or write mem
+        int dev = 0;
     };
-    std::vector<Slot> slot_;
+    // (never destroyed: the HIP runtime may be gone when static objects are)
+    static PinnedPool &get() {
+        static PinnedPool *pool = new PinnedPool;
+        return *pool;
+    }
+    void join() {
+        std::lock_guard<std::mutex> lk(mu_);
+        ++users_;
+    }
+    void leave() {
+        std::lock_guard<std::mutex> lk(mu_);
+        if (--users_) return;
+        for (Slot &q : free_) {  // (nothing is borrowed: a user returns what it has before it leaves)
+            (void)hipEventDestroy(q.ev);
+            (void)hipHostFree(q.mem);
+        }
+        free_.clear();
+        made_.clear();
+    }
+    // up to `want` slots of device dev, which is current
+    std::vector<Slot> borrow(int want, int dev) {
+        std::vector<Slot> got;
+        std::lock_guard<std::mutex> lk(mu_);
+        got.reserve(want);
+        int &made = made_[dev];
+        free_.reserve(SLOTS * made_.size());  // room for every slot there can be: giving back cannot fail
+        for (size_t q = free_.size(); q-- > 0 && (int)got.size() < want;)
+            if (free_[q].dev == dev) {
+                got.push_back(free_[q]);
+                free_.erase(free_.begin() + q);
+            }
+        while ((int)got.size() < want && made < SLOTS) {
+            Slot s;
+            s.dev = dev;
+            if (hipHostMalloc(reinterpret_cast<void **>(&s.mem), PIECE, hipHostMallocDefault) != hipSuccess) break;
+            if (hipEventCreateWithFlags(&s.ev, hipEventDisableTiming) != hipSuccess) {
+                (void)hipHostFree(s.mem);
+                break;
+            }
+            got.push_back(s);
+            ++made;
+        }
+        if ((int)got.size() < want) (void)hipGetLastError();  // (fewer pieces, or a plain copy)
+        return got;
+    }
+    void give_back(const std::vector<Slot> &s) {
+        std::lock_guard<std::mutex> lk(mu_);
+        free_.insert(free_.end(), s.begin(), s.end());
+    }
+
+  private:
+    static constexpr int SLOTS = 8;
+    std::mutex mu_;
+    std::vector<Slot> free_;
+    std::map<int, int> made_;
+    int users_ = 0;
+};
+
+class HostPipe {
+  public:
+    HostPipe() { PinnedPool::get().join(); }
+    HostPipe(const HostPipe &) = delete;
+    HostPipe &operator=(const HostPipe &) = delete;
+    ~HostPipe() { PinnedPool::get().leave(); }
+
+    // device -> host after the work enqueued on s so far; returns when dst holds the data
+    hipError_t down(void *dst, const void *src, size_t bytes, hipStream_t s) {
+        return copy<true>(static_cast<char *>(dst), static_cast<const char *>(src), bytes, s);
+    }
+    // host -> device, ordered on s; returns when src may change
+    hipError_t up(void *dst, const void *src, size_t bytes, hipStream_t s) {
+        return copy<false>(static_cast<char *>(dst), static_cast<const char *>(src), bytes, s);
+    }
+
+  private:
+    static constexpr size_t CHUNK = PinnedPool::PIECE, MIN = 2u << 20;  // below MIN the threads cost more than they save
 
     static int slots_for(size_t bytes) {
         const int hw = (int)std::thread::hardware_concurrency();
-        return (int)std::min<size_t>(std::min(SLOTS, std::max(1, hw)), (bytes + CHUNK / 2 - 1) / (CHUNK / 2));
+        return (int)std::min<size_t>(std::min(8, std::max(1, hw)), (bytes + CHUNK / 2 - 1) / (CHUNK / 2));
     }
-    bool ready(size_t bytes) {
-        const size_t want = (size_t)slots_for(bytes);
-        while (slot_.size() < want) {
-            Slot q;
-            if (hipHostMalloc(reinterpret_cast<void **>(&q.mem), CHUNK, hipHostMallocDefault) != hipSuccess) break;
-            if (hipEventCreateWithFlags(&q.ev, hipEventDisableTiming) != hipSuccess) {
-                (void)hipHostFree(q.mem);
-                break;
+    template <bool DOWN>
+    hipError_t copy(char *dst, const char *src, size_t bytes, hipStream_t s) {
+        if (bytes >= MIN) {
+            int dev = 0;
+            hipError_t e = hipGetDevice(&dev);
+            if (e) return e;
+            std::vector<PinnedPool::Slot> slot;
+            try {
+                slot = PinnedPool::get().borrow(slots_for(bytes), dev);
+            } catch (...) {  // out of memory: a plain copy
             }
-            slot_.push_back(q);
+            if (!slot.empty()) {
+                e = run<DOWN>(slot, dev, dst, src, bytes, s);
+                PinnedPool::get().give_back(slot);
+                return e;
+            }
         }
-        if (slot_.size() < want) (void)hipGetLastError();  // (fewer chunks, or a plain copy)
-        return !slot_.empty();
+        const hipError_t e = hipMemcpyAsync(dst, src, bytes, DOWN ? hipMemcpyDeviceToHost : hipMemcpyHostToDevice, s);
+        return e ? e : hipStreamSynchronize(s);
     }
 
     template <bool DOWN>
-    hipError_t run(char *dst, const char *src, size_t bytes, hipStream_t s) {
-        const int T = std::min((int)slot_.size(), slots_for(bytes));
+    hipError_t run(const std::vector<PinnedPool::Slot> &slot, int dev, char *dst, const char *src, size_t bytes,
+                   hipStream_t s) {
+        const int T = (int)slot.size();
         // equal pieces of at most CHUNK, whole pages, a multiple of the threads
         const size_t rounds = (bytes + (size_t)T * CHUNK - 1) / ((size_t)T * CHUNK);
         const size_t piece = std::min(CHUNK, ((bytes + rounds * T - 1) / (rounds * T) + 4095) / 4096 * 4096);
         const size_t n = (bytes + piece - 1) / piece;
-        int dev = 0;
-        hipError_t e0 = hipGetDevice(&dev);
-        if (e0) return e0;
         std::atomic<size_t> next{0};
         std::atomic<int> err{0};
         std::mutex mu;
         auto work = [&](int t) {
-            Slot &q = slot_[t];
+            const PinnedPool::Slot &q = slot[t];
+            bool busy = false;  // the event marks a copy that may still read mem
             hipError_t e = hipSetDevice(dev);
             while (!e && !err.load()) {
                 const size_t c = next.fetch_add(1);
                 if (c >= n) break;
                 const size_t off = c * piece, len = std::min(piece, bytes - off);
-                if (q.busy) e = hipEventSynchronize(q.ev);
+                if (busy) e = hipEventSynchronize(q.ev);
                 if (e) break;
-                q.busy = false;
                 if (!DOWN) std::memcpy(q.mem, src + off, len);
                 {
                     std::lock_guard<std::mutex> lk(mu);  // the event marks this thread's copy
                     e = DOWN ? hipMemcpyAsync(q.mem, src + off, len, hipMemcpyDeviceToHost, s)
                              : hipMemcpyAsync(dst + off, q.mem, len, hipMemcpyHostToDevice, s);
+                    busy = e == hipSuccess;
                     if (!e) e = hipEventRecord(q.ev, s);
                 }
-                if (e) break;
-                q.busy = true;
-                if (DOWN) {
-                    if ((e = hipEventSynchronize(q.ev))) break;
-                    q.busy = false;
-                    std::memcpy(dst + off, q.mem, len);
-                }
+                if (e || !DOWN) continue;
+                e = hipEventSynchronize(q.ev);
+                busy = e != hipSuccess;
+                if (!e) std::memcpy(dst + off, q.mem, len);
             }
+            // the piece goes back to the pool: nothing may use it any more
+            if (busy && hipEventSynchronize(q.ev) != hipSuccess) (void)hipStreamSynchronize(s);
             if (e) err.store((int)e);
         };
         std::vector<std::thread> pool;
