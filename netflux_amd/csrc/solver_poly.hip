@@ -4,16 +4,25 @@
 // slot field with one coalesced load.
 //   w      [6][N]     NONE, or bit 31 = the cell is the face's j side,
 //                     bit 30 = boundary, bits 0-29 = neighbour cell or ghost id
-//   ns     [6][N]     interior: the neighbour's slot of the same face;
-//                     boundary: the boundary type
+//   ns     [6][N]     the neighbour's slot of the same face
 //   geo    [6][6][N]  S of the face (as stored, i -> j), then r of this side
-//   U, U_old, R  [5][N];  V [5][NT] (cells, then ghosts);  FV [6][5][N]
-//   reconstructed face values of each slot;  grad [15][N], psi [5][N]
-// Kernels per stage: prim (U -> V), cell ghosts, sweep A (gradient, min/max,
-// limiter, face values; second order only), sweep B (flux balance and the
-// stage update).  Each follows the CPU solver's loops (src/Solver.cpp:54-230,
-// include/Numerics.hpp:86-292) with the same operations in the same order;
-// gradient, limiter and R are stored only when they are to be exported.
+//   U, R   [5][N];  V [5][NT] (cells, then ghosts);  FV [7][5][P], P = max(N,
+//   ghosts): reconstructed face values of each slot, and (slot 6) the ghosts
+//   of the boundary faces' values;  grad [15][N], psi [5][N]
+// A stage is two kernels: sweep A (gradient, min/max, limiter, face values;
+// second order only; the CFL steps where asked) and sweep B (flux balance,
+// stage update, primvars of the new state, residual sums).  Boundary ghosts
+// are formed at the end of the sweep that stores what they depend on, one face
+// per lane of the block's first lanes (in launches of their own a step took
+// 91.0 against 79.3 us at 12^3, 444 against 437 us at 80^3).  Each follows the CPU solver's loops
+// (src/Solver.cpp:54-230, include/Numerics.hpp:86-292) with the same
+// operations in the same order; gradient, limiter and R are stored only when
+// they are to be exported.
+//
+// U^n stays in Ua (it is U_old of the next stages), stages write Ub, the last
+// one Ua.  Primvars: X of U^n, Y of U1, Z of U2; sweep B of the last stage
+// stores X.  The CFL step of the primvars the last stage reads is the next
+// step's dt (src/Solver.cpp:248), reduced with the residual by one kernel.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -40,44 +49,117 @@ using V3 = Vec3T<double>;
 
 struct PolyDev {
     uint32_t N, NT, G;
+    size_t P;  // plane stride of FV
     const uint32_t *w;
     const uint8_t *ns;
     const double *geo, *vol, *dS;
-    // boundary faces, for the cell ghosts: cell i, ghost j, S, type
+    // boundary faces in device cell order: cell i, its slot, ghost j, S, type
     const uint32_t *bi, *bj;
+    const uint8_t *bslot, *bbc;
     const double *bS;
-    const uint8_t *bbc;
-    const int *stop;  // device-resident run: every kernel returns once it is set (null: no check)
+    const uint32_t *boff;  // [blocks + 1] first boundary face of each block's cells
+    FarField<double> fs;
+    const int *stop;  // kernels return if one of stop[0 .. nstop) is set
+    int nstop;
 };
 constexpr uint32_t BND = 0x40000000u, IDX = 0x3FFFFFFFu;
 
-__device__ __forceinline__ bool stopped(const int *stop) { return stop && *stop; }
+__device__ __forceinline__ bool stopped(const PolyDev &m) {
+    for (int q = 0; q < m.nstop; ++q)
+        if (m.stop[q]) return true;
+    return false;
+}
 
 __device__ __forceinline__ double geo(const PolyDev &m, int s, int q, uint32_t c) {
     return m.geo[((size_t)s * 6 + q) * m.N + c];
 }
 
-__global__ __launch_bounds__(PB) void k_poly_prim(const double *U, double *V, uint32_t N, uint32_t NT,
-                                                  const int *stop) {
+// sum or minimum over the block in a fixed tree; valid in thread 0
+template <bool MIN>
+__device__ __forceinline__ double tree(double v, double *sh) {
+    sh[threadIdx.x] = v;
+    __syncthreads();
+    for (int h = PB / 2; h > 0; h >>= 1) {
+        if ((int)threadIdx.x < h) {
+            const double a = sh[threadIdx.x], b = sh[threadIdx.x + h];
+            sh[threadIdx.x] = MIN ? smin(a, b) : a + b;
+        }
+        __syncthreads();
+    }
+    return sh[0];
+}
+
+// set_constant_ghost_values (src/Solver.cpp:300-330) of boundary face b
+__device__ __forceinline__ void ghost_cell(const PolyDev &m, uint32_t b, double *V) {
+    const uint32_t i = m.bi[b], j = m.bj[b];
+    double vd[5], vg[5];
+#pragma unroll
+    for (int k = 0; k < 5; ++k) vd[k] = V[k * (size_t)m.NT + i];
+    const V3 S = {m.bS[b], m.bS[m.G + b], m.bS[2 * (size_t)m.G + b]};
+    ghost_value<double>((int)m.bbc[b], vd, S, m.fs, vg);
+#pragma unroll
+    for (int k = 0; k < 5; ++k) V[k * (size_t)m.NT + j] = vg[k];
+}
+// ghost of its reconstructed face state (src/Solver.cpp:210-212)
+__device__ __forceinline__ void ghost_face(const PolyDev &m, uint32_t b, double *FV) {
+    const uint32_t i = m.bi[b], s = m.bslot[b];
+    double vd[5], vg[5];
+#pragma unroll
+    for (int k = 0; k < 5; ++k) vd[k] = FV[(s * 5 + k) * m.P + i];
+    const V3 S = {m.bS[b], m.bS[m.G + b], m.bS[2 * (size_t)m.G + b]};
+    ghost_d((int)m.bbc[b], vd, S, m.fs, vg);
+#pragma unroll
+    for (int k = 0; k < 5; ++k) FV[(30 + k) * m.P + (m.bj[b] - m.N)] = vg[k];
+}
+// The block's boundary faces, one per lane of its first lanes.  The range is
+// loaded at the start of a sweep and kept there by the asm: at its end every
+// block would wait for these scalar loads.
+struct BndFaces {
+    uint32_t b0, b1;
+};
+__device__ __forceinline__ BndFaces bnd_faces(const PolyDev &m, uint32_t lb) {
+    BndFaces r{m.boff[lb], m.boff[lb + 1]};
+    asm volatile("" : "+s"(r.b0), "+s"(r.b1));
+    return r;
+}
+template <typename F>
+__device__ __forceinline__ void block_ghosts(BndFaces r, F ghost) {
+    if (r.b0 == r.b1) return;  // the same for the whole block
+    __syncthreads();           // every lane's values are stored
+    for (uint32_t b = r.b0 + threadIdx.x; b < r.b1; b += PB) ghost(b);
+}
+
+__global__ __launch_bounds__(PB) void k_poly_prim(const double *U, double *V, uint32_t N, uint32_t NT) {
     const uint32_t c = blockIdx.x * PB + threadIdx.x;
-    if (c >= N || stopped(stop)) return;
+    if (c >= N) return;
     double u[5], v[5];
     for (int k = 0; k < 5; ++k) u[k] = U[k * (size_t)N + c];
     cons_to_prim_d(u, v);
     for (int k = 0; k < 5; ++k) V[k * (size_t)NT + c] = v[k];
 }
 
-// set_constant_ghost_values (src/Solver.cpp:300-330)
-__global__ __launch_bounds__(PB) void k_poly_ghost(PolyDev m, double *V, FarField<double> fs) {
+__global__ __launch_bounds__(PB) void k_poly_ghost(PolyDev m, double *V) {
     const uint32_t b = blockIdx.x * PB + threadIdx.x;
-    if (b >= m.G || stopped(m.stop)) return;
-    const uint32_t i = m.bi[b], j = m.bj[b];
-    double vd[5], vg[5];
-    for (int k = 0; k < 5; ++k) vd[k] = V[k * (size_t)m.NT + i];
-    const V3 S = {m.bS[b], m.bS[m.G + b], m.bS[2 * (size_t)m.G + b]};
-    ghost_value<double>((int)m.bbc[b], vd, S, fs, vg);
-    for (int k = 0; k < 5; ++k) V[k * (size_t)m.NT + j] = vg[k];
+    if (b < m.G && !stopped(m)) ghost_cell(m, b, V);
 }
+
+// calc_timestep of a cell (src/Solver.cpp:232-274)
+__device__ __forceinline__ double cell_step(const PolyDev &m, uint32_t c, const double *v, double CFL) {
+    const double cs = sound_speed_prim(v);
+    const double sx = (std::fabs(v[1]) + cs) * m.dS[c];
+    const double sy = (std::fabs(v[2]) + cs) * m.dS[(size_t)m.N + c];
+    const double sz = (std::fabs(v[3]) + cs) * m.dS[2 * (size_t)m.N + c];
+    return CFL * m.vol[c] / ((sx + sy) + sz);
+}
+
+struct SweepA {
+    const double *V;
+    int limiter;
+    double *FV;
+    double *grad, *psi;  // exported, or null
+    double CFL;
+    double *dt_part, *dt_cell;  // per-block minimum of the cells' CFL steps, the steps themselves; or null
+};
 
 // Green-Gauss (Numerics.hpp:86-128), max/min (:253-292), Barth (:148-250)
 // and the reconstructed face values (Solver.hpp:81-112) of one cell.  The
@@ -85,11 +167,16 @@ __global__ __launch_bounds__(PB) void k_poly_ghost(PolyDev m, double *V, FarFiel
 // (rdiv: the quotient of a plain division), the Barth limiter takes two
 // divisions per variable over the largest positive and most negative face
 // Delta_2 (barth_psi_hilo), and the face-centroid vectors are read once.
-__global__ __launch_bounds__(PB) void k_poly_sweepA(PolyDev m, const double *V, int limiter, double *FV,
-                                                    double *grad, double *psi) {
-    const uint32_t c = logical_block(blockIdx.x, gridDim.x, 1) * PB + threadIdx.x;  // XCD-contiguous
-    if (c >= m.N || stopped(m.stop)) return;
+// Bound by HBM: 600 bytes per hexahedron (288 of geometry, 240 of face values).
+__global__ __launch_bounds__(PB) void k_poly_sweepA(PolyDev m, SweepA a) {
+    __shared__ double sh[PB];
+    const uint32_t lb = logical_block(blockIdx.x, gridDim.x, 1);  // XCD-contiguous
+    const BndFaces br = bnd_faces(m, lb);
+    if (stopped(m)) return;  // the same for every thread of the block
+    const bool live = lb * PB + threadIdx.x < m.N;
+    const uint32_t c = live ? lb * PB + threadIdx.x : m.N - 1;
     const size_t NT = m.NT, N = m.N;
+    const double *V = a.V;
     double vc[5];
 #pragma unroll
     for (int k = 0; k < 5; ++k) vc[k] = V[k * NT + c];
@@ -145,7 +232,7 @@ __global__ __launch_bounds__(PB) void k_poly_sweepA(PolyDev m, const double *V, 
 #pragma unroll
     for (int k = 0; k < 5; ++k) {
         ps[k] = 1.0;  // SolverData.cpp:17 (no limiter)
-        if (limiter) {
+        if (a.limiter) {
             double hi = 0.0, lo = 0.0;
 #pragma unroll
             for (int s = 0; s < 6; ++s) {
@@ -157,46 +244,89 @@ __global__ __launch_bounds__(PB) void k_poly_sweepA(PolyDev m, const double *V, 
             ps[k] = barth_psi_hilo(hi, lo, vmax[k], vmin[k], vc[k]);
         }
     }
+    if (live) {
 #pragma unroll
-    for (int s = 0; s < 6; ++s) {
-        if (s >= nfc) break;
+        for (int s = 0; s < 6; ++s) {
+            if (s >= nfc) break;
 #pragma unroll
-        for (int k = 0; k < 5; ++k) {
-            const double D = (g[k] * r[s].x + g[k + 5] * r[s].y) + g[k + 10] * r[s].z;
-            FV[((size_t)s * 5 + k) * N + c] = vc[k] + ps[k] * D;
+            for (int k = 0; k < 5; ++k) {
+                const double D = (g[k] * r[s].x + g[k + 5] * r[s].y) + g[k + 10] * r[s].z;
+                a.FV[(s * 5 + k) * m.P + c] = vc[k] + ps[k] * D;
+            }
+        }
+        if (a.grad) {
+            for (int q = 0; q < 15; ++q) a.grad[q * N + c] = g[q];
+            for (int k = 0; k < 5; ++k) a.psi[k * N + c] = ps[k];
         }
     }
-    if (grad) {
-        for (int q = 0; q < 15; ++q) grad[q * N + c] = g[q];
-        for (int k = 0; k < 5; ++k) psi[k * N + c] = ps[k];
+    block_ghosts(br, [&](uint32_t b) { ghost_face(m, b, a.FV); });
+    if (a.dt_part) {
+        const double x = cell_step(m, c, vc, a.CFL);
+        if (a.dt_cell && live) a.dt_cell[c] = x;  // local time stepping: each cell's own CFL step
+        const double t = tree<true>(live ? smin(DBL_MAX, x) : DBL_MAX, sh);
+        if (threadIdx.x == 0) a.dt_part[lb] = t;
     }
 }
 
-struct StageArgs {
+struct SweepB {
     const double *V, *FV;  // FV == nullptr: first order (face values = cell values)
-    double *U;
-    const double *Uo;
-    double *R;     // stored when not null
-    double *Rrho;  // the density flux balance, stored when not null (residual norm)
-    int *bad;
-    int flux;    // 0 Rusanov, 1 HLLC
-    int kind;    // 0: U + dt/vol R, 1: RK3 stage 2, 2: RK3 stage 3, -1: no update
+    const double *U, *Uo;  // state entering the stage, U^n
+    double *Uout;          // (may alias either)
+    double *Vout;          // primvars and cell ghosts of Uout, or null
+    double *R;             // stored when not null
+    double *res_part;      // per-block sums of R_rho^2, or null
+    int *bad;              // cells with a non-finite flux balance are counted, or null
+    int flux;              // 0 Rusanov, 1 HLLC
+    int kind;              // 0: U + dt/vol R, 1: RK3 stage 2, 2: RK3 stage 3, -1: no update
     double dt;
-    const double *dtp;  // the step's dt in device memory (device-resident run), or null: dt
-    const double *dtc;  // per-cell steps (local time stepping), or null
-    FarField<double> fs;
+    const double *dtp;    // the step's dt in device memory (device-resident run), or null: dt
+    const double *dtc;    // per-cell steps (local time stepping), or null
+    const int *zero_old;  // U_old counts as zero while set (the first step)
 };
 
+// the stage update (src/Solver.cpp:83-133) of a cell
+__device__ __forceinline__ void stage_update(const PolyDev &m, const SweepB &a, uint32_t c, bool live, const double *R) {
+    const size_t N = m.N;
+    const double vol = m.vol[c], dt = a.dtc ? a.dtc[c] : (a.dtp ? *a.dtp : a.dt);
+    const bool zero = a.kind > 0 && *a.zero_old;
+    double un[5], v[5];
+#pragma unroll
+    for (int k = 0; k < 5; ++k) {
+        const double u = a.U[k * N + c], uo = a.kind > 0 && !zero ? a.Uo[k * N + c] : 0.0;
+        if (a.kind == 0) un[k] = u + dt / vol * R[k];
+        else if (a.kind == 1) un[k] = 3.0 / 4.0 * uo + 1.0 / 4.0 * u + 1.0 / 4.0 * dt / vol * R[k];
+        else un[k] = 1.0 / 3.0 * uo + 2.0 / 3.0 * u + 2.0 / 3.0 * dt / vol * R[k];
+    }
+    if (live) {
+#pragma unroll
+        for (int k = 0; k < 5; ++k) a.Uout[k * N + c] = un[k];
+        if (a.Vout) {
+            cons_to_prim_d(un, v);
+#pragma unroll
+            for (int k = 0; k < 5; ++k) a.Vout[k * (size_t)m.NT + c] = v[k];
+        }
+    }
+}
+
 // inviscid_fluxes (src/Solver.cpp:144-230) gathered per cell, the validity
-// check (src/SolverData.cpp:66-79) and the stage update (src/Solver.cpp:83-133)
-__global__ __launch_bounds__(PB) void k_poly_sweepB(PolyDev m, StageArgs a) {
-    const uint32_t c = logical_block(blockIdx.x, gridDim.x, 1) * PB + threadIdx.x;  // XCD-contiguous
-    if (c >= m.N || stopped(m.stop)) return;
+// check (src/SolverData.cpp:66-79) and the stage update.  Bound by HBM: about
+// 570 bytes per hexahedron (144 of face vectors, 240 of face values, which
+// the neighbours' reads find in L2).  The primvars stored here instead of in
+// a pass over U, U^n left in place instead of copied to U_old, the residual
+// and dt partials formed where their inputs are in registers: a step of 7
+// launches instead of 17, 102 -> 79 us at 12^3, 234 -> 216 at 64^3, 804 -> 775
+// at 96^3 hexahedra.
+__global__ __launch_bounds__(PB) void k_poly_sweepB(PolyDev m, SweepB a) {
+    __shared__ double sh[PB];
+    const uint32_t lb = logical_block(blockIdx.x, gridDim.x, 1);  // XCD-contiguous
+    const BndFaces br = bnd_faces(m, lb);
+    if (stopped(m)) return;  // the same for every thread of the block
+    const bool live = lb * PB + threadIdx.x < m.N;
+    const uint32_t c = live ? lb * PB + threadIdx.x : m.N - 1;
     const size_t NT = m.NT, N = m.N;
     double R[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
     // slot words first, then every face's loads without waiting on them;
-    // absent slots and boundary faces read the cell's own entries (in
-    // bounds) and are masked afterwards
+    // absent slots read the cell's own entries (in bounds)
     uint32_t w[6], qs[6];
     int nfc = 0;
 #pragma unroll
@@ -209,15 +339,17 @@ __global__ __launch_bounds__(PB) void k_poly_sweepB(PolyDev m, StageArgs a) {
         if (w[s] != NONE) nfc = s + 1;
 #pragma unroll
     for (int s = 0; s < 6; ++s) {
-        const bool inner = s < nfc && !(w[s] & BND);
-        const uint32_t n = inner ? (w[s] & IDX) : c, q = inner ? qs[s] : (uint32_t)s;
+        // the other side: the neighbour's slot of this face, or the ghost
+        const uint32_t id = w[s] & IDX;
+        const bool bnd = s < nfc && (w[s] & BND);
+        const uint32_t n = s < nfc ? (bnd && a.FV ? id - m.N : id) : c, q = s < nfc ? (bnd ? 6u : qs[s]) : (uint32_t)s;
         const V3 S = {geo(m, s, 0, c), geo(m, s, 1, c), geo(m, s, 2, c)};
         double own[5], oth[5], UO[5], UN[5], F[5];
-        for (int k = 0; k < 5; ++k) own[k] = a.FV ? a.FV[((size_t)s * 5 + k) * N + c] : a.V[k * NT + c];
-        for (int k = 0; k < 5; ++k) oth[k] = a.FV ? a.FV[((size_t)q * 5 + k) * N + n] : a.V[k * NT + n];
+#pragma unroll
+        for (int k = 0; k < 5; ++k) own[k] = a.FV ? a.FV[(s * 5 + k) * m.P + c] : a.V[k * NT + c];
+#pragma unroll
+        for (int k = 0; k < 5; ++k) oth[k] = a.FV ? a.FV[(q * 5 + k) * m.P + n] : a.V[k * NT + n];
         if (s >= nfc) break;
-        if (w[s] & BND)  // the cell is the face's i side; ghost of its face value
-            ghost_d((int)qs[s], own, S, a.fs, oth);
         const bool sj = (w[s] & SIDE_J) != 0;
         prim_to_cons(own, UO);
         prim_to_cons(oth, UN);
@@ -236,144 +368,145 @@ __global__ __launch_bounds__(PB) void k_poly_sweepB(PolyDev m, StageArgs a) {
         }
     }
     bool ok = true;
+#pragma unroll
     for (int k = 0; k < 5; ++k) {
-        if (a.R) a.R[k * N + c] = R[k];
+        if (a.R && live) a.R[k * N + c] = R[k];
         ok = ok && std::isfinite(R[k]);
     }
-    if (a.Rrho) a.Rrho[c] = R[0];
-    if (!ok && a.bad) atomicAdd(a.bad, 1);
-    if (a.kind < 0) return;
-    const double vol = m.vol[c], dt = a.dtc ? a.dtc[c] : (a.dtp ? *a.dtp : a.dt);
-    for (int k = 0; k < 5; ++k) {
-        const size_t q = k * N + c;
-        const double u = a.U[q];
-        if (a.kind == 0) a.U[q] = u + dt / vol * R[k];
-        else if (a.kind == 1) a.U[q] = 3.0 / 4.0 * a.Uo[q] + 1.0 / 4.0 * u + 1.0 / 4.0 * dt / vol * R[k];
-        else a.U[q] = 1.0 / 3.0 * a.Uo[q] + 2.0 / 3.0 * u + 2.0 / 3.0 * dt / vol * R[k];
+    if (!ok && a.bad && live) atomicAdd(a.bad, 1);
+    if (a.kind >= 0) {
+        stage_update(m, a, c, live, R);
+        if (a.Vout) block_ghosts(br, [&](uint32_t b) { ghost_cell(m, b, a.Vout); });
+    }
+    if (a.res_part) {
+        const double s = tree<false>(live ? R[0] * R[0] : 0.0, sh);
+        if (threadIdx.x == 0) a.res_part[lb] = s;
     }
 }
 
-// the stage update alone, after the host has checked the flux balance
-__global__ __launch_bounds__(PB) void k_poly_update(PolyDev m, double *U, const double *Uo, const double *R,
-                                                    int kind, double dt_all, const double *dtc) {
-    const uint32_t c = blockIdx.x * PB + threadIdx.x;
-    if (c >= m.N) return;
-    const double vol = m.vol[c], dt = dtc ? dtc[c] : dt_all;
-    for (int k = 0; k < 5; ++k) {
-        const size_t q = k * (size_t)m.N + c;
-        const double u = U[q];
-        if (kind == 0) U[q] = u + dt / vol * R[q];
-        else if (kind == 1) U[q] = 3.0 / 4.0 * Uo[q] + 1.0 / 4.0 * u + 1.0 / 4.0 * dt / vol * R[q];
-        else U[q] = 1.0 / 3.0 * Uo[q] + 2.0 / 3.0 * u + 2.0 / 3.0 * dt / vol * R[q];
-    }
+// the stage update alone, where the flux balance R had no bad cell (m.stop
+// covers its counter)
+__global__ __launch_bounds__(PB) void k_poly_update(PolyDev m, SweepB a) {
+    const uint32_t lb = blockIdx.x;
+    const BndFaces br = bnd_faces(m, lb);
+    if (stopped(m)) return;
+    const bool live = lb * PB + threadIdx.x < m.N;
+    const uint32_t c = live ? lb * PB + threadIdx.x : m.N - 1;
+    double R[5];
+#pragma unroll
+    for (int k = 0; k < 5; ++k) R[k] = a.R[k * (size_t)m.N + c];
+    stage_update(m, a, c, live, R);
+    if (a.Vout) block_ghosts(br, [&](uint32_t b) { ghost_cell(m, b, a.Vout); });
 }
 
-// calc_timestep (src/Solver.cpp:232-274): per-block minimum of the cell steps
-__global__ __launch_bounds__(PB) void k_poly_dt(PolyDev m, const double *V, double CFL, double *part,
-                                                double *dt_cell) {
+// per-block minimum of the cell steps of the primvars V
+__global__ __launch_bounds__(PB) void k_poly_dt(PolyDev m, const double *V, double CFL, double *part, double *dt_cell) {
     __shared__ double sh[PB];
-    if (stopped(m.stop)) return;  // the same for every thread of the block
+    if (stopped(m)) return;  // the same for every thread of the block
     const uint32_t c = blockIdx.x * PB + threadIdx.x;
     double t = DBL_MAX;
     if (c < m.N) {
         double v[5];
         for (int k = 0; k < 5; ++k) v[k] = V[k * (size_t)m.NT + c];
-        const double cs = sound_speed_prim(v);
-        const double sx = (std::fabs(v[1]) + cs) * m.dS[c];
-        const double sy = (std::fabs(v[2]) + cs) * m.dS[(size_t)m.N + c];
-        const double sz = (std::fabs(v[3]) + cs) * m.dS[2 * (size_t)m.N + c];
-        const double x = CFL * m.vol[c] / ((sx + sy) + sz);
-        if (dt_cell) dt_cell[c] = x;  // local time stepping: each cell's own CFL step
+        const double x = cell_step(m, c, v, CFL);
+        if (dt_cell) dt_cell[c] = x;
         t = smin(t, x);
     }
-    sh[threadIdx.x] = t;
-    __syncthreads();
-    for (int h = PB / 2; h > 0; h >>= 1) {
-        if ((int)threadIdx.x < h) sh[threadIdx.x] = smin(sh[threadIdx.x], sh[threadIdx.x + h]);
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) part[blockIdx.x] = sh[0];
+    t = tree<true>(t, sh);
+    if (threadIdx.x == 0) part[blockIdx.x] = t;
 }
 
-// per-block sums of x^2 (the residual norm), fixed order
-__global__ __launch_bounds__(PB) void k_poly_sumsq(const double *x, uint32_t n, double *part, const int *stop) {
-    __shared__ double sh[PB];
-    if (stopped(stop)) return;  // the same for every thread of the block
-    const uint32_t c = blockIdx.x * PB + threadIdx.x;
-    sh[threadIdx.x] = c < n ? x[c] * x[c] : 0.0;
-    __syncthreads();
-    for (int h = PB / 2; h > 0; h >>= 1) {
-        if ((int)threadIdx.x < h) sh[threadIdx.x] += sh[threadIdx.x + h];
-        __syncthreads();
+// Run state on the device: flags [0] stop, [1] converged, [2] invalid dt, [3]
+// steps completed (the index of the step in progress), so a graph of several
+// steps can be replayed unchanged.
+struct RunDev {
+    int *flags;            // null: a step driven from the host
+    double *dtdev;         // the next step's dt
+    double *dts, *hres;    // per step of a run: dt, residual
+    double *runp;          // {drop, ref}: ref is the first residual since the state was set, or negative when this
+                           // run's first step is that residual (a first residual of 0 never converges)
+    int *zero_old;         // U_old counts as zero (before the first step)
+    int *bad;              // [3] bad cells of each stage (checked steps)
+    double *host;          // pinned: residual, dt, bad[3]
+};
+
+// partials in a fixed order: each thread a strided sum (or minimum), then a tree
+template <bool MIN>
+__device__ __forceinline__ double all_parts(const double *part, uint32_t nb, double *sh) {
+    constexpr int Q = 8;  // loads in flight
+    double v = MIN ? DBL_MAX : 0.0;
+    for (uint32_t i0 = threadIdx.x; i0 < nb; i0 += Q * PB) {
+        double x[Q];
+#pragma unroll
+        for (int q = 0; q < Q; ++q) x[q] = part[i0 + q * PB < nb ? i0 + q * PB : i0];
+#pragma unroll
+        for (int q = 0; q < Q; ++q)
+            if (i0 + q * PB < nb) v = MIN ? smin(v, x[q]) : v + x[q];
     }
-    if (threadIdx.x == 0) part[blockIdx.x] = sh[0];
+    return tree<MIN>(v, sh);
+}
+__device__ __forceinline__ bool valid_dt(double dt) { return (dt - dt == 0.0) && dt > 0.0; }
+
+// dt of the first step: minimum of the block partials, or the one in place;
+// and a run's flags, drop and reference
+__global__ __launch_bounds__(PB) void k_poly_begin(RunDev r, const double *part, uint32_t nb, double drop, double ref) {
+    __shared__ double sh[PB];
+    double dt = 0.0;
+    if (part) dt = all_parts<true>(part, nb, sh);
+    if (threadIdx.x) return;
+    if (part) r.dtdev[0] = dt;
+    else dt = r.dtdev[0];
+    r.host[1] = dt;
+    if (!r.flags) return;
+    const bool ok = valid_dt(dt);
+    r.flags[0] = r.flags[2] = ok ? 0 : 1;
+    r.flags[1] = r.flags[3] = 0;
+    r.runp[0] = drop;
+    r.runp[1] = ref;
+    r.dts[0] = dt;
 }
 
-// Device-resident run, one block each.  flags: [0] stop, [1] converged,
-// [2] invalid dt, [3] steps completed (the index of the step in progress), so
-// a graph of several steps can be replayed unchanged.
-// The step's dt: minimum of the block partials (calc_timestep).
-__global__ __launch_bounds__(PB) void k_poly_step_dt(const double *part, uint32_t nb, int *flags, double *dtdev,
-                                                     double *dts) {
-    __shared__ double sh[PB];
-    if (flags[0]) return;
-    const int k = flags[3];  // this step's index: the steps completed so far
-    double t = DBL_MAX;
-    for (uint32_t q = threadIdx.x; q < nb; q += PB) t = smin(t, part[q]);
-    sh[threadIdx.x] = t;
-    __syncthreads();
-    for (int h = PB / 2; h > 0; h >>= 1) {
-        if ((int)threadIdx.x < h) sh[threadIdx.x] = smin(sh[threadIdx.x], sh[threadIdx.x + h]);
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        const double dt = sh[0];
-        dts[k] = dt;
-        if (!((dt - dt == 0.0) && dt > 0.0)) {
-            flags[2] = 1;
-            flags[0] = 1;
-        } else {
-            dtdev[0] = dt;
+// The end of a step, one block: the residual (sum of the block partials, its
+// square root), the drop test, and the next step's dt with its test.
+__global__ __launch_bounds__(PB) void k_poly_end(RunDev r, const double *res_part, const double *dt_part, uint32_t nb) {
+    __shared__ double sh[2][PB];
+    if (r.flags && r.flags[0]) return;
+    const double s = all_parts<false>(res_part, nb, sh[0]), dt = all_parts<true>(dt_part, nb, sh[1]);
+    if (threadIdx.x) return;
+    const double res = sqrt(s);
+    if (!r.flags) {
+        r.host[0] = res;
+        r.host[1] = dt;
+        bool bad = false;
+        for (int q = 0; q < 3; ++q) {
+            bad = bad || r.bad[q];
+            r.host[2 + q] = r.bad[q];
+            r.bad[q] = 0;
         }
+        if (bad) return;
+        *r.zero_old = 0;
+        r.dtdev[0] = dt;
+        return;
+    }
+    const int k = r.flags[3];
+    r.hres[k] = res;
+    r.flags[3] = k + 1;
+    *r.zero_old = 0;
+    r.dtdev[0] = dt;
+    r.dts[k + 1] = dt;
+    const double drop = r.runp[0], ref = r.runp[1];
+    const double r0 = ref >= 0.0 ? ref : r.hres[0];
+    if (drop > 0.0 && r0 > 0.0 && res / r0 <= drop) {
+        r.flags[1] = 1;
+        r.flags[0] = 1;
+    }
+    if (!valid_dt(dt)) {  // an error only if a further step was asked for
+        r.flags[2] = 1;
+        r.flags[0] = 1;
     }
 }
 
-// The step's residual: sum of the block partials in a fixed order (each
-// thread a strided sum, then a tree), its square root, and the drop test.
-// runp = {drop, ref}: ref is the first residual since the state was set, or
-// negative when this run's first step is that residual (the host loop's
-// hist[0]; a first residual of 0 never converges, as there).  Read from
-// device memory so a captured graph serves any drop and reference.
-__global__ __launch_bounds__(PB) void k_poly_step_res(const double *part, uint32_t nb, int *flags, double *hres,
-                                                      const double *runp) {
-    __shared__ double sh[PB];
-    if (flags[0]) return;
-    const int k = flags[3];
-    double v = 0.0;
-    for (uint32_t q = threadIdx.x; q < nb; q += PB) v += part[q];
-    sh[threadIdx.x] = v;
-    __syncthreads();
-    for (int h = PB / 2; h > 0; h >>= 1) {
-        if ((int)threadIdx.x < h) sh[threadIdx.x] += sh[threadIdx.x + h];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        const double r = sqrt(sh[0]);
-        hres[k] = r;
-        flags[3] = k + 1;
-        const double drop = runp[0], ref = runp[1];
-        const double r0 = ref >= 0.0 ? ref : hres[0];
-        if (drop > 0.0 && r0 > 0.0 && r / r0 <= drop) {
-            flags[1] = 1;
-            flags[0] = 1;
-        }
-    }
-}
-
-__global__ __launch_bounds__(PB) void k_poly_copy(double *dst, const double *src, size_t n, const int *stop) {
-    const size_t q = (size_t)blockIdx.x * PB + threadIdx.x;
-    if (q < n && !stopped(stop)) dst[q] = src[q];
-}
+__global__ void k_poly_set(int *p, int v) { *p = v; }
 
 // reference-order AoS [N][cols] <-> [cols][N] in device cell order
 __global__ __launch_bounds__(PB) void k_poly_aos_in(const double *aos, const uint32_t *perm, double *soa, uint32_t N,
@@ -399,22 +532,24 @@ __global__ __launch_bounds__(PB) void k_poly_fill(double *p, double v, size_t n)
 struct PolyPath {
     hipStream_t st = nullptr;
     nf_params prm{};
-    FarField<double> fs{};
     PolyDev m{};
     nf_fv_sizes sizes{};
-    double *U = nullptr, *Uo = nullptr, *V = nullptr, *Ve = nullptr, *FV = nullptr;
-    double *grad = nullptr, *psi = nullptr, *R = nullptr, *part = nullptr;
-    double *Rrho = nullptr;
+    double *Ua = nullptr, *Ub = nullptr, *X = nullptr, *Y = nullptr, *Z = nullptr, *FV = nullptr;
+    double *grad = nullptr, *psi = nullptr, *R = nullptr, *dt_part = nullptr, *res_part = nullptr;
     double *dtc = nullptr;  // [N] per-cell steps (local time stepping)
-    int *flags = nullptr;   // device-resident run flags
-    double *dtdev = nullptr, *dts = nullptr, *hres = nullptr;  // its dt, and per step dt and residual
-    int run_cap = 0;
-    double *runp = nullptr;  // device {drop, ref} of the current run
+    RunDev run{};           // run.flags: set for the kernels of a device-resident run only
+    int *flags = nullptr;
+    int64_t run_cap = 0;
+    uint32_t *boff = nullptr;
     hipGraphExec_t graph = nullptr;  // check_every steps of nf_run, captured once per K and buffers
     int graph_K = 0;
-    int *bad = nullptr;
     bool aux_valid = false;  // grad / psi / R hold nf_eval_flux_balance of the current state
     // run state since the last set_state / set_freestream
+    bool split = false;      // a failed stage left the state in Ub (U_old still in Ua)
+    bool x_prim = false;     // X holds prim of the state, ghosts included
+    bool dt_valid = false;   // dtdev (and dt) hold the next step's dt; else it is that of X
+    bool old_zero = false;   // U_old counts as zero
+    double dt = 0.0;
     // kernel timing (nf_time_kernels): HIP events around each launch
     bool timing = false;
     std::vector<std::pair<const char *, std::pair<hipEvent_t, hipEvent_t>>> pending;
@@ -427,10 +562,15 @@ struct PolyPath {
     double time = 0.0;
     bool converged = false;
     std::vector<void *> owned;
+    double *state() const { return split ? Ub : Ua; }
+    bool second() const { return prm.spatial_order == NF_SECOND_ORDER; }
+    bool rk3() const { return prm.time_scheme == NF_TVD_RK3; }
+    uint32_t blocks() const { return (m.N + PB - 1) / PB; }
     ~PolyPath() {
         if (st) (void)hipStreamSynchronize(st);
         if (graph) (void)hipGraphExecDestroy(graph);
         for (void *p : owned) (void)hipFree(p);
+        if (run.host) (void)hipHostFree(run.host);
     }
 };
 
@@ -516,72 +656,141 @@ int tflush(PolyPath *P, std::string &err) {
     return NF_OK;
 }
 
-// evaluate_flux_balance of U into R (and the stage update when kind >= 0):
-// primvars into V, ghosts, sweep A for second order, sweep B
-// lts_dt: also store each cell's CFL step of these primvars (first stage of a
-// locally time-stepped step); the update then uses the per-cell steps
-// stop, dtp: device-resident run (kernels return once *stop is set; the dt is
-// read from *dtp)
-int flux_balance(PolyPath *P, double *V, int kind, double dt, bool aux, bool res, bool lts_dt, std::string &err,
-                 const int *stop = nullptr, const double *dtp = nullptr) {
-    PolyDev m = P->m;
-    m.stop = stop;
-    const bool check = P->prm.check_physical_validity != 0;
+// primvars of U into V, cell ghosts included.  timed: one launch each in the
+// kernel timing
+int prim_of(PolyPath *P, const double *U, double *V, bool timed, std::string &err) {
     int rc;
     hipEvent_t e = nullptr;
-    if ((rc = tstart(P, &e, err))) return rc;
-    hipLaunchKernelGGL(k_poly_prim, grid(m.N), dim3(PB), 0, P->st, (const double *)P->U, V, m.N, m.NT, stop);
-    if ((rc = tstop(P, "poly_prim", e, err)) || (rc = tstart(P, &e, err))) return rc;
-    if (m.G) hipLaunchKernelGGL(k_poly_ghost, grid(m.G), dim3(PB), 0, P->st, m, V, P->fs);
-    if ((rc = tstop(P, "poly_ghost", e, err))) return rc;
-    const bool lts = P->prm.local_time_step != 0 && kind >= 0;
-    if (lts_dt)
-        hipLaunchKernelGGL(k_poly_dt, grid(m.N), dim3(PB), 0, P->st, m, (const double *)V, P->prm.CFL, P->part,
-                           P->dtc);
-    const bool second = P->prm.spatial_order == NF_SECOND_ORDER;
-    if (second) {
-        if ((rc = tstart(P, &e, err))) return rc;
-        hipLaunchKernelGGL(k_poly_sweepA, grid(m.N), dim3(PB), 0, P->st, m, (const double *)V,
-                           P->prm.limiter != NF_LIMITER_NONE ? 1 : 0, P->FV, aux ? P->grad : nullptr,
-                           aux ? P->psi : nullptr);
-        if ((rc = tstop(P, "poly_sweepA", e, err))) return rc;
+    if (timed && (rc = tstart(P, &e, err))) return rc;
+    hipLaunchKernelGGL(k_poly_prim, grid(P->m.N), dim3(PB), 0, P->st, U, V, P->m.N, P->m.NT);
+    if (timed && ((rc = tstop(P, "poly_prim", e, err)) || (rc = tstart(P, &e, err)))) return rc;
+    if (P->m.G) {
+        PolyDev m = P->m;
+        m.nstop = 0;
+        hipLaunchKernelGGL(k_poly_ghost, grid(m.G), dim3(PB), 0, P->st, m, V);
     }
-    StageArgs a;
-    a.V = V;
-    a.FV = second ? P->FV : nullptr;
-    a.U = P->U;
-    a.Uo = P->Uo;
-    a.R = (aux || check) ? P->R : nullptr;
-    a.Rrho = res ? P->Rrho : nullptr;
-    a.bad = check ? P->bad : nullptr;
-    a.flux = P->prm.inv_flux_scheme == NF_FLUX_HLLC ? 1 : 0;
-    a.kind = check ? -1 : kind;
-    a.dt = dt;
-    a.dtp = dtp;
-    a.dtc = lts ? P->dtc : nullptr;
-    a.fs = P->fs;
-    if (check) PHIP(hipMemsetAsync(P->bad, 0, sizeof(int), P->st));
-    if ((rc = tstart(P, &e, err))) return rc;
-    hipLaunchKernelGGL(k_poly_sweepB, grid(m.N), dim3(PB), 0, P->st, m, a);
+    if (timed && (rc = tstop(P, "poly_ghost", e, err))) return rc;
     PHIP(hipGetLastError());
-    if ((rc = tstop(P, "poly_sweepB", e, err))) return rc;
-    if (check) {
-        int nbad = 0;
-        PHIP(hipMemcpyAsync(&nbad, P->bad, sizeof(int), hipMemcpyDeviceToHost, P->st));
-        PHIP(hipStreamSynchronize(P->st));
-        if (nbad > 0) {
-            err = std::to_string(nbad) + " cells with unphysical values detected in the flux_balance field of the "
-                                         "Euler solver";
-            return NF_E_NONPHYSICAL;
-        }
-        if (kind >= 0) {
-            hipLaunchKernelGGL(k_poly_update, grid(m.N), dim3(PB), 0, P->st, m, P->U, (const double *)P->Uo,
-                               (const double *)P->R, kind, dt, (const double *)a.dtc);
-            PHIP(hipGetLastError());
-        }
-    }
     return NF_OK;
 }
+
+// X = prim of the state (where it is not already)
+int ensure_x(PolyPath *P, std::string &err) {
+    if (P->x_prim) return NF_OK;
+    const int rc = prim_of(P, P->state(), P->X, false, err);
+    P->x_prim = rc == NF_OK;
+    return rc;
+}
+
+// one flux balance from the primvars V: sweep A for second order, sweep B.
+// a: what sweep B does with it; dt_part, dt_cell: the CFL steps of V too
+int flux_balance(PolyPath *P, const PolyDev &m, const double *V, SweepB a, bool aux, double *dt_part, double *dt_cell,
+                 std::string &err) {
+    int rc;
+    hipEvent_t e = nullptr;
+    if (P->second()) {
+        if ((rc = tstart(P, &e, err))) return rc;
+        const SweepA x{V, P->prm.limiter != NF_LIMITER_NONE ? 1 : 0, P->FV, aux ? P->grad : nullptr,
+                       aux ? P->psi : nullptr, P->prm.CFL, dt_part, dt_cell};
+        hipLaunchKernelGGL(k_poly_sweepA, dim3(P->blocks()), dim3(PB), 0, P->st, m, x);
+        if ((rc = tstop(P, "poly_sweepA", e, err))) return rc;
+    } else if (dt_part) {
+        hipLaunchKernelGGL(k_poly_dt, dim3(P->blocks()), dim3(PB), 0, P->st, m, V, P->prm.CFL, dt_part, dt_cell);
+    }
+    a.V = V;
+    a.FV = P->second() ? P->FV : nullptr;
+    a.flux = P->prm.inv_flux_scheme == NF_FLUX_HLLC ? 1 : 0;
+    a.zero_old = P->run.zero_old;
+    if ((rc = tstart(P, &e, err))) return rc;
+    hipLaunchKernelGGL(k_poly_sweepB, dim3(P->blocks()), dim3(PB), 0, P->st, m, a);
+    PHIP(hipGetLastError());
+    return tstop(P, "poly_sweepB", e, err);
+}
+
+// The stages of one step (Solver::step, src/Solver.cpp:34-52, 83-133): dt
+// given, or (device-resident run) from dtdev, with kernels that return once
+// flags[0] is set.  With the flux-balance check (host-driven steps) an update
+// runs only where no cell of its or an earlier stage was bad.  Leaves the
+// partials of the residual and of the next dt.
+int stages(PolyPath *P, bool on_device, double dt, std::string &err) {
+    const bool rk3 = P->rk3(), second = P->second(), lts = P->prm.local_time_step != 0;
+    const bool check = P->prm.check_physical_validity != 0;
+    const int n = rk3 ? 3 : 1;
+    int rc;
+    if ((rc = ensure_x(P, err))) return rc;
+    // (a first-order Euler step's sweep B reads its neighbours' values in X)
+    const bool store_x = rk3 || second;
+    double *const Vin[3] = {P->X, P->Y, P->Z};
+    for (int s = 0; s < n; ++s) {
+        const bool last = s + 1 == n;
+        PolyDev m = P->m;
+        m.stop = on_device ? P->flags : P->run.bad;
+        m.nstop = on_device ? 1 : (check ? s : 0);
+        SweepB a{};
+        a.U = s == 0 ? P->state() : P->Ub;
+        a.Uo = P->Ua;
+        a.Uout = last ? P->Ua : P->Ub;
+        a.Vout = last ? (store_x ? P->X : nullptr) : Vin[s + 1];
+        a.R = check ? P->R : nullptr;
+        a.res_part = s == 0 ? P->res_part : nullptr;
+        a.bad = check ? P->run.bad + s : nullptr;
+        a.kind = check ? -1 : s;
+        a.dt = dt;
+        a.dtp = on_device ? P->run.dtdev : nullptr;
+        a.dtc = lts ? P->dtc : nullptr;
+        // (kernel timing: the primvars and ghosts of the stage in launches of their own)
+        if (P->timing && (rc = prim_of(P, a.U, Vin[s], true, err))) return rc;
+        if ((rc = flux_balance(P, m, Vin[s], a, false, last || (lts && s == 0) ? P->dt_part : nullptr,
+                               lts && s == 0 ? P->dtc : nullptr, err)))
+            return rc;
+        if (check) {
+            m.nstop = s + 1;
+            a.kind = s;
+            a.zero_old = P->run.zero_old;
+            hipLaunchKernelGGL(k_poly_update, dim3(P->blocks()), dim3(PB), 0, P->st, m, a);
+        }
+    }
+    P->x_prim = store_x;
+    PHIP(hipGetLastError());
+    return NF_OK;
+}
+
+int step_end(PolyPath *P, bool on_device, std::string &err) {
+    RunDev r = P->run;
+    r.flags = on_device ? P->flags : nullptr;
+    hipLaunchKernelGGL(k_poly_end, dim3(1), dim3(PB), 0, P->st, r, (const double *)P->res_part,
+                       (const double *)P->dt_part, P->blocks());
+    PHIP(hipGetLastError());
+    return NF_OK;
+}
+
+// dt of the first step where it is not in place, and (on_device) a run's start
+int begin(PolyPath *P, bool on_device, double drop, double ref, std::string &err) {
+    RunDev r = P->run;
+    r.flags = on_device ? P->flags : nullptr;
+    if (!P->dt_valid) {
+        PolyDev m = P->m;
+        m.nstop = 0;
+        hipLaunchKernelGGL(k_poly_dt, dim3(P->blocks()), dim3(PB), 0, P->st, m, (const double *)P->X, P->prm.CFL,
+                           P->dt_part, (double *)nullptr);
+    }
+    hipLaunchKernelGGL(k_poly_begin, dim3(1), dim3(PB), 0, P->st, r,
+                       (const double *)(P->dt_valid ? nullptr : P->dt_part), P->blocks(), drop, ref);
+    PHIP(hipGetLastError());
+    return NF_OK;
+}
+
+int set_old_zero(PolyPath *P, bool zero, std::string &err) {
+    P->old_zero = zero;
+    hipLaunchKernelGGL(k_poly_set, dim3(1), dim3(1), 0, P->st, P->run.zero_old, zero ? 1 : 0);
+    PHIP(hipGetLastError());
+    return NF_OK;
+}
+
+std::string bad_cells(int n) {
+    return std::to_string(n) + " cells with unphysical values detected in the flux_balance field of the Euler solver";
+}
+
 }  // namespace
 
 int poly_create(const PrimalMesh &pm, const FVGrid &g, const nf_params &p, hipStream_t st, PolyPath **out,
@@ -596,7 +805,6 @@ int poly_create(const PrimalMesh &pm, const FVGrid &g, const nf_params &p, hipSt
     PolyPath *P = hold.get();
     P->st = st;
     P->prm = p;
-    P->fs = make_farfield<double>(p.primvars_inf);
     const uint32_t N = g.N, NT = g.NT, Fint = g.Fint, F = g.F;
     P->sizes = {N, NT, Fint, F, (uint32_t)g.pfirst.size()};
     if (NT - 1 > IDX) {
@@ -618,11 +826,17 @@ int poly_create(const PrimalMesh &pm, const FVGrid &g, const nf_params &p, hipSt
     std::vector<uint8_t> ns((size_t)6 * N, 0), cnt(N, 0);
     std::vector<double> geo((size_t)36 * N, 0.0);
     const uint32_t G = F - Fint;
-    std::vector<uint32_t> bi(G), bj(G);
+    // boundary faces in device cell order: bat[b] = reference boundary face
+    std::vector<uint32_t> bat(G), bpos(G);
+    for (uint32_t b = 0; b < G; ++b) bat[b] = b;
+    auto bcell = [&](uint32_t b) { return iperm[g.ij[2 * (size_t)(Fint + b)]]; };
+    std::stable_sort(bat.begin(), bat.end(), [&](uint32_t a, uint32_t b) { return bcell(a) < bcell(b); });
+    for (uint32_t b = 0; b < G; ++b) bpos[bat[b]] = b;
+    std::vector<uint32_t> bi(G), bj(G), boff((N + PB - 1) / PB + 1, 0);
     std::vector<double> bS((size_t)3 * G);
-    std::vector<uint8_t> bbc(G);
+    std::vector<uint8_t> bbc(G), bslot(G);
     for (size_t q = 0; q < g.pfirst.size(); ++q)
-        for (uint32_t f = g.pfirst[q]; f < g.pfirst[q] + g.pn[q]; ++f) bbc[f - Fint] = (uint8_t)g.pbc[q];
+        for (uint32_t f = g.pfirst[q]; f < g.pfirst[q] + g.pn[q]; ++f) bbc[bpos[f - Fint]] = (uint8_t)g.pbc[q];
     auto put_geo = [&](uint32_t c, int s, uint32_t f, const std::vector<double> &r) {
         for (int d = 0; d < 3; ++d) {
             geo[((size_t)s * 6 + d) * N + c] = g.S[3 * (size_t)f + d];
@@ -645,41 +859,53 @@ int poly_create(const PrimalMesh &pm, const FVGrid &g, const nf_params &p, hipSt
             ns[(size_t)sj * N + j] = (uint8_t)si;
             put_geo(j, sj, f, g.rj);
         } else {
-            const uint32_t b = f - Fint;
+            const uint32_t b = bpos[f - Fint];
             w[(size_t)si * N + i] = j | BND;
-            ns[(size_t)si * N + i] = bbc[b];
             bi[b] = i;
             bj[b] = j;
+            bslot[b] = (uint8_t)si;
+            boff[i / PB + 1]++;
             for (int d = 0; d < 3; ++d) bS[(size_t)d * G + b] = g.S[3 * (size_t)f + d];
         }
         put_geo(i, si, f, g.ri);
     }
+    for (size_t q = 1; q < boff.size(); ++q) boff[q] += boff[q - 1];
     std::vector<double> vol(N), dS((size_t)3 * N);
     for (uint32_t c = 0; c < N; ++c) {
         vol[c] = g.vol[P->perm[c]];
         for (int d = 0; d < 3; ++d) dS[d * (size_t)N + c] = g.dS[3 * (size_t)P->perm[c] + d];
     }
     uint32_t *dw, *dbi, *dbj;
-    uint8_t *dns, *dbbc;
+    uint8_t *dns, *dbbc, *dbslot;
     double *dgeo, *dvol, *ddS, *dbS;
+    const size_t plane = std::max(N, G);
+    const uint32_t nblk = (N + PB - 1) / PB;
     int rc;
     if ((rc = alloc(P, &dw, w.size(), err)) || (rc = alloc(P, &dns, ns.size(), err)) ||
         (rc = alloc(P, &dgeo, geo.size(), err)) || (rc = alloc(P, &dvol, N, err)) ||
         (rc = alloc(P, &ddS, 3 * (size_t)N, err)) || (rc = alloc(P, &dbi, G, err)) || (rc = alloc(P, &dbj, G, err)) ||
-        (rc = alloc(P, &dbS, 3 * (size_t)G, err)) || (rc = alloc(P, &dbbc, G, err)))
+        (rc = alloc(P, &dbS, 3 * (size_t)G, err)) || (rc = alloc(P, &dbbc, G, err)) ||
+        (rc = alloc(P, &dbslot, G, err)) || (rc = alloc(P, &P->boff, boff.size(), err)))
         return rc;
     if ((rc = upload(dw, w, err)) || (rc = upload(dns, ns, err)) || (rc = upload(dgeo, geo, err)) ||
         (rc = upload(dvol, vol, err)) || (rc = upload(ddS, dS, err)) || (rc = upload(dbi, bi, err)) ||
-        (rc = upload(dbj, bj, err)) || (rc = upload(dbS, bS, err)) || (rc = upload(dbbc, bbc, err)))
+        (rc = upload(dbj, bj, err)) || (rc = upload(dbS, bS, err)) || (rc = upload(dbbc, bbc, err)) ||
+        (rc = upload(dbslot, bslot, err)) || (rc = upload(P->boff, boff, err)))
         return rc;
-    P->m = {N, NT, G, dw, dns, dgeo, dvol, ddS, dbi, dbj, dbS, dbbc};
-    if ((rc = alloc(P, &P->U, 5 * (size_t)N, err)) || (rc = alloc(P, &P->Uo, 5 * (size_t)N, err)) ||
-        (rc = alloc(P, &P->V, 5 * (size_t)NT, err)) || (rc = alloc(P, &P->Ve, 5 * (size_t)NT, err)) ||
-        (rc = alloc(P, &P->FV, 30 * (size_t)N, err)) || (rc = alloc(P, &P->grad, 15 * (size_t)N, err)) ||
-        (rc = alloc(P, &P->psi, 5 * (size_t)N, err)) || (rc = alloc(P, &P->R, 5 * (size_t)N, err)) ||
-        (rc = alloc(P, &P->part, (N + PB - 1) / PB, err)) || (rc = alloc(P, &P->bad, 1, err)) ||
-        (rc = alloc(P, &P->Rrho, N, err)) || (rc = alloc(P, &P->dtc, N, err)))
+    P->m = {N, NT, G, plane, dw, dns, dgeo, dvol, ddS, dbi, dbj, dbslot, dbbc, dbS,
+            P->boff, make_farfield<double>(p.primvars_inf), nullptr, 0};
+    if ((rc = alloc(P, &P->Ua, 5 * (size_t)N, err)) || (rc = alloc(P, &P->Ub, 5 * (size_t)N, err)) ||
+        (rc = alloc(P, &P->X, 5 * (size_t)NT, err)) || (rc = alloc(P, &P->Y, 5 * (size_t)NT, err)) ||
+        (rc = alloc(P, &P->Z, 5 * (size_t)NT, err)) || (rc = alloc(P, &P->FV, 35 * plane, err)) ||
+        (rc = alloc(P, &P->grad, 15 * (size_t)N, err)) || (rc = alloc(P, &P->psi, 5 * (size_t)N, err)) ||
+        (rc = alloc(P, &P->R, 5 * (size_t)N, err)) || (rc = alloc(P, &P->dt_part, nblk, err)) ||
+        (rc = alloc(P, &P->res_part, nblk, err)) || (rc = alloc(P, &P->dtc, N, err)) ||
+        (rc = alloc(P, &P->flags, 4, err)) || (rc = alloc(P, &P->run.dtdev, 1, err)) ||
+        (rc = alloc(P, &P->run.runp, 2, err)) || (rc = alloc(P, &P->run.zero_old, 1, err)) ||
+        (rc = alloc(P, &P->run.bad, 3, err)))
         return rc;
+    PHIP(hipMemset(P->run.bad, 0, 3 * sizeof(int)));
+    PHIP(hipHostMalloc(reinterpret_cast<void **>(&P->run.host), 8 * sizeof(double), hipHostMallocDefault));
     if ((rc = poly_set_freestream(P, err))) return rc;
     *out = hold.release();
     return NF_OK;
@@ -695,6 +921,7 @@ static void reset_run(PolyPath *P) {
     P->time = 0.0;
     P->converged = false;
     P->aux_valid = false;
+    P->split = P->dt_valid = P->x_prim = false;
 }
 
 int poly_set_freestream(PolyPath *P, std::string &err) {
@@ -703,15 +930,13 @@ int poly_set_freestream(PolyPath *P, std::string &err) {
     double U[5];
     prim_to_cons(P->prm.primvars_inf, U);
     for (int k = 0; k < 5; ++k) {
-        hipLaunchKernelGGL(k_poly_fill, grid(N), dim3(PB), 0, P->st, P->U + k * (size_t)N, U[k], (size_t)N);
-        hipLaunchKernelGGL(k_poly_fill, grid(N), dim3(PB), 0, P->st, P->V + k * (size_t)P->m.NT,
+        hipLaunchKernelGGL(k_poly_fill, grid(N), dim3(PB), 0, P->st, P->Ua + k * (size_t)N, U[k], (size_t)N);
+        hipLaunchKernelGGL(k_poly_fill, grid(N), dim3(PB), 0, P->st, P->X + k * (size_t)P->m.NT,
                            P->prm.primvars_inf[k], (size_t)N);
     }
-    if (P->prm.rk3_zero_old_first_step)
-        hipLaunchKernelGGL(k_poly_fill, grid(5 * (size_t)N), dim3(PB), 0, P->st, P->Uo, 0.0, 5 * (size_t)N);
-    else
-        PHIP(hipMemcpyAsync(P->Uo, P->U, 5 * (size_t)N * 8, hipMemcpyDeviceToDevice, P->st));
-    PHIP(hipGetLastError());
+    // (X is V_inf, which the first dt is taken from, and not prim(U) bit for bit)
+    int rc;
+    if ((rc = set_old_zero(P, P->prm.rk3_zero_old_first_step != 0, err))) return rc;
     PHIP(hipStreamSynchronize(P->st));
     return NF_OK;
 }
@@ -730,28 +955,21 @@ int poly_set_state(PolyPath *P, const double *U, const double *U_old, std::strin
     }
     int rc;
     reset_run(P);
-    if ((rc = put_soa(P, P->U, U, 5, err))) return rc;
-    hipLaunchKernelGGL(k_poly_prim, grid(N), dim3(PB), 0, P->st, (const double *)P->U, P->V, N, P->m.NT,
-                       (const int *)nullptr);
-    if (zero)
-        hipLaunchKernelGGL(k_poly_fill, grid(5 * (size_t)N), dim3(PB), 0, P->st, P->Uo, 0.0, 5 * (size_t)N);
-    else
-        PHIP(hipMemcpyAsync(P->Uo, P->U, 5 * (size_t)N * 8, hipMemcpyDeviceToDevice, P->st));
-    PHIP(hipGetLastError());
+    if ((rc = put_soa(P, P->Ua, U, 5, err)) || (rc = ensure_x(P, err)) || (rc = set_old_zero(P, zero, err))) return rc;
     PHIP(hipStreamSynchronize(P->st));
     return NF_OK;
 }
 
+// the dt the last step left, or that of the primvars as set
 int poly_calc_timestep(PolyPath *P, double *dt_out, std::string &err) {
-    const uint32_t nb = (P->m.N + PB - 1) / PB;
-    hipLaunchKernelGGL(k_poly_dt, dim3(nb), dim3(PB), 0, P->st, P->m, (const double *)P->V, P->prm.CFL, P->part,
-                       (double *)nullptr);
-    PHIP(hipGetLastError());
-    std::vector<double> part(nb);
-    PHIP(hipMemcpyAsync(part.data(), P->part, nb * 8, hipMemcpyDeviceToHost, P->st));
-    PHIP(hipStreamSynchronize(P->st));
-    double dt = DBL_MAX;
-    for (double x : part) dt = smin(dt, x);
+    int rc;
+    if (!P->dt_valid) {
+        if ((rc = begin(P, false, 0.0, 0.0, err))) return rc;
+        PHIP(hipStreamSynchronize(P->st));
+        P->dt = P->run.host[1];
+        P->dt_valid = true;
+    }
+    const double dt = P->dt;
     if (dt_out) *dt_out = dt;
     if (!((dt - dt == 0.0) && dt > 0.0)) {
         char buf[96];
@@ -762,47 +980,59 @@ int poly_calc_timestep(PolyPath *P, double *dt_out, std::string &err) {
     return NF_OK;
 }
 
-// Solver::step (src/Solver.cpp:34-52, 83-133)
+// Solver::step (src/Solver.cpp:34-52, 83-133), one synchronisation
 int poly_step(PolyPath *P, double dt, std::string &err) {
     int rc;
     P->aux_valid = false;
-    const bool rk3 = P->prm.time_scheme == NF_TVD_RK3, lts = P->prm.local_time_step != 0;
-    // the residual is the flux balance of U^n (first stage), as in the batched path
-    if ((rc = flux_balance(P, P->V, 0, dt, false, true, lts, err))) return rc;
-    if (rk3) {
-        if ((rc = flux_balance(P, P->V, 1, dt, false, false, false, err))) return rc;
-        if ((rc = flux_balance(P, P->V, 2, dt, false, false, false, err))) return rc;
-    }
-    PHIP(hipMemcpyAsync(P->Uo, P->U, 5 * (size_t)P->m.N * 8, hipMemcpyDeviceToDevice, P->st));
-    // residual norm ||R_rho||_2 of the first stage
-    const uint32_t nb = (P->m.N + PB - 1) / PB;
-    hipLaunchKernelGGL(k_poly_sumsq, dim3(nb), dim3(PB), 0, P->st, (const double *)P->Rrho, P->m.N, P->part,
-                       (const int *)nullptr);
-    PHIP(hipGetLastError());
-    std::vector<double> part(nb);
-    PHIP(hipMemcpyAsync(part.data(), P->part, nb * 8, hipMemcpyDeviceToHost, P->st));
+    if ((rc = stages(P, false, dt, err)) || (rc = step_end(P, false, err))) return rc;
     PHIP(hipStreamSynchronize(P->st));
-    // the summation order of k_poly_step_res, so both loops give the same bits
-    std::vector<double> acc(PB, 0.0);
-    for (uint32_t q = 0; q < nb; ++q) acc[q % PB] += part[q];
-    for (int h = PB / 2; h > 0; h >>= 1)
-        for (int t = 0; t < h; ++t) acc[t] += acc[t + h];
-    P->hist.push_back(std::sqrt(acc[0]));
+    for (int s = 0; s < 3; ++s) {
+        const int n = (int)P->run.host[2 + s];
+        if (n == 0) continue;
+        // the state is the failed stage's input, U_old what it was
+        P->split = P->split || s > 0;
+        P->x_prim = P->dt_valid = false;
+        if ((rc = ensure_x(P, err))) return rc;
+        err = bad_cells(n);
+        return NF_E_NONPHYSICAL;
+    }
+    P->hist.push_back(P->run.host[0]);  // the flux balance of U^n (first stage), as in the batched path
     P->time += dt;
+    P->dt = P->run.host[1];
+    P->dt_valid = true;
+    P->split = P->old_zero = false;
     return NF_OK;
 }
 
-// the flux balance of the current state, once, with its own primvar buffer:
-// the primvars a following calc_timestep reads are left as the last step set them
+// the flux balance of the current state, once, with a primvar buffer of the
+// stages: those the next dt or step reads are left as the last step set them
 int poly_eval_flux_balance(PolyPath *P, std::string &err) {
     int rc;
-    if ((rc = flux_balance(P, P->Ve, -1, 0.0, true, false, false, err))) return rc;
+    const bool check = P->prm.check_physical_validity != 0, timing = P->timing;
+    PolyDev m = P->m;
+    m.nstop = 0;
+    SweepB a{};
+    a.R = P->R;
+    a.bad = check ? P->run.bad : nullptr;
+    a.kind = -1;
+    P->timing = false;
+    rc = prim_of(P, P->state(), P->Y, false, err);
+    if (!rc) rc = flux_balance(P, m, P->Y, a, true, nullptr, nullptr, err);
+    P->timing = timing;
+    if (rc) return rc;
+    int bad = 0;
+    if (check) PHIP(hipMemcpyAsync(&bad, P->run.bad, sizeof bad, hipMemcpyDeviceToHost, P->st));
     PHIP(hipStreamSynchronize(P->st));
+    if (bad) {
+        PHIP(hipMemset(P->run.bad, 0, sizeof bad));
+        err = bad_cells(bad);
+        return NF_E_NONPHYSICAL;
+    }
     P->aux_valid = true;
     return NF_OK;
 }
 
-int poly_get_state(PolyPath *P, double *U, std::string &err) { return get_soa(P, P->U, 5, U, err); }
+int poly_get_state(PolyPath *P, double *U, std::string &err) { return get_soa(P, P->state(), 5, U, err); }
 
 // The Driver loop (calc_timestep, step) for n steps, stopping after the step
 // whose residual norm is at most drop times the first step's; a run that has
@@ -845,7 +1075,9 @@ static int poly_run_host(PolyPath *P, const nf_run_opts *o, nf_run_stats *stats,
     return rc;
 }
 
-// HIP-event durations of each kernel over n steps of the Driver loop
+// HIP-event durations of each kernel over n steps of the Driver loop, with
+// each stage's primvars and cell ghosts formed once more by the launches that
+// form them after a state change
 int poly_time_kernels(PolyPath *P, int32_t n_steps, nf_kernel_time *out, int32_t max, int32_t *n_out,
                       std::string &err) {
     if (n_steps < 1 || !out) return NF_E_ARG;
@@ -875,29 +1107,9 @@ int poly_time_kernels(PolyPath *P, int32_t n_steps, nf_kernel_time *out, int32_t
 // One step of the device-resident run: the same kernels and values as
 // calc_timestep + step, with dt, residual and the stop test on the device.
 static int enqueue_run_step(PolyPath *P, std::string &err) {
-    PolyDev m = P->m;
-    m.stop = P->flags;
-    const uint32_t nb = (m.N + PB - 1) / PB;
-    hipLaunchKernelGGL(k_poly_dt, dim3(nb), dim3(PB), 0, P->st, m, (const double *)P->V, P->prm.CFL, P->part,
-                       (double *)nullptr);
-    hipLaunchKernelGGL(k_poly_step_dt, dim3(1), dim3(PB), 0, P->st, (const double *)P->part, nb, P->flags,
-                       P->dtdev, P->dts);
-    PHIP(hipGetLastError());
-    const bool rk3 = P->prm.time_scheme == NF_TVD_RK3, lts = P->prm.local_time_step != 0;
     int rc;
-    if ((rc = flux_balance(P, P->V, 0, 0.0, false, true, lts, err, P->flags, P->dtdev))) return rc;
-    if (rk3) {
-        if ((rc = flux_balance(P, P->V, 1, 0.0, false, false, false, err, P->flags, P->dtdev))) return rc;
-        if ((rc = flux_balance(P, P->V, 2, 0.0, false, false, false, err, P->flags, P->dtdev))) return rc;
-    }
-    hipLaunchKernelGGL(k_poly_copy, grid(5 * (size_t)m.N), dim3(PB), 0, P->st, P->Uo, (const double *)P->U,
-                       5 * (size_t)m.N, (const int *)P->flags);
-    hipLaunchKernelGGL(k_poly_sumsq, dim3(nb), dim3(PB), 0, P->st, (const double *)P->Rrho, m.N, P->part,
-                       (const int *)P->flags);
-    hipLaunchKernelGGL(k_poly_step_res, dim3(1), dim3(PB), 0, P->st, (const double *)P->part, nb, P->flags,
-                       P->hres, (const double *)P->runp);
-    PHIP(hipGetLastError());
-    return NF_OK;
+    if ((rc = stages(P, true, 0.0, err))) return rc;
+    return step_end(P, true, err);
 }
 
 // nf_run: check_every steps, captured once as a HIP graph (use_graph) or
@@ -911,29 +1123,25 @@ int poly_run(PolyPath *P, const nf_run_opts *o, nf_run_stats *stats, std::string
     const double drop = o->residual_drop;
     int rc;
     P->aux_valid = false;
-    if (!P->flags && ((rc = alloc(P, &P->flags, 4, err)) || (rc = alloc(P, &P->dtdev, 1, err)) ||
-                      (rc = alloc(P, &P->runp, 2, err))))
-        return rc;
-    if (o->n_steps > P->run_cap) {  // per-step history buffers, grown (the graph refers to them)
-        const int cap = std::max(o->n_steps, 1024);
+    if ((int64_t)o->n_steps + 1 > P->run_cap) {  // per-step history buffers, grown (the graph refers to them)
+        const int64_t cap = std::max<int64_t>((int64_t)o->n_steps + 1, 1024);
         PHIP(hipStreamSynchronize(P->st));
         if (P->graph) {
             (void)hipGraphExecDestroy(P->graph);
             P->graph = nullptr;
         }
-        for (double *old : {P->dts, P->hres}) {
+        for (double *old : {P->run.dts, P->run.hres}) {
             if (!old) continue;
             P->owned.erase(std::find(P->owned.begin(), P->owned.end(), (void *)old));
             PHIP(hipFree(old));
         }
-        P->dts = P->hres = nullptr;
-        if ((rc = alloc(P, &P->dts, cap, err)) || (rc = alloc(P, &P->hres, cap, err))) return rc;
+        P->run.dts = P->run.hres = nullptr;
+        P->run_cap = 0;
+        if ((rc = alloc(P, &P->run.dts, cap, err)) || (rc = alloc(P, &P->run.hres, cap, err))) return rc;
         P->run_cap = cap;
     }
-    PHIP(hipMemsetAsync(P->flags, 0, 4 * sizeof(int), P->st));
     // this run's drop and reference (negative: the run's own first residual)
-    const double runp[2] = {drop, P->hist.empty() ? -1.0 : P->hist.front()};
-    PHIP(hipMemcpyAsync(P->runp, runp, sizeof runp, hipMemcpyHostToDevice, P->st));
+    if ((rc = begin(P, true, drop, P->hist.empty() ? -1.0 : P->hist.front(), err))) return rc;
     hipEvent_t e0, e1;
     PHIP(hipEventCreate(&e0));
     PHIP(hipEventCreate(&e1));
@@ -943,7 +1151,10 @@ int poly_run(PolyPath *P, const nf_run_opts *o, nf_run_stats *stats, std::string
     if (!(drop > 0.0 && P->converged)) {
         while (queued < o->n_steps && !flags[0]) {
             const int chunk = std::min(K, o->n_steps - queued);
-            if (o->use_graph && chunk == K && K > 1) {
+            // a graph starts from prim(U) in X, whatever was the case when it
+            // was captured, and from the state in Ua
+            if ((rc = ensure_x(P, err))) return rc;
+            if (o->use_graph && chunk == K && K > 1 && !P->split) {
                 if (!P->graph || P->graph_K != K) {
                     if (P->graph) (void)hipGraphExecDestroy(P->graph);
                     P->graph = nullptr;
@@ -952,6 +1163,7 @@ int poly_run(PolyPath *P, const nf_run_opts *o, nf_run_stats *stats, std::string
                     for (int q = 0; q < K; ++q)
                         if ((rc = enqueue_run_step(P, err))) {
                             (void)hipStreamEndCapture(P->st, &gr);
+                            P->x_prim = false;
                             return rc;
                         }
                     PHIP(hipStreamEndCapture(P->st, &gr));
@@ -961,9 +1173,16 @@ int poly_run(PolyPath *P, const nf_run_opts *o, nf_run_stats *stats, std::string
                     P->graph_K = K;
                 }
                 PHIP(hipGraphLaunch(P->graph, P->st));
+                P->x_prim = P->rk3() || P->second();
             } else {
-                for (int q = 0; q < chunk; ++q)
+                for (int q = 0; q < chunk; ++q) {
                     if ((rc = enqueue_run_step(P, err))) return rc;
+                    if (!P->split) continue;
+                    // the state moves to Ua with the step, if that is taken
+                    PHIP(hipMemcpyAsync(flags, P->flags, sizeof flags, hipMemcpyDeviceToHost, P->st));
+                    PHIP(hipStreamSynchronize(P->st));
+                    P->split = flags[3] == 0;
+                }
             }
             queued += chunk;
             PHIP(hipMemcpyAsync(flags, P->flags, sizeof flags, hipMemcpyDeviceToHost, P->st));
@@ -978,8 +1197,11 @@ int poly_run(PolyPath *P, const nf_run_opts *o, nf_run_stats *stats, std::string
     (void)hipEventDestroy(e1);
     const int done = flags[3];
     std::vector<double> dts(done + 1), res(done);
-    if (done + flags[2] > 0) PHIP(hipMemcpy(dts.data(), P->dts, (done + flags[2]) * 8, hipMemcpyDeviceToHost));
-    if (done > 0) PHIP(hipMemcpy(res.data(), P->hres, done * 8, hipMemcpyDeviceToHost));
+    PHIP(hipMemcpy(dts.data(), P->run.dts, (done + 1) * 8, hipMemcpyDeviceToHost));
+    if (done > 0) PHIP(hipMemcpy(res.data(), P->run.hres, done * 8, hipMemcpyDeviceToHost));
+    P->dt = dts[done];
+    P->dt_valid = true;
+    if (done > 0) P->old_zero = false;
     for (int k = 0; k < done; ++k) {
         P->time += dts[k];
         P->hist.push_back(res[k]);
@@ -996,7 +1218,7 @@ int poly_run(PolyPath *P, const nf_run_opts *o, nf_run_stats *stats, std::string
         stats->fell_back = 0;
         stats->pad = 0;
     }
-    if (flags[2]) {
+    if (flags[2] && !flags[1] && done < o->n_steps) {
         char buf[96];
         std::snprintf(buf, sizeof buf, "Invalid dt calculated (dt = %f)", dts[done]);
         err = buf;
@@ -1014,13 +1236,17 @@ int poly_get_residuals(PolyPath *P, double *out, int32_t max, int32_t *n_out) {
 
 int poly_get_field(PolyPath *P, int32_t which, double *out, std::string &err) {
     switch (which) {
-    case NF_FIELD_PRIM:  // prim(U) into Ve with row stride N for the export
-        hipLaunchKernelGGL(k_poly_prim, grid(P->m.N), dim3(PB), 0, P->st, (const double *)P->U, P->Ve, P->m.N,
-                           P->m.N, (const int *)nullptr);
+    case NF_FIELD_PRIM:  // prim(U) with row stride N for the export
+        hipLaunchKernelGGL(k_poly_prim, grid(P->m.N), dim3(PB), 0, P->st, (const double *)P->state(), P->Y, P->m.N,
+                           P->m.N);
         PHIP(hipGetLastError());
-        return get_soa(P, P->Ve, 5, out, err);
+        return get_soa(P, P->Y, 5, out, err);
     case NF_FIELD_STATE_OLD:
-        return get_soa(P, P->Uo, 5, out, err);
+        if (P->old_zero) {
+            std::memset(out, 0, 5 * (size_t)P->m.N * 8);
+            return NF_OK;
+        }
+        return get_soa(P, P->Ua, 5, out, err);
     case NF_FIELD_LIMITER:
     case NF_FIELD_GRADIENT:
     case NF_FIELD_RESIDUAL:
