@@ -68,6 +68,7 @@ namespace nf {
 
 constexpr int BLOCK = 256;  // threads of the auxiliary kernels; instance padding unit
 constexpr int TILE = 64;    // cells per layout tile
+constexpr uint32_t HALO_LDS = 53760;  // most LDS bytes of a halo block (three per CU)
 
 // load through a global-address-space pointer (keeps the compiler from
 // falling back to flat loads, which also count against the LDS counter)
@@ -108,6 +109,14 @@ struct DevMesh {
     const double *gx, *gy, *gz;
     const uint2 *cell_ln;
     const uint32_t *nbr;
+    // per BLOCK cells: the distinct states its cells need from outside, entries
+    // [hal_off[b], hal_off[b+1]) of hal (device cell, or bit 31 and boundary
+    // face); cell_nb: per cell 4 x u16, the place of each slot's neighbour --
+    // below BLOCK the block's own cell, then the halo's entries -- and bit 15
+    // on a boundary slot.  null: some block's halo is too large
+    const uint32_t *hal_off, *hal;
+    const uint2 *cell_nb;
+    uint32_t nstride;  // entries of the longest node table
     const uint32_t *fcode;
     const uint32_t *blk_inst;  // [blocks] instance of each 256-cell block (32-bit: scalar loads)
     const uint32_t *inst_end;  // [instances] one past the instance's last device cell
@@ -234,20 +243,20 @@ __device__ __forceinline__ NodeTableLoad node_table_issue(const DevMesh &m, uint
 }
 template <int B>
 __device__ __forceinline__ NodeView node_table_finish(const DevMesh &m, uint32_t p, const NodeTableLoad &t,
-                                                      double *lds, CellGeo &g) {
+                                                      double *lds, CellGeo &g, uint32_t stride = 256) {
     const uint32_t lane = p & 63u, wv = threadIdx.x >> 6;
-    double *w = lds + wv * 768;  // [3][256] per wave
+    double *w = lds + wv * 3 * stride;  // [3][stride] per wave
     if (lane < t.n) {
         w[lane] = t.x;
-        w[256 + lane] = t.y;
-        w[512 + lane] = t.z;
+        w[stride + lane] = t.y;
+        w[2 * stride + lane] = t.z;
     }
     if (t.n > 64) {  // uniform per wave
         const uint32_t o0 = m.grp_off[p >> 6];
         for (uint32_t i = lane + 64; i < t.n; i += 64) {
             w[i] = m.gx[o0 + i];
-            w[256 + i] = m.gy[o0 + i];
-            w[512 + i] = m.gz[o0 + i];
+            w[stride + i] = m.gy[o0 + i];
+            w[2 * stride + i] = m.gz[o0 + i];
         }
     }
     // LDS operations of one wave complete in order; the fences keep the
@@ -255,7 +264,7 @@ __device__ __forceinline__ NodeView node_table_finish(const DevMesh &m, uint32_t
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    NodeView v{w, {t.q.x & 0xFFFFu, t.q.x >> 16, t.q.y & 0xFFFFu, t.q.y >> 16}, 256};
+    NodeView v{w, {t.q.x & 0xFFFFu, t.q.x >> 16, t.q.y & 0xFFFFu, t.q.y >> 16}, stride};
     g.p0 = nv_node(v, 0);
     g.p1 = nv_node(v, 1);
     g.p2 = nv_node(v, 2);
@@ -678,6 +687,153 @@ __global__ __launch_bounds__(B) NF_SWEEP_ATTR void k_sweepA(DevMesh m, SweepAArg
     if (a.dt_part) {
         const double v = block_reduce<true, B>(dtc, sh);
         if (threadIdx.x == 0) a.dt_part[L.lb] = v;
+    }
+}
+
+// Sweep A over blocks of 256 cells whose halo fits (second order).  In Morton
+// order a block's 1,024 neighbours are 830 of its own cells and some 200
+// states outside.  The block gathers those once, one state per lane,
+// converts each once, and keeps them beside its own states in LDS, where a
+// variable's neighbour values are read when they are used.  In k_sweepA every
+// lane gathers and converts its outside neighbours under a mask and holds 40
+// registers of neighbour values through the sweep: 2 waves per SIMD, here 4
+// (128 registers; LDS as large as the context's largest halo and node table,
+// 28 to 34 KB).  TVD-RK3 step, farfield box / bump channel, k_sweepA -> here:
+// 215k / 202k cells 156 / 149 -> 143 / 138 us, 998k / 1,054k 488 / 510 ->
+// 449 / 487, 3.95M / 4.14M 1,929 / 1,904 -> 1,742 / 1,778.  With 3 waves the
+// same to 1 %: what is left is memory (650 B per cell and stage in both
+// sweeps, 4.4 TB/s at 3.95M cells).
+template <int ORDER, bool FROM_U, bool FUSE>
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_sweepA_halo(DevMesh m, SweepAArgs a) {
+    constexpr int B = BLOCK;
+    static_assert(ORDER != 0, "a first-order sweep needs no neighbours");
+    __shared__ double sh[B / 64];
+    // node tables, in whose place the face values on their way out are, and
+    // [cell][5] the states of the block and of its halo
+    extern __shared__ __align__(16) double lds[];
+    double *vs = lds + 12 * m.nstride;
+    const LaneCell L = lane_cell<B>(m, a.xcd_remap);
+    const uint32_t h0 = m.hal_off[L.lb], nh = m.hal_off[L.lb + 1] - h0;
+    BndRange br{0, 0};
+    if (FUSE) br = bnd_range<B>(a.bnd.boff, L.lb);
+    if (m.st[L.inst].stop) return;
+    const uint32_t c = L.c, t = threadIdx.x, p = L.lb * B + t, lane = t & 63u;
+    const bool live = L.live;
+
+    const uint32_t hw = m.hal[h0 + (t < nh ? t : 0)];  // (one entry past the end is there)
+    const uint32_t code = m.fcode[c];
+    const uint2 nb = m.cell_nb[p];
+    const NodeTableLoad ntl = node_table_issue(m, p);
+    __builtin_amdgcn_sched_barrier(0);
+    double Vc[5], Vh[5];
+#pragma unroll
+    for (int k = 0; k < 5; ++k) Vc[k] = a.V[tix(c, k)];
+    auto halo_load = [&](uint32_t w) {
+        const double *src = ((w & 0x80000000u) ? a.Gc : a.V) + tix(w & 0x1FFFFFFFu, 0);
+#pragma unroll
+        for (int k = 0; k < 5; ++k) Vh[k] = ldg(src + k * TILE);
+    };
+    auto halo_store = [&](uint32_t h, uint32_t w) {
+        if (FROM_U && !(w & 0x80000000u)) {  // (ghosts are primvars already)
+            const double Uh[5] = {Vh[0], Vh[1], Vh[2], Vh[3], Vh[4]};
+            cons_to_prim_d(Uh, Vh);
+        }
+#pragma unroll
+        for (int k = 0; k < 5; ++k) vs[5 * (B + h) + k] = Vh[k];
+    };
+    if (t < nh) halo_load(hw);
+    __builtin_amdgcn_sched_barrier(0);
+    CellGeo g;
+    const NodeView nv = node_table_finish<B>(m, p, ntl, lds, g, m.nstride);
+    if (FROM_U) {
+        const double Uc[5] = {Vc[0], Vc[1], Vc[2], Vc[3], Vc[4]};
+        cons_to_prim_d(Uc, Vc);
+    }
+#pragma unroll
+    for (int k = 0; k < 5; ++k) vs[5 * t + k] = Vc[k];
+    if (t < nh) halo_store(t, hw);
+    for (uint32_t h = t + B; h < nh; h += B) {
+        const uint32_t w = m.hal[h0 + h];
+        halo_load(w);
+        halo_store(h, w);
+    }
+    cell_geo(m, g);
+    V3d S[4], r[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) face_geo(m, g, nv, (code >> (8 * s)) & 0xFFu, S[s], &r[s]);
+    __syncthreads();  // every wave's states are in LDS
+
+    const uint32_t nbw[4] = {nb.x & 0xFFFFu, nb.x >> 16, nb.y & 0xFFFFu, nb.y >> 16};
+    const double *vn[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) vn[s] = vs + 5 * (nbw[s] & 0x7FFFu);
+    // face normals as the cell adds them: -S where the cell is the
+    // reference's neighbour j (cell j subtracts tmp/vol); in place, as
+    // the time step below uses |S| only
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+        const uint32_t mneg = ((code >> (8 * s + 7)) & 1u) ? 0u : 0x80000000u;
+        S[s] = {flip(S[s].x, mneg), flip(S[s].y, mneg), flip(S[s].z, mneg)};
+    }
+    double *vt = lds + (t >> 6) * 3 * m.nstride;  // (the wave's node table: dead)
+    // one variable at a time, as in tileA_run
+#pragma unroll
+    for (int k = 0; k < 5; ++k) {
+        const double Vk = vs[5 * t + k];  // (kept there: ten registers fewer)
+        double Vn[4];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) Vn[s] = vn[s][k];
+        double g0 = 0.0, g1 = 0.0, g2 = 0.0;
+        double vmax = Vk, vmin = Vk;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const double uf = 0.5 * (Vk + Vn[s]);
+            g0 = g0 + rdiv(uf * S[s].x, g.ivol);
+            g1 = g1 + rdiv(uf * S[s].y, g.ivol);
+            g2 = g2 + rdiv(uf * S[s].z, g.ivol);
+            if (ORDER == 2) {
+                vmax = dmax(vmax, Vn[s]);
+                vmin = dmin(vmin, Vn[s]);
+            }
+        }
+        double delta[4];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) delta[s] = (g0 * r[s].x + g1 * r[s].y) + g2 * r[s].z;
+        const double psi = (ORDER == 2) ? barth_psi_d(delta, vmax, vmin, Vk) : 1.0;
+        // 16-byte stores through the wave's slice, as in tileA_run
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+        for (int s = 0; s < 4; ++s) vt[s * TILE + lane] = Vk + psi * delta[s];
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        const double2 v0 = reinterpret_cast<const double2 *>(vt)[lane];
+        const double2 v1 = reinterpret_cast<const double2 *>(vt)[lane + TILE];
+        double *row = a.FV + fix(p & ~63u, lane >> 5, k) + 2 * (lane & 31u);
+        *reinterpret_cast<double2 *>(row) = v0;
+        *reinterpret_cast<double2 *>(row + 2 * 5 * TILE) = v1;
+        if (live && a.grad_aux) {
+            const size_t o = a.aux_row[c];
+            a.grad_aux[15 * o + k] = g0;
+            a.grad_aux[15 * o + k + 5] = g1;
+            a.grad_aux[15 * o + k + 10] = g2;
+            a.psi_aux[5 * o + k] = psi;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    if (FUSE) bnd_ghosts<B, GhostOf::FV>(a.bnd, br, L.inst, a.FV);
+    if (a.dt_part) {
+        uint32_t w[4];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) w[s] = nbw[s] << 16;  // (bit 31: boundary)
+#pragma unroll
+        for (int k = 0; k < 5; ++k) Vc[k] = vs[5 * t + k];
+        const double tc = cell_dt(Vc, S, w, g.vol, a.CFL);
+        if (a.dt_cell && live) a.dt_cell[c] = tc;
+        const double v = block_reduce<true, B>((live && tc < DBL_MAX) ? tc : DBL_MAX, sh);
+        if (t == 0) a.dt_part[L.lb] = v;
     }
 }
 

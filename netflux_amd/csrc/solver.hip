@@ -301,6 +301,10 @@ struct nf_ctx {
     uint32_t *grp_off = nullptr;          // 64-cell group node tables
     double *gx = nullptr, *gy = nullptr, *gz = nullptr;
     uint2 *cell_ln = nullptr;
+    uint32_t *hal_off = nullptr, *hal = nullptr;  // block halos of sweep A; null: gathered per lane
+    uint2 *cell_nb = nullptr;
+    uint32_t nstride = 86;  // node table entries per 64 cells: at least the face values' 256 doubles
+    uint32_t halo_lds = 0;  // LDS bytes of a halo block
     uint32_t *blk_inst = nullptr;
     uint32_t *inst_end = nullptr;
     InstState *st = nullptr;
@@ -368,7 +372,8 @@ int dalloc(nf_ctx *ctx, T **p, size_t n) {
 
 DevMesh devmesh(const nf_ctx *c) {
     return DevMesh{3.0,         6.0,       c->nodes, c->cnodes, c->grp_off,  c->gx,       c->gy,
-                   c->gz,       c->cell_ln, c->nbr,   c->fcode,  c->blk_inst, c->inst_end, c->st};
+                   c->gz,       c->cell_ln, c->nbr,   c->hal_off, c->hal,    c->cell_nb, c->nstride, c->fcode,
+                   c->blk_inst, c->inst_end, c->st};
 }
 
 const RedTable &red(const nf_ctx *c) { return c->block == 128 ? c->red128 : c->red256; }
@@ -484,6 +489,11 @@ hipError_t launch_sweepB(hipStream_t s, uint32_t ncell, bool hllc, const DevMesh
 constexpr uint32_t FUSE_MAX_CELLS = 1024 * BLOCK;
 bool fused_ghosts(const nf_ctx *ctx) { return ctx->Ncell <= FUSE_MAX_CELLS; }
 
+// sweep A with block halos: second order, 256-cell blocks, every halo fits.
+// (Cells in an order without locality have up to 1,024 outside neighbours per
+// block; their gather is the same work either way.)
+bool use_halo(const nf_ctx *ctx, int order) { return order != 0 && ctx->block == BLOCK && ctx->cell_nb; }
+
 // sweep A of the current primvars, or (U set, FP64) of prim(U) of that state.
 // dt: per-block CFL minima into dt_part; dtc: per-cell CFL steps into dt_cell
 // (local time stepping); aux: keep the gradient and limiter fields.
@@ -511,6 +521,17 @@ int run_sweepA(nf_ctx *ctx, bool dt, bool aux, bool dtc = false, const double *U
                        ctx->perm_dev, bnd_args(ctx, ctx->Gf)};
     const char *name = order == 2 ? "sweepA_barth" : (order == 1 ? "sweepA_nolim" : "sweepA_first");
     return launch_fn(ctx, name, [&] {
+        if (use_halo(ctx, order)) {
+            auto go = [&](auto from_u, auto fused) {
+                const dim3 g(ctx->Ncell / BLOCK), b(BLOCK);
+                const uint32_t lds = ctx->halo_lds;
+                if (order == 1) hipLaunchKernelGGL((k_sweepA_halo<1, from_u(), fused()>), g, b, lds, ctx->stream, m, a);
+                else hipLaunchKernelGGL((k_sweepA_halo<2, from_u(), fused()>), g, b, lds, ctx->stream, m, a);
+                return hipGetLastError();
+            };
+            if (U) return fuse ? go(std::true_type{}, std::true_type{}) : go(std::true_type{}, std::false_type{});
+            return fuse ? go(std::false_type{}, std::true_type{}) : go(std::false_type{}, std::false_type{});
+        }
         auto go = [&](auto from_u, auto fused) {
             return ctx->block == 128
                        ? launch_sweepA<128, from_u(), fused()>(ctx->stream, ctx->Ncell, order, m, a)
@@ -1084,6 +1105,46 @@ int create(int32_t n, const nf_mesh_desc *descs, const nf_params *prms, nf_ctx *
             grp_off.push_back(grp_off.back() + cnt);
         }
     }
+    // block halos of sweep A: distinct outside states in first-use order
+    std::vector<uint32_t> hal_off(1, 0), hal;
+    std::vector<uint2> cell_nb(cell0);
+    for (size_t g = 0; g + 1 < grp_off.size(); ++g) ctx->nstride = std::max(ctx->nstride, grp_off[g + 1] - grp_off[g]);
+    ctx->nstride = (ctx->nstride + 1) & ~1u;
+    {
+        std::vector<uint32_t> stamp(cell0, UINT32_MAX), loc(cell0);
+        for (uint32_t b = 0; b < cell0 / BLOCK; ++b) {
+            uint32_t cnt = 0;
+            for (uint32_t p = b * BLOCK; p < (b + 1) * BLOCK; ++p) {
+                if (p >= inst_end[blk_inst[b]]) {  // padding: as the last cell, in this block too
+                    cell_nb[p] = cell_nb[p - 1];
+                    continue;
+                }
+                uint32_t l[4];
+                for (int q = 0; q < 4; ++q) {
+                    const uint32_t w = nbr[4 * (size_t)p + q], idx = w & NBR_INDEX_MASK;
+                    if (w & NBR_BOUNDARY) {  // (its cell's alone)
+                        hal.push_back(NBR_BOUNDARY | idx);
+                        l[q] = 0x8000u | (BLOCK + cnt++);
+                    } else if (idx / BLOCK == b) {
+                        l[q] = idx % BLOCK;
+                    } else {
+                        if (stamp[idx] != b) {
+                            stamp[idx] = b;
+                            loc[idx] = BLOCK + cnt++;
+                            hal.push_back(idx);
+                        }
+                        l[q] = loc[idx];
+                    }
+                }
+                cell_nb[p] = make_uint2(l[0] | l[1] << 16, l[2] | l[3] << 16);
+            }
+            ctx->halo_lds = std::max(ctx->halo_lds, cnt);
+            hal_off.push_back((uint32_t)hal.size());
+        }
+    }
+    ctx->halo_lds = 8 * (12 * ctx->nstride + 5 * (BLOCK + ctx->halo_lds));
+    const bool halos = ctx->halo_lds <= HALO_LDS;
+    hal.push_back(0);  // (read, not used, by a block without a halo)
     ctx->Ncell = (uint32_t)cell0;
     ctx->nbf = (uint32_t)bface.size();
 
@@ -1099,6 +1160,14 @@ int create(int32_t n, const nf_mesh_desc *descs, const nf_params *prms, nf_ctx *
     if ((rc = dalloc(ctx, &ctx->gy, gy.size()))) return rc;
     if ((rc = dalloc(ctx, &ctx->gz, gz.size()))) return rc;
     if ((rc = dalloc(ctx, &ctx->cell_ln, cell_ln.size()))) return rc;
+    if (halos) {
+        if ((rc = dalloc(ctx, &ctx->hal_off, hal_off.size()))) return rc;
+        if ((rc = dalloc(ctx, &ctx->hal, hal.size()))) return rc;
+        if ((rc = dalloc(ctx, &ctx->cell_nb, cell_nb.size()))) return rc;
+        HIPC(hipMemcpy(ctx->hal_off, hal_off.data(), hal_off.size() * 4, hipMemcpyHostToDevice));
+        HIPC(hipMemcpy(ctx->hal, hal.data(), hal.size() * 4, hipMemcpyHostToDevice));
+        HIPC(hipMemcpy(ctx->cell_nb, cell_nb.data(), cell_nb.size() * sizeof(uint2), hipMemcpyHostToDevice));
+    }
     if ((rc = dalloc(ctx, &ctx->blk_inst, blk_inst.size()))) return rc;
     if ((rc = dalloc(ctx, &ctx->inst_end, inst_end.size()))) return rc;
     if ((rc = dalloc(ctx, &ctx->st, (size_t)n))) return rc;
