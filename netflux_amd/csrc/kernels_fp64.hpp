@@ -68,7 +68,7 @@ namespace nf {
 
 constexpr int BLOCK = 256;  // threads of the auxiliary kernels; instance padding unit
 constexpr int TILE = 64;    // cells per layout tile
-constexpr uint32_t HALO_LDS = 53760;  // most LDS bytes of a halo block (three per CU)
+constexpr uint32_t FACE_LDS = 53728;  // most LDS bytes of a block of k_sweepA_face (three per CU)
 
 // load through a global-address-space pointer (keeps the compiler from
 // falling back to flat loads, which also count against the LDS counter)
@@ -103,20 +103,27 @@ struct DevMesh {
     const double *nodes;
     const uint32_t *cnodes;
     // per 64-cell group: its distinct nodes' coordinates, SoA, entries
-    // [grp_off[g], grp_off[g+1]); cell_ln: the group-local entry of each
-    // cell's four nodes (4 x u16)
+    // [grp_off[g], grp_off[g+1]); cell_ln: per cell 4 x u16, the byte
+    // offsets of its nodes in the group's [node][3] table
     const uint32_t *grp_off;
     const double *gx, *gy, *gz;
     const uint2 *cell_ln;
     const uint32_t *nbr;
-    // per BLOCK cells: the distinct states its cells need from outside, entries
-    // [hal_off[b], hal_off[b+1]) of hal (device cell, or bit 31 and boundary
-    // face); cell_nb: per cell 4 x u16, the place of each slot's neighbour --
-    // below BLOCK the block's own cell, then the halo's entries -- and bit 15
-    // on a boundary slot.  null: some block's halo is too large
-    const uint32_t *hal_off, *hal;
-    const uint2 *cell_nb;
-    uint32_t nstride;  // entries of the longest node table
+    // per BLOCK cells, null if some block has too many records: faces between
+    // two of its cells, numbers [foff[b], foff[b+1]), and records of its other
+    // cell sides, [roff[b], roff[b+1]).  Per record: hal, the cell of the
+    // face's other side (or bit 31 and boundary face); rec, that side's record
+    // (or bit 31 and boundary face), bit 30 set if the record's own side is
+    // the reference owner's; rS [tile][3][64], the face vector.  Per cell
+    // 4 x u16: cell_nb, where a slot's neighbour state is -- below BLOCK the
+    // block's own cell, then the records' -- and bit 15 on a boundary slot;
+    // cell_fx, the place of a slot's side among the block's 2 nf + nr (owner
+    // sides of its faces, their other sides, records) and bit 15 on an owner's
+    // side.  nstride: most nodes of a node table; nent: most nf + nr
+    const uint32_t *foff, *roff, *hal, *rec;
+    const uint2 *cell_nb, *cell_fx;
+    const double *rS, *vol;
+    uint32_t nstride, nent;
     const uint32_t *fcode;
     const uint32_t *blk_inst;  // [blocks] instance of each 256-cell block (32-bit: scalar loads)
     const uint32_t *inst_end;  // [instances] one past the instance's last device cell
@@ -186,31 +193,34 @@ __device__ __forceinline__ void load_cell(const DevMesh &m, uint32_t c, CellGeo 
     cell_geo(m, g);
 }
 
-// Node coordinates in LDS, rows x, y, z of `stride` entries each; l[q] is
-// the entry of the lane's q-th cell node.  Selecting a face's nodes by index
-// from LDS replaces register selects.
+// Node coordinates in LDS, [entry][3].  l holds the byte offsets of the four
+// cell nodes' entries, 16 bits each: one byte permute selects a face's node,
+// its three coordinates follow at constant offsets (with separate rows and
+// the offsets in four registers the selects were 5 % of sweep A's
+// instructions).
 struct NodeView {
     const double *lds;
-    uint32_t l[4];
-    uint32_t stride;
+    uint2 l;
 };
 __device__ __forceinline__ V3d nv_node(const NodeView &v, uint32_t q) {
-    const uint32_t i = q == 0 ? v.l[0] : (q == 1 ? v.l[1] : (q == 2 ? v.l[2] : v.l[3]));
-    return {v.lds[i], v.lds[v.stride + i], v.lds[2 * v.stride + i]};
+    const uint32_t o = __builtin_amdgcn_perm(v.l.y, v.l.x, 0x0c0c0100u + q * 0x0202u);
+    const double *w = reinterpret_cast<const double *>(reinterpret_cast<const char *>(v.lds) + o);
+    return {w[0], w[1], w[2]};
 }
 
 // Per-lane staging (boundary-face kernels): lane t writes its four nodes at
-// entries q*B + t; only its own entries are read, so no barrier is needed.
+// entries 4 t + q; only its own entries are read, so no barrier is needed.
 template <int B>
 __device__ __forceinline__ NodeView stage_nodes(double *lds, const CellGeo &g) {
     const uint32_t t = threadIdx.x;
     const V3d P[4] = {g.p0, g.p1, g.p2, g.p3};
-    NodeView v{lds, {t, B + t, 2 * B + t, 3 * B + t}, 4 * B};
+    const uint32_t o = 96 * t;
+    NodeView v{lds, make_uint2(o | (o + 24) << 16, (o + 48) | (o + 72) << 16)};
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-        lds[q * B + t] = P[q].x;
-        lds[4 * B + q * B + t] = P[q].y;
-        lds[8 * B + q * B + t] = P[q].z;
+        lds[12 * t + 3 * q] = P[q].x;
+        lds[12 * t + 3 * q + 1] = P[q].y;
+        lds[12 * t + 3 * q + 2] = P[q].z;
     }
     return v;
 }
@@ -245,18 +255,18 @@ template <int B>
 __device__ __forceinline__ NodeView node_table_finish(const DevMesh &m, uint32_t p, const NodeTableLoad &t,
                                                       double *lds, CellGeo &g, uint32_t stride = 256) {
     const uint32_t lane = p & 63u, wv = threadIdx.x >> 6;
-    double *w = lds + wv * 3 * stride;  // [3][stride] per wave
+    double *w = lds + wv * 3 * stride;  // [stride][3] per wave
     if (lane < t.n) {
-        w[lane] = t.x;
-        w[stride + lane] = t.y;
-        w[2 * stride + lane] = t.z;
+        w[3 * lane] = t.x;
+        w[3 * lane + 1] = t.y;
+        w[3 * lane + 2] = t.z;
     }
     if (t.n > 64) {  // uniform per wave
         const uint32_t o0 = m.grp_off[p >> 6];
         for (uint32_t i = lane + 64; i < t.n; i += 64) {
-            w[i] = m.gx[o0 + i];
-            w[stride + i] = m.gy[o0 + i];
-            w[2 * stride + i] = m.gz[o0 + i];
+            w[3 * i] = m.gx[o0 + i];
+            w[3 * i + 1] = m.gy[o0 + i];
+            w[3 * i + 2] = m.gz[o0 + i];
         }
     }
     // LDS operations of one wave complete in order; the fences keep the
@@ -264,7 +274,7 @@ __device__ __forceinline__ NodeView node_table_finish(const DevMesh &m, uint32_t
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    NodeView v{w, {t.q.x & 0xFFFFu, t.q.x >> 16, t.q.y & 0xFFFFu, t.q.y >> 16}, stride};
+    NodeView v{w, t.q};
     g.p0 = nv_node(v, 0);
     g.p1 = nv_node(v, 1);
     g.p2 = nv_node(v, 2);
@@ -410,14 +420,15 @@ struct BndArgs {
     const uint8_t *bbc;          // boundary type
     const double *bS;            // [3][nb] S_ij of each boundary face (cell -> ghost)
     uint32_t nb;                 // boundary faces
+    const uint32_t *brec;        // record of each boundary face (GhostOf::REC)
     const FarField<double> *fs;  // [instances]
     double *out;                 // [nb/64][5][64], tiled like V
 };
 
 // what a ghost is formed from: V (set_constant_ghost_values, src/Solver.cpp:
 // 300-330), the primvars of the state U, or the reconstructed face states FV
-// (src/Solver.cpp:210-212)
-enum class GhostOf { V, U, FV };
+// (src/Solver.cpp:210-212), or their records
+enum class GhostOf { V, U, FV, REC };
 
 // The face vector comes precomputed from the host face graph: the same cross
 // product and sign the sweeps evaluate from the nodes, so the same bits.
@@ -427,7 +438,8 @@ __device__ __forceinline__ void bnd_ghost(const BndArgs &a, uint32_t b, uint32_t
     const V3d S = {a.bS[b], a.bS[a.nb + b], a.bS[2 * (size_t)a.nb + b]};
     double Vd[5], Vg[5];
 #pragma unroll
-    for (int k = 0; k < 5; ++k) Vd[k] = OF == GhostOf::FV ? src[fix(c, w >> 29, k)] : src[tix(c, k)];
+    for (int k = 0; k < 5; ++k)
+        Vd[k] = OF == GhostOf::FV ? src[fix(c, w >> 29, k)] : src[tix(OF == GhostOf::REC ? a.brec[b] : c, k)];
     if (OF == GhostOf::U) {
         const double Ud[5] = {Vd[0], Vd[1], Vd[2], Vd[3], Vd[4]};
         cons_to_prim_d(Ud, Vd);
@@ -459,7 +471,8 @@ __global__ __launch_bounds__(BLOCK) void k_ghost(BndArgs a, const double *src) {
 struct SweepAArgs {
     const double *V;   // [tile][5][64] primvars (FROM_U = false) or the state U (FROM_U)
     const double *Gc;  // [nb/64][5][64] ghost of the cell-centre state
-    double *FV;        // [tile][4][5][64]
+    double *FV;        // [tile][4][5][64]; k_sweepA_face: per block [5][nf] fluxes of its own faces
+    double *H;         // k_sweepA_face: [tile][5][64] face values of the records
     double *dt_part;   // per-block CFL dt minimum, or null
     double *dt_cell;   // [N] per-cell CFL step (local time stepping), or null
     double CFL;
@@ -468,6 +481,7 @@ struct SweepAArgs {
     double *psi_aux;   // [N][5] or null
     const uint32_t *aux_row;  // device cell -> row of grad_aux and psi_aux (reference cell)
     BndArgs bnd;       // FUSE: ghosts of the reconstructed face states (out: Gf)
+    int hllc;          // k_sweepA_face: the flux
 };
 
 // One 64-cell tile of sweep A: its loads (tileA_issue) and the rest
@@ -690,39 +704,46 @@ __global__ __launch_bounds__(B) NF_SWEEP_ATTR void k_sweepA(DevMesh m, SweepAArg
     }
 }
 
-// Sweep A over blocks of 256 cells whose halo fits (second order).  In Morton
-// order a block's 1,024 neighbours are 830 of its own cells and some 200
-// states outside.  The block gathers those once, one state per lane,
-// converts each once, and keeps them beside its own states in LDS, where a
-// variable's neighbour values are read when they are used.  In k_sweepA every
-// lane gathers and converts its outside neighbours under a mask and holds 40
-// registers of neighbour values through the sweep: 2 waves per SIMD, here 4
-// (128 registers; LDS as large as the context's largest halo and node table,
-// 28 to 34 KB).  TVD-RK3 step, farfield box / bump channel, k_sweepA -> here:
-// 215k / 202k cells 156 / 149 -> 143 / 138 us, 998k / 1,054k 488 / 510 ->
-// 449 / 487, 3.95M / 4.14M 1,929 / 1,904 -> 1,742 / 1,778.  With 3 waves the
-// same to 1 %: what is left is memory (650 B per cell and stage in both
-// sweeps, 4.4 TB/s at 3.95M cells).
+// Second-order sweeps over the faces of blocks of 256 cells, as long as every
+// block's LDS fits (any order with locality).  Of a block's 1,024 cell sides
+// some 830 belong to 415 faces between its own cells; the other 200 are its
+// records.  Sweep A gathers and converts the records' outside states once,
+// one per lane, and keeps them in LDS beside the block's own; reconstructs
+// every cell; passes the face values through LDS; and one lane per face then
+// evaluates the flux of a face of the block, once instead of once from either
+// side.  It stores those fluxes and the records' face values, 97 B per cell;
+// sweep B evaluates the records' fluxes only, and sums every cell's four in
+// slot order.  Against the sweeps that gather per lane and pass all 160 B of
+// face values through memory (k_sweepA, k_sweepB): 470 instead of 650 B per
+// cell and stage, 620 instead of 1,024 flux evaluations per block.  TVD-RK3
+// step, farfield box / bump channel: 63k / 60k cells 63.5 / 63.5 -> 60.7 /
+// 61.5 us, 215k / 202k 156 / 149 -> 136 / 130, 998k / 1,054k 488 / 510 -> 382
+// / 415, 3.95M / 4.14M 1,929 / 1,904 -> 1,471 / 1,593.
+//
+// Sweep A is bound by its phases between barriers: the vector units are busy
+// 60 % of its time, memory moves 2.1 TB/s.  52 KB of LDS hold three blocks per
+// CU; the face values in two halves (33 KB, 128 registers, four blocks) cost
+// more in barriers than they gain: 382 -> 410 us at 998k cells.
 template <int ORDER, bool FROM_U, bool FUSE>
-__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_sweepA_halo(DevMesh m, SweepAArgs a) {
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(3, 3))) void k_sweepA_face(DevMesh m, SweepAArgs a) {
     constexpr int B = BLOCK;
     static_assert(ORDER != 0, "a first-order sweep needs no neighbours");
     __shared__ double sh[B / 64];
-    // node tables, in whose place the face values on their way out are, and
-    // [cell][5] the states of the block and of its halo
+    // node tables and [cell][5] the states of the block and of its halo; later
+    // [5][1024] the face values of all cell sides and [3][512] face vectors
     extern __shared__ __align__(16) double lds[];
     double *vs = lds + 12 * m.nstride;
     const LaneCell L = lane_cell<B>(m, a.xcd_remap);
-    const uint32_t h0 = m.hal_off[L.lb], nh = m.hal_off[L.lb + 1] - h0;
+    const uint32_t f0 = m.foff[L.lb], nf = m.foff[L.lb + 1] - f0, r0 = m.roff[L.lb], nr = m.roff[L.lb + 1] - r0;
     BndRange br{0, 0};
     if (FUSE) br = bnd_range<B>(a.bnd.boff, L.lb);
     if (m.st[L.inst].stop) return;
-    const uint32_t c = L.c, t = threadIdx.x, p = L.lb * B + t, lane = t & 63u;
+    const uint32_t c = L.c, t = threadIdx.x, p = L.lb * B + t;
     const bool live = L.live;
 
-    const uint32_t hw = m.hal[h0 + (t < nh ? t : 0)];  // (one entry past the end is there)
+    const uint32_t hw = m.hal[r0 + (t < nr ? t : 0)];  // (one entry past the end is there)
     const uint32_t code = m.fcode[c];
-    const uint2 nb = m.cell_nb[p];
+    const uint2 nb = m.cell_nb[p], fx = m.cell_fx[p];
     const NodeTableLoad ntl = node_table_issue(m, p);
     __builtin_amdgcn_sched_barrier(0);
     double Vc[5], Vh[5];
@@ -741,7 +762,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4, 4))) v
 #pragma unroll
         for (int k = 0; k < 5; ++k) vs[5 * (B + h) + k] = Vh[k];
     };
-    if (t < nh) halo_load(hw);
+    if (t < nr) halo_load(hw);
     __builtin_amdgcn_sched_barrier(0);
     CellGeo g;
     const NodeView nv = node_table_finish<B>(m, p, ntl, lds, g, m.nstride);
@@ -751,9 +772,9 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4, 4))) v
     }
 #pragma unroll
     for (int k = 0; k < 5; ++k) vs[5 * t + k] = Vc[k];
-    if (t < nh) halo_store(t, hw);
-    for (uint32_t h = t + B; h < nh; h += B) {
-        const uint32_t w = m.hal[h0 + h];
+    if (t < nr) halo_store(t, hw);
+    for (uint32_t h = t + B; h < nr; h += B) {
+        const uint32_t w = m.hal[r0 + h];
         halo_load(w);
         halo_store(h, w);
     }
@@ -775,8 +796,9 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4, 4))) v
         const uint32_t mneg = ((code >> (8 * s + 7)) & 1u) ? 0u : 0x80000000u;
         S[s] = {flip(S[s].x, mneg), flip(S[s].y, mneg), flip(S[s].z, mneg)};
     }
-    double *vt = lds + (t >> 6) * 3 * m.nstride;  // (the wave's node table: dead)
-    // one variable at a time, as in tileA_run
+    double Vf[4][5];
+    // one variable at a time, as in tileA_run; the face values wait in registers
+    // until every wave has read its neighbours' states
 #pragma unroll
     for (int k = 0; k < 5; ++k) {
         const double Vk = vs[5 * t + k];  // (kept there: ten registers fewer)
@@ -800,20 +822,8 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4, 4))) v
 #pragma unroll
         for (int s = 0; s < 4; ++s) delta[s] = (g0 * r[s].x + g1 * r[s].y) + g2 * r[s].z;
         const double psi = (ORDER == 2) ? barth_psi_d(delta, vmax, vmin, Vk) : 1.0;
-        // 16-byte stores through the wave's slice, as in tileA_run
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
-        for (int s = 0; s < 4; ++s) vt[s * TILE + lane] = Vk + psi * delta[s];
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        const double2 v0 = reinterpret_cast<const double2 *>(vt)[lane];
-        const double2 v1 = reinterpret_cast<const double2 *>(vt)[lane + TILE];
-        double *row = a.FV + fix(p & ~63u, lane >> 5, k) + 2 * (lane & 31u);
-        *reinterpret_cast<double2 *>(row) = v0;
-        *reinterpret_cast<double2 *>(row + 2 * 5 * TILE) = v1;
+        for (int s = 0; s < 4; ++s) Vf[s][k] = Vk + psi * delta[s];
         if (live && a.grad_aux) {
             const size_t o = a.aux_row[c];
             a.grad_aux[15 * o + k] = g0;
@@ -823,23 +833,90 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4, 4))) v
         }
         __builtin_amdgcn_sched_barrier(0);
     }
-    if (FUSE) bnd_ghosts<B, GhostOf::FV>(a.bnd, br, L.inst, a.FV);
+    double tc = DBL_MAX;
     if (a.dt_part) {
+#pragma unroll
+        for (int k = 0; k < 5; ++k) Vc[k] = vs[5 * t + k];
         uint32_t w[4];
 #pragma unroll
         for (int s = 0; s < 4; ++s) w[s] = nbw[s] << 16;  // (bit 31: boundary)
-#pragma unroll
-        for (int k = 0; k < 5; ++k) Vc[k] = vs[5 * t + k];
-        const double tc = cell_dt(Vc, S, w, g.vol, a.CFL);
+        tc = cell_dt(Vc, S, w, g.vol, a.CFL);
         if (a.dt_cell && live) a.dt_cell[c] = tc;
+    }
+    __syncthreads();
+    // every side's values, and each own face's vector from its owner, to LDS
+    double *fS = lds + 5 * 4 * B;
+    if (live) {
+        const uint32_t pos[4] = {fx.x & 0x7FFFu, (fx.x >> 16) & 0x7FFFu, fx.y & 0x7FFFu, (fx.y >> 16) & 0x7FFFu};
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+#pragma unroll
+            for (int k = 0; k < 5; ++k) lds[k * 4 * B + pos[s]] = Vf[s][k];
+            if (pos[s] < nf) {
+                fS[pos[s]] = S[s].x;
+                fS[2 * B + pos[s]] = S[s].y;
+                fS[4 * B + pos[s]] = S[s].z;
+            }
+        }
+    }
+    __syncthreads();
+    for (uint32_t h = t; h < nr; h += B) {
+#pragma unroll
+        for (int k = 0; k < 5; ++k) a.H[tix(r0 + h, k)] = lds[k * 4 * B + 2 * nf + h];
+    }
+    for (uint32_t f = t; f < nf; f += B) {
+        double Vo[5], Vn[5], UO[5], UN[5], F[5];
+#pragma unroll
+        for (int k = 0; k < 5; ++k) {
+            Vo[k] = lds[k * 4 * B + f];
+            Vn[k] = lds[k * 4 * B + nf + f];
+        }
+        const V3d Sf = {fS[f], fS[2 * B + f], fS[4 * B + f]};
+        prim_to_cons(Vo, UO);
+        prim_to_cons(Vn, UN);
+        if (a.hllc) hllc_d(UO, UN, Sf, F);
+        else rusanov_side(UO, UN, Sf, 0u, F);
+#pragma unroll
+        for (int k = 0; k < 5; ++k) a.FV[5 * (size_t)f0 + k * (size_t)nf + f] = F[k];
+    }
+    if (FUSE) bnd_ghosts<B, GhostOf::REC>(a.bnd, br, L.inst, a.H);
+    if (a.dt_part) {
         const double v = block_reduce<true, B>((live && tc < DBL_MAX) ? tc : DBL_MAX, sh);
         if (t == 0) a.dt_part[L.lb] = v;
     }
 }
 
+// Face vectors of the records and cell volumes, with the sweeps' arithmetic.
+__global__ __launch_bounds__(BLOCK) void k_rec_geo(DevMesh m, double *rS, double *vol) {
+    __shared__ double lds[12 * BLOCK];
+    const LaneCell L = lane_cell<BLOCK>(m, 0);
+    const uint32_t p = L.lb * BLOCK + threadIdx.x;
+    const uint32_t nf = m.foff[L.lb + 1] - m.foff[L.lb], r0 = m.roff[L.lb], code = m.fcode[L.c];
+    const uint2 fx = m.cell_fx[p];
+    const NodeTableLoad ntl = node_table_issue(m, p);
+    CellGeo g;
+    const NodeView nv = node_table_finish<BLOCK>(m, p, ntl, lds, g);
+    cell_geo(m, g);
+    vol[p] = g.vol;
+    if (!L.live) return;
+    const uint32_t pos[4] = {fx.x & 0x7FFFu, (fx.x >> 16) & 0x7FFFu, fx.y & 0x7FFFu, (fx.y >> 16) & 0x7FFFu};
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+        if (pos[s] < 2 * nf) continue;
+        V3d S;
+        face_geo(m, g, nv, (code >> (8 * s)) & 0xFFu, S, nullptr);
+        const uint32_t r = r0 + pos[s] - 2 * nf;
+        const size_t o = ((size_t)(r >> 6) * 3) * TILE + (r & 63u);
+        rS[o] = S.x;
+        rS[o + TILE] = S.y;
+        rS[o + 2 * TILE] = S.z;
+    }
+}
+
 // ---------------------------------------------------------------------------
 struct SweepBArgs {
-    const double *FV;       // [tile][4][5][64]
+    const double *FV;       // [tile][4][5][64]; k_sweepB_face: per block [5][nf] fluxes
+    const double *H;        // k_sweepB_face: [tile][5][64] face values of the records
     const double *Gf;       // [nb/64][5][64] ghost of the reconstructed face state
     const double *U;        // [tile][5][64] state entering the stage
     const double *Uo;       // U_old (U^n)
@@ -854,6 +931,54 @@ struct SweepBArgs {
     double *Rst, *fst;      // checked stage: R [tile][5][64] and f [cell] for k_apply, no update
     BndArgs bnd;            // FUSE: ghosts of the updated cell states (out: Gc), where it updates
 };
+
+// The end of sweep B of a cell with flux balance R: checks, what is kept of R,
+// the stage's update and the residual.
+template <int B, bool FUSE>
+__device__ __forceinline__ void finish_cell(const DevMesh &m, const SweepBArgs &a, const LaneCell &L, BndRange br,
+                                            InstState &st, const double *R, bool zero_old, const double *Up,
+                                            const double *Uop, const Rcp &ivol, double *sh) {
+    const uint32_t c = L.c;
+    const bool live = L.live;
+    if (live && a.check) {
+        bool ok = true;
+#pragma unroll
+        for (int k = 0; k < 5; ++k) ok = ok && (R[k] - R[k] == 0.0);
+        if (!ok) atomicAdd(&st.bad_flux, 1);
+    }
+    if (a.R_aux) {
+        if (live) {
+#pragma unroll
+            for (int k = 0; k < 5; ++k) a.R_aux[5 * (size_t)a.aux_row[c] + k] = R[k];
+        }
+    } else {
+        const double dt = a.dt_cell ? a.dt_cell[c] : st.dt;
+        // Solver::TVD_RK3 / explicit_euler (src/Solver.cpp:98-132)
+        const double f = rdiv(a.kind == 1 ? dt : (a.kind == 2 ? 1.0 / 4.0 * dt : 2.0 / 3.0 * dt), ivol);
+        if (a.Rst) {
+            if (live) {
+#pragma unroll
+                for (int k = 0; k < 5; ++k) a.Rst[tix(c, k)] = R[k];
+                a.fst[c] = f;
+            }
+        } else {
+            double Un[5], Vnew[5];
+            stage_combine(a.kind, zero_old, f, Up, Uop, R, Un);
+            cons_to_prim_d(Un, Vnew);
+            if (live) {
+#pragma unroll
+                for (int k = 0; k < 5; ++k) a.Uout[tix(c, k)] = Un[k];
+                if (!(Vnew[0] > 0.0) || !(Vnew[4] > 0.0) || !(Un[4] > 0.0)) atomicAdd(&st.bad_state, 1);
+            }
+            if (FUSE) bnd_ghosts<B, GhostOf::U>(a.bnd, br, L.inst, a.Uout);
+        }
+    }
+    if (a.res_part) {
+        const double r2 = live ? R[0] * R[0] : 0.0;
+        const double v = block_reduce<false, B>(r2, sh);
+        if (threadIdx.x == 0) a.res_part[L.lb] = v;
+    }
+}
 
 // FLUX: 0 Rusanov, 1 HLLC
 template <int B, int FLUX, bool FUSE>
@@ -936,44 +1061,91 @@ __global__ __launch_bounds__(B) NF_SWEEPB_ATTR void k_sweepB(DevMesh m, SweepBAr
         // faces' values are live at once
         asm volatile("" : "+v"(R[0]), "+v"(R[1]), "+v"(R[2]), "+v"(R[3]), "+v"(R[4]) : : "memory");
     }
-    if (live && a.check) {
-        bool ok = true;
+    finish_cell<B, FUSE>(m, a, L, br, st, R, zero_old, Up, Uop, g.ivol, sh);
+}
+
+// The records' fluxes, then every cell's flux balance from LDS.  156 B per cell
+// move at 3.3 TB/s (998k cells: 48 us); bound by the latency of a block's
+// loads with four waves per SIMD.  Five waves spill: 382 -> 472 us per step.
+template <int FLUX, bool FUSE>
+__global__ __launch_bounds__(BLOCK) void k_sweepB_face(DevMesh m, SweepBArgs a) {
+    constexpr int B = BLOCK;
+    __shared__ double sh[B / 64];
+    extern __shared__ __align__(16) double fl[];  // [5][nent] fluxes of the block's faces, then of its records
+    const LaneCell L = lane_cell<B>(m, a.xcd_remap);
+    const uint32_t f0 = m.foff[L.lb], nf = m.foff[L.lb + 1] - f0, r0 = m.roff[L.lb], nr = m.roff[L.lb + 1] - r0;
+    BndRange br{0, 0};
+    if (FUSE) br = bnd_range<B>(a.bnd.boff, L.lb);
+    InstState &st = m.st[L.inst];
+    if (st.stop) return;
+    const uint32_t c = L.c, t = threadIdx.x;
+    const uint32_t rw = m.rec[r0 + (t < nr ? t : 0)];  // (one entry past the end is there)
+    const uint2 fx = m.cell_fx[L.lb * B + t];
+    double F[2][5];  // (a block has at most 2 B faces)
 #pragma unroll
-        for (int k = 0; k < 5; ++k) ok = ok && (R[k] - R[k] == 0.0);
-        if (!ok) atomicAdd(&st.bad_flux, 1);
-    }
-    if (a.R_aux) {
-        if (live) {
+    for (int q = 0; q < 2; ++q)
+        if (t + q * B < nf) {
 #pragma unroll
-            for (int k = 0; k < 5; ++k) a.R_aux[5 * (size_t)a.aux_row[c] + k] = R[k];
+            for (int k = 0; k < 5; ++k) F[q][k] = a.FV[5 * (size_t)f0 + k * (size_t)nf + t + q * B];
         }
-    } else {
-        const double dt = a.dt_cell ? a.dt_cell[c] : st.dt;
-        // Solver::TVD_RK3 / explicit_euler (src/Solver.cpp:98-132)
-        const double f = rdiv(a.kind == 1 ? dt : (a.kind == 2 ? 1.0 / 4.0 * dt : 2.0 / 3.0 * dt), g.ivol);
-        if (a.Rst) {
-            if (live) {
+    const bool zero_old = st.uold_zero;
+    const double vol = m.vol[c];
+    double Up[5], Uop[5];
+    {
+        const double *uo = (a.kind == 1 || zero_old) ? a.U : a.Uo;
 #pragma unroll
-                for (int k = 0; k < 5; ++k) a.Rst[tix(c, k)] = R[k];
-                a.fst[c] = f;
+        for (int k = 0; k < 5; ++k) {
+            Up[k] = a.U[tix(c, k)];
+            Uop[k] = uo[tix(c, k)];
+        }
+    }
+    auto rec_flux = [&](uint32_t h, uint32_t w) {
+        const uint32_t r = r0 + h;
+        const double *src = ((w & 0x80000000u) ? a.Gf : a.H) + tix(w & 0x1FFFFFFFu, 0);
+        const double *sp = m.rS + (size_t)(r >> 6) * 3 * TILE + (r & 63u);
+        double Vo[5], Vn[5], UO[5], UN[5], G[5];
+#pragma unroll
+        for (int k = 0; k < 5; ++k) {
+            Vo[k] = a.H[tix(r, k)];
+            Vn[k] = ldg(src + k * TILE);
+        }
+        const V3d S = {sp[0], sp[TILE], sp[2 * TILE]};
+        prim_to_cons(Vo, UO);
+        prim_to_cons(Vn, UN);
+        const bool own = w & 0x40000000u;
+        if (FLUX == 1) {
+            double UL[5], UR[5];
+#pragma unroll
+            for (int k = 0; k < 5; ++k) {
+                UL[k] = own ? UO[k] : UN[k];
+                UR[k] = own ? UN[k] : UO[k];
             }
+            hllc_d(UL, UR, S, G);
         } else {
-            double Un[5], Vnew[5];
-            stage_combine(a.kind, zero_old, f, Up, Uop, R, Un);
-            cons_to_prim_d(Un, Vnew);
-            if (live) {
-#pragma unroll
-                for (int k = 0; k < 5; ++k) a.Uout[tix(c, k)] = Un[k];
-                if (!(Vnew[0] > 0.0) || !(Vnew[4] > 0.0) || !(Un[4] > 0.0)) atomicAdd(&st.bad_state, 1);
-            }
-            if (FUSE) bnd_ghosts<B, GhostOf::U>(a.bnd, br, L.inst, a.Uout);
+            rusanov_side(UO, UN, S, own ? 0u : 0x80000000u, G);
         }
+#pragma unroll
+        for (int k = 0; k < 5; ++k) fl[k * m.nent + nf + h] = G[k];
+    };
+    if (t < nr) rec_flux(t, rw);
+    for (uint32_t h = t + B; h < nr; h += B) rec_flux(h, m.rec[r0 + h]);
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+        if (t + q * B < nf) {
+#pragma unroll
+            for (int k = 0; k < 5; ++k) fl[k * m.nent + t + q * B] = F[q][k];
+        }
+    __syncthreads();
+    double R[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+    const uint32_t fw[4] = {fx.x & 0xFFFFu, fx.x >> 16, fx.y & 0xFFFFu, fx.y >> 16};
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+        const uint32_t pos = fw[s] & 0x7FFFu, e = pos < nf ? pos : pos - nf;
+        const uint32_t sub = (fw[s] & 0x8000u) << 16;  // R_i -= F, R_j += F
+#pragma unroll
+        for (int k = 0; k < 5; ++k) R[k] = R[k] + flip(fl[k * m.nent + e], sub);
     }
-    if (a.res_part) {
-        const double r2 = live ? R[0] * R[0] : 0.0;
-        const double v = block_reduce<false, B>(r2, sh);
-        if (threadIdx.x == 0) a.res_part[L.lb] = v;
-    }
+    finish_cell<B, FUSE>(m, a, L, br, st, R, zero_old, Up, Uop, rcp_of(vol), sh);
 }
 
 __global__ __launch_bounds__(BLOCK) void k_apply(DevMesh m, ApplyArgs a) { apply_stage_cell<double>(m, a); }

@@ -301,10 +301,13 @@ struct nf_ctx {
     uint32_t *grp_off = nullptr;          // 64-cell group node tables
     double *gx = nullptr, *gy = nullptr, *gz = nullptr;
     uint2 *cell_ln = nullptr;
-    uint32_t *hal_off = nullptr, *hal = nullptr;  // block halos of sweep A; null: gathered per lane
-    uint2 *cell_nb = nullptr;
-    uint32_t nstride = 86;  // node table entries per 64 cells: at least the face values' 256 doubles
-    uint32_t halo_lds = 0;  // LDS bytes of a halo block
+    // faces and records of the blocks (DevMesh); null: gathered per lane
+    uint32_t *foff = nullptr, *roff = nullptr, *hal = nullptr, *rec = nullptr, *brec = nullptr;
+    uint2 *cell_nb = nullptr, *cell_fx = nullptr;
+    double *rS = nullptr, *vol = nullptr;
+    uint32_t nstride = 1, nent = 0;
+    uint32_t face_lds = 0;  // LDS bytes of a block of k_sweepA_face
+    size_t rec_at = 0;  // records' place in FV
     uint32_t *blk_inst = nullptr;
     uint32_t *inst_end = nullptr;
     InstState *st = nullptr;
@@ -372,7 +375,8 @@ int dalloc(nf_ctx *ctx, T **p, size_t n) {
 
 DevMesh devmesh(const nf_ctx *c) {
     return DevMesh{3.0,         6.0,       c->nodes, c->cnodes, c->grp_off,  c->gx,       c->gy,
-                   c->gz,       c->cell_ln, c->nbr,   c->hal_off, c->hal,    c->cell_nb, c->nstride, c->fcode,
+                   c->gz,       c->cell_ln, c->nbr,   c->foff,    c->roff,  c->hal,
+                   c->rec,      c->cell_nb,  c->cell_fx, c->rS,   c->vol,   c->nstride, c->nent,  c->fcode,
                    c->blk_inst, c->inst_end, c->st};
 }
 
@@ -429,7 +433,7 @@ int refresh_v(nf_ctx *ctx) {
 }
 
 BndArgs bnd_args(const nf_ctx *c, double *out) {
-    return {c->bface, c->boff, c->binst, c->bbc, c->bS, c->nbf, c->fs, out};
+    return {c->bface, c->boff, c->binst, c->bbc, c->bS, c->nbf, c->brec, c->fs, out};
 }
 mx::BndArgsMx bnd_args_mx(const nf_ctx *c, float *out) {
     return {c->bface, c->boff, c->binst, c->bbc, c->nbf, c->fs32, out};
@@ -448,6 +452,16 @@ int run_ghost_cell(nf_ctx *ctx, const double *U) {
     return LAUNCH("ghost_cell", k_ghost<GhostOf::V>, g, b, bnd_args(ctx, ctx->Gc), (const double *)ctx->V);
 }
 
+int order_of(const nf_ctx *ctx) {
+    if (ctx->prm.spatial_order == NF_FIRST_ORDER) return 0;
+    return ctx->prm.limiter == NF_LIMITER_NONE ? 1 : 2;
+}
+
+// The sweeps over block faces (k_sweepA_face): second order, 256-cell blocks,
+// every block's LDS fits.  Cells in an order without locality have up to 1,024
+// outside neighbours per block; their gather is the same work either way.
+bool use_faces(const nf_ctx *ctx) { return order_of(ctx) != 0 && ctx->block == BLOCK && ctx->cell_nb; }
+
 // ghosts of the reconstructed face states
 int run_ghost_face(nf_ctx *ctx) {
     if (ctx->nbf == 0) return NF_OK;
@@ -455,13 +469,11 @@ int run_ghost_face(nf_ctx *ctx) {
         return launch_fn(ctx, "ghost_face_mx", [&] {
             return mx::launch_ghost_mx(true, ctx->stream, devmesh(ctx), bnd_args_mx(ctx, ctx->Gf32), ctx->FV32);
         });
+    if (use_faces(ctx))
+        return LAUNCH("ghost_face", k_ghost<GhostOf::REC>, dim3((ctx->nbf + BLOCK - 1) / BLOCK), dim3(BLOCK),
+                      bnd_args(ctx, ctx->Gf), (const double *)(ctx->FV + ctx->rec_at));
     return LAUNCH("ghost_face", k_ghost<GhostOf::FV>, dim3((ctx->nbf + BLOCK - 1) / BLOCK), dim3(BLOCK),
                   bnd_args(ctx, ctx->Gf), (const double *)ctx->FV);
-}
-
-int order_of(const nf_ctx *ctx) {
-    if (ctx->prm.spatial_order == NF_FIRST_ORDER) return 0;
-    return ctx->prm.limiter == NF_LIMITER_NONE ? 1 : 2;
 }
 
 template <int B, bool FROM_U, bool FUSE>
@@ -489,11 +501,6 @@ hipError_t launch_sweepB(hipStream_t s, uint32_t ncell, bool hllc, const DevMesh
 constexpr uint32_t FUSE_MAX_CELLS = 1024 * BLOCK;
 bool fused_ghosts(const nf_ctx *ctx) { return ctx->Ncell <= FUSE_MAX_CELLS; }
 
-// sweep A with block halos: second order, 256-cell blocks, every halo fits.
-// (Cells in an order without locality have up to 1,024 outside neighbours per
-// block; their gather is the same work either way.)
-bool use_halo(const nf_ctx *ctx, int order) { return order != 0 && ctx->block == BLOCK && ctx->cell_nb; }
-
 // sweep A of the current primvars, or (U set, FP64) of prim(U) of that state.
 // dt: per-block CFL minima into dt_part; dtc: per-cell CFL steps into dt_cell
 // (local time stepping); aux: keep the gradient and limiter fields.
@@ -516,17 +523,17 @@ int run_sweepA(nf_ctx *ctx, bool dt, bool aux, bool dtc = false, const double *U
             return mx::launch_sweepA_mx(order, ctx->block, fuse, ctx->Ncell, ctx->stream, m, x);
         });
     }
-    const SweepAArgs a{U ? U : ctx->V, ctx->Gc, ctx->FV, dt ? ctx->dt_part : nullptr, dtc ? ctx->dt_cell : nullptr,
+    const SweepAArgs a{U ? U : ctx->V, ctx->Gc, ctx->FV, ctx->FV + ctx->rec_at, dt ? ctx->dt_part : nullptr, dtc ? ctx->dt_cell : nullptr,
                        ctx->prm.CFL, ctx->xcd_remap, aux ? ctx->grad_aux : nullptr, aux ? ctx->psi_aux : nullptr,
-                       ctx->perm_dev, bnd_args(ctx, ctx->Gf)};
+                       ctx->perm_dev, bnd_args(ctx, ctx->Gf), ctx->prm.inv_flux_scheme == NF_FLUX_HLLC};
     const char *name = order == 2 ? "sweepA_barth" : (order == 1 ? "sweepA_nolim" : "sweepA_first");
     return launch_fn(ctx, name, [&] {
-        if (use_halo(ctx, order)) {
+        if (use_faces(ctx)) {
             auto go = [&](auto from_u, auto fused) {
                 const dim3 g(ctx->Ncell / BLOCK), b(BLOCK);
-                const uint32_t lds = ctx->halo_lds;
-                if (order == 1) hipLaunchKernelGGL((k_sweepA_halo<1, from_u(), fused()>), g, b, lds, ctx->stream, m, a);
-                else hipLaunchKernelGGL((k_sweepA_halo<2, from_u(), fused()>), g, b, lds, ctx->stream, m, a);
+                const uint32_t lds = ctx->face_lds;
+                if (order == 1) hipLaunchKernelGGL((k_sweepA_face<1, from_u(), fused()>), g, b, lds, ctx->stream, m, a);
+                else hipLaunchKernelGGL((k_sweepA_face<2, from_u(), fused()>), g, b, lds, ctx->stream, m, a);
                 return hipGetLastError();
             };
             if (U) return fuse ? go(std::true_type{}, std::true_type{}) : go(std::true_type{}, std::false_type{});
@@ -570,12 +577,19 @@ int run_sweepB(nf_ctx *ctx, int kind, const double *U, double *Uout, bool res, b
                          [&] { return mx::launch_apply_mx(dim3(ctx->Ncell / BLOCK), ctx->stream, m, ap); });
     }
     // (FP64: prim(Uout) is not stored; the next sweep A evaluates it from U)
-    const SweepBArgs a{ctx->FV, ctx->Gf, U, ctx->Ua, Uout, dtc, kind, res ? ctx->res_part : nullptr,
+    const SweepBArgs a{ctx->FV, ctx->FV + ctx->rec_at, ctx->Gf, U, ctx->Ua, Uout, dtc, kind, res ? ctx->res_part : nullptr,
                        ctx->prm.check_physical_validity, ctx->xcd_remap, aux ? ctx->R_aux : nullptr, ctx->perm_dev, Rst, fst,
                        bnd_args(ctx, ctx->Gc)};
     const bool hllc = ctx->prm.inv_flux_scheme == NF_FLUX_HLLC;
     if ((rc = launch_fn(ctx, "sweepB", [&] {
              auto go = [&](auto fused) {
+                 if (use_faces(ctx)) {
+                     const dim3 g(ctx->Ncell / BLOCK), b(BLOCK);
+                     const uint32_t lds = 5 * 8 * ctx->nent;
+                     if (hllc) hipLaunchKernelGGL((k_sweepB_face<1, fused()>), g, b, lds, ctx->stream, m, a);
+                     else hipLaunchKernelGGL((k_sweepB_face<0, fused()>), g, b, lds, ctx->stream, m, a);
+                     return hipGetLastError();
+                 }
                  return ctx->block == 128 ? launch_sweepB<128, fused()>(ctx->stream, ctx->Ncell, hllc, m, a)
                                           : launch_sweepB<256, fused()>(ctx->stream, ctx->Ncell, hllc, m, a);
              };
@@ -1100,51 +1114,75 @@ int create(int32_t n, const nf_mesh_desc *descs, const nf_params *prms, nf_ctx *
                     }
                     l[q] = loc[v];
                 }
-                cell_ln[p] = make_uint2(l[0] | l[1] << 16, l[2] | l[3] << 16);
+                cell_ln[p] = make_uint2(24 * (l[0] | l[1] << 16), 24 * (l[2] | l[3] << 16));
             }
             grp_off.push_back(grp_off.back() + cnt);
         }
     }
-    // block halos of sweep A: distinct outside states in first-use order
-    std::vector<uint32_t> hal_off(1, 0), hal;
-    std::vector<uint2> cell_nb(cell0);
-    for (size_t g = 0; g + 1 < grp_off.size(); ++g) ctx->nstride = std::max(ctx->nstride, grp_off[g + 1] - grp_off[g]);
-    ctx->nstride = (ctx->nstride + 1) & ~1u;
+    // faces and records of the blocks, in first-use order
+    const size_t guess = cell0 + 4 * BLOCK;  // (200 records per block in Morton order)
+    std::vector<uint32_t> foff(1, 0), roff(1, 0), hal, rec, rec_side, side_rec(4 * cell0), brec(bface.size());
+    std::vector<uint2> cell_nb(cell0), cell_fx(cell0);
+    uint32_t nrmax = 0;
     {
-        std::vector<uint32_t> stamp(cell0, UINT32_MAX), loc(cell0);
+        for (auto *v : {&hal, &rec, &rec_side}) v->reserve(guess);
+        auto pack = [](const uint32_t *l) { return make_uint2(l[0] | l[1] << 16, l[2] | l[3] << 16); };
+        uint32_t face[4 * BLOCK];
         for (uint32_t b = 0; b < cell0 / BLOCK; ++b) {
-            uint32_t cnt = 0;
-            for (uint32_t p = b * BLOCK; p < (b + 1) * BLOCK; ++p) {
-                if (p >= inst_end[blk_inst[b]]) {  // padding: as the last cell, in this block too
-                    cell_nb[p] = cell_nb[p - 1];
-                    continue;
-                }
+            uint32_t nf = 0, nr = 0;
+            const uint32_t p0 = b * BLOCK, end = std::min(p0 + BLOCK, inst_end[blk_inst[b]]);
+            for (uint32_t p = p0; p < end; ++p) {
                 uint32_t l[4];
-                for (int q = 0; q < 4; ++q) {
-                    const uint32_t w = nbr[4 * (size_t)p + q], idx = w & NBR_INDEX_MASK;
-                    if (w & NBR_BOUNDARY) {  // (its cell's alone)
-                        hal.push_back(NBR_BOUNDARY | idx);
-                        l[q] = 0x8000u | (BLOCK + cnt++);
-                    } else if (idx / BLOCK == b) {
-                        l[q] = idx % BLOCK;
+                for (uint32_t q = 0; q < 4; ++q) {
+                    const uint32_t i = 4 * p + q, w = nbr[i], idx = w & NBR_INDEX_MASK;
+                    if ((w & NBR_BOUNDARY) || idx / BLOCK != b) {
+                        l[q] = (w & NBR_BOUNDARY) >> 16 | (BLOCK + nr);
+                        hal.push_back((w & NBR_BOUNDARY) | idx);
+                        side_rec[i] = roff.back() + nr;
+                        face[i - 4 * p0] = nr++;
                     } else {
-                        if (stamp[idx] != b) {
-                            stamp[idx] = b;
-                            loc[idx] = BLOCK + cnt++;
-                            hal.push_back(idx);
-                        }
-                        l[q] = loc[idx];
+                        const uint32_t j = 4 * idx + ((w >> 29) & 3u);  // the other side
+                        l[q] = idx - p0;
+                        face[i - 4 * p0] = j < i ? face[j - 4 * p0] : nf++;
                     }
                 }
-                cell_nb[p] = make_uint2(l[0] | l[1] << 16, l[2] | l[3] << 16);
+                cell_nb[p] = pack(l);
             }
-            ctx->halo_lds = std::max(ctx->halo_lds, cnt);
-            hal_off.push_back((uint32_t)hal.size());
+            for (uint32_t p = p0; p < end; ++p) {
+                uint32_t l[4];
+                for (uint32_t q = 0; q < 4; ++q) {
+                    const uint32_t i = 4 * p + q, w = nbr[i], own = (fcode[p] >> (8 * q + 7)) & 1u;
+                    const bool out = (w & NBR_BOUNDARY) || (w & NBR_INDEX_MASK) / BLOCK != b;
+                    l[q] = own << 15 | (face[i - 4 * p0] + (out ? 2 * nf : (own ? 0 : nf)));
+                    if (out) {
+                        rec.push_back(own << 30);
+                        rec_side.push_back(i);
+                    }
+                }
+                cell_fx[p] = pack(l);
+            }
+            for (uint32_t p = end; p < p0 + BLOCK; ++p) {  // padding: as the last cell
+                cell_nb[p] = cell_nb[end - 1];
+                cell_fx[p] = cell_fx[end - 1];
+            }
+            ctx->nent = std::max(ctx->nent, nf + nr);
+            nrmax = std::max(nrmax, nr);
+            foff.push_back(foff.back() + nf);
+            roff.push_back(roff.back() + nr);
         }
+        for (size_t r = 0; r < rec.size(); ++r) {
+            const uint32_t w = nbr[rec_side[r]], idx = w & NBR_INDEX_MASK;
+            if (w & NBR_BOUNDARY) brec[idx] = (uint32_t)r;
+            rec[r] |= (w & NBR_BOUNDARY) ? w & (NBR_BOUNDARY | NBR_INDEX_MASK) : side_rec[4 * idx + ((w >> 29) & 3u)];
+        }
+        hal.push_back(0);  // (read, not used, by a block without records)
+        rec.push_back(0);
+        for (size_t g = 0; g + 1 < grp_off.size(); ++g)
+            ctx->nstride = std::max(ctx->nstride, grp_off[g + 1] - grp_off[g]);
     }
-    ctx->halo_lds = 8 * (12 * ctx->nstride + 5 * (BLOCK + ctx->halo_lds));
-    const bool halos = ctx->halo_lds <= HALO_LDS;
-    hal.push_back(0);  // (read, not used, by a block without a halo)
+    ctx->rec_at = (5 * (size_t)foff.back() + 63) / 64 * 64;
+    ctx->face_lds = 8 * std::max<uint32_t>(12 * ctx->nstride + 5 * (BLOCK + nrmax), 26 * BLOCK);
+    const bool faces = ctx->face_lds <= FACE_LDS;
     ctx->Ncell = (uint32_t)cell0;
     ctx->nbf = (uint32_t)bface.size();
 
@@ -1160,11 +1198,21 @@ int create(int32_t n, const nf_mesh_desc *descs, const nf_params *prms, nf_ctx *
     if ((rc = dalloc(ctx, &ctx->gy, gy.size()))) return rc;
     if ((rc = dalloc(ctx, &ctx->gz, gz.size()))) return rc;
     if ((rc = dalloc(ctx, &ctx->cell_ln, cell_ln.size()))) return rc;
-    if (halos) {
-        if ((rc = dalloc(ctx, &ctx->hal_off, hal_off.size()))) return rc;
+    if (faces) {
         if ((rc = dalloc(ctx, &ctx->hal, hal.size()))) return rc;
         if ((rc = dalloc(ctx, &ctx->cell_nb, cell_nb.size()))) return rc;
-        HIPC(hipMemcpy(ctx->hal_off, hal_off.data(), hal_off.size() * 4, hipMemcpyHostToDevice));
+        if ((rc = dalloc(ctx, &ctx->foff, foff.size()))) return rc;
+        if ((rc = dalloc(ctx, &ctx->roff, roff.size()))) return rc;
+        if ((rc = dalloc(ctx, &ctx->rec, rec.size()))) return rc;
+        if ((rc = dalloc(ctx, &ctx->brec, brec.size()))) return rc;
+        if ((rc = dalloc(ctx, &ctx->cell_fx, cell_fx.size()))) return rc;
+        if ((rc = dalloc(ctx, &ctx->rS, 3 * ((rec.size() + 63) / 64 * 64)))) return rc;
+        if ((rc = dalloc(ctx, &ctx->vol, NC))) return rc;
+        HIPC(hipMemcpy(ctx->foff, foff.data(), foff.size() * 4, hipMemcpyHostToDevice));
+        HIPC(hipMemcpy(ctx->roff, roff.data(), roff.size() * 4, hipMemcpyHostToDevice));
+        HIPC(hipMemcpy(ctx->rec, rec.data(), rec.size() * 4, hipMemcpyHostToDevice));
+        if (ctx->nbf) HIPC(hipMemcpy(ctx->brec, brec.data(), brec.size() * 4, hipMemcpyHostToDevice));
+        HIPC(hipMemcpy(ctx->cell_fx, cell_fx.data(), cell_fx.size() * sizeof(uint2), hipMemcpyHostToDevice));
         HIPC(hipMemcpy(ctx->hal, hal.data(), hal.size() * 4, hipMemcpyHostToDevice));
         HIPC(hipMemcpy(ctx->cell_nb, cell_nb.data(), cell_nb.size() * sizeof(uint2), hipMemcpyHostToDevice));
     }
@@ -1180,7 +1228,7 @@ int create(int32_t n, const nf_mesh_desc *descs, const nf_params *prms, nf_ctx *
         if ((rc = dalloc(ctx, &ctx->Gf32, 5 * ((size_t)ctx->nbf + TILE - 1) / TILE * TILE))) return rc;
     } else {
         if ((rc = dalloc(ctx, &ctx->V, 5 * NC))) return rc;
-        if ((rc = dalloc(ctx, &ctx->FV, 20 * NC))) return rc;
+        if ((rc = dalloc(ctx, &ctx->FV, 20 * NC + 512))) return rc;
         if ((rc = dalloc(ctx, &ctx->Gc, 5 * ((size_t)ctx->nbf + TILE - 1) / TILE * TILE))) return rc;
         if ((rc = dalloc(ctx, &ctx->Gf, 5 * ((size_t)ctx->nbf + TILE - 1) / TILE * TILE))) return rc;
     }
@@ -1212,6 +1260,11 @@ int create(int32_t n, const nf_mesh_desc *descs, const nf_params *prms, nf_ctx *
     HIPC(hipMemcpy(ctx->cell_ln, cell_ln.data(), cell_ln.size() * sizeof(uint2), hipMemcpyHostToDevice));
     HIPC(hipMemcpy(ctx->blk_inst, blk_inst.data(), blk_inst.size() * 4, hipMemcpyHostToDevice));
     HIPC(hipMemcpy(ctx->inst_end, inst_end.data(), inst_end.size() * 4, hipMemcpyHostToDevice));
+    if (faces) {
+        hipLaunchKernelGGL(k_rec_geo, dim3(ctx->Ncell / BLOCK), dim3(BLOCK), 0, ctx->stream, devmesh(ctx), ctx->rS, ctx->vol);
+        HIPC(hipGetLastError());
+        HIPC(hipStreamSynchronize(ctx->stream));
+    }
     if (ctx->nbf) {
         HIPC(hipMemcpy(ctx->bface, bface.data(), bface.size() * 4, hipMemcpyHostToDevice));
         HIPC(hipMemcpy(ctx->bbc, bbc.data(), bbc.size(), hipMemcpyHostToDevice));
@@ -1743,7 +1796,7 @@ int nf_set_precision(nf_ctx *ctx, int32_t precision) {
     }
     if (!mixed && !ctx->V) {
         if ((rc = dalloc(ctx, &ctx->V, 5 * NC))) return rc;
-        if ((rc = dalloc(ctx, &ctx->FV, 20 * NC))) return rc;
+        if ((rc = dalloc(ctx, &ctx->FV, 20 * NC + 512))) return rc;
         if ((rc = dalloc(ctx, &ctx->Gc, 5 * ((size_t)ctx->nbf + TILE - 1) / TILE * TILE))) return rc;
         if ((rc = dalloc(ctx, &ctx->Gf, 5 * ((size_t)ctx->nbf + TILE - 1) / TILE * TILE))) return rc;
     }
