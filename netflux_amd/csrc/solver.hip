@@ -495,10 +495,11 @@ hipError_t launch_sweepB(hipStream_t s, uint32_t ncell, bool hllc, const DevMesh
 // Boundary ghosts at the end of the sweeps (FUSE) or in launches of their own:
 // a launch costs 4 to 6 us whatever it does, a boundary block's ghosts 4 to 8
 // us at the end of a sweep, hidden only while blocks do not queue for CUs.
-// Step at 63k / 196k / 303k / 584k farfield cells, us: separate 78.7 / 135 /
-// 184 / 276, fused 63.0 / 133 / 190 / 295; mixed precision 67.3 / 109 / 145 /
-// 208 and 54.5 / 97 / 145 / 217.
-constexpr uint32_t FUSE_MAX_CELLS = 1024 * BLOCK;
+// Step of farfield boxes, us, separate / fused: 63k cells 76.5 / 60.7, 215k 145
+// / 136, 329k 176 / 171, 511k 221 / 222, 795k 306 / 311; of channels 349k 184 /
+// 175, 480k 215 / 210, 829k 315 / 317; mixed precision, box 63k 67 / 54, 303k
+// 145 / 145, 444k 176 / 180, channel 294k 147 / 141, 480k 190 / 188.
+constexpr uint32_t FUSE_MAX_CELLS = 1536 * BLOCK;
 bool fused_ghosts(const nf_ctx *ctx) { return ctx->Ncell <= FUSE_MAX_CELLS; }
 
 // sweep A of the current primvars, or (U set, FP64) of prim(U) of that state.

@@ -115,3 +115,22 @@ def test_wall_boxes_match_oracle(n):
     g.run(12, check_every=4)
     o.run(12)
     np.testing.assert_array_equal(g.get_solver_data().get_solution(), o.get("U"))
+
+
+@pytest.mark.parametrize("precision,block", [("fp64", 256), ("fp64", 128), ("mixed", 256)])
+def test_large_batch_equals_single(precision, block):
+    """The ghosts in launches of their own: a batch of 1,800 blocks against
+    its meshes alone, whose sweeps store them."""
+    print(f"[case] separate ghosts, {precision}, block {block}", flush=True)
+    mesh = nf.Mesh.box((36, 34, 33), jitter=0.1, patches=("FarField", "SlipWall", "NoSlipWall") * 2)
+    cfg = pulse_config(precision=precision, rk3_zero_old_first_step=False)
+    b = nf.BatchSolver(cfg, [mesh, nf.Mesh.box((34, 33, 33), patches=("SlipWall",) * 6)])
+    assert sum(b.N) > 1700 * 256
+    U = pulse_state(mesh)
+    g = nf.EulerSolver(cfg, mesh)
+    for s in (b, g):
+        s.set_launch(block)
+        s.set_state(*((0, U) if s is b else (U,)))
+        s.run(5, check_every=2)
+    np.testing.assert_array_equal(b.get_solution(0), g.get_solver_data().get_solution())
+    np.testing.assert_array_equal(b.residuals(0), g.residuals())
