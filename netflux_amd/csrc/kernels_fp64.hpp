@@ -890,6 +890,100 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(3, 3))) v
     }
 }
 
+// Faces and records of the blocks, numbered in the order of the cells' slots.
+// COUNT: foff[b + 1], roff[b + 1] = their numbers.  Otherwise, from the
+// offsets, the tables of DevMesh but rec, and side_rec [cell][4], the record
+// of each side.
+struct FaceTables {
+    uint32_t *foff, *roff, *hal, *rec, *brec, *side_rec;
+    uint2 *cell_nb, *cell_fx;
+};
+template <bool COUNT>
+__global__ __launch_bounds__(BLOCK) void k_block_faces(DevMesh m, FaceTables o) {
+    __shared__ uint32_t sum[BLOCK];      // faces | records << 16
+    __shared__ uint16_t face[4 * BLOCK];
+    __shared__ uint2 last[2];
+    const uint32_t b = blockIdx.x, t = threadIdx.x, p0 = b * BLOCK, p = p0 + t;
+    const bool live = p < m.inst_end[m.blk_inst[b]];
+    const uint4 w4 = *reinterpret_cast<const uint4 *>(m.nbr + 4 * (size_t)p);
+    const uint32_t w[4] = {w4.x, w4.y, w4.z, w4.w};
+    bool out[4], first[4];
+    uint32_t j[4], n = 0;
+#pragma unroll
+    for (uint32_t q = 0; q < 4; ++q) {
+        const uint32_t idx = w[q] & 0x1FFFFFFFu;
+        out[q] = (w[q] & 0x80000000u) || idx / BLOCK != b;
+        j[q] = 4 * (idx - p0) + ((w[q] >> 29) & 3u);  // the other side's place in the block
+        first[q] = !out[q] && 4 * t + q < j[q];
+        if (live) n += (first[q] ? 1u : 0u) + (out[q] ? 0x10000u : 0u);
+    }
+    sum[t] = n;
+    __syncthreads();
+    for (uint32_t d = 1; d < BLOCK; d *= 2) {
+        const uint32_t v = t >= d ? sum[t - d] : 0;
+        __syncthreads();
+        sum[t] += v;
+        __syncthreads();
+    }
+    const uint32_t nf = sum[BLOCK - 1] & 0xFFFFu, nr = sum[BLOCK - 1] >> 16;
+    if (COUNT) {
+        if (t == 0) o.foff[b + 1] = nf, o.roff[b + 1] = nr;
+        return;
+    }
+    uint32_t f = (sum[t] - n) & 0xFFFFu, h = (sum[t] - n) >> 16, nb[4], fx[4];
+#pragma unroll
+    for (uint32_t q = 0; q < 4; ++q)
+        if (live && first[q]) face[4 * t + q] = (uint16_t)f++;
+    __syncthreads();
+    const uint32_t code = m.fcode[p];
+#pragma unroll
+    for (uint32_t q = 0; q < 4; ++q) {
+        if (!live) continue;
+        const uint32_t own = (code >> (8 * q + 7)) & 1u;
+        if (out[q]) {
+            const uint32_t r = o.roff[b] + h;
+            o.hal[r] = w[q] & 0x9FFFFFFFu;
+            o.side_rec[4 * (size_t)p + q] = r;
+            nb[q] = (w[q] & 0x80000000u) >> 16 | (BLOCK + h);
+            fx[q] = own << 15 | (2 * nf + h++);
+        } else {
+            const uint32_t g = face[first[q] ? 4 * t + q : j[q]];
+            nb[q] = j[q] / 4;
+            fx[q] = own << 15 | (own ? g : nf + g);
+        }
+    }
+    if (live) {
+        const uint2 a = make_uint2(nb[0] | nb[1] << 16, nb[2] | nb[3] << 16);
+        const uint2 c = make_uint2(fx[0] | fx[1] << 16, fx[2] | fx[3] << 16);
+        o.cell_nb[p] = a;
+        o.cell_fx[p] = c;
+        if (t == BLOCK - 1 || p + 1 == m.inst_end[m.blk_inst[b]]) last[0] = a, last[1] = c;
+    }
+    __syncthreads();
+    if (!live) o.cell_nb[p] = last[0], o.cell_fx[p] = last[1];  // padding: as the last cell
+}
+
+// rec and brec, once every block has numbered its records
+__global__ __launch_bounds__(BLOCK) void k_link_records(DevMesh m, FaceTables o) {
+    const uint32_t b = blockIdx.x, p = b * BLOCK + threadIdx.x;
+    if (b + 1 == gridDim.x && threadIdx.x == 0) {  // (read, not used, by a block without records)
+        const uint32_t n = o.roff[gridDim.x];
+        o.hal[n] = 0;
+        o.rec[n] = 0;
+    }
+    if (p >= m.inst_end[m.blk_inst[b]]) return;
+    const uint32_t code = m.fcode[p];
+    for (uint32_t q = 0; q < 4; ++q) {
+        const uint32_t w = m.nbr[4 * (size_t)p + q], idx = w & 0x1FFFFFFFu;
+        const bool bnd = w & 0x80000000u;
+        if (!bnd && idx / BLOCK == b) continue;
+        const uint32_t r = o.side_rec[4 * (size_t)p + q];
+        if (bnd) o.brec[idx] = r;
+        o.rec[r] = ((code >> (8 * q + 7)) & 1u) << 30 |
+                   (bnd ? 0x80000000u | idx : o.side_rec[4 * (size_t)idx + ((w >> 29) & 3u)]);
+    }
+}
+
 // Face vectors of the records and cell volumes, with the sweeps' arithmetic.
 __global__ __launch_bounds__(BLOCK) void k_rec_geo(DevMesh m, double *rS, double *vol) {
     __shared__ double lds[12 * BLOCK];

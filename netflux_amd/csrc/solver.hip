@@ -502,6 +502,59 @@ hipError_t launch_sweepB(hipStream_t s, uint32_t ncell, bool hllc, const DevMesh
 constexpr uint32_t FUSE_MAX_CELLS = 1536 * BLOCK;
 bool fused_ghosts(const nf_ctx *ctx) { return ctx->Ncell <= FUSE_MAX_CELLS; }
 
+// The block faces of an FP64 context (DevMesh), on the device: as host loops
+// they were 15 of the 150 ms that a context of 500k cells takes.  The sides'
+// records pass through FV, which no sweep has written for a later one yet.
+int build_faces(nf_ctx *ctx) {
+    if (order_of(ctx) == 0) return NF_OK;
+    int rc;
+    const uint32_t nblk = ctx->Ncell / BLOCK;
+    std::vector<uint32_t> foff(nblk + 1), roff(nblk + 1);
+    FaceTables o{};
+    o.side_rec = reinterpret_cast<uint32_t *>(ctx->FV);
+    if ((rc = dalloc(ctx, &o.foff, nblk + 1))) return rc;
+    if ((rc = dalloc(ctx, &o.roff, nblk + 1))) return rc;
+    hipLaunchKernelGGL(k_block_faces<true>, dim3(nblk), dim3(BLOCK), 0, ctx->stream, devmesh(ctx), o);
+    HIPC(hipGetLastError());
+    HIPC(hipStreamSynchronize(ctx->stream));
+    HIPC(hipMemcpy(foff.data(), o.foff, foff.size() * 4, hipMemcpyDeviceToHost));
+    HIPC(hipMemcpy(roff.data(), o.roff, roff.size() * 4, hipMemcpyDeviceToHost));
+    foff[0] = roff[0] = 0;
+    uint32_t nrmax = 0;
+    for (uint32_t b = 0; b < nblk; ++b) {
+        ctx->nent = std::max(ctx->nent, foff[b + 1] + roff[b + 1]);
+        nrmax = std::max(nrmax, roff[b + 1]);
+        foff[b + 1] += foff[b];
+        roff[b + 1] += roff[b];
+    }
+    ctx->face_lds = 8 * std::max<uint32_t>(12 * ctx->nstride + 5 * (BLOCK + nrmax), 26 * BLOCK);
+    if (ctx->face_lds > FACE_LDS) return NF_OK;
+    const size_t nr = roff[nblk];
+    ctx->rec_at = (5 * (size_t)foff[nblk] + 63) / 64 * 64;
+    if ((rc = dalloc(ctx, &o.hal, nr + 1))) return rc;
+    if ((rc = dalloc(ctx, &o.rec, nr + 1))) return rc;
+    if ((rc = dalloc(ctx, &o.brec, ctx->nbf))) return rc;
+    if ((rc = dalloc(ctx, &o.cell_nb, ctx->Ncell))) return rc;
+    if ((rc = dalloc(ctx, &o.cell_fx, ctx->Ncell))) return rc;
+    if ((rc = dalloc(ctx, &ctx->rS, 3 * ((nr + 63) / 64 * 64)))) return rc;
+    if ((rc = dalloc(ctx, &ctx->vol, ctx->Ncell))) return rc;
+    HIPC(hipMemcpy(o.foff, foff.data(), foff.size() * 4, hipMemcpyHostToDevice));
+    HIPC(hipMemcpy(o.roff, roff.data(), roff.size() * 4, hipMemcpyHostToDevice));
+    hipLaunchKernelGGL(k_block_faces<false>, dim3(nblk), dim3(BLOCK), 0, ctx->stream, devmesh(ctx), o);
+    hipLaunchKernelGGL(k_link_records, dim3(nblk), dim3(BLOCK), 0, ctx->stream, devmesh(ctx), o);
+    ctx->foff = o.foff;
+    ctx->roff = o.roff;
+    ctx->hal = o.hal;
+    ctx->rec = o.rec;
+    ctx->brec = o.brec;
+    ctx->cell_fx = o.cell_fx;
+    hipLaunchKernelGGL(k_rec_geo, dim3(nblk), dim3(BLOCK), 0, ctx->stream, devmesh(ctx), ctx->rS, ctx->vol);
+    HIPC(hipGetLastError());
+    HIPC(hipStreamSynchronize(ctx->stream));
+    ctx->cell_nb = o.cell_nb;  // (from here on the sweeps use them)
+    return NF_OK;
+}
+
 // sweep A of the current primvars, or (U set, FP64) of prim(U) of that state.
 // dt: per-block CFL minima into dt_part; dtc: per-cell CFL steps into dt_cell
 // (local time stepping); aux: keep the gradient and limiter fields.
@@ -1120,70 +1173,8 @@ int create(int32_t n, const nf_mesh_desc *descs, const nf_params *prms, nf_ctx *
             grp_off.push_back(grp_off.back() + cnt);
         }
     }
-    // faces and records of the blocks, in first-use order
-    const size_t guess = cell0 + 4 * BLOCK;  // (200 records per block in Morton order)
-    std::vector<uint32_t> foff(1, 0), roff(1, 0), hal, rec, rec_side, side_rec(4 * cell0), brec(bface.size());
-    std::vector<uint2> cell_nb(cell0), cell_fx(cell0);
-    uint32_t nrmax = 0;
-    {
-        for (auto *v : {&hal, &rec, &rec_side}) v->reserve(guess);
-        auto pack = [](const uint32_t *l) { return make_uint2(l[0] | l[1] << 16, l[2] | l[3] << 16); };
-        uint32_t face[4 * BLOCK];
-        for (uint32_t b = 0; b < cell0 / BLOCK; ++b) {
-            uint32_t nf = 0, nr = 0;
-            const uint32_t p0 = b * BLOCK, end = std::min(p0 + BLOCK, inst_end[blk_inst[b]]);
-            for (uint32_t p = p0; p < end; ++p) {
-                uint32_t l[4];
-                for (uint32_t q = 0; q < 4; ++q) {
-                    const uint32_t i = 4 * p + q, w = nbr[i], idx = w & NBR_INDEX_MASK;
-                    if ((w & NBR_BOUNDARY) || idx / BLOCK != b) {
-                        l[q] = (w & NBR_BOUNDARY) >> 16 | (BLOCK + nr);
-                        hal.push_back((w & NBR_BOUNDARY) | idx);
-                        side_rec[i] = roff.back() + nr;
-                        face[i - 4 * p0] = nr++;
-                    } else {
-                        const uint32_t j = 4 * idx + ((w >> 29) & 3u);  // the other side
-                        l[q] = idx - p0;
-                        face[i - 4 * p0] = j < i ? face[j - 4 * p0] : nf++;
-                    }
-                }
-                cell_nb[p] = pack(l);
-            }
-            for (uint32_t p = p0; p < end; ++p) {
-                uint32_t l[4];
-                for (uint32_t q = 0; q < 4; ++q) {
-                    const uint32_t i = 4 * p + q, w = nbr[i], own = (fcode[p] >> (8 * q + 7)) & 1u;
-                    const bool out = (w & NBR_BOUNDARY) || (w & NBR_INDEX_MASK) / BLOCK != b;
-                    l[q] = own << 15 | (face[i - 4 * p0] + (out ? 2 * nf : (own ? 0 : nf)));
-                    if (out) {
-                        rec.push_back(own << 30);
-                        rec_side.push_back(i);
-                    }
-                }
-                cell_fx[p] = pack(l);
-            }
-            for (uint32_t p = end; p < p0 + BLOCK; ++p) {  // padding: as the last cell
-                cell_nb[p] = cell_nb[end - 1];
-                cell_fx[p] = cell_fx[end - 1];
-            }
-            ctx->nent = std::max(ctx->nent, nf + nr);
-            nrmax = std::max(nrmax, nr);
-            foff.push_back(foff.back() + nf);
-            roff.push_back(roff.back() + nr);
-        }
-        for (size_t r = 0; r < rec.size(); ++r) {
-            const uint32_t w = nbr[rec_side[r]], idx = w & NBR_INDEX_MASK;
-            if (w & NBR_BOUNDARY) brec[idx] = (uint32_t)r;
-            rec[r] |= (w & NBR_BOUNDARY) ? w & (NBR_BOUNDARY | NBR_INDEX_MASK) : side_rec[4 * idx + ((w >> 29) & 3u)];
-        }
-        hal.push_back(0);  // (read, not used, by a block without records)
-        rec.push_back(0);
-        for (size_t g = 0; g + 1 < grp_off.size(); ++g)
-            ctx->nstride = std::max(ctx->nstride, grp_off[g + 1] - grp_off[g]);
-    }
-    ctx->rec_at = (5 * (size_t)foff.back() + 63) / 64 * 64;
-    ctx->face_lds = 8 * std::max<uint32_t>(12 * ctx->nstride + 5 * (BLOCK + nrmax), 26 * BLOCK);
-    const bool faces = ctx->face_lds <= FACE_LDS;
+    for (size_t g = 0; g + 1 < grp_off.size(); ++g)
+        ctx->nstride = std::max(ctx->nstride, grp_off[g + 1] - grp_off[g]);
     ctx->Ncell = (uint32_t)cell0;
     ctx->nbf = (uint32_t)bface.size();
 
@@ -1199,24 +1190,6 @@ int create(int32_t n, const nf_mesh_desc *descs, const nf_params *prms, nf_ctx *
     if ((rc = dalloc(ctx, &ctx->gy, gy.size()))) return rc;
     if ((rc = dalloc(ctx, &ctx->gz, gz.size()))) return rc;
     if ((rc = dalloc(ctx, &ctx->cell_ln, cell_ln.size()))) return rc;
-    if (faces) {
-        if ((rc = dalloc(ctx, &ctx->hal, hal.size()))) return rc;
-        if ((rc = dalloc(ctx, &ctx->cell_nb, cell_nb.size()))) return rc;
-        if ((rc = dalloc(ctx, &ctx->foff, foff.size()))) return rc;
-        if ((rc = dalloc(ctx, &ctx->roff, roff.size()))) return rc;
-        if ((rc = dalloc(ctx, &ctx->rec, rec.size()))) return rc;
-        if ((rc = dalloc(ctx, &ctx->brec, brec.size()))) return rc;
-        if ((rc = dalloc(ctx, &ctx->cell_fx, cell_fx.size()))) return rc;
-        if ((rc = dalloc(ctx, &ctx->rS, 3 * ((rec.size() + 63) / 64 * 64)))) return rc;
-        if ((rc = dalloc(ctx, &ctx->vol, NC))) return rc;
-        HIPC(hipMemcpy(ctx->foff, foff.data(), foff.size() * 4, hipMemcpyHostToDevice));
-        HIPC(hipMemcpy(ctx->roff, roff.data(), roff.size() * 4, hipMemcpyHostToDevice));
-        HIPC(hipMemcpy(ctx->rec, rec.data(), rec.size() * 4, hipMemcpyHostToDevice));
-        if (ctx->nbf) HIPC(hipMemcpy(ctx->brec, brec.data(), brec.size() * 4, hipMemcpyHostToDevice));
-        HIPC(hipMemcpy(ctx->cell_fx, cell_fx.data(), cell_fx.size() * sizeof(uint2), hipMemcpyHostToDevice));
-        HIPC(hipMemcpy(ctx->hal, hal.data(), hal.size() * 4, hipMemcpyHostToDevice));
-        HIPC(hipMemcpy(ctx->cell_nb, cell_nb.data(), cell_nb.size() * sizeof(uint2), hipMemcpyHostToDevice));
-    }
     if ((rc = dalloc(ctx, &ctx->blk_inst, blk_inst.size()))) return rc;
     if ((rc = dalloc(ctx, &ctx->inst_end, inst_end.size()))) return rc;
     if ((rc = dalloc(ctx, &ctx->st, (size_t)n))) return rc;
@@ -1261,11 +1234,7 @@ int create(int32_t n, const nf_mesh_desc *descs, const nf_params *prms, nf_ctx *
     HIPC(hipMemcpy(ctx->cell_ln, cell_ln.data(), cell_ln.size() * sizeof(uint2), hipMemcpyHostToDevice));
     HIPC(hipMemcpy(ctx->blk_inst, blk_inst.data(), blk_inst.size() * 4, hipMemcpyHostToDevice));
     HIPC(hipMemcpy(ctx->inst_end, inst_end.data(), inst_end.size() * 4, hipMemcpyHostToDevice));
-    if (faces) {
-        hipLaunchKernelGGL(k_rec_geo, dim3(ctx->Ncell / BLOCK), dim3(BLOCK), 0, ctx->stream, devmesh(ctx), ctx->rS, ctx->vol);
-        HIPC(hipGetLastError());
-        HIPC(hipStreamSynchronize(ctx->stream));
-    }
+    if (!ctx->mixed && (rc = build_faces(ctx))) return rc;
     if (ctx->nbf) {
         HIPC(hipMemcpy(ctx->bface, bface.data(), bface.size() * 4, hipMemcpyHostToDevice));
         HIPC(hipMemcpy(ctx->bbc, bbc.data(), bbc.size(), hipMemcpyHostToDevice));
@@ -1800,6 +1769,7 @@ int nf_set_precision(nf_ctx *ctx, int32_t precision) {
         if ((rc = dalloc(ctx, &ctx->FV, 20 * NC + 512))) return rc;
         if ((rc = dalloc(ctx, &ctx->Gc, 5 * ((size_t)ctx->nbf + TILE - 1) / TILE * TILE))) return rc;
         if ((rc = dalloc(ctx, &ctx->Gf, 5 * ((size_t)ctx->nbf + TILE - 1) / TILE * TILE))) return rc;
+        if ((rc = build_faces(ctx))) return rc;
     }
     HIPC(hipStreamSynchronize(ctx->stream));
     ctx->mixed = mixed;
