@@ -44,6 +44,7 @@ struct RedArgs {
     int cap;
     double drop;
     double *out;   // residuals go to out[instance] instead
+    InstState *host;  // the final states also go here (pinned host memory), or null
 };
 
 template <bool MIN>
@@ -105,7 +106,10 @@ template <bool ONE>
 __global__ __launch_bounds__(BLOCK) void k_finish(RedArgs a) {
     __shared__ double sh[2][BLOCK / 64];
     const uint32_t i = blockIdx.x;
-    if (!a.out && a.st[i].stop) return;
+    if (!a.out && a.st[i].stop) {
+        if (a.host && threadIdx.x == 0) a.host[i] = a.st[i];
+        return;
+    }
     const uint32_t b0 = ONE ? a.first[a.c0[i]] : a.c0[i], nb = ONE ? a.n[a.c0[i]] : a.nc[i];
     double s = 0.0, v = DBL_MAX;
     if (a.res_part) s = red_blocks<false>(ONE ? a.res_part : a.red_res, b0, nb, sh[0]);
@@ -113,6 +117,7 @@ __global__ __launch_bounds__(BLOCK) void k_finish(RedArgs a) {
     if (threadIdx.x == 0) {
         if (a.res_part) finish_res(a, i, s);
         if (a.dt_part) finish_dt(a, i, v);
+        if (a.host) a.host[i] = a.st[i];
     }
 }
 
@@ -130,20 +135,17 @@ __global__ __launch_bounds__(BLOCK) void k_reduce(RedArgs a) {
 
 // op 0: clear the run flags of every instance (err, stop, converged, error
 // counters); op 2: the same, but a converged instance stays converged and
-// stopped; op 1: set dt of instance `which`
+// stopped; op 1: as 0, and set dt of instance `which`
 __global__ void k_flags(InstState *st, int n, int op, int which, double dt) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    if (op == 0 || op == 2) {
-        const int keep = op == 2 && st[i].converged;
-        st[i].err = 0;
-        st[i].stop = keep;
-        st[i].converged = keep;
-        st[i].bad_flux = 0;
-        st[i].bad_state = 0;
-    } else if (i == which) {
-        st[i].dt = dt;
-    }
+    const int keep = op == 2 && st[i].converged;
+    st[i].err = 0;
+    st[i].stop = keep;
+    st[i].converged = keep;
+    st[i].bad_flux = 0;
+    st[i].bad_state = 0;
+    if (op == 1 && i == which) st[i].dt = dt;
 }
 
 // fresh run state of instance i (nstep = 0, time = 0)
@@ -311,6 +313,8 @@ struct nf_ctx {
     uint32_t *blk_inst = nullptr;
     uint32_t *inst_end = nullptr;
     InstState *st = nullptr;
+    InstState *host_st = nullptr;  // single mesh: its state after the last host step or time step (pinned)
+    bool host_st_valid = false;    // nothing has changed st since
     double *Ua = nullptr, *Ub = nullptr, *V = nullptr, *FV = nullptr;
     float *V32 = nullptr, *FV32 = nullptr;
     uint32_t nbf = 0;
@@ -611,6 +615,7 @@ int run_sweepA(nf_ctx *ctx, bool dt, bool aux, bool dtc = false, const double *U
 int run_sweepB(nf_ctx *ctx, int kind, const double *U, double *Uout, bool res, bool aux) {
     int rc;
     const bool fuse = fused_ghosts(ctx);
+    ctx->host_st_valid = false;  // (its error counters)
     if (!fuse && (rc = run_ghost_face(ctx))) return rc;
     const DevMesh m = devmesh(ctx);
     const double *dtc = ctx->prm.local_time_step ? ctx->dt_cell : nullptr;
@@ -656,10 +661,10 @@ int run_sweepB(nf_ctx *ctx, int kind, const double *U, double *Uout, bool res, b
 
 // reductions of the last sweeps' partials: res (into the histories, or out)
 // and dt (advance: at the end of a step)
-int reduce(nf_ctx *ctx, bool res, double drop, double *out, bool dt, int advance) {
+int reduce(nf_ctx *ctx, bool res, double drop, double *out, bool dt, int advance, InstState *host = nullptr) {
     const RedTable &r = red(ctx);
     const RedArgs a{dt ? ctx->dt_part : nullptr, res ? ctx->res_part : nullptr, r.first, r.n, r.inst_c0, r.inst_nc,
-                    ctx->red_dt, ctx->red_res, ctx->st, advance, ctx->hist, ctx->hist_cap, drop, out};
+                    ctx->red_dt, ctx->red_res, ctx->st, advance, ctx->hist, ctx->hist_cap, drop, out, host};
     if (r.nchunk == ctx->n_inst) return LAUNCH("reduce", k_finish<true>, dim3(ctx->n_inst), dim3(BLOCK), a);
     int rc;
     if ((rc = LAUNCH("reduce_chunks", k_reduce, dim3(r.nchunk), dim3(BLOCK), a))) return rc;
@@ -672,8 +677,9 @@ int reduce(nf_ctx *ctx, bool res, double drop, double *out, bool dt, int advance
 // the reference's next calc_timestep sees (src/Solver.cpp:248);
 // k_finish installs that dt for the following step.  U^n (= U_old after
 // the first step) stays in Ua; stages write Ub, the last stage writes Ua.
-int enqueue_step(nf_ctx *ctx, double drop) {
+int enqueue_step(nf_ctx *ctx, double drop, InstState *host = nullptr) {
     int rc;
+    ctx->host_st_valid = false;
     const bool rk3 = ctx->prm.time_scheme == NF_TVD_RK3;
     const bool lts = ctx->prm.local_time_step;
     // each stage's sweep A evaluates the primvars of its input state
@@ -690,27 +696,42 @@ int enqueue_step(nf_ctx *ctx, double drop) {
     }
     if (!ctx->mixed)
         for (Inst &I : ctx->inst) I.v_stale = true;
-    return reduce(ctx, !early, drop, nullptr, true, 1);
+    return reduce(ctx, !early, drop, nullptr, true, 1, host);
 }
 
 // dt of the current primvars with a standalone sweep A
-int enqueue_timestep(nf_ctx *ctx) {
+int enqueue_timestep(nf_ctx *ctx, InstState *host = nullptr) {
     int rc;
+    ctx->host_st_valid = false;
     if ((rc = run_sweepA(ctx, true, false))) return rc;
-    return reduce(ctx, false, 0.0, nullptr, true, 0);
+    return reduce(ctx, false, 0.0, nullptr, true, 0, host);
 }
 
 int clear_flags(nf_ctx *ctx, bool keep_converged = false) {
+    ctx->host_st_valid = false;
     hipLaunchKernelGGL(k_flags, dim3((ctx->n_inst + 63) / 64), dim3(64), 0, ctx->stream, ctx->st, ctx->n_inst,
                        keep_converged ? 2 : 0, 0, 0.0);
     HIPC(hipGetLastError());
     return NF_OK;
 }
 
+// the run states; no wait and no copy if the last work on the stream was a
+// host step or a time step that left them in host_st
 int read_states(nf_ctx *ctx, std::vector<InstState> &h) {
     h.resize(ctx->n_inst);
+    if (ctx->host_st_valid) {
+        h[0] = *ctx->host_st;
+        return NF_OK;
+    }
     HIPC(hipStreamSynchronize(ctx->stream));
     HIPC(hipMemcpy(h.data(), ctx->st, h.size() * sizeof(InstState), hipMemcpyDeviceToHost));
+    return NF_OK;
+}
+
+// after work that leaves the state in host_st
+int wait_host_st(nf_ctx *ctx) {
+    HIPC(hipStreamSynchronize(ctx->stream));
+    ctx->host_st_valid = ctx->host_st != nullptr;
     return NF_OK;
 }
 
@@ -816,6 +837,7 @@ int after_state_set(nf_ctx *ctx, int i, bool uold_zero) {
                            ctx->V + (size_t)5 * I.cell0, I.Npad);
         HIPC(hipGetLastError());
     }
+    ctx->host_st_valid = false;
     hipLaunchKernelGGL(k_reset_inst, dim3(1), dim3(64), 0, ctx->stream, ctx->st, i, (int)uold_zero, I.rref);
     HIPC(hipGetLastError());
     HIPC(hipStreamSynchronize(ctx->stream));
@@ -1193,6 +1215,7 @@ int create(int32_t n, const nf_mesh_desc *descs, const nf_params *prms, nf_ctx *
     if ((rc = dalloc(ctx, &ctx->blk_inst, blk_inst.size()))) return rc;
     if ((rc = dalloc(ctx, &ctx->inst_end, inst_end.size()))) return rc;
     if ((rc = dalloc(ctx, &ctx->st, (size_t)n))) return rc;
+    if (n == 1) HIPC(hipHostMalloc((void **)&ctx->host_st, sizeof(InstState), hipHostMallocDefault));
     if ((rc = dalloc(ctx, &ctx->Ua, 5 * NC))) return rc;
     if ((rc = dalloc(ctx, &ctx->Ub, 5 * NC))) return rc;
     if (ctx->mixed) {
@@ -1285,15 +1308,23 @@ bool valid_inst(const nf_ctx *ctx, int32_t i) {
     return ctx && i >= 0 && i < ctx->n_inst;
 }
 
-// one step of a single-instance context with the dt held on the device
-int step_device_dt(nf_ctx *ctx) {
+// one step of a single-instance context with the dt held on the device, or
+// *dt.  One wait per step: its last kernel leaves the run state in host
+// memory, from which the step's errors, the next calc_timestep and the next
+// step's history are read (with a wait and a copy for each of them and two
+// launches for flags and dt, calc_timestep and step of 750 cells took 128 us, now
+// 75).
+int step_device_dt(nf_ctx *ctx, const double *dt = nullptr) {
     int rc;
-    if ((rc = clear_flags(ctx))) return rc;
     std::vector<InstState> h;
     if ((rc = read_states(ctx, h))) return rc;
     if ((rc = ensure_hist(ctx, h[0].nstep + 2))) return rc;
-    if ((rc = enqueue_step(ctx, -1.0))) return rc;
+    ctx->host_st_valid = false;
+    hipLaunchKernelGGL(k_flags, dim3(1), dim3(64), 0, ctx->stream, ctx->st, 1, dt ? 1 : 0, 0, dt ? *dt : 0.0);
+    HIPC(hipGetLastError());
+    if ((rc = enqueue_step(ctx, -1.0, ctx->host_st))) return rc;
     if (ctx->timing && (rc = flush_timing(ctx))) return rc;
+    if ((rc = wait_host_st(ctx))) return rc;
     ctx->inst[0].dt_valid = true;
     ctx->aux_valid = false;
     return check_errors(ctx);
@@ -1468,6 +1499,7 @@ int restore(nf_ctx *ctx, const Snapshot &s) {
     HIPC(hipMemcpy(ctx->Ua, s.U.data(), n5 * sizeof(double), hipMemcpyHostToDevice));
     if (ctx->mixed) HIPC(hipMemcpy(ctx->V32, s.V32.data(), n5 * sizeof(float), hipMemcpyHostToDevice));
     else HIPC(hipMemcpy(ctx->V, s.V.data(), n5 * sizeof(double), hipMemcpyHostToDevice));
+    ctx->host_st_valid = false;
     HIPC(hipMemcpy(ctx->st, s.st.data(), s.st.size() * sizeof(InstState), hipMemcpyHostToDevice));
     for (size_t i = 0; i < ctx->inst.size(); ++i) {
         ctx->inst[i].dt_valid = s.dt_valid[i];
@@ -1495,6 +1527,7 @@ int nf_destroy(nf_ctx *ctx) {
     nf::poly_destroy(ctx->poly);
     if (ctx->graph) (void)hipGraphExecDestroy(ctx->graph);
     for (void *p : ctx->owned) (void)hipFree(p);
+    if (ctx->host_st) (void)hipHostFree(ctx->host_st);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
     return NF_OK;
@@ -1551,7 +1584,8 @@ int nf_calc_timestep(nf_ctx *ctx, double *dt_out) {
     int rc;
     if (!ctx->inst[0].dt_valid) {
         if ((rc = clear_flags(ctx))) return rc;
-        if ((rc = enqueue_timestep(ctx))) return rc;
+        if ((rc = enqueue_timestep(ctx, ctx->host_st))) return rc;
+        if ((rc = wait_host_st(ctx))) return rc;
         ctx->inst[0].dt_valid = true;
     }
     std::vector<InstState> h;
@@ -1569,9 +1603,7 @@ int nf_calc_timestep(nf_ctx *ctx, double *dt_out) {
 int nf_step(nf_ctx *ctx, double dt) {
     if (ctx && ctx->poly) return nf::poly_step(ctx->poly, dt, ctx->err);
     if (!single(ctx)) return NF_E_ARG;
-    hipLaunchKernelGGL(k_flags, dim3(1), dim3(64), 0, ctx->stream, ctx->st, 1, 1, 0, dt);
-    HIPC(hipGetLastError());
-    return step_device_dt(ctx);
+    return step_device_dt(ctx, &dt);
 }
 
 int nf_run(nf_ctx *ctx, const nf_run_opts *o, nf_run_stats *st) {
@@ -1710,6 +1742,7 @@ int nf_inst_set_residual_ref(nf_ctx *ctx, int32_t i, double ref) {
     int rc;
     if ((rc = read_states(ctx, h))) return rc;
     h[i].rref = ctx->inst[i].rref;
+    ctx->host_st_valid = false;
     HIPC(hipMemcpy(ctx->st + i, &h[i], sizeof(InstState), hipMemcpyHostToDevice));
     return NF_OK;
 }
