@@ -513,16 +513,16 @@ int build_faces(nf_ctx *ctx) {
     if (order_of(ctx) == 0) return NF_OK;
     int rc;
     const uint32_t nblk = ctx->Ncell / BLOCK;
-    std::vector<uint32_t> foff(nblk + 1), roff(nblk + 1);
+    std::vector<uint32_t> off(2 * (nblk + 1));  // foff, roff
+    uint32_t *foff = off.data(), *roff = foff + nblk + 1;
     FaceTables o{};
     o.side_rec = reinterpret_cast<uint32_t *>(ctx->FV);
-    if ((rc = dalloc(ctx, &o.foff, nblk + 1))) return rc;
-    if ((rc = dalloc(ctx, &o.roff, nblk + 1))) return rc;
+    if ((rc = dalloc(ctx, &o.foff, off.size()))) return rc;
+    o.roff = o.foff + nblk + 1;
     hipLaunchKernelGGL(k_block_faces<true>, dim3(nblk), dim3(BLOCK), 0, ctx->stream, devmesh(ctx), o);
     HIPC(hipGetLastError());
     HIPC(hipStreamSynchronize(ctx->stream));
-    HIPC(hipMemcpy(foff.data(), o.foff, foff.size() * 4, hipMemcpyDeviceToHost));
-    HIPC(hipMemcpy(roff.data(), o.roff, roff.size() * 4, hipMemcpyDeviceToHost));
+    HIPC(hipMemcpy(off.data(), o.foff, off.size() * 4, hipMemcpyDeviceToHost));
     foff[0] = roff[0] = 0;
     uint32_t nrmax = 0;
     for (uint32_t b = 0; b < nblk; ++b) {
@@ -535,15 +535,17 @@ int build_faces(nf_ctx *ctx) {
     if (ctx->face_lds > FACE_LDS) return NF_OK;
     const size_t nr = roff[nblk];
     ctx->rec_at = (5 * (size_t)foff[nblk] + 63) / 64 * 64;
-    if ((rc = dalloc(ctx, &o.hal, nr + 1))) return rc;
-    if ((rc = dalloc(ctx, &o.rec, nr + 1))) return rc;
-    if ((rc = dalloc(ctx, &o.brec, ctx->nbf))) return rc;
-    if ((rc = dalloc(ctx, &o.cell_nb, ctx->Ncell))) return rc;
-    if ((rc = dalloc(ctx, &o.cell_fx, ctx->Ncell))) return rc;
-    if ((rc = dalloc(ctx, &ctx->rS, 3 * ((nr + 63) / 64 * 64)))) return rc;
-    if ((rc = dalloc(ctx, &ctx->vol, ctx->Ncell))) return rc;
-    HIPC(hipMemcpy(o.foff, foff.data(), foff.size() * 4, hipMemcpyHostToDevice));
-    HIPC(hipMemcpy(o.roff, roff.data(), roff.size() * 4, hipMemcpyHostToDevice));
+    const size_t nrp = (nr + 64) / 64 * 64, nbp = (ctx->nbf + 63) / 64 * 64, NC = ctx->Ncell;
+    uint32_t *tab = nullptr;  // one allocation for all
+    if ((rc = dalloc(ctx, &tab, 6 * nrp + 6 * NC + 2 * nrp + nbp))) return rc;
+    ctx->rS = reinterpret_cast<double *>(tab);
+    ctx->vol = ctx->rS + 3 * nrp;
+    o.cell_nb = reinterpret_cast<uint2 *>(ctx->vol + NC);
+    o.cell_fx = o.cell_nb + NC;
+    o.hal = reinterpret_cast<uint32_t *>(o.cell_fx + NC);
+    o.rec = o.hal + nrp;
+    o.brec = o.rec + nrp;
+    HIPC(hipMemcpy(o.foff, off.data(), off.size() * 4, hipMemcpyHostToDevice));
     hipLaunchKernelGGL(k_block_faces<false>, dim3(nblk), dim3(BLOCK), 0, ctx->stream, devmesh(ctx), o);
     hipLaunchKernelGGL(k_link_records, dim3(nblk), dim3(BLOCK), 0, ctx->stream, devmesh(ctx), o);
     ctx->foff = o.foff;
@@ -725,6 +727,13 @@ int read_states(nf_ctx *ctx, std::vector<InstState> &h) {
     }
     HIPC(hipStreamSynchronize(ctx->stream));
     HIPC(hipMemcpy(h.data(), ctx->st, h.size() * sizeof(InstState), hipMemcpyDeviceToHost));
+    return NF_OK;
+}
+
+// (made by the first host step: pinned memory costs as much to make and free
+// as a third of a small context)
+int ensure_host_st(nf_ctx *ctx) {
+    if (!ctx->host_st) HIPC(hipHostMalloc((void **)&ctx->host_st, sizeof(InstState), hipHostMallocDefault));
     return NF_OK;
 }
 
@@ -1215,7 +1224,6 @@ int create(int32_t n, const nf_mesh_desc *descs, const nf_params *prms, nf_ctx *
     if ((rc = dalloc(ctx, &ctx->blk_inst, blk_inst.size()))) return rc;
     if ((rc = dalloc(ctx, &ctx->inst_end, inst_end.size()))) return rc;
     if ((rc = dalloc(ctx, &ctx->st, (size_t)n))) return rc;
-    if (n == 1) HIPC(hipHostMalloc((void **)&ctx->host_st, sizeof(InstState), hipHostMallocDefault));
     if ((rc = dalloc(ctx, &ctx->Ua, 5 * NC))) return rc;
     if ((rc = dalloc(ctx, &ctx->Ub, 5 * NC))) return rc;
     if (ctx->mixed) {
@@ -1318,7 +1326,7 @@ int step_device_dt(nf_ctx *ctx, const double *dt = nullptr) {
     int rc;
     std::vector<InstState> h;
     if ((rc = read_states(ctx, h))) return rc;
-    if ((rc = ensure_hist(ctx, h[0].nstep + 2))) return rc;
+    if ((rc = ensure_hist(ctx, h[0].nstep + 2)) || (rc = ensure_host_st(ctx))) return rc;
     ctx->host_st_valid = false;
     hipLaunchKernelGGL(k_flags, dim3(1), dim3(64), 0, ctx->stream, ctx->st, 1, dt ? 1 : 0, 0, dt ? *dt : 0.0);
     HIPC(hipGetLastError());
@@ -1699,7 +1707,7 @@ int nf_get_field(nf_ctx *ctx, int32_t which, double *out) {
         if (!ctx->aux_valid) return fail(ctx, NF_E_ARG, "call nf_eval_flux_balance first");
         // (the sweeps stored them in reference order)
         HIPC(ctx->pipe.down(out, which == NF_FIELD_LIMITER ? ctx->psi_aux : (which == NF_FIELD_GRADIENT ? ctx->grad_aux : ctx->R_aux),
-                            (which == NF_FIELD_GRADIENT ? 15 : 5) * (size_t)ctx->inst[0].N * sizeof(double), ctx->stream));
+                            (which == NF_FIELD_GRADIENT ? 15 : 5) * (size_t)ctx->inst[0].N * sizeof(double), ctx->stream, true));
         return NF_OK;
     default:
         return fail(ctx, NF_E_ARG, "unknown field");

@@ -30,6 +30,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <initializer_list>
 #include <map>
 #include <memory>
 #include <new>
@@ -523,9 +524,16 @@ __global__ __launch_bounds__(PB) void k_poly_aos_out(const double *soa, const ui
     const size_t r = (size_t)cols * perm[d];
     for (int k = 0; k < cols; ++k) aos[r + k] = soa[k * (size_t)N + d];
 }
-__global__ __launch_bounds__(PB) void k_poly_fill(double *p, double v, size_t n) {
-    const size_t q = (size_t)blockIdx.x * PB + threadIdx.x;
-    if (q < n) p[q] = v;
+struct Five {
+    double v[5];
+};
+__global__ __launch_bounds__(PB) void k_poly_fill(double *U, Five u, double *X, Five x, size_t NT, uint32_t n) {
+    const uint32_t q = blockIdx.x * PB + threadIdx.x;
+    if (q >= n) return;
+    for (int k = 0; k < 5; ++k) {
+        U[k * (size_t)n + q] = u.v[k];
+        X[k * NT + q] = x.v[k];
+    }
 }
 }  // namespace
 
@@ -587,6 +595,25 @@ namespace {
 template <typename T> int alloc(PolyPath *P, T **p, size_t n, std::string &err) {
     PHIP(hipMalloc((void **)p, std::max<size_t>(n, 1) * sizeof(T)));
     P->owned.push_back(*p);
+    return NF_OK;
+}
+// several arrays in one allocation (a context of 2k cells has 28 arrays, and
+// as many calls were a tenth of its creation)
+struct Slot {
+    void **p;
+    size_t bytes;
+    template <typename T> Slot(T **q, size_t n) : p((void **)q), bytes((std::max<size_t>(n, 1) * sizeof(T) + 255) & ~(size_t)255) {}
+};
+int alloc_all(PolyPath *P, std::initializer_list<Slot> slots, std::string &err) {
+    size_t n = 0;
+    for (const Slot &q : slots) n += q.bytes;
+    char *base = nullptr;
+    int rc;
+    if ((rc = alloc(P, &base, n, err))) return rc;
+    for (const Slot &q : slots) {
+        *q.p = base;
+        base += q.bytes;
+    }
     return NF_OK;
 }
 template <typename T> int upload(T *dst, const std::vector<T> &src, std::string &err) {
@@ -755,7 +782,17 @@ int stages(PolyPath *P, bool on_device, double dt, std::string &err) {
     return NF_OK;
 }
 
+// the pinned results of begin and step_end, made by the first of them: they cost
+// as much to make and free as a quarter of a small context
+int ensure_host(PolyPath *P, std::string &err) {
+    if (!P->run.host)
+        PHIP(hipHostMalloc(reinterpret_cast<void **>(&P->run.host), 8 * sizeof(double), hipHostMallocDefault));
+    return NF_OK;
+}
+
 int step_end(PolyPath *P, bool on_device, std::string &err) {
+    int rc;
+    if ((rc = ensure_host(P, err))) return rc;
     RunDev r = P->run;
     r.flags = on_device ? P->flags : nullptr;
     hipLaunchKernelGGL(k_poly_end, dim3(1), dim3(PB), 0, P->st, r, (const double *)P->res_part,
@@ -766,6 +803,8 @@ int step_end(PolyPath *P, bool on_device, std::string &err) {
 
 // dt of the first step where it is not in place, and (on_device) a run's start
 int begin(PolyPath *P, bool on_device, double drop, double ref, std::string &err) {
+    int rc;
+    if ((rc = ensure_host(P, err))) return rc;
     RunDev r = P->run;
     r.flags = on_device ? P->flags : nullptr;
     if (!P->dt_valid) {
@@ -881,11 +920,10 @@ int poly_create(const PrimalMesh &pm, const FVGrid &g, const nf_params &p, hipSt
     const size_t plane = std::max(N, G);
     const uint32_t nblk = (N + PB - 1) / PB;
     int rc;
-    if ((rc = alloc(P, &dw, w.size(), err)) || (rc = alloc(P, &dns, ns.size(), err)) ||
-        (rc = alloc(P, &dgeo, geo.size(), err)) || (rc = alloc(P, &dvol, N, err)) ||
-        (rc = alloc(P, &ddS, 3 * (size_t)N, err)) || (rc = alloc(P, &dbi, G, err)) || (rc = alloc(P, &dbj, G, err)) ||
-        (rc = alloc(P, &dbS, 3 * (size_t)G, err)) || (rc = alloc(P, &dbbc, G, err)) ||
-        (rc = alloc(P, &dbslot, G, err)) || (rc = alloc(P, &P->boff, boff.size(), err)))
+    if ((rc = alloc_all(P, {{&dw, w.size()}, {&dns, ns.size()}, {&dgeo, geo.size()}, {&dvol, N},
+                            {&ddS, 3 * (size_t)N}, {&dbi, G}, {&dbj, G}, {&dbS, 3 * (size_t)G}, {&dbbc, G},
+                            {&dbslot, G}, {&P->boff, boff.size()}},
+                        err)))
         return rc;
     if ((rc = upload(dw, w, err)) || (rc = upload(dns, ns, err)) || (rc = upload(dgeo, geo, err)) ||
         (rc = upload(dvol, vol, err)) || (rc = upload(ddS, dS, err)) || (rc = upload(dbi, bi, err)) ||
@@ -894,18 +932,14 @@ int poly_create(const PrimalMesh &pm, const FVGrid &g, const nf_params &p, hipSt
         return rc;
     P->m = {N, NT, G, plane, dw, dns, dgeo, dvol, ddS, dbi, dbj, dbslot, dbbc, dbS,
             P->boff, make_farfield<double>(p.primvars_inf), nullptr, 0};
-    if ((rc = alloc(P, &P->Ua, 5 * (size_t)N, err)) || (rc = alloc(P, &P->Ub, 5 * (size_t)N, err)) ||
-        (rc = alloc(P, &P->X, 5 * (size_t)NT, err)) || (rc = alloc(P, &P->Y, 5 * (size_t)NT, err)) ||
-        (rc = alloc(P, &P->Z, 5 * (size_t)NT, err)) || (rc = alloc(P, &P->FV, 35 * plane, err)) ||
-        (rc = alloc(P, &P->grad, 15 * (size_t)N, err)) || (rc = alloc(P, &P->psi, 5 * (size_t)N, err)) ||
-        (rc = alloc(P, &P->R, 5 * (size_t)N, err)) || (rc = alloc(P, &P->dt_part, nblk, err)) ||
-        (rc = alloc(P, &P->res_part, nblk, err)) || (rc = alloc(P, &P->dtc, N, err)) ||
-        (rc = alloc(P, &P->flags, 4, err)) || (rc = alloc(P, &P->run.dtdev, 1, err)) ||
-        (rc = alloc(P, &P->run.runp, 2, err)) || (rc = alloc(P, &P->run.zero_old, 1, err)) ||
-        (rc = alloc(P, &P->run.bad, 3, err)))
+    if ((rc = alloc_all(P, {{&P->Ua, 5 * (size_t)N}, {&P->Ub, 5 * (size_t)N}, {&P->X, 5 * (size_t)NT},
+                            {&P->Y, 5 * (size_t)NT}, {&P->Z, 5 * (size_t)NT}, {&P->FV, 35 * plane},
+                            {&P->grad, 15 * (size_t)N}, {&P->psi, 5 * (size_t)N}, {&P->R, 5 * (size_t)N},
+                            {&P->dt_part, nblk}, {&P->res_part, nblk}, {&P->dtc, N}, {&P->flags, 4},
+                            {&P->run.dtdev, 1}, {&P->run.runp, 2}, {&P->run.zero_old, 1}, {&P->run.bad, 3}},
+                        err)))
         return rc;
     PHIP(hipMemset(P->run.bad, 0, 3 * sizeof(int)));
-    PHIP(hipHostMalloc(reinterpret_cast<void **>(&P->run.host), 8 * sizeof(double), hipHostMallocDefault));
     if ((rc = poly_set_freestream(P, err))) return rc;
     *out = hold.release();
     return NF_OK;
@@ -927,13 +961,11 @@ static void reset_run(PolyPath *P) {
 int poly_set_freestream(PolyPath *P, std::string &err) {
     const uint32_t N = P->m.N;
     reset_run(P);
-    double U[5];
-    prim_to_cons(P->prm.primvars_inf, U);
-    for (int k = 0; k < 5; ++k) {
-        hipLaunchKernelGGL(k_poly_fill, grid(N), dim3(PB), 0, P->st, P->Ua + k * (size_t)N, U[k], (size_t)N);
-        hipLaunchKernelGGL(k_poly_fill, grid(N), dim3(PB), 0, P->st, P->X + k * (size_t)P->m.NT,
-                           P->prm.primvars_inf[k], (size_t)N);
-    }
+    Five U, V;
+    prim_to_cons(P->prm.primvars_inf, U.v);
+    std::copy(P->prm.primvars_inf, P->prm.primvars_inf + 5, V.v);
+    hipLaunchKernelGGL(k_poly_fill, grid(N), dim3(PB), 0, P->st, P->Ua, U, P->X, V, (size_t)P->m.NT, N);
+    PHIP(hipGetLastError());
     // (X is V_inf, which the first dt is taken from, and not prim(U) bit for bit)
     int rc;
     if ((rc = set_old_zero(P, P->prm.rk3_zero_old_first_step != 0, err))) return rc;
