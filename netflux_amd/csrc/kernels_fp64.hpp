@@ -721,7 +721,7 @@ __global__ __launch_bounds__(B) NF_SWEEP_ATTR void k_sweepA(DevMesh m, SweepAArg
 // / 415, 3.95M / 4.14M 1,929 / 1,904 -> 1,471 / 1,593.
 //
 // Sweep A is bound by its phases between barriers: the vector units are busy
-// 60 % of its time, memory moves 2.1 TB/s.  52 KB of LDS hold three blocks per
+// 60 % of its time, memory moves 2.9 TB/s (207 B per cell).  52 KB of LDS hold three blocks per
 // CU; the face values in two halves (33 KB, 128 registers, four blocks) cost
 // more in barriers than they gain: 382 -> 410 us at 998k cells.
 template <int ORDER, bool FROM_U, bool FUSE>
@@ -1162,9 +1162,9 @@ __global__ __launch_bounds__(B) NF_SWEEPB_ATTR void k_sweepB(DevMesh m, SweepBAr
     finish_cell<B, FUSE>(m, a, L, br, st, R, zero_old, Up, Uop, g.ivol, sh);
 }
 
-// The records' fluxes, then every cell's flux balance from LDS.  156 B per cell
-// move at 3.3 TB/s (998k cells: 48 us); bound by the latency of a block's
-// loads with four waves per SIMD.  Five waves spill: 382 -> 472 us per step.
+// The records' fluxes, then every cell's flux balance from LDS.  273 B per cell
+// move at 5.7 TB/s (998k cells: 48 us): bound by memory, with the vector units
+// busy 23 % of the time.  Five waves per SIMD spill: 382 -> 472 us per step.
 template <int FLUX, bool FUSE>
 __global__ __launch_bounds__(BLOCK) void k_sweepB_face(DevMesh m, SweepBArgs a) {
     constexpr int B = BLOCK;

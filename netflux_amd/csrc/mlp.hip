@@ -698,14 +698,18 @@ int nf_mlp_create(uint64_t seed, nf_mlp **out) {
     nf_mlp *mm = hold.get();
     HIPM(hipGetDevice(&mm->device));
     HIPM(hipStreamCreateWithFlags(&mm->stream, hipStreamNonBlocking));
-    HIPM(hipMalloc(&mm->p, NPARAM * sizeof(float)));
-    HIPM(hipMalloc(&mm->g, NPARAM * sizeof(float)));
-    HIPM(hipMalloc(&mm->m, NPARAM * sizeof(float)));
-    HIPM(hipMalloc(&mm->v, NPARAM * sizeof(float)));
-    HIPM(hipMalloc(&mm->pb, NPARAM * sizeof(__bf16)));
-    HIPM(hipMalloc(&mm->pt, NPT * sizeof(__bf16)));
+    // one allocation; the moments and pt, which start at zero, side by side
+    constexpr size_t ROW = (NPARAM * sizeof(float) + 255) & ~(size_t)255, TR = (NPT * sizeof(__bf16) + 255) & ~(size_t)255;
+    char *base = nullptr;
+    HIPM(hipMalloc(&base, 5 * ROW + TR + 27 * sizeof(float)));
+    mm->p = reinterpret_cast<float *>(base);  // (the one that is freed)
+    mm->g = reinterpret_cast<float *>(base + ROW);
+    mm->m = reinterpret_cast<float *>(base + 2 * ROW);
+    mm->v = reinterpret_cast<float *>(base + 3 * ROW);
+    mm->pt = reinterpret_cast<__bf16 *>(base + 4 * ROW);
+    mm->pb = reinterpret_cast<__bf16 *>(base + 4 * ROW + TR);
+    mm->norm = reinterpret_cast<float *>(base + 5 * ROW + TR);
     HIPM(hipMemset(mm->pt, 0, NPT * sizeof(__bf16)));
-    HIPM(hipMalloc(&mm->norm, 27 * sizeof(float)));
     // uniform(+-1/sqrt(fan_in)) weights and biases, a linear layer's default
     std::mt19937_64 rng(seed);
     std::vector<float> h(NPARAM);
@@ -730,8 +734,7 @@ int nf_mlp_destroy(nf_mlp *mm) {
     if (!mm) return NF_OK;
     if (mm->stream) (void)hipStreamSynchronize(mm->stream);
     for (void *q : mm->ws) (void)hipFree(q);
-    for (void *q : {(void *)mm->p, (void *)mm->g, (void *)mm->m, (void *)mm->v, (void *)mm->pb, (void *)mm->pt, (void *)mm->norm,
-                    (void *)mm->dx, (void *)mm->dy, (void *)mm->didx})
+    for (void *q : {(void *)mm->p, (void *)mm->dx, (void *)mm->dy, (void *)mm->didx})
         if (q) (void)hipFree(q);
     if (mm->stream) (void)hipStreamDestroy(mm->stream);
     delete mm;
@@ -751,8 +754,7 @@ int nf_mlp_set_params(nf_mlp *mm, const float *params) {
     if (!mm || !params) return NF_E_ARG;
     HIPM(hipStreamSynchronize(mm->stream));
     HIPM(hipMemcpy(mm->p, params, NPARAM * sizeof(float), hipMemcpyHostToDevice));
-    HIPM(hipMemset(mm->m, 0, NPARAM * sizeof(float)));
-    HIPM(hipMemset(mm->v, 0, NPARAM * sizeof(float)));
+    HIPM(hipMemset(mm->m, 0, (mm->v - mm->m + NPARAM) * sizeof(float)));  // both moments
     mm->adam_t = 0;
     hipLaunchKernelGGL(k_to_bf16, dim3((NPARAM + 255) / 256), dim3(256), 0, mm->stream, (const float *)mm->p, mm->pb,
                        mm->pt);
