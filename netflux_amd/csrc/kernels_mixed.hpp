@@ -239,7 +239,14 @@ __global__ __launch_bounds__(B) void k_sweepA_mx(DevMesh m, SweepAArgsMx a) {
     cell_geo(m, g);
     V3f S[4], r[4];
 #pragma unroll
-    for (int s = 0; s < 4; ++s) face_geo_mx(nv, g, (code >> (8 * s)) & 0xFFu, S[s], &r[s]);
+    for (int s = 0; s < 4; ++s) {
+        face_geo_mx(nv, g, (code >> (8 * s)) & 0xFFu, S[s], &r[s]);
+        // formed here: sunk to their uses they keep the nodes of all faces alive
+        // (150 registers and 3 waves per SIMD; 116 and 4 so: step of a channel of
+        // 202k / 1,054k / 4.14M cells 107.8 / 290.8 / 1,342 -> 105.4 / 282.0 /
+        // 1,288 us, farfield boxes 1 to 2 %, no change below 150k; the same bits)
+        asm volatile("" : "+v"(S[s].x), "+v"(S[s].y), "+v"(S[s].z), "+v"(r[s].x), "+v"(r[s].y), "+v"(r[s].z));
+    }
     const float ivol = (float)(1.0 / g.vol);
     __builtin_amdgcn_sched_barrier(0);
     if (ORDER != 0) {
