@@ -13,7 +13,8 @@
 // The pinned pieces (8 of 4 MB for each device) belong to a pool, since making
 // them takes longer (1.3 ms) than most copies: a copy borrows those it can
 // get, under a lock, and returns them when its last piece has left; a copy that
-// gets none is a plain one.  The pool is given back with its last user.
+// gets none is a plain one.  The pool is given back with its last user.  It
+// also has the small records that kernels leave their results in.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -29,7 +30,7 @@ namespace nf {
 
 class PinnedPool {
   public:
-    static constexpr size_t PIECE = 4u << 20;
+    static constexpr size_t PIECE = 4u << 20, RECORD = 128;
     struct Slot {
         char *mem = nullptr;
         hipEvent_t ev = nullptr;
@@ -53,6 +54,35 @@ class PinnedPool {
         }
         free_.clear();
         made_.clear();
+        for (char *p : page_) (void)hipHostFree(p);
+        page_.clear();
+        rec_.clear();
+    }
+    // a record of up to RECORD bytes, which kernels can store to on any device;
+    // null if there is no memory.  (Making and freeing pinned memory of its own
+    // cost a small context a quarter of its life.)
+    void *record() {
+        std::lock_guard<std::mutex> lk(mu_);
+        try {
+            if (rec_.empty()) {
+                constexpr size_t PAGE = 4096;
+                page_.reserve(page_.size() + 1);
+                rec_.reserve((page_.size() + 1) * (PAGE / RECORD));  // giving back cannot fail
+                char *p = nullptr;
+                if (hipHostMalloc(reinterpret_cast<void **>(&p), PAGE, hipHostMallocPortable) != hipSuccess) return nullptr;
+                page_.push_back(p);
+                for (size_t o = 0; o < PAGE; o += RECORD) rec_.push_back(p + o);
+            }
+        } catch (...) {
+            return nullptr;
+        }
+        char *r = rec_.back();
+        rec_.pop_back();
+        return r;
+    }
+    void give_record(void *r) {
+        std::lock_guard<std::mutex> lk(mu_);
+        rec_.push_back(static_cast<char *>(r));
     }
     // up to `want` slots of device dev, which is current
     std::vector<Slot> borrow(int want, int dev) {
@@ -89,6 +119,7 @@ class PinnedPool {
     static constexpr int SLOTS = 8;
     std::mutex mu_;
     std::vector<Slot> free_;
+    std::vector<char *> page_, rec_;  // pages of records, free records
     std::map<int, int> made_;
     int users_ = 0;
 };

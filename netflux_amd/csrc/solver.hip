@@ -730,11 +730,11 @@ int read_states(nf_ctx *ctx, std::vector<InstState> &h) {
     return NF_OK;
 }
 
-// (made by the first host step: pinned memory costs as much to make and free
-// as a third of a small context)
+// (taken by the first host step)
 int ensure_host_st(nf_ctx *ctx) {
-    if (!ctx->host_st) HIPC(hipHostMalloc((void **)&ctx->host_st, sizeof(InstState), hipHostMallocDefault));
-    return NF_OK;
+    static_assert(sizeof(InstState) <= nf::PinnedPool::RECORD, "");
+    if (!ctx->host_st) ctx->host_st = static_cast<InstState *>(nf::PinnedPool::get().record());
+    return ctx->host_st ? NF_OK : fail(ctx, NF_E_HIP, "no pinned host memory");
 }
 
 // after work that leaves the state in host_st
@@ -1535,7 +1535,7 @@ int nf_destroy(nf_ctx *ctx) {
     nf::poly_destroy(ctx->poly);
     if (ctx->graph) (void)hipGraphExecDestroy(ctx->graph);
     for (void *p : ctx->owned) (void)hipFree(p);
-    if (ctx->host_st) (void)hipHostFree(ctx->host_st);
+    if (ctx->host_st) nf::PinnedPool::get().give_record(ctx->host_st);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
     return NF_OK;

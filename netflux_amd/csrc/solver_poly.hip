@@ -576,7 +576,7 @@ struct PolyPath {
         if (st) (void)hipStreamSynchronize(st);
         if (graph) (void)hipGraphExecDestroy(graph);
         for (void *p : owned) (void)hipFree(p);
-        if (run.host) (void)hipHostFree(run.host);
+        if (run.host) PinnedPool::get().give_record(run.host);
     }
 };
 
@@ -780,12 +780,12 @@ int stages(PolyPath *P, bool on_device, double dt, std::string &err) {
     return NF_OK;
 }
 
-// the pinned results of begin and step_end, made by the first of them: they cost
-// as much to make and free as a quarter of a small context
+// the pinned results of begin and step_end, taken by the first of them
 int ensure_host(PolyPath *P, std::string &err) {
-    if (!P->run.host)
-        PHIP(hipHostMalloc(reinterpret_cast<void **>(&P->run.host), 8 * sizeof(double), hipHostMallocDefault));
-    return NF_OK;
+    if (!P->run.host) P->run.host = static_cast<double *>(PinnedPool::get().record());
+    if (P->run.host) return NF_OK;
+    err = "no pinned host memory";
+    return NF_E_HIP;
 }
 
 int step_end(PolyPath *P, bool on_device, std::string &err) {

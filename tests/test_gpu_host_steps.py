@@ -47,3 +47,31 @@ def test_state_seen_between_calls(kw):
     host(1)
     assert len(s.residuals()) == 1
     np.testing.assert_array_equal(s.residuals(), ref.residuals()[:1])
+
+
+def test_many_contexts_alive():
+    """More contexts than a page of pinned records holds, stepped in turn and
+    given back out of order; new ones take the freed records."""
+    print("[case] host steps of 40 contexts", flush=True)
+    mesh = nf.Mesh.box((3, 2, 2), patches=("SlipWall",) * 6)
+    hexes = nf.Mesh.hex_box(2, patches=("SlipWall",) * 6)
+    out = {}
+    for m in (mesh, hexes):
+        cfg = sod_config(rk3_zero_old_first_step=False)
+        U = pulse_state(m, mach=0.0)
+        live = [nf.EulerSolver(cfg, m) for _ in range(40)]
+        for s in live:
+            s.set_state(U, U)
+        for _ in range(2):
+            for s in live:
+                s.calc_timestep(cfg)
+                s.step(cfg)
+        del live[::2], s
+        again = nf.EulerSolver(cfg, m)
+        again.set_state(U, U)
+        for _ in range(2):
+            again.calc_timestep(cfg)
+            again.step(cfg)
+        for s in live:
+            np.testing.assert_array_equal(s.get_solver_data().get_solution(), again.get_solver_data().get_solution())
+            np.testing.assert_array_equal(s.residuals(), again.residuals())
