@@ -34,6 +34,7 @@
 
 #include <cstdint>
 
+#include "face_record.hpp"
 #include "fp64_math.hpp"
 #include "physics.hpp"
 
@@ -113,8 +114,7 @@ struct DevMesh {
     // two of its cells, numbers [foff[b], foff[b+1]), and records of its other
     // cell sides, [roff[b], roff[b+1]).  Per record: hal, the cell of the
     // face's other side (or bit 31 and boundary face); rec, that side's record
-    // (or bit 31 and boundary face), bit 30 set if the record's own side is
-    // the reference owner's; rS [tile][3][64], the face vector.  Per cell
+    // (face_record.hpp); rS [tile][3][64], the face vector.  Per cell
     // 4 x u16: cell_nb, where a slot's neighbour state is -- below BLOCK the
     // block's own cell, then the records' -- and bit 15 on a boundary slot;
     // cell_fx, the place of a slot's side among the block's 2 nf + nr (owner
@@ -979,8 +979,8 @@ __global__ __launch_bounds__(BLOCK) void k_link_records(DevMesh m, FaceTables o)
         if (!bnd && idx / BLOCK == b) continue;
         const uint32_t r = o.side_rec[4 * (size_t)p + q];
         if (bnd) o.brec[idx] = r;
-        o.rec[r] = ((code >> (8 * q + 7)) & 1u) << 30 |
-                   (bnd ? 0x80000000u | idx : o.side_rec[4 * (size_t)idx + ((w >> 29) & 3u)]);
+        o.rec[r] = rec_word(bnd, (code >> (8 * q + 7)) & 1u,
+                            bnd ? idx : o.side_rec[4 * (size_t)idx + ((w >> 29) & 3u)]);
     }
 }
 
@@ -1199,7 +1199,7 @@ __global__ __launch_bounds__(BLOCK) void k_sweepB_face(DevMesh m, SweepBArgs a) 
     }
     auto rec_flux = [&](uint32_t h, uint32_t w) {
         const uint32_t r = r0 + h;
-        const double *src = ((w & 0x80000000u) ? a.Gf : a.H) + tix(w & 0x1FFFFFFFu, 0);
+        const double *src = ((w & REC_BOUNDARY) ? a.Gf : a.H) + tix(rec_index(w), 0);
         const double *sp = m.rS + (size_t)(r >> 6) * 3 * TILE + (r & 63u);
         double Vo[5], Vn[5], UO[5], UN[5], G[5];
 #pragma unroll
@@ -1210,7 +1210,7 @@ __global__ __launch_bounds__(BLOCK) void k_sweepB_face(DevMesh m, SweepBArgs a) 
         const V3d S = {sp[0], sp[TILE], sp[2 * TILE]};
         prim_to_cons(Vo, UO);
         prim_to_cons(Vn, UN);
-        const bool own = w & 0x40000000u;
+        const bool own = w & REC_OWNER;
         if (FLUX == 1) {
             double UL[5], UR[5];
 #pragma unroll

@@ -533,7 +533,8 @@ int build_faces(nf_ctx *ctx) {
     }
     ctx->face_lds = 8 * std::max<uint32_t>(12 * ctx->nstride + 5 * (BLOCK + nrmax), 26 * BLOCK);
     if (ctx->face_lds > FACE_LDS) return NF_OK;
-    const size_t nr = roff[nblk];
+    const size_t nr = roff[nblk];  // (at most 4 x 2^29: the sums are in range)
+    if (nr > REC_MAX) return NF_OK;
     ctx->rec_at = (5 * (size_t)foff[nblk] + 63) / 64 * 64;
     const size_t nrp = (nr + 64) / 64 * 64, nbp = (ctx->nbf + 63) / 64 * 64, NC = ctx->Ncell;
     uint32_t *tab = nullptr;  // one allocation for all
