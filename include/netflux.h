@@ -312,9 +312,10 @@ int nf_mlp_predict(nf_mlp *m, const float *x, int64_t n, float *y);
  * DEVICE arrays x [n][6] -> y [n][5], at most 16384 samples per call (more:
  * NF_E_ARG), enqueued on `stream` (a hipStream_t; null: the network's own
  * stream) without synchronising and without allocating.  One kernel, whose
- * activations stay on the CU: calls share no buffer.  The device that was
- * current at nf_mlp_create must be current.  Same results as nf_mlp_predict,
- * bit for bit. */
+ * activations stay on the CU: calls share no buffer, and may overlap.  Where y
+ * lies over x (in place), x goes through a buffer of the network first, and
+ * such calls on one network must not overlap.  The device that was current at
+ * nf_mlp_create must be current.  Same results as nf_mlp_predict, bit for bit. */
 int nf_mlp_predict_noalloc(nf_mlp *m, const float *x, int64_t n, float *y, void *stream);
 /* mean squared error of the normalised outputs over one batch of n <= 2^20
  * samples and its gradient with respect to the FP32 parameters */

@@ -500,14 +500,22 @@ __global__ __launch_bounds__(256) void k_to_bf16(const float *p, __bf16 *pb, __b
     if (i < NPARAM) put_bf16(i, p[i], pb, pt);
 }
 
+__global__ __launch_bounds__(256) void k_copy(const float *x, float *y, int n) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n) y[i] = x[i];
+}
+
 }  // namespace
 
 // ---------------------------------------------------------------------------
+constexpr int64_t NOALLOC_MAX = 16384;  // samples per nf_mlp_predict_noalloc call
+
 struct nf_mlp {
     std::string err;
     hipStream_t stream = nullptr;
     float *p = nullptr, *g = nullptr, *m = nullptr, *v = nullptr;  // FP32 [NPARAM]
     __bf16 *pb = nullptr, *pt = nullptr;                           // BF16 copy, transposes (PT2..)
+    float *xcopy = nullptr;  // inputs of a predict_noalloc call whose outputs lie over them, [NOALLOC_MAX][IN]
     float *norm = nullptr;  // device: in_shift[6], in_scale[6], out_shift[5], out_scale[5], out_iscale[5]
     float hnorm[27] = {};
     bool norm_set = false;  // false: training sets it from the data
@@ -666,10 +674,6 @@ hipError_t predict_device(nf_mlp *m, const float *x, int64_t n, float *y, hipStr
 }  // namespace nf
 
 // ============================================================================
-namespace {
-constexpr int64_t NOALLOC_MAX = 16384;  // samples per nf_mlp_predict_noalloc call
-}
-
 extern "C" {
 
 int64_t nf_mlp_n_params(void) { return NPARAM; }
@@ -685,7 +689,16 @@ int nf_mlp_predict_noalloc(nf_mlp *mm, const float *x, int64_t n, float *y, void
     HIPM(hipGetDevice(&dev));
     if (dev != mm->device)
         return fail(mm, NF_E_ARG, "nf_mlp_predict_noalloc: the network's device must be current");
-    HIPM(infer(mm, x, 1, IN, y, 1, OUT, n, stream ? static_cast<hipStream_t>(stream) : mm->stream));
+    const hipStream_t s = stream ? static_cast<hipStream_t>(stream) : mm->stream;
+    // y over x: a block's outputs would replace inputs that another block has
+    // not read yet
+    const uintptr_t xa = reinterpret_cast<uintptr_t>(x), ya = reinterpret_cast<uintptr_t>(y);
+    if (xa < ya + OUT * n * sizeof(float) && ya < xa + IN * n * sizeof(float)) {
+        hipLaunchKernelGGL(k_copy, dim3((unsigned)((IN * n + 255) / 256)), dim3(256), 0, s, x, mm->xcopy, (int)(IN * n));
+        HIPM(hipGetLastError());
+        x = mm->xcopy;
+    }
+    HIPM(infer(mm, x, 1, IN, y, 1, OUT, n, s));
     return NF_OK;
 }
 
@@ -701,7 +714,7 @@ int nf_mlp_create(uint64_t seed, nf_mlp **out) {
     // one allocation; the moments and pt, which start at zero, side by side
     constexpr size_t ROW = (NPARAM * sizeof(float) + 255) & ~(size_t)255, TR = (NPT * sizeof(__bf16) + 255) & ~(size_t)255;
     char *base = nullptr;
-    HIPM(hipMalloc(&base, 5 * ROW + TR + 27 * sizeof(float)));
+    HIPM(hipMalloc(&base, 5 * ROW + TR + (32 + IN * NOALLOC_MAX) * sizeof(float)));
     mm->p = reinterpret_cast<float *>(base);  // (the one that is freed)
     mm->g = reinterpret_cast<float *>(base + ROW);
     mm->m = reinterpret_cast<float *>(base + 2 * ROW);
@@ -709,6 +722,7 @@ int nf_mlp_create(uint64_t seed, nf_mlp **out) {
     mm->pt = reinterpret_cast<__bf16 *>(base + 4 * ROW);
     mm->pb = reinterpret_cast<__bf16 *>(base + 4 * ROW + TR);
     mm->norm = reinterpret_cast<float *>(base + 5 * ROW + TR);
+    mm->xcopy = mm->norm + 32;
     HIPM(hipMemset(mm->pt, 0, NPT * sizeof(__bf16)));
     // uniform(+-1/sqrt(fan_in)) weights and biases, a linear layer's default
     std::mt19937_64 rng(seed);
