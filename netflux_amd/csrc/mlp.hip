@@ -543,11 +543,13 @@ int fail(nf_mlp *m, int code, const std::string &msg) {
     if (m) m->err = msg;
     return code;
 }
-#define HIPM(expr)                                                                       \
-    do {                                                                                 \
-        hipError_t e_ = (expr);                                                          \
-        if (e_ != hipSuccess)                                                            \
-            return fail(mm, NF_E_HIP, std::string(#expr) + ": " + hipGetErrorString(e_)); \
+#define HIPM(expr)                                                                          \
+    do {                                                                                    \
+        hipError_t e_ = (expr);                                                             \
+        if (e_ != hipSuccess) {                                                             \
+            (void)hipGetLastError(); /* reported here, not by the next call's launches */   \
+            return fail(mm, NF_E_HIP, std::string(#expr) + ": " + hipGetErrorString(e_));   \
+        }                                                                                   \
     } while (0)
 
 int ensure_ws(nf_mlp *mm, int n) {

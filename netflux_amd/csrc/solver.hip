@@ -363,8 +363,10 @@ int fail(nf_ctx *c, int code, const std::string &msg) {
 #define HIPC(expr)                                                                         \
     do {                                                                                   \
         hipError_t e_ = (expr);                                                            \
-        if (e_ != hipSuccess)                                                              \
+        if (e_ != hipSuccess) {                                                            \
+            (void)hipGetLastError(); /* reported here, not by the next call's launches */  \
             return fail(ctx, NF_E_HIP, std::string(#expr) + ": " + hipGetErrorString(e_)); \
+        }                                                                                  \
     } while (0)
 
 template <typename T>

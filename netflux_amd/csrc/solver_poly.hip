@@ -585,6 +585,7 @@ namespace {
     do {                                                                            \
         hipError_t e_ = (expr);                                                     \
         if (e_ != hipSuccess) {                                                     \
+            (void)hipGetLastError(); /* not reported again by the next call */      \
             err = std::string(#expr) + ": " + hipGetErrorString(e_);                \
             return NF_E_HIP;                                                        \
         }                                                                           \

@@ -1,0 +1,71 @@
+"""What the library's host code does when device memory runs out: the call
+reports it, and the next call that fits neither uses freed or missing arrays
+nor is refused.  On the CPU, over a HIP runtime without a device
+(fake_hip.cpp) whose allocations fail from a given size on; each case runs in
+a process of its own, since the library binds to one runtime."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+PRELUDE = """
+import ctypes as C, sys
+sys.path.insert(0, {root!r})
+hip = C.CDLL({fake!r}, mode=C.RTLD_GLOBAL)
+hip.fake_allocated.restype = C.c_size_t
+hip.fake_fail_above.argtypes = [C.c_size_t]
+ANY = 2**64 - 1
+import numpy as np
+import netflux_amd as nf
+from netflux_amd.mlp import Mlp
+
+def fails(call):
+    try:
+        call()
+    except RuntimeError as e:
+        assert "out of memory" in str(e), e
+        return True
+
+def allocates(call):
+    before = hip.fake_allocated()
+    call()
+    return hip.fake_allocated() - before
+"""
+
+
+@pytest.fixture(scope="module")
+def run(tmp_path_factory):
+    fake = tmp_path_factory.mktemp("fake_hip") / "fake_hip.so"
+    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-o", fake, os.path.join(HERE, "fake_hip.cpp")],
+                   check=True)
+
+    def go(body):
+        code = PRELUDE.format(root=os.path.dirname(HERE), fake=str(fake)) + body
+        p = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=120)
+        assert p.returncode == 0, p.stderr
+
+    return go
+
+
+def test_failure_is_reported_once(run):
+    """The runtime keeps the error of a failed allocation; a launch of the next
+    call must not find it."""
+    run("""
+net = Mlp(1)
+hip.fake_fail_above(50 << 20)
+assert fails(lambda: net.predict(np.ones((3000000, 6), np.float32)))
+net.predict(np.ones((256, 6), np.float32))
+from tests.mixed_meshes import mixed_box
+cfg = nf.Config(density_fs=1.0, pressure_fs=0.7, check_physical_validity=False)
+for mesh in (nf.Mesh.box(3), mixed_box((2, 2, 2))):
+    s = nf.EulerSolver(cfg, mesh)
+    U = s.get_solver_data().get_solution()
+    s.set_state(U)
+    hip.fake_fail_above(100 << 10)
+    assert fails(lambda: s.run(100000))  # its history of 800 KB
+    hip.fake_fail_above(ANY)
+    s.set_state(U)
+""")
