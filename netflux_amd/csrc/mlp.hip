@@ -554,6 +554,7 @@ int fail(nf_mlp *m, int code, const std::string &msg) {
 
 int ensure_ws(nf_mlp *mm, int n) {
     if (n <= mm->cap) return NF_OK;
+    mm->cap = 0;  // (until every array is there)
     for (void *q : mm->ws) (void)hipFree(q);
     mm->ws.clear();
     const int cap = (n + 255) / 256 * 256;

@@ -69,3 +69,17 @@ for mesh in (nf.Mesh.box(3), mixed_box((2, 2, 2))):
     hip.fake_fail_above(ANY)
     s.set_state(U)
 """)
+
+
+def test_network_workspace_that_could_not_grow(run):
+    run("""
+net = Mlp(1)
+x, y = np.ones((300000, 6), np.float32), np.ones((300000, 5), np.float32)
+net.loss_grad(x[:256], y[:256])
+hip.fake_fail_above(100 << 20)  # the 154 MB arrays of the larger batch
+assert fails(lambda: net.loss_grad(x, y))
+hip.fake_fail_above(ANY)
+# the arrays of the first call went to make room
+assert allocates(lambda: net.loss_grad(x[:256], y[:256])) > 128 * 256 * 4 * 3
+assert allocates(lambda: net.loss_grad(x[:256], y[:256])) == 0
+""")
