@@ -1802,18 +1802,19 @@ int nf_set_precision(nf_ctx *ctx, int32_t precision) {
         return fail(ctx, NF_E_ARG, "the HLLC flux is implemented in FP64 only");
     int rc;
     const size_t NC = ctx->Ncell;
-    if (mixed && !ctx->V32) {
-        if ((rc = dalloc(ctx, &ctx->V32, 5 * NC))) return rc;
-        if ((rc = dalloc(ctx, &ctx->FV32, 20 * NC))) return rc;
-        if ((rc = dalloc(ctx, &ctx->Gc32, 5 * ((size_t)ctx->nbf + TILE - 1) / TILE * TILE))) return rc;
-        if ((rc = dalloc(ctx, &ctx->Gf32, 5 * ((size_t)ctx->nbf + TILE - 1) / TILE * TILE))) return rc;
-    }
-    if (!mixed && !ctx->V) {
-        if ((rc = dalloc(ctx, &ctx->V, 5 * NC))) return rc;
-        if ((rc = dalloc(ctx, &ctx->FV, 20 * NC + 512))) return rc;
-        if ((rc = dalloc(ctx, &ctx->Gc, 5 * ((size_t)ctx->nbf + TILE - 1) / TILE * TILE))) return rc;
-        if ((rc = dalloc(ctx, &ctx->Gf, 5 * ((size_t)ctx->nbf + TILE - 1) / TILE * TILE))) return rc;
-        if ((rc = build_faces(ctx))) return rc;
+    const size_t NG = 5 * (((size_t)ctx->nbf + TILE - 1) / TILE * TILE);
+    // (each array by itself: a switch that failed for want of memory has some)
+    auto ensure = [&](auto **p, size_t n) { return *p ? NF_OK : dalloc(ctx, p, n); };
+    if (mixed) {
+        if ((rc = ensure(&ctx->V32, 5 * NC)) || (rc = ensure(&ctx->FV32, 20 * NC)) ||
+            (rc = ensure(&ctx->Gc32, NG)) || (rc = ensure(&ctx->Gf32, NG)))
+            return rc;
+    } else {
+        const bool first = !ctx->Gf;
+        if ((rc = ensure(&ctx->V, 5 * NC)) || (rc = ensure(&ctx->FV, 20 * NC + 512)) ||
+            (rc = ensure(&ctx->Gc, NG)) || (rc = ensure(&ctx->Gf, NG)))
+            return rc;
+        if (first && (rc = build_faces(ctx))) return rc;
     }
     HIPC(hipStreamSynchronize(ctx->stream));
     ctx->mixed = mixed;

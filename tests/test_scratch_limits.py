@@ -83,3 +83,18 @@ hip.fake_fail_above(ANY)
 assert allocates(lambda: net.loss_grad(x[:256], y[:256])) > 128 * 256 * 4 * 3
 assert allocates(lambda: net.loss_grad(x[:256], y[:256])) == 0
 """)
+
+
+@pytest.mark.parametrize("now,then,limit", [("mixed", "fp64", 4 << 20), ("fp64", "mixed", 2 << 20)])
+def test_precision_switch_without_room(run, now, then, limit):
+    # 48,000 cells: the new precision's primvars (1.9 or 1 MB) fit, its face values (7.7 or 3.8 MB) do not
+    run(f"""
+cfg = nf.Config(density_fs=1.0, pressure_fs=0.7, precision={now!r})
+s = nf.EulerSolver(cfg, nf.Mesh.box(20))
+hip.fake_fail_above({limit})
+for _ in range(2):
+    assert fails(lambda: s.set_precision({then!r}))
+hip.fake_fail_above(ANY)
+assert allocates(lambda: s.set_precision({then!r})) > {limit}
+assert allocates(lambda: (s.set_precision({now!r}), s.set_precision({then!r}))) == 0
+""")
