@@ -511,15 +511,22 @@ bool fused_ghosts(const nf_ctx *ctx) { return ctx->Ncell <= FUSE_MAX_CELLS; }
 // The block faces of an FP64 context (DevMesh), on the device: as host loops
 // they were 15 of the 150 ms that a context of 500k cells takes.  The sides'
 // records pass through FV, which no sweep has written for a later one yet.
+// The last of a context's arrays: one that has no room for them (some 50 B per
+// cell) does without, its sweeps gather per lane.
 int build_faces(nf_ctx *ctx) {
     if (order_of(ctx) == 0) return NF_OK;
-    int rc;
+    auto room = [&](uint32_t **p, size_t n) {
+        if (hipMalloc((void **)p, n * sizeof(uint32_t)) == hipSuccess) return true;
+        (void)hipGetLastError();
+        return false;
+    };
     const uint32_t nblk = ctx->Ncell / BLOCK;
     std::vector<uint32_t> off(2 * (nblk + 1));  // foff, roff
     uint32_t *foff = off.data(), *roff = foff + nblk + 1;
     FaceTables o{};
     o.side_rec = reinterpret_cast<uint32_t *>(ctx->FV);
-    if ((rc = dalloc(ctx, &o.foff, off.size()))) return rc;
+    if (!room(&o.foff, off.size())) return NF_OK;
+    ctx->owned.push_back(o.foff);
     o.roff = o.foff + nblk + 1;
     hipLaunchKernelGGL(k_block_faces<true>, dim3(nblk), dim3(BLOCK), 0, ctx->stream, devmesh(ctx), o);
     HIPC(hipGetLastError());
@@ -540,7 +547,8 @@ int build_faces(nf_ctx *ctx) {
     ctx->rec_at = (5 * (size_t)foff[nblk] + 63) / 64 * 64;
     const size_t nrp = (nr + 64) / 64 * 64, nbp = (ctx->nbf + 63) / 64 * 64, NC = ctx->Ncell;
     uint32_t *tab = nullptr;  // one allocation for all
-    if ((rc = dalloc(ctx, &tab, 6 * nrp + 6 * NC + 2 * nrp + nbp))) return rc;
+    if (!room(&tab, 6 * nrp + 6 * NC + 2 * nrp + nbp)) return NF_OK;
+    ctx->owned.push_back(tab);
     ctx->rS = reinterpret_cast<double *>(tab);
     ctx->vol = ctx->rS + 3 * nrp;
     o.cell_nb = reinterpret_cast<uint2 *>(ctx->vol + NC);
@@ -1268,7 +1276,6 @@ int create(int32_t n, const nf_mesh_desc *descs, const nf_params *prms, nf_ctx *
     HIPC(hipMemcpy(ctx->cell_ln, cell_ln.data(), cell_ln.size() * sizeof(uint2), hipMemcpyHostToDevice));
     HIPC(hipMemcpy(ctx->blk_inst, blk_inst.data(), blk_inst.size() * 4, hipMemcpyHostToDevice));
     HIPC(hipMemcpy(ctx->inst_end, inst_end.data(), inst_end.size() * 4, hipMemcpyHostToDevice));
-    if (!ctx->mixed && (rc = build_faces(ctx))) return rc;
     if (ctx->nbf) {
         HIPC(hipMemcpy(ctx->bface, bface.data(), bface.size() * 4, hipMemcpyHostToDevice));
         HIPC(hipMemcpy(ctx->bbc, bbc.data(), bbc.size(), hipMemcpyHostToDevice));
@@ -1301,6 +1308,7 @@ int create(int32_t n, const nf_mesh_desc *descs, const nf_params *prms, nf_ctx *
     }
     if ((rc = ensure_hist(ctx, 1024))) return rc;
     if ((rc = ensure_stage(ctx))) return rc;
+    if (!ctx->mixed && (rc = build_faces(ctx))) return rc;
     for (int i = 0; i < n; ++i)
         if ((rc = set_freestream(ctx, i))) return rc;
     *out = hold.release();

@@ -2,7 +2,8 @@
 // memory is host memory, copies are copies, kernels do nothing.  Loaded with
 // RTLD_GLOBAL before libnetflux.so, its functions are the ones that are called.
 // fake_fail_above(n): device allocations of more than n bytes fail from now on;
-// fake_fail_host(1): so do pinned ones.
+// fake_capacity(n): those that would take the total above n bytes;
+// fake_fail_host(1): pinned ones.
 #include <atomic>
 #include <cstddef>
 #include <cstdlib>
@@ -10,13 +11,16 @@
 
 typedef int err_t;
 static constexpr err_t OOM = 2;
-static std::atomic<size_t> fail_above{~(size_t)0}, allocated{0};
+static constexpr size_t HEAD = 256;  // the size of an allocation, in front of it
+static std::atomic<size_t> fail_above{~(size_t)0}, capacity{~(size_t)0}, allocated{0}, live{0};
 static std::atomic<int> fail_host{0}, last{0};
 
 extern "C" {
 void fake_fail_above(size_t n) { fail_above = n; }
+void fake_capacity(size_t n) { capacity = n; }
 void fake_fail_host(int on) { fail_host = on; }
 size_t fake_allocated() { return allocated; }  // bytes of all successful device allocations so far
+size_t fake_live() { return live; }            // bytes of those not freed
 
 err_t hipGetDeviceCount(int *n) { return *n = 1, 0; }
 err_t hipGetDevice(int *d) { return *d = 0, 0; }
@@ -24,12 +28,23 @@ err_t hipSetDevice(int) { return 0; }
 const char *hipGetErrorString(err_t) { return "out of memory"; }
 err_t hipGetLastError() { return last.exchange(0); }
 err_t hipMalloc(void **p, size_t n) {
-    if (n > fail_above) return last = OOM;
+    if (n > fail_above || live + n > capacity) return last = OOM;
+    char *q = static_cast<char *>(std::calloc(n + HEAD, 1));
+    if (!q) return last = OOM;
+    std::memcpy(q, &n, sizeof n);
     allocated += n;
-    *p = std::calloc(n + 1, 1);
-    return *p ? 0 : OOM;
+    live += n;
+    *p = q + HEAD;
+    return 0;
 }
-err_t hipFree(void *p) { return std::free(p), 0; }
+err_t hipFree(void *p) {
+    if (!p) return 0;
+    char *q = static_cast<char *>(p) - HEAD;
+    size_t n;
+    std::memcpy(&n, q, sizeof n);
+    live -= n;
+    return std::free(q), 0;
+}
 err_t hipHostMalloc(void **p, size_t n, unsigned) {
     if (fail_host) return last = OOM;
     *p = std::calloc(n, 1);

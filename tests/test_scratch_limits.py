@@ -16,7 +16,8 @@ import ctypes as C, sys
 sys.path.insert(0, {root!r})
 hip = C.CDLL({fake!r}, mode=C.RTLD_GLOBAL)
 hip.fake_allocated.restype = C.c_size_t
-hip.fake_fail_above.argtypes = [C.c_size_t]
+hip.fake_live.restype = C.c_size_t
+hip.fake_fail_above.argtypes = hip.fake_capacity.argtypes = [C.c_size_t]
 ANY = 2**64 - 1
 import numpy as np
 import netflux_amd as nf
@@ -97,4 +98,35 @@ for _ in range(2):
 hip.fake_fail_above(ANY)
 assert allocates(lambda: s.set_precision({then!r})) > {limit}
 assert allocates(lambda: (s.set_precision({now!r}), s.set_precision({then!r}))) == 0
+""")
+
+
+def test_context_without_room_for_the_face_tables(run):
+    """The tables of the sweeps over block faces are what a context can do
+    without: one that fits only without them is made all the same, and every
+    array made with a context comes before them."""
+    run("""
+cfg = nf.Config(density_fs=1.0, pressure_fs=0.7, check_physical_validity=True, local_time_step=True)
+mesh = nf.Mesh.box(20)
+first = nf.Config(density_fs=1.0, pressure_fs=0.7, check_physical_validity=True, local_time_step=True, spatial_order="First")
+import gc
+def made(c):
+    s = nf.EulerSolver(c, mesh)
+    n = hip.fake_live()
+    del s
+    gc.collect()
+    assert hip.fake_live() == 0
+    return n
+full, least = made(cfg), made(first)  # (first order has no use for the tables)
+assert full - least > 24 * mesh.n_cells
+hip.fake_capacity(full - 1)
+assert made(cfg) < full
+hip.fake_capacity(least)
+assert made(cfg) == least
+hip.fake_capacity(least - 1)
+try:
+    made(cfg)
+except RuntimeError:
+    sys.exit(0)
+sys.exit("a context without room for its arrays was made")
 """)
