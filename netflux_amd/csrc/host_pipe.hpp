@@ -69,7 +69,10 @@ class PinnedPool {
                 page_.reserve(page_.size() + 1);
                 rec_.reserve((page_.size() + 1) * (PAGE / RECORD));  // giving back cannot fail
                 char *p = nullptr;
-                if (hipHostMalloc(reinterpret_cast<void **>(&p), PAGE, hipHostMallocPortable) != hipSuccess) return nullptr;
+                if (hipHostMalloc(reinterpret_cast<void **>(&p), PAGE, hipHostMallocPortable) != hipSuccess) {
+                    (void)hipGetLastError();  // (the user does without)
+                    return nullptr;
+                }
                 page_.push_back(p);
                 for (size_t o = 0; o < PAGE; o += RECORD) rec_.push_back(p + o);
             }

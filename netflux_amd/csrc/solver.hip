@@ -741,11 +741,10 @@ int read_states(nf_ctx *ctx, std::vector<InstState> &h) {
     return NF_OK;
 }
 
-// (taken by the first host step)
-int ensure_host_st(nf_ctx *ctx) {
+// (taken by the first host step; without one the states are copied)
+void ensure_host_st(nf_ctx *ctx) {
     static_assert(sizeof(InstState) <= nf::PinnedPool::RECORD, "");
     if (!ctx->host_st) ctx->host_st = static_cast<InstState *>(nf::PinnedPool::get().record());
-    return ctx->host_st ? NF_OK : fail(ctx, NF_E_HIP, "no pinned host memory");
 }
 
 // after work that leaves the state in host_st
@@ -1337,7 +1336,8 @@ int step_device_dt(nf_ctx *ctx, const double *dt = nullptr) {
     int rc;
     std::vector<InstState> h;
     if ((rc = read_states(ctx, h))) return rc;
-    if ((rc = ensure_hist(ctx, h[0].nstep + 2)) || (rc = ensure_host_st(ctx))) return rc;
+    if ((rc = ensure_hist(ctx, h[0].nstep + 2))) return rc;
+    ensure_host_st(ctx);
     ctx->host_st_valid = false;
     hipLaunchKernelGGL(k_flags, dim3(1), dim3(64), 0, ctx->stream, ctx->st, 1, dt ? 1 : 0, 0, dt ? *dt : 0.0);
     HIPC(hipGetLastError());

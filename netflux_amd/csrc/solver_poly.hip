@@ -426,7 +426,7 @@ struct RunDev {
                            // run's first step is that residual (a first residual of 0 never converges)
     int *zero_old;         // U_old counts as zero (before the first step)
     int *bad;              // [3] bad cells of each stage (checked steps)
-    double *host;          // pinned: residual, dt, bad[3]
+    double *host;          // residual, dt, bad[3]: pinned, or where there was none dev_res
 };
 
 // partials in a fixed order: each thread a strided sum (or minimum), then a tree
@@ -544,6 +544,7 @@ struct PolyPath {
     double *grad = nullptr, *psi = nullptr, *R = nullptr, *dt_part = nullptr, *res_part = nullptr;
     double *dtc = nullptr;  // [N] per-cell steps (local time stepping)
     RunDev run{};           // run.flags: set for the kernels of a device-resident run only
+    double *dev_res = nullptr, res[5] = {};  // results without pinned memory, and on the host (read_results)
     int *flags = nullptr;
     int64_t run_cap = 0;
     uint32_t *boff = nullptr;
@@ -576,7 +577,7 @@ struct PolyPath {
         if (st) (void)hipStreamSynchronize(st);
         if (graph) (void)hipGraphExecDestroy(graph);
         for (void *p : owned) (void)hipFree(p);
-        if (run.host) PinnedPool::get().give_record(run.host);
+        if (run.host && run.host != dev_res) PinnedPool::get().give_record(run.host);
     }
 };
 
@@ -781,17 +782,22 @@ int stages(PolyPath *P, bool on_device, double dt, std::string &err) {
     return NF_OK;
 }
 
-// the pinned results of begin and step_end, taken by the first of them
-int ensure_host(PolyPath *P, std::string &err) {
+// where begin and step_end leave their results, taken by the first of them
+void ensure_host(PolyPath *P) {
     if (!P->run.host) P->run.host = static_cast<double *>(PinnedPool::get().record());
-    if (P->run.host) return NF_OK;
-    err = "no pinned host memory";
-    return NF_E_HIP;
+    if (!P->run.host) P->run.host = P->dev_res;
+}
+// the results, after the work enqueued so far
+int read_results(PolyPath *P, std::string &err) {
+    if (P->run.host == P->dev_res)
+        PHIP(hipMemcpyAsync(P->res, P->dev_res, sizeof P->res, hipMemcpyDeviceToHost, P->st));
+    PHIP(hipStreamSynchronize(P->st));
+    if (P->run.host != P->dev_res) std::copy(P->run.host, P->run.host + 5, P->res);
+    return NF_OK;
 }
 
 int step_end(PolyPath *P, bool on_device, std::string &err) {
-    int rc;
-    if ((rc = ensure_host(P, err))) return rc;
+    ensure_host(P);
     RunDev r = P->run;
     r.flags = on_device ? P->flags : nullptr;
     hipLaunchKernelGGL(k_poly_end, dim3(1), dim3(PB), 0, P->st, r, (const double *)P->res_part,
@@ -802,8 +808,7 @@ int step_end(PolyPath *P, bool on_device, std::string &err) {
 
 // dt of the first step where it is not in place, and (on_device) a run's start
 int begin(PolyPath *P, bool on_device, double drop, double ref, std::string &err) {
-    int rc;
-    if ((rc = ensure_host(P, err))) return rc;
+    ensure_host(P);
     RunDev r = P->run;
     r.flags = on_device ? P->flags : nullptr;
     if (!P->dt_valid) {
@@ -935,7 +940,7 @@ int poly_create(const PrimalMesh &pm, const FVGrid &g, const nf_params &p, hipSt
                             {&P->Y, 5 * (size_t)NT}, {&P->Z, 5 * (size_t)NT}, {&P->FV, 35 * plane},
                             {&P->grad, 15 * (size_t)N}, {&P->psi, 5 * (size_t)N}, {&P->R, 5 * (size_t)N},
                             {&P->dt_part, nblk}, {&P->res_part, nblk}, {&P->dtc, N}, {&P->flags, 4},
-                            {&P->run.dtdev, 1}, {&P->run.runp, 2}, {&P->run.zero_old, 1}, {&P->run.bad, 3}},
+                            {&P->run.dtdev, 1}, {&P->dev_res, 5}, {&P->run.runp, 2}, {&P->run.zero_old, 1}, {&P->run.bad, 3}},
                         err)))
         return rc;
     PHIP(hipMemset(P->run.bad, 0, 3 * sizeof(int)));
@@ -995,9 +1000,8 @@ int poly_set_state(PolyPath *P, const double *U, const double *U_old, std::strin
 int poly_calc_timestep(PolyPath *P, double *dt_out, std::string &err) {
     int rc;
     if (!P->dt_valid) {
-        if ((rc = begin(P, false, 0.0, 0.0, err))) return rc;
-        PHIP(hipStreamSynchronize(P->st));
-        P->dt = P->run.host[1];
+        if ((rc = begin(P, false, 0.0, 0.0, err)) || (rc = read_results(P, err))) return rc;
+        P->dt = P->res[1];
         P->dt_valid = true;
     }
     const double dt = P->dt;
@@ -1015,10 +1019,9 @@ int poly_calc_timestep(PolyPath *P, double *dt_out, std::string &err) {
 int poly_step(PolyPath *P, double dt, std::string &err) {
     int rc;
     P->aux_valid = false;
-    if ((rc = stages(P, false, dt, err)) || (rc = step_end(P, false, err))) return rc;
-    PHIP(hipStreamSynchronize(P->st));
+    if ((rc = stages(P, false, dt, err)) || (rc = step_end(P, false, err)) || (rc = read_results(P, err))) return rc;
     for (int s = 0; s < 3; ++s) {
-        const int n = (int)P->run.host[2 + s];
+        const int n = (int)P->res[2 + s];
         if (n == 0) continue;
         // the state is the failed stage's input, U_old what it was
         P->split = P->split || s > 0;
@@ -1027,9 +1030,9 @@ int poly_step(PolyPath *P, double dt, std::string &err) {
         err = bad_cells(n);
         return NF_E_NONPHYSICAL;
     }
-    P->hist.push_back(P->run.host[0]);  // the flux balance of U^n (first stage), as in the batched path
+    P->hist.push_back(P->res[0]);  // the flux balance of U^n (first stage), as in the batched path
     P->time += dt;
-    P->dt = P->run.host[1];
+    P->dt = P->res[1];
     P->dt_valid = true;
     P->split = P->old_zero = false;
     return NF_OK;

@@ -130,3 +130,20 @@ except RuntimeError:
     sys.exit(0)
 sys.exit("a context without room for its arrays was made")
 """)
+
+
+def test_host_steps_without_pinned_memory(run):
+    """The pinned record of a host-driven step's results, and the pinned pieces
+    of large copies, are what a context can do without."""
+    run("""
+from tests.mixed_meshes import mixed_box
+hip.fake_fail_host(1)
+cfg = nf.Config(density_fs=1.0, pressure_fs=0.7)
+cfg.delta_time = 1e-3
+for mesh in (nf.Mesh.box(3), nf.Mesh.box(24), mixed_box((3, 2, 2))):
+    s = nf.EulerSolver(cfg, mesh)
+    U = s.get_solver_data().get_solution()
+    for _ in range(2):
+        s.set_state(U)
+        s.step(cfg)
+""")
