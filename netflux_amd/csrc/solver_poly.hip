@@ -1186,9 +1186,10 @@ int poly_run(PolyPath *P, const nf_run_opts *o, nf_run_stats *stats, std::string
         while (queued < o->n_steps && !flags[0]) {
             const int chunk = std::min(K, o->n_steps - queued);
             // a graph starts from prim(U) in X, whatever was the case when it
-            // was captured, and from the state in Ua
+            // was captured, and from the state in Ua (a split state exists only
+            // with the flux-balance check, whose runs went to the host loop)
             if ((rc = ensure_x(P, err))) return rc;
-            if (o->use_graph && chunk == K && K > 1 && !P->split) {
+            if (o->use_graph && chunk == K && K > 1) {
                 if (!P->graph || P->graph_K != K) {
                     if (P->graph) (void)hipGraphExecDestroy(P->graph);
                     P->graph = nullptr;
@@ -1209,14 +1210,8 @@ int poly_run(PolyPath *P, const nf_run_opts *o, nf_run_stats *stats, std::string
                 PHIP(hipGraphLaunch(P->graph, P->st));
                 P->x_prim = P->rk3() || P->second();
             } else {
-                for (int q = 0; q < chunk; ++q) {
+                for (int q = 0; q < chunk; ++q)
                     if ((rc = enqueue_run_step(P, err))) return rc;
-                    if (!P->split) continue;
-                    // the state moves to Ua with the step, if that is taken
-                    PHIP(hipMemcpyAsync(flags, P->flags, sizeof flags, hipMemcpyDeviceToHost, P->st));
-                    PHIP(hipStreamSynchronize(P->st));
-                    P->split = flags[3] == 0;
-                }
             }
             queued += chunk;
             PHIP(hipMemcpyAsync(flags, P->flags, sizeof flags, hipMemcpyDeviceToHost, P->st));
