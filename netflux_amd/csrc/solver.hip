@@ -99,9 +99,10 @@ __device__ __forceinline__ void finish_dt(const RedArgs &a, uint32_t i, double v
 }
 
 // One block per instance: everything, where no instance has more than one
-// chunk (RCHUNK blocks, 524,288 cells), from the partials (ONE); else the
-// second level, from the chunks' results of k_reduce.  The step's residual
-// and dt go through one launch (two with chunks), not two (four).
+// chunk (RCHUNK sweep blocks: 524,288 cells, in 128-cell blocks 262,144), from
+// the partials (ONE); else the second level, from the chunks' results of
+// k_reduce.  The step's residual and dt go through one launch (two with
+// chunks), not two (four).
 template <bool ONE>
 __global__ __launch_bounds__(BLOCK) void k_finish(RedArgs a) {
     __shared__ double sh[2][BLOCK / 64];
