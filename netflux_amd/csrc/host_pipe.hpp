@@ -145,7 +145,12 @@ class HostPipe {
     }
 
   private:
-    static constexpr size_t CHUNK = PinnedPool::PIECE, MIN = 2u << 20;  // below MIN the threads cost more than they save
+    // Below this many bytes the threads cost more than they save.  Upwards the
+    // runtime's own copy is at 39 GB/s and the threads' start shows for longer:
+    // nf_set_state of 5.9 / 13.2 / 26.5 / 39.9 MB 215 / 413 / 775 / 1,476 us plain,
+    // 271 / 506 / 795 / 1,168 through the pieces; nf_get_state of 1.9 / 3.3 / 13.2
+    // MB 145 / 253 / 918 plain, 143 / 222 / 658 through them.
+    static constexpr size_t CHUNK = PinnedPool::PIECE, MIN_DOWN = 2u << 20, MIN_UP = 32u << 20;
 
     static int slots_for(size_t bytes) {
         const int hw = (int)std::thread::hardware_concurrency();
@@ -153,7 +158,7 @@ class HostPipe {
     }
     template <bool DOWN>
     hipError_t copy(char *dst, const char *src, size_t bytes, hipStream_t s, bool idle = false) {
-        if (bytes >= MIN) {
+        if (bytes >= (DOWN ? MIN_DOWN : MIN_UP)) {
             int dev = 0;
             hipError_t e = hipGetDevice(&dev);
             if (e) return e;
