@@ -531,8 +531,8 @@ int build_faces(nf_ctx *ctx) {
     o.roff = o.foff + nblk + 1;
     hipLaunchKernelGGL(k_block_faces<true>, dim3(nblk), dim3(BLOCK), 0, ctx->stream, devmesh(ctx), o);
     HIPC(hipGetLastError());
+    HIPC(hipMemcpyAsync(off.data(), o.foff, off.size() * 4, hipMemcpyDeviceToHost, ctx->stream));
     HIPC(hipStreamSynchronize(ctx->stream));
-    HIPC(hipMemcpy(off.data(), o.foff, off.size() * 4, hipMemcpyDeviceToHost));
     foff[0] = roff[0] = 0;
     uint32_t nrmax = 0;
     for (uint32_t b = 0; b < nblk; ++b) {
@@ -557,7 +557,7 @@ int build_faces(nf_ctx *ctx) {
     o.hal = reinterpret_cast<uint32_t *>(o.cell_fx + NC);
     o.rec = o.hal + nrp;
     o.brec = o.rec + nrp;
-    HIPC(hipMemcpy(o.foff, off.data(), off.size() * 4, hipMemcpyHostToDevice));
+    HIPC(hipMemcpyAsync(o.foff, off.data(), off.size() * 4, hipMemcpyHostToDevice, ctx->stream));
     hipLaunchKernelGGL(k_block_faces<false>, dim3(nblk), dim3(BLOCK), 0, ctx->stream, devmesh(ctx), o);
     hipLaunchKernelGGL(k_link_records, dim3(nblk), dim3(BLOCK), 0, ctx->stream, devmesh(ctx), o);
     ctx->foff = o.foff;
@@ -1029,15 +1029,16 @@ int build_red_table(nf_ctx *ctx, uint32_t B, RedTable &r) {
         nc.push_back((uint32_t)first.size() - c0.back());
     }
     r.nchunk = (int)first.size();
+    // one array for the four (as eight, and their copies, the two tables were a
+    // tenth of a small context's creation)
+    std::vector<uint32_t> all(first);
+    for (const auto *v : {&n, &c0, &nc}) all.insert(all.end(), v->begin(), v->end());
     int rc;
-    if ((rc = dalloc(ctx, &r.first, first.size()))) return rc;
-    if ((rc = dalloc(ctx, &r.n, n.size()))) return rc;
-    if ((rc = dalloc(ctx, &r.inst_c0, c0.size()))) return rc;
-    if ((rc = dalloc(ctx, &r.inst_nc, nc.size()))) return rc;
-    HIPC(hipMemcpy(r.first, first.data(), first.size() * 4, hipMemcpyHostToDevice));
-    HIPC(hipMemcpy(r.n, n.data(), n.size() * 4, hipMemcpyHostToDevice));
-    HIPC(hipMemcpy(r.inst_c0, c0.data(), c0.size() * 4, hipMemcpyHostToDevice));
-    HIPC(hipMemcpy(r.inst_nc, nc.data(), nc.size() * 4, hipMemcpyHostToDevice));
+    if ((rc = dalloc(ctx, &r.first, all.size()))) return rc;
+    r.n = r.first + first.size();
+    r.inst_c0 = r.n + n.size();
+    r.inst_nc = r.inst_c0 + c0.size();
+    HIPC(hipMemcpy(r.first, all.data(), all.size() * 4, hipMemcpyHostToDevice));
     return NF_OK;
 }
 

@@ -13,13 +13,15 @@ typedef int err_t;
 static constexpr err_t OOM = 2;
 static constexpr size_t HEAD = 256;  // the size of an allocation, in front of it
 static std::atomic<size_t> fail_above{~(size_t)0}, capacity{~(size_t)0}, allocated{0}, live{0};
-static std::atomic<int> fail_host{0}, last{0};
+static std::atomic<int> fail_host{0}, last{0}, allocations{0}, waits{0};
 
 extern "C" {
 void fake_fail_above(size_t n) { fail_above = n; }
 void fake_capacity(size_t n) { capacity = n; }
 void fake_fail_host(int on) { fail_host = on; }
 size_t fake_allocated() { return allocated; }  // bytes of all successful device allocations so far
+int fake_allocations() { return allocations; }
+int fake_waits() { return waits; }             // blocking copies and waits for a stream
 size_t fake_live() { return live; }            // bytes of those not freed
 
 err_t hipGetDeviceCount(int *n) { return *n = 1, 0; }
@@ -32,6 +34,7 @@ err_t hipMalloc(void **p, size_t n) {
     char *q = static_cast<char *>(std::calloc(n + HEAD, 1));
     if (!q) return last = OOM;
     std::memcpy(q, &n, sizeof n);
+    ++allocations;
     allocated += n;
     live += n;
     *p = q + HEAD;
@@ -51,7 +54,7 @@ err_t hipHostMalloc(void **p, size_t n, unsigned) {
     return *p ? 0 : OOM;
 }
 err_t hipHostFree(void *p) { return std::free(p), 0; }
-err_t hipMemcpy(void *d, const void *s, size_t n, int) { return std::memmove(d, s, n), 0; }
+err_t hipMemcpy(void *d, const void *s, size_t n, int) { return ++waits, std::memmove(d, s, n), 0; }
 err_t hipMemcpyAsync(void *d, const void *s, size_t n, int, void *) { return std::memmove(d, s, n), 0; }
 err_t hipMemcpy2DAsync(void *d, size_t dp, const void *s, size_t sp, size_t w, size_t h, int, void *) {
     for (size_t q = 0; q < h; ++q) std::memmove((char *)d + q * dp, (const char *)s + q * sp, w);
@@ -62,7 +65,7 @@ err_t hipMemsetAsync(void *d, int v, size_t n, void *) { return std::memset(d, v
 static char handle;
 err_t hipStreamCreateWithFlags(void **s, unsigned) { return *s = &handle, 0; }
 err_t hipStreamDestroy(void *) { return 0; }
-err_t hipStreamSynchronize(void *) { return 0; }
+err_t hipStreamSynchronize(void *) { return ++waits, 0; }
 err_t hipEventCreate(void **e) { return *e = &handle, 0; }
 err_t hipEventCreateWithFlags(void **e, unsigned) { return *e = &handle, 0; }
 err_t hipEventDestroy(void *) { return 0; }
