@@ -10,11 +10,11 @@
 // 11.3 ms (14 of them the comparison of U with U_old when both are the same
 // array), nf_get_state into fresh pages 49.0 -> 12.3 ms.
 //
-// The pinned pieces (8 of 4 MB for each device) belong to a pool, since making
-// them takes longer (1.3 ms) than most copies: a copy borrows those it can
-// get, under a lock, and returns them when its last piece has left; a copy that
-// gets none is a plain one.  The pool is given back with its last user.  It
-// also has the small records that kernels leave their results in.
+// The pinned pieces (up to 8 of 4 MB for each device) belong to a pool: a copy
+// borrows those it can get, under a lock, and returns them when its last piece
+// has left; a copy that gets none is a plain one.  The pool is given back with
+// its last user.  It also has the small records that kernels leave their
+// results in.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -87,8 +87,8 @@ class PinnedPool {
         std::lock_guard<std::mutex> lk(mu_);
         rec_.push_back(static_cast<char *>(r));
     }
-    // up to `want` slots of device dev, which is current
-    std::vector<Slot> borrow(int want, int dev) {
+    // up to `want` slots of device dev, which is current; make: new ones too
+    std::vector<Slot> borrow(int want, int dev, bool make) {
         std::vector<Slot> got;
         std::lock_guard<std::mutex> lk(mu_);
         got.reserve(want);
@@ -99,7 +99,7 @@ class PinnedPool {
                 got.push_back(free_[q]);
                 free_.erase(free_.begin() + q);
             }
-        while ((int)got.size() < want && made < SLOTS) {
+        while (make && (int)got.size() < want && made < SLOTS) {
             Slot s;
             s.dev = dev;
             if (hipHostMalloc(reinterpret_cast<void **>(&s.mem), PIECE, hipHostMallocDefault) != hipSuccess) break;
@@ -151,6 +151,12 @@ class HostPipe {
     // 271 / 506 / 795 / 1,168 through the pieces; nf_get_state of 1.9 / 3.3 / 13.2
     // MB 145 / 253 / 918 plain, 143 / 222 / 658 through them.
     static constexpr size_t CHUNK = PinnedPool::PIECE, MIN_DOWN = 2u << 20, MIN_UP = 32u << 20;
+    // Pieces that are not there yet are made by a copy of at least this size, or
+    // by a user's second: where memory comes in small pages making them takes
+    // 1.3 ms, more than one smaller copy gains (a lone context's only nf_get_state
+    // of 15.3 MB took 2.0 ms with, 1.3 without).
+    static constexpr size_t MIN_MAKE = 32u << 20;
+    int large_ = 0;  // copies of this user that could have made pieces
 
     static int slots_for(size_t bytes) {
         const int hw = (int)std::thread::hardware_concurrency();
@@ -163,8 +169,9 @@ class HostPipe {
             hipError_t e = hipGetDevice(&dev);
             if (e) return e;
             std::vector<PinnedPool::Slot> slot;
+            const bool make = bytes >= MIN_MAKE || large_++ > 0;
             try {
-                slot = PinnedPool::get().borrow(slots_for(bytes), dev);
+                slot = PinnedPool::get().borrow(slots_for(bytes), dev, make);
             } catch (...) {  // out of memory: a plain copy
             }
             if (!slot.empty()) {
