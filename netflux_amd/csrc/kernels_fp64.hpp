@@ -705,7 +705,9 @@ __global__ __launch_bounds__(B) NF_SWEEP_ATTR void k_sweepA(DevMesh m, SweepAArg
 }
 
 // Second-order sweeps over the faces of blocks of 256 cells, as long as every
-// block's LDS fits (any order with locality).  Of a block's 1,024 cell sides
+// block's LDS fits: with the Morton order (at most some 330 records per block)
+// and the input order of a generated box (360), not with reverse Cuthill-McKee,
+// whose fronts give a block up to 1,024 records.  Of a block's 1,024 cell sides
 // some 830 belong to 415 faces between its own cells; the other 200 are its
 // records.  Sweep A gathers and converts the records' outside states once,
 // one per lane, and keeps them in LDS beside the block's own; reconstructs

@@ -6,9 +6,9 @@
 // (kernels_fp64.hpp), with FP32 V [tile][5][64], FV [tile][4][5][64] and
 // ghost states.  Face geometry is formed in FP64 from the nodes and rounded
 // once: S from the face's own node order, so the two cells of a face hold
-// bit-identical FP32 normals, and each face flux is evaluated by both cells
-// with identical FP32 arithmetic -- the FP64 flux balance conserves exactly.
-// This header is compiled with floating-point contraction enabled.
+// bit-identical FP32 normals.  Each face flux is evaluated by both cells, in
+// FP32 with contraction enabled (rusanov_side_f: the two can differ in their
+// last bits).
 #pragma once
 #include "kernels_fp64.hpp"
 
@@ -97,14 +97,13 @@ __device__ __forceinline__ void prim_to_cons_f(const float *V, float *U) {
 }
 
 // Rusanov flux seen from one cell (see rusanov_side): F for UL = own if the
-// cell is the owner (mneg = 0), UL = neighbour otherwise
+// cell is the owner (mneg = 0), UL = neighbour otherwise.  The two cells of a
+// face evaluate this with UO and UN swapped, and this header is compiled with
+// -ffp-contract=fast (which an fp contract pragma does not limit): a fused FO +
+// FN rounds the owner's product on one side and the neighbour's on the other,
+// so the two fluxes can differ in their last FP32 bits and interior faces
+// conserve to FP32 rounding only.
 __device__ __forceinline__ void rusanov_side_f(const float *UO, const float *UN, V3f S, uint32_t mneg, float *F) {
-    // No contraction here: the two cells of a face evaluate this with UO and
-    // UN swapped, and a fused FO + FN would round the owner's product on one
-    // side and the neighbour's on the other.  Unfused, every operation is
-    // either symmetric in (UO, UN) or exactly negated, so both cells get the
-    // same flux bit for bit and interior faces conserve exactly.
-#pragma clang fp contract(off)
     const float z = S.x * S.x + S.y * S.y + S.z * S.z;
     const float area = fsqrt(z);
     const float ia = frcp(area);

@@ -465,8 +465,9 @@ int order_of(const nf_ctx *ctx) {
 }
 
 // The sweeps over block faces (k_sweepA_face): second order, 256-cell blocks,
-// every block's LDS fits.  Cells in an order without locality have up to 1,024
-// outside neighbours per block; their gather is the same work either way.
+// every block's LDS fits.  Cells in an order without locality, and in reverse
+// Cuthill-McKee order, have up to 1,024 outside neighbours per block; their
+// gather is the same work either way.
 bool use_faces(const nf_ctx *ctx) { return order_of(ctx) != 0 && ctx->block == BLOCK && ctx->cell_nb; }
 
 // ghosts of the reconstructed face states
