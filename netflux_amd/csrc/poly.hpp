@@ -16,10 +16,11 @@
 namespace nf {
 
 struct PolyPath;
+class HostPipe;
 
-// NF_OK or an NF_E_* status with the message in err
-int poly_create(const PrimalMesh &pm, const FVGrid &g, const nf_params &p, hipStream_t st, PolyPath **out,
-                std::string &err);
+// NF_OK or an NF_E_* status with the message in err; st and pipe are the context's
+int poly_create(const PrimalMesh &pm, const FVGrid &g, const nf_params &p, hipStream_t st, HostPipe &pipe,
+                PolyPath **out, std::string &err);
 void poly_destroy(PolyPath *P);
 nf_fv_sizes poly_sizes(const PolyPath *P);
 int poly_set_freestream(PolyPath *P, std::string &err);

@@ -1090,7 +1090,7 @@ int create(int32_t n, const nf_mesh_desc *descs, const nf_params *prms, nf_ctx *
         ctx->n_inst = 0;
         HIPC(hipGetDevice(&ctx->device));
         HIPC(hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking));
-        const int rc = nf::poly_create(pm, g, p0, ctx->stream, &ctx->poly, ctx->err);
+        const int rc = nf::poly_create(pm, g, p0, ctx->stream, ctx->pipe, &ctx->poly, ctx->err);
         if (rc) {
             (void)hipStreamDestroy(ctx->stream);
             return rc;

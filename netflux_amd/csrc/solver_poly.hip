@@ -563,7 +563,7 @@ struct PolyPath {
     std::map<std::string, std::pair<double, int>> ktime;
     std::vector<uint32_t> perm;  // device cell -> reference cell
     uint32_t *perm_dev = nullptr;  // the same on the device (made on first state transfer)
-    HostPipe pipe;                 // large arrays across the boundary
+    HostPipe *pipe = nullptr;      // the context's: large arrays across the boundary
     double *stage = nullptr;       // [15][N] AoS staging of state and field transfers
     std::vector<double> hist;    // residual norm of each step (flux balance of U^n)
     double time = 0.0;
@@ -636,7 +636,7 @@ int put_soa(PolyPath *P, double *dst, const double *aos, int cols, std::string &
     const uint32_t N = P->m.N;
     int rc;
     if ((rc = ensure_stage(P, err))) return rc;
-    PHIP(P->pipe.up(P->stage, aos, (size_t)cols * N * 8, P->st));
+    PHIP(P->pipe->up(P->stage, aos, (size_t)cols * N * 8, P->st));
     hipLaunchKernelGGL(k_poly_aos_in, grid(N), dim3(PB), 0, P->st, (const double *)P->stage,
                        (const uint32_t *)P->perm_dev, dst, N, cols);
     PHIP(hipGetLastError());
@@ -650,7 +650,7 @@ int get_soa(PolyPath *P, const double *src, int cols, double *aos, std::string &
     hipLaunchKernelGGL(k_poly_aos_out, grid(N), dim3(PB), 0, P->st, src, (const uint32_t *)P->perm_dev, P->stage,
                        N, cols);
     PHIP(hipGetLastError());
-    PHIP(P->pipe.down(aos, P->stage, (size_t)cols * N * 8, P->st));
+    PHIP(P->pipe->down(aos, P->stage, (size_t)cols * N * 8, P->st));
     return NF_OK;
 }
 
@@ -836,8 +836,8 @@ std::string bad_cells(int n) {
 
 }  // namespace
 
-int poly_create(const PrimalMesh &pm, const FVGrid &g, const nf_params &p, hipStream_t st, PolyPath **out,
-                std::string &err) {
+int poly_create(const PrimalMesh &pm, const FVGrid &g, const nf_params &p, hipStream_t st, HostPipe &pipe,
+                PolyPath **out, std::string &err) {
     (void)pm;
     *out = nullptr;
     if (p.precision != NF_PREC_FP64) {
@@ -847,6 +847,7 @@ int poly_create(const PrimalMesh &pm, const FVGrid &g, const nf_params &p, hipSt
     std::unique_ptr<PolyPath> hold(new PolyPath);
     PolyPath *P = hold.get();
     P->st = st;
+    P->pipe = &pipe;
     P->prm = p;
     const uint32_t N = g.N, NT = g.NT, Fint = g.Fint, F = g.F;
     P->sizes = {N, NT, Fint, F, (uint32_t)g.pfirst.size()};
