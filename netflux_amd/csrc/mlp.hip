@@ -710,7 +710,10 @@ int nf_mlp_create(uint64_t seed, nf_mlp **out) {
     *out = nullptr;
     int ndev = 0;
     if (hipGetDeviceCount(&ndev) != hipSuccess || ndev == 0) return NF_E_NOGPU;
-    std::unique_ptr<nf_mlp> hold(new nf_mlp);
+    struct Destroy {  // (where the creation fails)
+        void operator()(nf_mlp *m) const { (void)nf_mlp_destroy(m); }
+    };
+    std::unique_ptr<nf_mlp, Destroy> hold(new nf_mlp);
     nf_mlp *mm = hold.get();
     HIPM(hipGetDevice(&mm->device));
     HIPM(hipStreamCreateWithFlags(&mm->stream, hipStreamNonBlocking));

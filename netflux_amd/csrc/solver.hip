@@ -1043,6 +1043,11 @@ int build_red_table(nf_ctx *ctx, uint32_t B, RedTable &r) {
     return NF_OK;
 }
 
+// a context whose creation fails gives back what it has
+struct Destroy {
+    void operator()(nf_ctx *c) const { (void)nf_destroy(c); }
+};
+
 int create(int32_t n, const nf_mesh_desc *descs, const nf_params *prms, nf_ctx **out) {
     if (!descs || !prms || !out || n < 1 || n > 65535) return NF_E_ARG;
     *out = nullptr;
@@ -1084,21 +1089,18 @@ int create(int32_t n, const nf_mesh_desc *descs, const nf_params *prms, nf_ctx *
         } catch (const nf::MeshError &) {
             return NF_E_MESH;
         }
-        std::unique_ptr<nf_ctx> hold(new nf_ctx);
+        std::unique_ptr<nf_ctx, Destroy> hold(new nf_ctx);
         nf_ctx *ctx = hold.get();
         ctx->prm = p0;
         ctx->n_inst = 0;
         HIPC(hipGetDevice(&ctx->device));
         HIPC(hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking));
         const int rc = nf::poly_create(pm, g, p0, ctx->stream, ctx->pipe, &ctx->poly, ctx->err);
-        if (rc) {
-            (void)hipStreamDestroy(ctx->stream);
-            return rc;
-        }
+        if (rc) return rc;
         *out = hold.release();
         return NF_OK;
     }
-    std::unique_ptr<nf_ctx> hold(new nf_ctx);
+    std::unique_ptr<nf_ctx, Destroy> hold(new nf_ctx);
     nf_ctx *ctx = hold.get();
     ctx->prm = p0;
     ctx->n_inst = n;

@@ -158,3 +158,35 @@ s = nf.EulerSolver(nf.Config(density_fs=1.0, pressure_fs=0.7), nf.Mesh.box(6))
 assert hip.fake_allocations() <= 41, hip.fake_allocations()
 assert hip.fake_waits() <= 31, hip.fake_waits()
 """)
+
+
+def test_failed_creation_gives_everything_back(run):
+    """A context or network that does not fit leaves no device memory behind,
+    so that a smaller one fits where it would have without the attempt."""
+    run("""
+import gc
+from tests.mixed_meshes import mixed_box
+cfg = nf.Config(density_fs=1.0, pressure_fs=0.7)
+def creation_fails(make):
+    try:
+        make()
+    except RuntimeError:
+        return True
+for large, small in ((nf.Mesh.box(20), nf.Mesh.box(5)), (mixed_box((12, 12, 12)), mixed_box((3, 3, 3)))):
+    s = nf.EulerSolver(cfg, large)
+    need = hip.fake_live()
+    del s
+    gc.collect()
+    for part in (0.2, 0.5, 0.9):  # fails early, halfway and late
+        hip.fake_capacity(int(part * need))
+        assert creation_fails(lambda: nf.EulerSolver(cfg, large))
+        gc.collect()
+        assert hip.fake_live() == 0, (part, hip.fake_live())
+    s = nf.EulerSolver(cfg, small)
+    del s
+    gc.collect()
+    hip.fake_capacity(ANY)
+hip.fake_capacity(100000)
+assert creation_fails(lambda: Mlp(1))
+assert hip.fake_live() == 0
+""")
